@@ -303,6 +303,15 @@ def test_between_one_and_two_workgroups_per_cu(b, h, m, n, d, causal):
     run_all(q, k, causal, what=f"finer tiles b{b} h{h} m{m} n{n} d{d}", reductions=("sum", "max"))
 
 
+@pytest.mark.parametrize("b,h,m,n,d", [(1, 33, 1100, 1100, 64), (2, 16, 2048, 2048, 32), (3, 11, 1900, 2100, 136),
+                                       (1, 40, 1537, 1500, 128), (1, 7, 9000, 9000, 16)])
+def test_causal_launches_that_are_on_the_chip_at_once(b, h, m, n, d):
+    """One to two workgroups per CU with the mask: the second half of the tiles is dealt in reverse.  Every tile
+    of every head is still taken once (heads that do and do not divide the CU count)."""
+    q, k = _inputs.randn_pair(b, h, m, n, d, seed=m + d)
+    run_all(q, k, True, what=f"{b}x{h} {m}x{n}x{d}", reductions=["sum", "max"])
+
+
 @pytest.mark.parametrize("m", [100, 128, 300, 384, 600])
 def test_row_sweep_block_choice(m):
     """Query counts for which the row sweep keeps one 32-row block per wave (M <= 128 and ragged M
