@@ -1769,16 +1769,22 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(const float* __restrict__
 
 // ---------------------------------------------------------------------------------------------
 // Keep-mask of the k largest scores of every row (what a pruning caller does with the reduced
-// columns).  One workgroup of 1024 threads per row.  Floats are mapped to integers of the same order and
-// the key T of the k-th largest element is found from the top bits down; keys equal to T are kept from
-// the lowest column up until k are kept.
+// columns).  Floats are mapped to integers of the same order and the key T of the k-th largest element is
+// found from the top down; keys equal to T are kept from the lowest column up until k are kept.
 //
-// Rows of up to 32768 columns (topk_mask_kernel): thread t owns keys [t*VPT, t*VPT + VPT) in registers
-// (VPT = 8 or 32) and T is built bit by bit: T | bit is accepted when at least k keys are >= it.  A pass
-// is one compare and one add per key, one cross-lane sum, one LDS add per wave and one barrier.
-// Longer rows (topk_mask_long_kernel) are re-read from memory in every pass, so T is found eight bits at
-// a time from a 256-bin histogram in LDS; a wave whose keys all fall into one bin (the usual case for
-// the top digits) adds its count with one atomic.
+// Rows that fit the registers of one workgroup (topk_mask_kernel): the row is read once, 16 bytes per lane and
+// load, and its keys stay in registers.  T is found by narrowing: the keys between the smallest and the
+// largest one are counted in 2 * T equal bins in LDS, the bin that holds the k-th largest one becomes the
+// range of the next count, and as soon as a bin holds few enough keys they are gathered and ranked against
+// each other.  A count takes 11 bits of the range (9 in the smaller workgroup), so at most three (four) are
+// needed, and one or two are for scores that are spread at all.  The search bit by bit that stood
+// here before took 34 passes of one barrier each and read the rows with every lane on a line of its own; this
+// one is bound by the vector instructions over the keys and the latency of eight or so barriers.  Kernel time, 32 rows:
+// 1024 columns fp32 11.9 -> 4.2 us, 8192 fp32 14.7 -> 5.8, fp16 18.6 -> 6.1, 32768 fp32 31.2 -> 14.3, fp16 44.3 -> 14.5;
+// with nine columns in ten equal 15.5 -> 7.7 (8192 fp32) and 31.8 -> 20.9 (32768 fp32).
+// Longer rows without scratch (topk_mask_long_kernel) are re-read from memory in every pass, so T is found
+// eight bits at a time from a 256-bin histogram in LDS; a wave whose keys all fall into one bin (the usual
+// case for the top digits) adds its count with one atomic.
 __device__ __forceinline__ uint32_t order_key(float x) {
   uint32_t b = __builtin_bit_cast(uint32_t, x);
   if (b == 0x80000000u) b = 0u;  // -0 and +0 are one value
@@ -1819,16 +1825,31 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
+// Largest v over the 64 lanes, as a wave-uniform value.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// Inclusive prefix sums over the 64 lanes.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);   // row_shr 1, 2, 4, 8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
 
 // Exclusive rank of this thread's first tie among the ties of the row, by column, given that thread t
 // owns a contiguous run of columns and has `mine` ties.
 __device__ __forceinline__ uint32_t ties_before(uint32_t mine, uint32_t* wave_eq, int lane, int wave) {
-  uint32_t incl = mine;   // inclusive scan over the wave
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t o = __shfl_up(incl, d);
-    if (lane >= d) incl += o;
-  }
+  const uint32_t incl = wave_scan(mine);
   if (lane == 63) wave_eq[wave] = incl;
   __syncthreads();
   uint32_t before = incl - mine;
@@ -1836,101 +1857,211 @@ __device__ __forceinline__ uint32_t ties_before(uint32_t mine, uint32_t* wave_eq
   return before;
 }
 
-template <int VPT, typename ET>
-__global__ __launch_bounds__(kTopkThreads) void topk_mask_kernel(const ET* __restrict__ scores,
-                                                                 uint8_t* __restrict__ mask,
-                                                                 float* __restrict__ threshold, int N, int k) {
-  constexpr int kW = kTopkThreads / 64;
-  __shared__ uint32_t cnt[34];       // one counter per pass: nothing to reset between passes
-  __shared__ uint32_t wave_eq[kW];
+// A row of at most T * VPT columns in the registers of one workgroup: thread t holds W consecutive columns
+// from (j * T + t) * W on, for j < VPT / W, so loads (16 bytes per lane) and stores (W bytes) are dense.
+template <int T, int VPT, typename ET>
+__global__ __launch_bounds__(T) void topk_mask_kernel(const ET* __restrict__ scores, uint8_t* __restrict__ mask,
+                                                      float* __restrict__ threshold, int N, int k) {
+  constexpr int kW = T / 64;
+  constexpr int W = 16 / (int)sizeof(ET);
+  constexpr int J = VPT / W;
+  constexpr int kBins = 2 * T, kBinBits = __builtin_ctz(kBins);
+  constexpr int kGather = T < 512 ? T : 512;   // keys that are ranked against each other, one per thread
+  static_assert(VPT % W == 0, "whole vectors");
+  __shared__ __attribute__((aligned(16))) uint32_t hist[kBins];
+  __shared__ __attribute__((aligned(16))) uint32_t cand[kGather];
+  __shared__ uint32_t wave_a[kW], wave_b[kW];
+  __shared__ uint32_t block_ties[J * kW];
+  __shared__ uint32_t sh_bin, sh_above, sh_count, sh_key, sh_need, sh_ties, sh_gathered;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const ET* s = scores + (int64_t)blockIdx.x * N;
   uint8_t* m = mask + (int64_t)blockIdx.x * N;
   const uint32_t kk = (uint32_t)min(max(k, 0), N);
-  const int base = tid * VPT;
 
+  // Keys; 0 stands for a column past N (no key is 0: -inf, the smallest value, has a positive one).
   uint32_t u[VPT];
-  // four elements per load when every row starts on such a boundary
-  if (rows_aligned_to_4(scores, N)) {
 #pragma unroll
-    for (int i = 0; i < VPT; i += 4) {
-      if (base + i < N) {
-        order_keys4(s + base + i, u + i);
+  for (int j = 0; j < J; ++j) {
+    const int col = (j * T + tid) * W;
+    ET v[W];
+    if (col + W <= N) {
+      __builtin_memcpy(v, s + col, 16);   // one load whatever the row's alignment
+#pragma unroll
+      for (int e = 0; e < W; ++e) u[j * W + e] = order_key(widen<ET>(v[e]));
+    } else {
+#pragma unroll
+      for (int e = 0; e < W; ++e) u[j * W + e] = (col + e < N) ? order_key(widen<ET>(s[col + e])) : 0u;
+    }
+  }
+
+  for (int i = tid; i < kBins; i += T) hist[i] = 0u;
+  if (tid == 0) sh_gathered = 0u;
+  uint32_t lo = 1u, range = 0xfffffffeu; // the k-th largest key is in [lo, lo + range]
+  uint32_t need = kk;                    // and is the need-th largest of the `ties` keys in there
+  uint32_t key = 0xffffffffu, ties = 0u; // k <= 0: nothing is kept
+  while (kk > 0) {
+    // the smallest and the largest key of the range (the smallest through its complement, where 0 is neutral)
+    uint32_t hi = 0u, nlo = 0u;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const bool in = u[i] - lo <= range;
+      hi = max(hi, in ? u[i] : 0u);
+      nlo = max(nlo, in ? ~u[i] : 0u);
+    }
+    hi = wave_max(hi);
+    nlo = wave_max(nlo);
+    if (lane == 0) {
+      wave_a[wave] = hi;
+      wave_b[wave] = nlo;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kW; ++w) {
+      hi = max(hi, wave_a[w]);
+      nlo = max(nlo, wave_b[w]);
+    }
+    lo = ~nlo;
+    range = hi - lo;
+    if (range == 0u && ties > 0u) {   // one value many times over
+      key = lo;
+      break;
+    }
+    const int bits = range ? 32 - __builtin_clz(range) : 0;
+    const int shift = max(bits - kBinBits, 0);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      // A bin that many lanes share (zeros, ties) serializes their atomics.  Where the first column of a vector shows
+      // that, the lanes that agree with the first live one add theirs together, key by key; doing so always
+      // costs 5 us on rows of 32768 columns.
+      const bool in0 = u[j * W] - lo <= range;
+      const uint64_t live0 = __builtin_amdgcn_ballot_w64(in0);
+      const uint32_t bin0 = (u[j * W] - lo) >> shift;
+      const uint32_t lead0 = __builtin_amdgcn_readlane(bin0, live0 ? __builtin_ctzll(live0) : 0);
+      if (__builtin_popcountll(__builtin_amdgcn_ballot_w64(in0 && bin0 == lead0)) <= 8) {
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+          const uint32_t d = u[j * W + e] - lo;
+          if (d <= range) atomicAdd(&hist[d >> shift], 1u);
+        }
       } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) u[i + e] = 0u;   // padding: below every candidate (candidates are >= 1)
+        for (int e = 0; e < W; ++e) {
+          const uint32_t d = u[j * W + e] - lo, bin = d >> shift;
+          const bool in = d <= range;
+          const uint64_t live = __builtin_amdgcn_ballot_w64(in);
+          const uint32_t lead = __builtin_amdgcn_readlane(bin, live ? __builtin_ctzll(live) : 0);
+          const uint64_t same = __builtin_amdgcn_ballot_w64(in && bin == lead);
+          if (same != 0 && lane == __builtin_ctzll(same)) atomicAdd(&hist[bin], (uint32_t)__builtin_popcountll(same));
+          if (in && bin != lead) atomicAdd(&hist[bin], 1u);
+        }
       }
     }
-  } else {
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) u[i] = (base + i < N) ? order_key(widen<ET>(s[base + i])) : 0u;
-  }
-  if (tid < 34) cnt[tid] = 0;
-  __syncthreads();
-
-  // number of this wave's keys that satisfy pred(key), as a wave-uniform value: every lane counts its
-  // own keys, one cross-lane sum per call
-  auto wave_count = [&](auto pred) {
-    uint32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) c += pred(u[i]) ? 1u : 0u;
-    return wave_sum(c);
-  };
-
-  uint32_t T = 0;
-  for (int b = 31; b >= 0; --b) {
-    const uint32_t cand = T | (1u << b);
-    const uint32_t c = wave_count([&](uint32_t x) { return x >= cand; });
-    if (lane == 0 && c != 0) atomicAdd(&cnt[31 - b], c);
     __syncthreads();
-    if (cnt[31 - b] >= kk) T = cand;
+    // thread t takes bins kBins - 1 - 2t and the one below: prefix sums are counts from the top
+    const uint32_t h0 = hist[kBins - 1 - 2 * tid], h1 = hist[kBins - 2 - 2 * tid];
+    const uint32_t incl = wave_scan(h0 + h1);
+    if (lane == 63) wave_a[wave] = incl;
+    __syncthreads();
+    uint32_t above = incl - h0 - h1;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) above += (w < wave) ? wave_a[w] : 0u;
+    if (above < need && above + h0 >= need) {
+      sh_bin = (uint32_t)(kBins - 1 - 2 * tid);
+      sh_above = above;
+      sh_count = h0;
+    } else if (above + h0 < need && above + h0 + h1 >= need) {
+      sh_bin = (uint32_t)(kBins - 2 - 2 * tid);
+      sh_above = above + h0;
+      sh_count = h1;
+    }
+    hist[kBins - 1 - 2 * tid] = 0u;
+    hist[kBins - 2 - 2 * tid] = 0u;
+    __syncthreads();
+    ties = sh_count;
+    need -= sh_above;
+    lo += sh_bin << shift;
+    range = min((1u << shift) - 1u, 0xffffffffu - lo);   // (past 2^32 it would take in the padding)
+    if (shift == 0) {
+      key = lo;
+      break;
+    }
+    if (ties <= (uint32_t)kGather) {
+      const uint32_t count = ties;
+#pragma unroll
+      for (int i = 0; i < VPT; ++i)
+        if (u[i] - lo <= range) cand[atomicAdd(&sh_gathered, 1u)] = u[i];
+      __syncthreads();
+      if (tid < (int)count) {
+        const uint32_t mine = cand[tid];
+        uint32_t gt = 0, eq = 0;
+        for (uint32_t i = 0; i < count; ++i) {
+          const uint32_t o = cand[i];
+          gt += o > mine ? 1u : 0u;
+          eq += o == mine ? 1u : 0u;
+        }
+        if (gt < need && gt + eq >= need) {   // the same for every key that ties with it
+          sh_key = mine;
+          sh_need = need - gt;
+          sh_ties = eq;
+        }
+      }
+      __syncthreads();
+      key = sh_key;
+      need = sh_need;
+      ties = sh_ties;
+      break;
+    }
   }
-  // T is the key of the k-th largest element (all ones if k == 0: nothing is kept)
-  {
-    const uint32_t na = wave_count([&](uint32_t x) { return x > T; });
-    const uint32_t ne = wave_count([&](uint32_t x) { return x == T; });
-    if (lane == 0) {
-      if (na) atomicAdd(&cnt[32], na);
-      if (ne) atomicAdd(&cnt[33], ne);
+  // `key` is the key of the k-th largest element; `need` of the `ties` keys equal to it are kept
+  if (tid == 0 && threshold) threshold[blockIdx.x] = key_value(key);
+
+  const bool drop_ties = need < ties;   // uniform: some ties are dropped, rank them by column
+  if (drop_ties) {
+    // ties per block of 64 * W columns, in column order, then their exclusive prefix sums
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      uint32_t c = 0;
+#pragma unroll
+      for (int e = 0; e < W; ++e) c += u[j * W + e] == key ? 1u : 0u;
+      c = wave_sum(c);
+      if (lane == 0) block_ties[j * kW + wave] = c;
     }
     __syncthreads();
-  }
-  const uint32_t above = cnt[32], ties = cnt[33];
-  const uint32_t need = (kk > above) ? kk - above : 0u;   // how many of the `ties` keys equal to T are kept
-  if (tid == 0 && threshold) threshold[blockIdx.x] = key_value(T);
-
-  uint32_t before = 0;
-  if (need < ties) {   // uniform over the workgroup: some ties are dropped, rank them by column
-    uint32_t mine = 0;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) mine += (u[i] == T) ? 1u : 0u;
-    before = ties_before(mine, wave_eq, lane, wave);
-  }
-
-  // the mask, VPT bytes per thread
-  const bool keep_all_ties = need >= ties;
-  uint8_t out[VPT];
-#pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    const bool eq = u[i] == T;
-    const bool keep = (kk > 0) && ((u[i] > T) || (eq && (keep_all_ties || before < need)));
-    if (eq) ++before;
-    out[i] = keep ? 1 : 0;
-  }
-  if ((N & 7) == 0 && (reinterpret_cast<uintptr_t>(mask) & 7) == 0) {
-#pragma unroll
-    for (int i = 0; i < VPT; i += 8) {
-      if (base + i < N) {
-        uint64_t w = 0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) w |= (uint64_t)out[i + e] << (8 * e);
-        *reinterpret_cast<uint64_t*>(m + base + i) = w;
+    if (wave == 0) {
+      uint32_t base = 0;
+      for (int i0 = 0; i0 < J * kW; i0 += 64) {
+        const uint32_t c = (i0 + lane < J * kW) ? block_ties[i0 + lane] : 0u;
+        const uint32_t incl = wave_scan(c);
+        if (i0 + lane < J * kW) block_ties[i0 + lane] = base + incl - c;
+        base += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
       }
     }
-  } else {
+    __syncthreads();
+  }
 #pragma unroll
-    for (int i = 0; i < VPT; ++i)
-      if (base + i < N) m[base + i] = out[i];
+  for (int j = 0; j < J; ++j) {
+    const int col = (j * T + tid) * W;
+    uint32_t rank = 0u;   // ties in front of this thread's columns
+    if (drop_ties) {
+      uint32_t mine = 0;
+#pragma unroll
+      for (int e = 0; e < W; ++e) mine += u[j * W + e] == key ? 1u : 0u;
+      rank = block_ties[j * kW + wave] + wave_scan(mine) - mine;
+    }
+    uint8_t out[W];
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      const bool eq = u[j * W + e] == key;
+      out[e] = (kk > 0 && (u[j * W + e] > key || (eq && rank < need))) ? 1 : 0;
+      if (drop_ties && eq) ++rank;
+    }
+    if (col + W <= N) {
+      __builtin_memcpy(m + col, out, W);
+    } else {
+#pragma unroll
+      for (int e = 0; e < W; ++e)
+        if (col + e < N) m[col + e] = out[e];
+    }
   }
 }
 
@@ -2635,8 +2766,9 @@ int topk_any(const ET* scores, uint8_t* mask, float* threshold, int64_t rows, in
     return 0;
   }
   const dim3 grid((unsigned)rows), block(kTopkThreads);
-  if (N <= 8 * kTopkThreads) hipLaunchKernelGGL((topk_mask_kernel<8, ET>), grid, block, 0, s, scores, mask, threshold, N, k);
-  else if (N <= 32 * kTopkThreads) hipLaunchKernelGGL((topk_mask_kernel<32, ET>), grid, block, 0, s, scores, mask, threshold, N, k);
+  if (N <= 8 * 256) hipLaunchKernelGGL((topk_mask_kernel<256, 8, ET>), grid, dim3(256), 0, s, scores, mask, threshold, N, k);
+  else if (N <= 8 * kTopkThreads) hipLaunchKernelGGL((topk_mask_kernel<kTopkThreads, 8, ET>), grid, block, 0, s, scores, mask, threshold, N, k);
+  else if (N <= 32 * kTopkThreads) hipLaunchKernelGGL((topk_mask_kernel<kTopkThreads, 32, ET>), grid, block, 0, s, scores, mask, threshold, N, k);
   else hipLaunchKernelGGL(topk_mask_long_kernel<ET>, grid, block, 0, s, scores, mask, threshold, N, k);
   return 0;
 }

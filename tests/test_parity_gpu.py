@@ -991,6 +991,32 @@ def test_topk_orders_nans_above_everything(n, dtype):
         assert torch.equal(torch.isnan(thr.cpu()), nans >= k), k
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("n", [63, 2047, 2048, 2049, 8191, 8193, 32761, 32768])
+def test_topk_narrowing(n, dtype):
+    """Rows that end the narrowing in each of its ways, at the edges of the three workgroup sizes: spread scores
+    (ranked after the first count), one value in most columns, two neighbouring values, values packed into one bin
+    of the first count by a far outlier on either side, everything equal; bases that are not 16-byte aligned."""
+    from oracle.colreduce_oracle import topk_mask_ref
+    g = torch.Generator().manual_seed(n)
+    r = torch.randn(7, n, generator=g)
+    r[1] = torch.where(r[1] < 1, torch.zeros(n), r[1])
+    r[2] = torch.where(r[2] < 0, torch.full((n,), 0.5), torch.full((n,), 0.5 + 2.0 ** -11))
+    r[3] = 1 + r[3].abs() * 1e-3
+    r[3, n // 2] = 6e4
+    r[4] = 1 + r[4].abs() * 1e-3
+    r[4, n // 3] = -6e4
+    r[5] = -3.25
+    r[6] = float("nan")
+    r[6, : n // 2] = -float("inf")
+    r = r.to(dtype)
+    dev = r.cuda()   # rows of an odd number of elements: their bases have every alignment
+    for k in (1, n // 4, n // 2 + 1, n - 1, n):
+        mask, thr = fca.topk_keep_mask(dev, k, return_threshold=True)
+        want = topk_mask_ref(r.float().numpy(), k)
+        assert (mask.cpu().numpy() == want).all(), (n, k, dtype)
+
+
 def test_topk_on_reduced_columns():
     from oracle.colreduce_oracle import topk_mask_ref
     q, k = _inputs.config4(heads=4, n=2048)
