@@ -71,6 +71,11 @@ def _declare(lib):
     lib.fcr_colreduce_to.restype = c.c_int
     lib.fcr_colreduce_to.argtypes = ([c.c_void_p, c.c_void_p, c.c_void_p, c.c_int, c.c_void_p] + common +
                                      [c.c_int, c.c_int, c.c_void_p])
+    lib.fcr_workspace_bytes.restype = c.c_size_t
+    lib.fcr_workspace_bytes.argtypes = [c.c_int] * 6
+    lib.fcr_colreduce_ws.restype = c.c_int
+    lib.fcr_colreduce_ws.argtypes = ([c.c_void_p] * 4 + [c.c_int, c.c_void_p, c.c_size_t] + common +
+                                     [c.c_int, c.c_int, c.c_void_p])
     lib.fcr_colreduce_static.restype = c.c_int
     lib.fcr_colreduce_static.argtypes = ([c.c_void_p, c.c_void_p, c.c_void_p] + common +
                                          [c.c_int, c.c_int, c.c_void_p])

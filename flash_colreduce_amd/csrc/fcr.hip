@@ -1745,6 +1745,164 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
 }
 
 // ---------------------------------------------------------------------------------------------
+// One query (a decoded token): every score is used by one row only, so there is nothing for a tile to share and
+// the call is the reading of the keys.  Workgroups stream disjoint ranges of keys from memory straight into
+// registers, LPR lanes per key row and 16 bytes per lane and load, multiply on the vector unit in fp32, and
+// leave the raw products (4 bytes per key, against a row of 16 to 1024) and one (maximum, sum) of 2^score in
+// scratch; a second launch merges those pairs and stores the columns.  No workgroup waits for another, and a key
+// meets no matrix instruction with fifteen rows of padding.
+// Bound by HBM: eight loads of 1 KiB are in flight per wave and eight waves per SIMD (64 registers, hence the launch
+// bound); the 26 vector instructions per load take a fifth of its time.  256 pairs of 9001 keys of 128 bf16: 146 us
+// with the single sweep -> 102 us, 5.8 TB/s of keys (a large copy on the same card: 5.2; 112 us with loads that
+// are not marked non-temporal); what the single sweep does not take gains more: 80 x 30011 x 256 bf16 448 -> 220,
+// 64 x 16384 x 192 fp32 696 -> 127, 256 x 4096 x 64 fp32 207 -> 46, and at the small end 8 x 1024 x 128 14.4 -> 10,
+// 512 x 128 x 128 11.2 -> 9.5, 2 x 64 x 64 10.3 -> 9.6.
+constexpr int kOneLoads = 8;
+constexpr int kOneCols = 4;   // columns per thread of the second launch
+
+// (m, l) stands for l * 2^m, the sum of 2^score over the keys seen so far; m is their maximum, -inf before the
+// first one.  A NaN or +inf score makes l a NaN, for good.
+__device__ __forceinline__ void one_query_merge(float& m, float& l, float m2, float l2) {
+  const float mx = fmaxf(m, m2);
+  const float ref = (mx == kNegInf) ? 0.f : mx;
+  l = l * fast_exp2(m - ref) + l2 * fast_exp2(m2 - ref);
+  m = mx;
+}
+__device__ __forceinline__ void one_query_merge_wave(float& m, float& l) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const float m2 = __shfl_xor(m, d), l2 = __shfl_xor(l, d);
+    one_query_merge(m, l, m2, l2);
+  }
+}
+
+// Sum over each aligned group of LPR lanes, in all of its lanes.
+template <int LPR>
+__device__ __forceinline__ float group_sum(float v) {
+  if constexpr (LPR >= 2) v += dpp_row<0xB1>(v);     // quad_perm [1,0,3,2]
+  if constexpr (LPR >= 4) v += dpp_row<0x4E>(v);     // quad_perm [2,3,0,1]
+  if constexpr (LPR >= 8) v += dpp_row<0x141>(v);    // row_half_mirror
+  if constexpr (LPR >= 16) v += dpp_row<0x140>(v);   // row_mirror
+  if constexpr (LPR >= 32) v += __shfl_xor(v, 16);
+  if constexpr (LPR >= 64) v += __shfl_xor(v, 32);
+  return v;
+}
+
+// The elements of a 16-byte granule as floats.
+template <int DT>
+__device__ __forceinline__ void granule_floats(u32x4 v, float (&f)[DT == FCR_DTYPE_F32 ? 4 : 8]) {
+  if constexpr (DT == FCR_DTYPE_F32) {
+    const f32x4 x = __builtin_bit_cast(f32x4, v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = x[e];
+  } else if constexpr (DT == FCR_DTYPE_F16) {
+    const f16x8 x = __builtin_bit_cast(f16x8, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = (float)x[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[2 * e] = __builtin_bit_cast(float, v[e] << 16);
+      f[2 * e + 1] = __builtin_bit_cast(float, v[e] & 0xffff0000u);
+    }
+  }
+}
+
+// Workgroup v takes keys [split * rows_wg, + rows_wg) of pair v / p.splits, split = v % p.splits.  scores: [BH, pitch].
+template <int DT, int LPR>
+__global__ __launch_bounds__(256, 8) void one_query_scores_kernel(const Params p, float* __restrict__ scores,
+                                                               int64_t pitch, int rows_wg) {
+  constexpr int E = DT == FCR_DTYPE_F32 ? 4 : 8;
+  constexpr int kRows = 64 / LPR;                               // key rows per load
+  constexpr int kSel = kOneLoads > LPR ? kOneLoads / LPR : 1;   // finished scores per lane and step
+  constexpr int kStep = kOneLoads * kRows;                      // key rows per wave and step
+  __shared__ float wave_m[4], wave_l[4];
+  const int lane = threadIdx.x & 63, g = lane & (LPR - 1), r0 = lane / LPR;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int bh = (int)blockIdx.x / p.splits, split = (int)blockIdx.x - bh * p.splits;
+  const int b = bh / p.H, h = bh - b * p.H;
+  const char* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh + (int64_t)g * 16;
+  const char* qb = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)g * 16;
+  const bool live = g < p.dgran;   // the lanes past the end of a row neither load nor count
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  float qf[E];
+  granule_floats<DT>(live ? *reinterpret_cast<const u32x4*>(qb) : zero, qf);
+  const int first = split * rows_wg, end = min(p.N, first + rows_wg);
+  float* out = scores + (int64_t)bh * pitch;
+  float m = kNegInf, l = 0.f;
+  for (int row = first + wave * kStep; row < end; row += 4 * kStep) {
+    u32x4 v[kOneLoads];
+#pragma unroll
+    for (int u = 0; u < kOneLoads; ++u) {
+      const u32x4* src = reinterpret_cast<const u32x4*>(kb + (int64_t)min(row + u * kRows + r0, p.N - 1) * p.k_sr);
+      v[u] = zero;
+      if (live) v[u] = __builtin_nontemporal_load(src);   // no one else reads this row
+    }
+    float done[kSel];
+#pragma unroll
+    for (int i = 0; i < kSel; ++i) done[i] = 0.f;
+#pragma unroll
+    for (int u = 0; u < kOneLoads; ++u) {
+      float f[E], s = 0.f;
+      granule_floats<DT>(v[u], f);
+#pragma unroll
+      for (int e = 0; e < E; ++e) s = fmaf(f[e], qf[e], s);
+      s = group_sum<LPR>(s);
+      if (g == (u & (LPR - 1))) done[u / LPR] = s;   // lane g of a group keeps load g's row (and every LPR-th after it)
+    }
+#pragma unroll
+    for (int i = 0; i < kSel; ++i) {
+      const int r = row + (i * LPR + g) * kRows + r0;
+      if (i * LPR + g < kOneLoads && r < end) {
+        out[r] = done[i];
+        one_query_merge(m, l, done[i] * p.scale2, 1.f);
+      }
+    }
+  }
+  one_query_merge_wave(m, l);
+  if (lane == 0) {
+    wave_m[wave] = m;
+    wave_l[wave] = l;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 4; ++w) one_query_merge(m, l, wave_m[w], wave_l[w]);
+    p.part[2 * (int64_t)blockIdx.x] = m;
+    p.part[2 * (int64_t)blockIdx.x + 1] = l;
+  }
+}
+
+// p.tiles workgroups of 256 * kOneCols columns per pair; also the row statistic and the status word (p.sync, if any).
+template <int MODE>
+__global__ __launch_bounds__(256) void one_query_columns_kernel(const Params p, const float* __restrict__ scores,
+                                                                int64_t pitch) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int bh = (int)blockIdx.x / p.tiles, tile = (int)blockIdx.x - bh * p.tiles;
+  const int col0 = tile * 256 * kOneCols + tid;
+  const float* src = scores + (int64_t)bh * pitch;
+  float a[kOneCols];
+#pragma unroll
+  for (int i = 0; i < kOneCols; ++i) a[i] = src[min(col0 + 256 * i, p.N - 1)];
+  float m = kNegInf, l = 0.f;
+  const float* part = p.part + 2 * (int64_t)bh * p.splits;
+  for (int s = lane; s < p.splits; s += 64) one_query_merge(m, l, part[2 * s], part[2 * s + 1]);
+  one_query_merge_wave(m, l);
+  if (tile == 0 && tid == 0) p.lse[bh] = m + fast_log2(l);
+  if (blockIdx.x == 0 && tid == 0 && p.sync) *p.sync = 0u;
+  const float ref = (m == kNegInf) ? 0.f : m, inv = 1.0f / l;   // no score above -inf: 0 * inf, NaN sums
+#pragma unroll
+  for (int i = 0; i < kOneCols; ++i) {
+    const int key = col0 + 256 * i;
+    const float v = fast_exp2(fmaf(a[i], p.scale2, -ref)) * inv;
+    if (key < p.N) {
+      if (MODE != kModeMax) store_column(p, p.out, true, bh, key, v);
+      if (MODE != kModeSum) store_column(p, MODE == kModeBoth ? p.out2 : p.out, false, bh, key, fmaxf(v, 0.f));   // drops a NaN
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // fp32 operands.  x = hi + lo with hi = fp16(x), lo = fp16(x - hi) carries 22 bits of x.  Packing
 // queries as [hi | hi | lo] and keys as [hi | lo | hi] along d makes the fp16 kernels compute
 // q_hi.k_hi + q_hi.k_lo + q_lo.k_hi, the product to about 2^-22 (the lo.lo term is dropped), with fp32
@@ -2514,6 +2672,36 @@ bool fused_shape(int64_t bh, int M, int N, FusedPlan& f) {
   return true;
 }
 
+// The path for one query (one_query_*_kernel): sizes of its launches and its scratch, which lies behind everything
+// fcr_lse_bytes asks for.  Any element type and any number of keys.
+struct OneQueryPlan {
+  int lanes;              // lanes per key row: the row's granules, rounded up to a power of two
+  int splits, rows_wg;    // key ranges per pair and their length
+  int64_t pitch;          // floats per pair of the score array
+  int64_t part_at, scores_at, floats;   // where the pairs and the scores start and the workspace ends, in floats
+};
+OneQueryPlan one_query_plan(int dtype, int64_t bh, int N, int D, int64_t base_floats) {
+  OneQueryPlan o;
+  const int dgran = D * elem_bytes(dtype) / 16;
+  for (o.lanes = 1; o.lanes < dgran;) o.lanes *= 2;
+  const int64_t step = 4 * kOneLoads * (64 / o.lanes);   // keys a workgroup reads at a time
+  // about 128 workgroups per CU, each with at least one step: they fit eight at a time, and many short ranges level
+  // the end and read memory more nearly in order (default cache policy, 256 pairs of 9001 bf16 keys of 128: 16 per CU 120 us, 32: 118,
+  // 64: 115, 128 and more: 112; token-major keys of 256 prefer 32: 237 against 243)
+  int64_t splits = 128ll * chip_cus() / bh;
+  const int64_t steps = (N + step - 1) / step;
+  if (splits > steps) splits = steps;
+  if (splits < 1) splits = 1;
+  const int64_t steps_wg = (steps + splits - 1) / splits;
+  o.rows_wg = (int)(steps_wg * step);
+  o.splits = (int)((steps + steps_wg - 1) / steps_wg);
+  o.pitch = ((int64_t)N + 63) / 64 * 64;
+  o.part_at = (base_floats + 63) / 64 * 64;
+  o.scores_at = o.part_at + (2 * bh * o.splits + 63) / 64 * 64;
+  o.floats = o.scores_at + bh * o.pitch;
+  return o;
+}
+
 int launched(const char* what) {
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) return 0;
@@ -2736,6 +2924,38 @@ void launch_sweeps(int dtype, int which, const Params& p, int ksteps, bool causa
   if (dtype == FCR_DTYPE_F16) (long_rows ? fcr_detail::sweeps_f16_long_rows : fcr_detail::sweeps_f16)(which, p, ksteps, causal, mode, s);
   else if (dtype == FCR_DTYPE_BF16) (long_rows ? fcr_detail::sweeps_bf16_long_rows : fcr_detail::sweeps_bf16)(which, p, ksteps, causal, mode, s);
   else (long_rows ? fcr_detail::sweeps_f32_long_rows : fcr_detail::sweeps_f32)(which, p, ksteps, causal, mode, s);
+}
+
+template <int DT>
+void launch_one_query_scores(const Params& p, const OneQueryPlan& o, float* scores, hipStream_t s) {
+  const dim3 grid((unsigned)p.total), block(256);
+  switch (o.lanes) {
+    case 1: hipLaunchKernelGGL((one_query_scores_kernel<DT, 1>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 2: hipLaunchKernelGGL((one_query_scores_kernel<DT, 2>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 4: hipLaunchKernelGGL((one_query_scores_kernel<DT, 4>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 8: hipLaunchKernelGGL((one_query_scores_kernel<DT, 8>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 16: hipLaunchKernelGGL((one_query_scores_kernel<DT, 16>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 32: hipLaunchKernelGGL((one_query_scores_kernel<DT, 32>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    default: hipLaunchKernelGGL((one_query_scores_kernel<DT, 64>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+  }
+}
+
+int launch_one_query(Params& p, int dtype, const OneQueryPlan& o, float* ws, int mode, hipStream_t s) {
+  float* const scores = ws + o.scores_at;
+  p.part = ws + o.part_at;
+  p.splits = o.splits;
+  p.total = (int)(p.bh_count * (int64_t)o.splits);
+  if (dtype == FCR_DTYPE_F16) launch_one_query_scores<FCR_DTYPE_F16>(p, o, scores, s);
+  else if (dtype == FCR_DTYPE_BF16) launch_one_query_scores<FCR_DTYPE_BF16>(p, o, scores, s);
+  else launch_one_query_scores<FCR_DTYPE_F32>(p, o, scores, s);
+  int rc = launched("one_query_scores_kernel");
+  if (rc) return rc;
+  p.tiles = (p.N + 256 * kOneCols - 1) / (256 * kOneCols);
+  const dim3 grid((unsigned)(p.bh_count * (int64_t)p.tiles)), block(256);
+  if (mode == kModeSum) hipLaunchKernelGGL(one_query_columns_kernel<kModeSum>, grid, block, 0, s, p, scores, o.pitch);
+  else if (mode == kModeMax) hipLaunchKernelGGL(one_query_columns_kernel<kModeMax>, grid, block, 0, s, p, scores, o.pitch);
+  else hipLaunchKernelGGL(one_query_columns_kernel<kModeBoth>, grid, block, 0, s, p, scores, o.pitch);
+  return launched("one_query_columns_kernel");
 }
 
 template <int VPT, typename ET>
@@ -3009,7 +3229,8 @@ void order_end(SweepOrder* o, hipStream_t s, bool launched_it) {
 }
 
 // Both sweeps of a call, writing `out` in its final form.  ws_bytes = bytes the caller's workspace is known
-// to have (0: what fcr_lse_bytes asks for).  Few queries against many keys take the single sweep.
+// to have (0: what fcr_lse_bytes asks for).  One query takes the path of its own where the workspace has room for
+// its scores, few queries against many keys take the single sweep.
 int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, float* ws, size_t ws_bytes, int dtype,
                int B, int H, int M, int N, int D, const int64_t q_strides[4], const int64_t k_strides[4], float scale,
                int mode, int causal, void* stream, void* out2 = nullptr) {
@@ -3017,9 +3238,26 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
   int rc = make_params(p, q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, true, causal != 0, mode);
   if (rc) return rc;
   const int ksteps = ksteps_of(dtype, D);
+  const bool single = __atomic_load_n(&g_single_sweep, __ATOMIC_RELAXED) != 0;
   FusedPlan f;
-  if (__atomic_load_n(&g_single_sweep, __ATOMIC_RELAXED) && dtype != FCR_DTYPE_F32 && ksteps <= 4 &&
-      fused_shape(p.bh_count, M, N, f) && (ws_bytes == 0 || (size_t)f.floats * sizeof(float) <= ws_bytes)) {
+  const bool fused = dtype != FCR_DTYPE_F32 && ksteps <= 4 && fused_shape(p.bh_count, M, N, f);
+  p.out = out;
+  p.out2 = out2;
+  p.out_fmt = res.fmt;
+  if (res.mean) {
+    p.mean_from = causal ? p.c : N;
+    p.inv_m = 1.0f / (float)M;
+  }
+  p.stream_once = ((int64_t)p.bh_count * N * p.dgran * 16 >= (1ll << 30)) ? 1 : 0;
+  if (single && M == 1 && ws_bytes != 0) {   // (the mask hides nothing from the only query)
+    const OneQueryPlan o = one_query_plan(dtype, p.bh_count, N, D, (int64_t)(fcr_lse_bytes(B, H, M, N, D) / sizeof(float)));
+    if ((size_t)o.floats * sizeof(float) <= ws_bytes) {
+      p.lse = ws;
+      p.sync = fused ? reinterpret_cast<unsigned*>(ws + f.sync_at) : nullptr;   // fcr_colreduce_status looks there
+      return launch_one_query(p, dtype, o, ws, mode, static_cast<hipStream_t>(stream));
+    }
+  }
+  if (single && fused) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     p.lse = ws;
     p.part = ws + f.part_at;
@@ -3029,17 +3267,9 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
     p.total = f.teams * f.splits;
     const long long polls = __atomic_load_n(&g_wait_polls, __ATOMIC_RELAXED);
     p.spin_limit = polls > 0x7fffffffll ? 0x7fffffff : (int)polls;
-    p.out = out;
-    p.out2 = out2;
-    p.out_fmt = res.fmt;
-    if (res.mean) {
-      p.mean_from = causal ? p.c : N;
-      p.inv_m = 1.0f / (float)M;
-    }
-    p.stream_once = ((int64_t)p.bh_count * N * p.dgran * 16 >= (1ll << 30)) ? 1 : 0;
     const int words = (int)(f.floats - f.part_at);   // the slots and the error word start at zero
     fcr_detail::fused_refused = false;
-    SweepOrder* const order = (ws_bytes == 0) ? order_begin(s) : nullptr;
+    SweepOrder* const order = order_begin(s);
     launch_sweeps(dtype, 3, p, ksteps, causal != 0, mode | (f.qh == 2 ? 4 : 0) | (f.nq == 2 ? 8 : 0), s,
                   reinterpret_cast<unsigned*>(p.part), words);
     const int lrc = fcr_detail::fused_refused ? 0 : launched("col_fused_kernel");
@@ -3129,6 +3359,37 @@ int fcr_colreduce_sum_max_to(const void* q, const void* k, void* out_sum, void* 
   res.mean = sum_reduction == FCR_REDUCE_MEAN;
   return whole_call(q, k, out_sum, res, lse_ws, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale, kModeBoth, causal,
                     stream, out_max);
+}
+
+size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D) {
+  const size_t base = fcr_lse_bytes(B, H, M, N, D);
+  if (base == 0 || (dtype != FCR_DTYPE_F16 && dtype != FCR_DTYPE_BF16 && dtype != FCR_DTYPE_F32)) return base;
+  if (M == 1)
+    return (size_t)one_query_plan(dtype, (int64_t)B * H, N, D, (int64_t)(base / sizeof(float))).floats * sizeof(float);
+  return base;
+}
+
+int fcr_colreduce_ws(const void* q, const void* k, void* out, void* out_max, int out_dtype, void* ws, size_t ws_bytes,
+                     int dtype, int B, int H, int M, int N, int D, const int64_t q_strides[4],
+                     const int64_t k_strides[4], float scale, int reduction, int causal, void* stream) {
+  if (!out || !ws) return fail(FCR_E_NULL, "null pointer argument");
+  if (reduction != FCR_REDUCE_SUM && reduction != FCR_REDUCE_MEAN && (reduction != FCR_REDUCE_MAX || out_max))
+    return fail(FCR_E_REDUCTION, out_max ? "with out_max, reduction must be FCR_REDUCE_SUM or FCR_REDUCE_MEAN"
+                                         : "reduction must be FCR_REDUCE_SUM, FCR_REDUCE_MAX or FCR_REDUCE_MEAN");
+  if (out_dtype != FCR_DTYPE_F16 && out_dtype != FCR_DTYPE_BF16 && out_dtype != FCR_DTYPE_F32)
+    return fail(FCR_E_DTYPE, "out_dtype must be FCR_DTYPE_F16, FCR_DTYPE_BF16 or FCR_DTYPE_F32");
+  if ((reinterpret_cast<uintptr_t>(ws) & 15) != 0) return fail(FCR_E_STRIDE, "the workspace must be 16-byte aligned");
+  const size_t need = fcr_lse_bytes(B, H, M, N, D);
+  if (ws_bytes < need) {
+    snprintf(g_err, sizeof(g_err), "the workspace has %zu bytes, fcr_lse_bytes asks for %zu", ws_bytes, need);
+    return FCR_E_SCRATCH;
+  }
+  ResultSpec res;
+  res.fmt = out_dtype;
+  res.mean = reduction == FCR_REDUCE_MEAN;
+  const int mode = out_max ? kModeBoth : reduction == FCR_REDUCE_MAX ? kModeMax : kModeSum;
+  return whole_call(q, k, out, res, static_cast<float*>(ws), ws_bytes, dtype, B, H, M, N, D, q_strides, k_strides, scale,
+                    mode, causal, stream, out_max);
 }
 
 int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, int B, int H, int M, int N, int D,

@@ -93,10 +93,10 @@ _REDUCTIONS = {"sum": _lib.REDUCE_SUM, "max": _lib.REDUCE_MAX, "mean": _lib.REDU
 
 
 @functools.lru_cache(maxsize=4096)
-def _lse_floats(dev_index: int, b: int, h: int, m: int, n: int, d: int) -> int:
-    """Floats of the row-statistics buffer (fcr_lse_bytes depends on the device's CU count, hence dev_index)."""
+def _ws_floats(dev_index: int, dtype: int, b: int, h: int, m: int, n: int, d: int) -> int:
+    """Floats of the workspace (fcr_workspace_bytes depends on the device's CU count, hence dev_index)."""
     with torch.cuda.device(dev_index):
-        return max(b * h * m, _lib.load().fcr_lse_bytes(b, h, m, n, d) // 4)
+        return max(b * h * m, _lib.load().fcr_workspace_bytes(dtype, b, h, m, n, d) // 4)
 
 
 def _raw_stream(dev: torch.device) -> int:
@@ -109,7 +109,7 @@ def _raw_stream(dev: torch.device) -> int:
 
 def _launch_to(query, key, reduction, is_causal, scale, res_dtype):
     """One reduction, finished on the device: the column kernel stores res_dtype and divides the means
-    (fcr_colreduce_to), so nothing is left for torch to do after the two launches.  Needs M, N, B*H > 0."""
+    (fcr_colreduce_ws), so nothing is left for torch to do after the two launches.  Needs M, N, B*H > 0."""
     b, h, m, d = query.shape
     n = key.shape[2]
     if scale is None:
@@ -118,23 +118,25 @@ def _launch_to(query, key, reduction, is_causal, scale, res_dtype):
     lib = _lib.load()
     dev = query.device
     index = dev.index if dev.index is not None else torch.cuda.current_device()
-    lse = torch.empty(_lse_floats(index, b, h, m, n, q.shape[3]), device=dev, dtype=torch.float32)
+    dtype = _DTYPES[q.dtype]
+    floats = _ws_floats(index, dtype, b, h, m, n, q.shape[3])
+    ws = torch.empty(floats, device=dev, dtype=torch.float32)
     out = torch.empty((b, h, n), device=dev, dtype=res_dtype)
-    args = (q.data_ptr(), k.data_ptr(), out.data_ptr(), _DTYPES[res_dtype], lse.data_ptr(), _DTYPES[q.dtype], b, h, m, n,
-            q.shape[3], _lib.strides4(q.stride()), _lib.strides4(k.stride()), float(scale), _REDUCTIONS[reduction],
+    args = (q.data_ptr(), k.data_ptr(), out.data_ptr(), None, _DTYPES[res_dtype], ws.data_ptr(), 4 * floats, dtype, b, h,
+            m, n, q.shape[3], _lib.strides4(q.stride()), _lib.strides4(k.stride()), float(scale), _REDUCTIONS[reduction],
             1 if is_causal else 0)
     if torch.cuda.current_device() == index:
-        rc = lib.fcr_colreduce_to(*args, _raw_stream(dev))
+        rc = lib.fcr_colreduce_ws(*args, _raw_stream(dev))
     else:
         with torch.cuda.device(index):
-            rc = lib.fcr_colreduce_to(*args, _raw_stream(dev))
+            rc = lib.fcr_colreduce_ws(*args, _raw_stream(dev))
     if rc:
         _lib.check(rc)
     return out
 
 
 def _launch_pair_to(query, key, sum_reduction, is_causal, scale, res_dtype):
-    """Sums (or means) and maxima from one call, finished on the device (fcr_colreduce_sum_max_to)."""
+    """Sums (or means) and maxima from one call, finished on the device (fcr_colreduce_ws)."""
     b, h, m, d = query.shape
     n = key.shape[2]
     if scale is None:
@@ -143,13 +145,15 @@ def _launch_pair_to(query, key, sum_reduction, is_causal, scale, res_dtype):
     lib = _lib.load()
     dev = query.device
     index = dev.index if dev.index is not None else torch.cuda.current_device()
-    lse = torch.empty(_lse_floats(index, b, h, m, n, q.shape[3]), device=dev, dtype=torch.float32)
+    dtype = _DTYPES[q.dtype]
+    floats = _ws_floats(index, dtype, b, h, m, n, q.shape[3])
+    ws = torch.empty(floats, device=dev, dtype=torch.float32)
     sums = torch.empty((b, h, n), device=dev, dtype=res_dtype)
     maxs = torch.empty((b, h, n), device=dev, dtype=res_dtype)
     with torch.cuda.device(index):
-        _lib.check(lib.fcr_colreduce_sum_max_to(
-            q.data_ptr(), k.data_ptr(), sums.data_ptr(), maxs.data_ptr(), _DTYPES[res_dtype], lse.data_ptr(),
-            _DTYPES[q.dtype], b, h, m, n, q.shape[3], _lib.strides4(q.stride()), _lib.strides4(k.stride()), float(scale),
+        _lib.check(lib.fcr_colreduce_ws(
+            q.data_ptr(), k.data_ptr(), sums.data_ptr(), maxs.data_ptr(), _DTYPES[res_dtype], ws.data_ptr(), 4 * floats,
+            dtype, b, h, m, n, q.shape[3], _lib.strides4(q.stride()), _lib.strides4(k.stride()), float(scale),
             _REDUCTIONS[sum_reduction], 1 if is_causal else 0, _raw_stream(dev)))
     return sums, maxs
 
@@ -168,7 +172,9 @@ def _launch(query, key, kinds, is_causal, scale):
     dev = query.device
     # the row statistics, followed by whatever scratch the row kernel wants for this shape
     index = dev.index if dev.index is not None else torch.cuda.current_device()
-    lse = torch.empty(_lse_floats(index, b, h, m, n, q.shape[3]), device=dev, dtype=torch.float32)
+    dtype = _DTYPES[q.dtype]
+    floats = _ws_floats(index, dtype, b, h, m, n, q.shape[3])
+    lse = torch.empty(floats, device=dev, dtype=torch.float32)
     outs = [torch.empty((b * h, n), device=dev, dtype=torch.float32) for _ in kinds]
     if b * h * m * n == 0:
         lse.fill_(float("-inf"))
@@ -177,18 +183,19 @@ def _launch(query, key, kinds, is_causal, scale):
     else:
         with torch.cuda.device(dev):
             stream = torch.cuda.current_stream(dev).cuda_stream
-            common = (_DTYPES[q.dtype], b, h, m, n, q.shape[3], _lib.strides4(q.stride()), _lib.strides4(k.stride()),
+            common = (dtype, b, h, m, n, q.shape[3], _lib.strides4(q.stride()), _lib.strides4(k.stride()),
                       float(scale))
             causal = int(bool(is_causal))
             if len(kinds) == 1:
                 red = _lib.REDUCE_MAX if kinds[0] == "max" else _lib.REDUCE_SUM
-                _lib.check(lib.fcr_colreduce(q.data_ptr(), k.data_ptr(), outs[0].data_ptr(), lse.data_ptr(),
-                                             *common, red, causal, stream))
+                _lib.check(lib.fcr_colreduce_ws(q.data_ptr(), k.data_ptr(), outs[0].data_ptr(), None, _lib.DTYPE_F32,
+                                                lse.data_ptr(), 4 * floats, *common, red, causal, stream))
             elif sorted(kinds) == ["max", "sum"]:
                 # both kinds from one column sweep (few queries against many keys: from the single sweep)
                 by_kind = dict(zip(kinds, outs))
-                _lib.check(lib.fcr_colreduce_sum_max(q.data_ptr(), k.data_ptr(), by_kind["sum"].data_ptr(),
-                                                     by_kind["max"].data_ptr(), lse.data_ptr(), *common, causal, stream))
+                _lib.check(lib.fcr_colreduce_ws(q.data_ptr(), k.data_ptr(), by_kind["sum"].data_ptr(),
+                                                by_kind["max"].data_ptr(), _lib.DTYPE_F32, lse.data_ptr(), 4 * floats,
+                                                *common, _lib.REDUCE_SUM, causal, stream))
             else:
                 _lib.check(lib.fcr_row_lse(q.data_ptr(), k.data_ptr(), lse.data_ptr(), *common, causal, stream))
                 for kind, o in zip(kinds, outs):
@@ -289,7 +296,7 @@ def flash_colreduce_multi(
         raise ValueError("reduction='max' needs at least one query row.")
     wanted = set(reductions)
     if m > 0 and b * h * n > 0 and res_dtype in _DTYPES and wanted in ({"sum", "max"}, {"mean", "max"}):
-        # the usual pair: both results leave the kernel in their final form (fcr_colreduce_sum_max_to)
+        # the usual pair: both results leave the kernel in their final form (fcr_colreduce_ws)
         sums, maxs = _launch_pair_to(query, key, "mean" if "mean" in wanted else "sum", is_causal, scale, res_dtype)
         out, seen = [], set()
         for r in reductions:   # an entry named twice gets a tensor of its own

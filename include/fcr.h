@@ -67,7 +67,7 @@ extern "C" {
 #define FCR_E_WAIT -8      /* fcr_colreduce_status: a workgroup of the single sweep gave up waiting for its team */
 
 /* fcr_set_option */
-#define FCR_OPT_SINGLE_SWEEP 0 /* 0: few queries against many keys take the two kernels as well (default 1) */
+#define FCR_OPT_SINGLE_SWEEP 0 /* 0: few queries against many keys, or one query, take the two kernels as well (default 1) */
 #define FCR_OPT_WAIT_POLLS 1   /* polls of a team's slots after which a workgroup gives up (default 2^20) */
 
 /* size of the built-in scratch buffer of fcr_colreduce_static, per GPU */
@@ -189,6 +189,20 @@ int fcr_colreduce_sum_max(const void* q, const void* k, float* out_sum, float* o
 int fcr_colreduce_to(const void* q, const void* k, void* out, int out_dtype, float* lse_ws, int dtype, int B,
                      int H, int M, int N, int D, const int64_t q_strides[4], const int64_t k_strides[4],
                      float scale, int reduction, int causal, void* stream);
+
+/*
+ * The whole operator with a workspace of known size: what fcr_colreduce_to (out_max NULL) and
+ * fcr_colreduce_sum_max_to (out_max given; reduction then names what `out` holds, sum or mean) compute, and with
+ * fcr_workspace_bytes(dtype, B, H, M, N, D) bytes by the fastest path for the problem: one query is read
+ * once, without the matrix instructions, and its scores wait in the workspace (4 bytes per key) for their row's
+ * sum.  With less, but at least fcr_lse_bytes, the call takes the path of the entry points above
+ * (FCR_E_SCRATCH below that); results agree to rounding either way.  ws must be 16-byte aligned, its first
+ * B*H*M floats hold the row statistics on return, its contents before the call are irrelevant.
+ */
+size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D);
+int fcr_colreduce_ws(const void* q, const void* k, void* out, void* out_max, int out_dtype, void* ws, size_t ws_bytes,
+                     int dtype, int B, int H, int M, int N, int D, const int64_t q_strides[4],
+                     const int64_t k_strides[4], float scale, int reduction, int causal, void* stream);
 
 /*
  * fcr_colreduce without the lse_ws argument, for callers that cannot allocate device memory (code under

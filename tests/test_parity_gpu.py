@@ -405,6 +405,77 @@ def test_single_sweep(b, h, m, n, d, causal, dtype):
 
 
 @pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,h,n,d,dtype", [
+    (1, 1, 1, 8, torch.float16),          # one key, one granule per row
+    (2, 3, 31, 16, torch.bfloat16),       # less than a step of a wave
+    (1, 2, 257, 24, torch.float16),       # three granules on four lanes
+    (3, 5, 1025, 72, torch.bfloat16),     # nine granules on sixteen lanes, one column past a workgroup's
+    (2, 4, 4097, 128, torch.float16),     # more than one key range per pair
+    (1, 3, 1000, 200, torch.bfloat16),    # 32 lanes per row
+    (1, 2, 333, 512, torch.float16),      # 64 lanes per row
+    (2, 2, 600, 4, torch.float32), (1, 3, 2049, 80, torch.float32), (1, 2, 777, 256, torch.float32),
+    (1, 1, 70001, 64, torch.float16),     # more key ranges than lanes in the merge
+])
+def test_one_query(b, h, n, d, dtype, causal):
+    """One query row (one_query_*_kernel): every lanes-per-row, ragged lengths, both layouts; the row statistics and
+    the status word of its workspace; and the other path through the C ABI."""
+    from flash_colreduce_amd import _lib
+    from flash_colreduce_amd.flash import _DTYPES as DT
+    q, k = _inputs.randn_pair(b, h, 1, n, d, seed=n + d, dtype=dtype)
+    what = f"one query b{b} h{h} n{n} d{d} {dtype}"
+    qd, kd = q.cuda(), k.cuda()
+    kt = kd.transpose(1, 2).contiguous().transpose(1, 2)   # token-major memory seen as heads
+    lib = _lib.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    nbytes = lib.fcr_workspace_bytes(DT[dtype], b, h, 1, n, d)
+    assert nbytes >= lib.fcr_lse_bytes(b, h, 1, n, d) + 4 * b * h * n
+    for red in REDUCTIONS:
+        want = colreduce_ref(q, k, red, causal)
+        got = fca.flash_colreduce(qd, kd, red, is_causal=causal, out_dtype=torch.float32)
+        check(got.cpu(), want, red, what)
+        assert torch.equal(got, fca.flash_colreduce(qd, kt, red, is_causal=causal, out_dtype=torch.float32))
+        assert torch.equal(fca.flash_colreduce(qd, kd, red, is_causal=causal), got.to(dtype))   # (means divide by one)
+        if red == "mean":
+            continue
+        ws = torch.full((nbytes // 4,), float("nan"), device="cuda")
+        one, other = (torch.empty(b, h, n, device="cuda") for _ in range(2))
+        code = _lib.REDUCE_MAX if red == "max" else _lib.REDUCE_SUM
+        common = (DT[dtype], b, h, 1, n, d, _lib.strides4(qd.stride()), _lib.strides4(kd.stride()), d ** -0.5, code,
+                  int(causal), stream)
+        _lib.check(lib.fcr_colreduce_ws(qd.data_ptr(), kd.data_ptr(), one.data_ptr(), None, _lib.DTYPE_F32,
+                                        ws.data_ptr(), nbytes, *common))
+        assert torch.equal(one, got)
+        torch.testing.assert_close(ws[: b * h].view(b, h, 1).double().cpu(), row_lse2_ref(q, k, causal), rtol=0, atol=3e-4)
+        assert lib.fcr_colreduce_status(ws.data_ptr(), DT[dtype], b, h, 1, n, d, stream) == 0
+        _lib.check(lib.fcr_colreduce_ws(qd.data_ptr(), kd.data_ptr(), other.data_ptr(), None, _lib.DTYPE_F32,
+                                        ws.data_ptr(), lib.fcr_lse_bytes(b, h, 1, n, d), *common))
+        torch.testing.assert_close(other, one, rtol=2e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_one_query_non_finite(dtype):
+    """One query: a NaN or +inf score makes the sums of its row NaN and its maxima 0, -inf scores count nothing (a row
+    of nothing else is a NaN row), scores far from zero keep their softmax."""
+    h, n, d = 6, 3000, 64
+    q, k = _inputs.randn_pair(1, h, 1, n, d, seed=12, dtype=torch.float32)
+    q[..., 0] = 1.0
+    k[0, 0, 2000, 5] = float("nan")
+    k[0, 1, 7, 0] = float("inf")
+    k[0, 2, 100:2900, 0] = -float("inf")
+    k[0, 3, :, 0] = -float("inf")
+    k[0, 4] *= 30.0
+    q, k = q.to(dtype), k.to(dtype)
+    s, m = fca.flash_colreduce_multi(q.cuda(), k.cuda(), ["sum", "max"], is_causal=True, out_dtype=torch.float32)
+    bad = [0, 1, 3]
+    assert torch.isnan(s[0, bad]).all() and (m[0, bad] == 0).all()
+    good = [2, 4, 5]
+    p = torch.softmax((q.double() @ k.double().transpose(2, 3))[0, good, 0] / math.sqrt(d), -1)
+    for got in (s, m):
+        # scaled |q||k| sums of up to 150 at 2^-24 per term, added up eight at a time: below 1e-4 of a probability
+        torch.testing.assert_close(got[0, good].double().cpu(), p, rtol=1e-4, atol=1e-30)
+
+
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("m", [64, 128])
 def test_single_sweep_scores_far_from_zero(m, causal):
     """Row sums of 2^score that overflow or vanish in fp32 (an enormous aligned key late in the sweep, rows
