@@ -154,6 +154,15 @@ inline int row_blocks_per_wave(int ksteps, int M, int N, int64_t bh, bool causal
   if (wgs2 < cus && N <= 1024) return 1;
   return (wgs2 >= cus && wgs2 < 2 * cus + (causal ? 1 : 0)) ? 1 : 2;
 }
+// fp32 operands that give at most one workgroup of 128 rows on every other CU: tiles of 64 rows, one 16-row group
+// per wave (NB = 0).  Such a launch lasts as long as one workgroup, whose sweep is all fp32 matrix instructions
+// (32 cycles per 16x16x4 and SIMD), and half the resident rows halve it.  With more workgroups than that the
+// halves only share the CUs.  16-bit operands spend their short sweeps on latency instead.  A row sweep of 16 chunks
+// or more is split over the idle CUs (row_splits) and keeps its tile.  Per call: 2 heads of 256 x 256 x 64 24.3 -> 18.6 us,
+// 32 of 512 x 512 x 128 72 -> 42, 16 of 900 x 900 x 64 70 -> 41, 16 of 1024 x 1024 x 256 212 -> 151, 8 of 2048 x 2048 x 128
+// 199 -> 141, 2 of 8192 x 8192 x 128 757 -> 527; just above the rule (32 heads of 1024 x 1024 x 128) 137 either way.
+inline bool half_tiles(bool f32, int64_t rows, int64_t bh) { return f32 && 2 * bh * ((rows + 127) / 128) <= chip_cus(); }
+inline bool row_half_tiles(bool f32, int M, int N, int64_t bh) { return N <= 15 * 64 && half_tiles(f32, M, bh); }
 inline int row_tile_rows(int ksteps, int M, int N, int64_t bh, bool causal) {
   return kWaves * 32 * row_blocks_per_wave(ksteps, M, N, bh, causal);
 }
@@ -245,9 +254,12 @@ __device__ __forceinline__ void map_block_split(const Params& p, bool longest_is
 // block b has b+1 (rows) or 8-b (columns) visible sub-tiles out of 8, so every wave gets 9 of the 36
 // and the four waves reach each barrier together.  With one block per wave, wave w keeps block w
 // of four.
+// With NB = 0 a wave keeps one group, w of four.
+__host__ __device__ constexpr int wave_group_count(int nb) { return nb ? 2 * nb : 1; }
 template <int NB>
-__device__ __forceinline__ void wave_groups(int tile, int wave, int (&rows)[2 * NB]) {
-  const int t0 = tile * (kWaves * 32 * NB);
+__device__ __forceinline__ void wave_groups(int tile, int wave, int (&rows)[wave_group_count(NB)]) {
+  const int t0 = tile * (kWaves * 16 * wave_group_count(NB));
+  if constexpr (NB == 0) rows[0] = t0 + 16 * wave;
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     // blocks w, 7-w (, 8+w, 15-w): even positions count up, odd ones count down inside a run of eight
@@ -640,8 +652,8 @@ struct NoAux {};
 template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE>
 __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(const Params p) {
   using Rg = Ring<KS>;
-  constexpr int NG = 2 * NB;
-  constexpr int kTileRows = kWaves * 32 * NB;
+  constexpr int NG = wave_group_count(NB);
+  constexpr int kTileRows = kWaves * 16 * NG;
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes];
   int bh, tile, split;
   map_block_split(p, CAUSAL, bh, tile, split);
@@ -824,8 +836,8 @@ inline int col_tile_blocks(int ksteps, int mode, int N, int64_t bh, bool causal)
 template <int DT, int KS, bool CAUSAL, int MODE, int NB>
 __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_reduce_kernel(const Params p) {
   using Rg = Ring<KS>;
-  constexpr int NG = 2 * NB;
-  constexpr int kTileRows = kWaves * 32 * NB;
+  constexpr int NG = wave_group_count(NB);
+  constexpr int kTileRows = kWaves * 16 * NG;
   constexpr int kRed = kWaves * NG * 4 * 64 * 4;      // end-of-sweep transpose buffer
   constexpr int kSmem = (Rg::kBytes > kRed) ? Rg::kBytes : kRed;
   __shared__ __attribute__((aligned(1024))) char smem[kSmem];
@@ -2582,7 +2594,10 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   if (rc) return rc;
   // the device is first asked (for its CU count) here, after every argument check
   const int ksteps = ksteps_of(dtype, D);
-  const int trows = by_keys ? kWaves * 32 * col_tile_blocks(ksteps, col_mode, N, bh, causal) : row_tile_rows(ksteps, M, N, bh, causal);
+  const bool f32 = dtype == FCR_DTYPE_F32;
+  const bool half = by_keys ? half_tiles(f32, N, bh) : row_half_tiles(f32, M, N, bh);
+  const int trows = half ? kWaves * 16
+                         : by_keys ? kWaves * 32 * col_tile_blocks(ksteps, col_mode, N, bh, causal) : row_tile_rows(ksteps, M, N, bh, causal);
   const int64_t tiles = ((by_keys ? N : M) + trows - 1) / trows;
   p.q = static_cast<const char*>(q);
   p.k = static_cast<const char*>(k);
@@ -2718,6 +2733,9 @@ void launch_lse_blocks(const Params& p, bool causal, hipStream_t s) {
 
 template <int DT, int KS>
 void launch_lse(const Params& p, bool causal, hipStream_t s) {
+  if constexpr (DT == FCR_DTYPE_F32) {
+    if (row_half_tiles(true, p.M, p.N, p.bh_count)) return launch_lse_blocks<DT, KS, 0, false>(p, causal, s);
+  }
   if constexpr (KS <= 4) {
     if (row_blocks_per_wave(KS, p.M, p.N, p.bh_count, causal) == 2) return launch_lse_blocks<DT, KS, 2, false>(p, causal, s);
   }
@@ -2731,6 +2749,13 @@ template <int DT, int KS, int MODE>
 void launch_col_mode(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(kThreads);
   constexpr int NB = col_blocks_per_wave(KS, MODE);
+  if constexpr (DT == FCR_DTYPE_F32) {
+    if (half_tiles(true, p.N, p.bh_count)) {
+      if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 0>), grid, block, 0, s, p);
+      else hipLaunchKernelGGL((col_reduce_kernel<DT, KS, false, MODE, 0>), grid, block, 0, s, p);
+      return;
+    }
+  }
   if constexpr (NB == 2) {
     if (col_tile_blocks(KS, MODE, p.N, p.bh_count, causal) == 1) {
       if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 1>), grid, block, 0, s, p);

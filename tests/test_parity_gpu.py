@@ -312,6 +312,20 @@ def test_causal_launches_that_are_on_the_chip_at_once(b, h, m, n, d):
     run_all(q, k, True, what=f"{b}x{h} {m}x{n}x{d}", reductions=["sum", "max"])
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,h,m,n,d", [(1, 2, 256, 256, 64), (1, 1, 2, 65, 4), (2, 3, 65, 63, 72), (1, 4, 191, 961, 128),
+                                       (1, 8, 960, 960, 132), (1, 128, 64, 128, 16), (1, 129, 64, 128, 32),
+                                       (1, 8, 1000, 2048, 256)])
+def test_fp32_tiles_of_64_rows(b, h, m, n, d, causal):
+    """fp32 launches that leave CUs idle take 64-row tiles: remainders of a tile, of a wave's 16 rows and of a chunk,
+    M > N, both sides of the split row sweep, the most and one more than the most workgroups of the rule."""
+    q, k = _inputs.randn_pair(b, h, m, n, d, seed=m + n, dtype=torch.float32)
+    run_all(q, k, causal, what=f"fp32 {b}x{h} {m}x{n}x{d}")
+    s, mx = fca.flash_colreduce_multi(q.cuda(), k.cuda(), ["sum", "max"], is_causal=causal)
+    check(s.cpu(), colreduce_ref(q, k, "sum", causal), "sum", "fp32 pair")
+    check(mx.cpu(), colreduce_ref(q, k, "max", causal), "max", "fp32 pair")
+
+
 @pytest.mark.parametrize("m", [100, 128, 300, 384, 600])
 def test_row_sweep_block_choice(m):
     """Query counts for which the row sweep keeps one 32-row block per wave (M <= 128 and ragged M
