@@ -2631,11 +2631,12 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
 // workgroup per CU; otherwise the keys of a tile are split so that about two per CU run, each
 // keeping at least four 64-key chunks.
 int row_splits(int B, int H, int M, int N, int ksteps) {
+  const int64_t chunks = (N + kChunk - 1) / kChunk;
+  if (chunks < 16) return 1;
   const int trows = row_tile_rows(ksteps, M, N, (int64_t)B * H, false);  // same with the mask when wgs < 256
   const int64_t wgs = (int64_t)B * H * ((M + trows - 1) / trows);
-  const int64_t chunks = (N + kChunk - 1) / kChunk;
   const int cus = chip_cus();
-  if (wgs >= cus || chunks < 16) return 1;
+  if (wgs >= cus) return 1;
   int64_t s = 2 * cus / wgs;
   if (s > chunks / 4) s = chunks / 4;
   if (s > 64) s = 64;
@@ -3022,9 +3023,10 @@ int topk_any(const ET* scores, uint8_t* mask, float* threshold, int64_t rows, in
 namespace {
 size_t fcr_lse_bytes_two_kernels(int B, int H, int M, int N) {
   // the most any row width asks for (the tile height, hence the split count, depends a little on the
-  // number of 64-byte k-steps of a row), so the size holds for every dtype and D
+  // number of 64-byte k-steps of a row), so the size holds for every dtype and D; from five k-steps on
+  // row_blocks_per_wave gives one block for all (every call comes here: 16 widths cost the host 0.5 us)
   int splits = 1;
-  for (int ks = 1; ks <= kMaxKStepsF32; ++ks) {
+  for (int ks = 1; ks <= 5; ++ks) {
     const int s = row_splits(B, H, M, N, ks);
     if (s > splits) splits = s;
   }
