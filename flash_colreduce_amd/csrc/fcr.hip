@@ -2570,6 +2570,12 @@ int fill_ranks(const Params& p, bool causal) {
   return (cus + p.group - 1) / p.group;
 }
 
+// Rows the kernels take: a multiple of 16 bytes, at most 1 KiB (and no product of D that could overflow).
+bool row_width_ok(int dtype, int D) {
+  const int esize = elem_bytes(dtype);
+  return D >= 1 && D <= 64 * kMaxKStepsF32 / esize && (D * esize) % 16 == 0;
+}
+
 int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H, int M, int N, int D,
                 const int64_t qs[4], const int64_t ks[4], float scale, bool by_keys, bool causal,
                 int col_mode = kModeSum) {
@@ -3391,7 +3397,7 @@ int fcr_colreduce_sum_max_to(const void* q, const void* k, void* out_sum, void* 
 size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D) {
   const size_t base = fcr_lse_bytes(B, H, M, N, D);
   if (base == 0 || (dtype != FCR_DTYPE_F16 && dtype != FCR_DTYPE_BF16 && dtype != FCR_DTYPE_F32)) return base;
-  if (M == 1)
+  if (M == 1 && row_width_ok(dtype, D))   // (a row the call rejects has no plan: no power of two of 64 lanes or less)
     return (size_t)one_query_plan(dtype, (int64_t)B * H, N, D, (int64_t)(base / sizeof(float))).floats * sizeof(float);
   return base;
 }

@@ -28,7 +28,8 @@ def test_library_exports_every_declared_symbol():
     assert {"fcr_version", "fcr_last_error", "fcr_lse_bytes", "fcr_row_lse", "fcr_col_reduce",
             "fcr_col_reduce_sum_max", "fcr_pack_f32", "fcr_colreduce", "fcr_colreduce_static",
             "fcr_colreduce_to", "fcr_topk_mask", "fcr_topk_mask_ws", "fcr_topk_mask_typed", "fcr_topk_bytes", "fcr_set_option",
-            "fcr_colreduce_status", "fcr_colreduce_sum_max", "fcr_colreduce_sum_max_to"} <= set(names)
+            "fcr_colreduce_status", "fcr_colreduce_sum_max", "fcr_colreduce_sum_max_to", "fcr_workspace_bytes",
+            "fcr_colreduce_ws"} <= set(names)
     for name in names:
         assert hasattr(lib, name), name
 
@@ -43,6 +44,20 @@ def test_version_and_sizes():
     # one workgroup per CU of 128 rows, and the status line
     assert lib.fcr_lse_bytes(1, 32, 128, 4096, 128) == (32 * 128 + 2 * 2 * 256 * 128 + 32) * 4
     assert lib.fcr_lse_bytes(-1, 3, 5, 7, 8) == 0 and lib.fcr_lse_bytes(1, 3, 0, 7, 8) == 0
+
+
+def test_workspace_size_of_one_query():
+    """One query asks for its scores and key ranges behind fcr_lse_bytes, for every row width the kernels take; for
+    any other width (which the call then rejects) and for more queries it is fcr_lse_bytes."""
+    lib = _lib.load()
+    for dtype, limit, step in ((0, 512, 8), (1, 512, 8), (2, 256, 4)):
+        for d in range(step, limit + 1, step):
+            assert lib.fcr_workspace_bytes(dtype, 2, 3, 1, 1000, d) >= lib.fcr_lse_bytes(2, 3, 1, 1000, d) + 4 * 6 * 1000
+        for d in (limit + step, 2 * limit, 1 << 20, 1 << 30, (1 << 31) - 1, step - 1, 0, -step):
+            assert lib.fcr_workspace_bytes(dtype, 2, 3, 1, 1000, d) == lib.fcr_lse_bytes(2, 3, 1, 1000, d)
+        assert lib.fcr_workspace_bytes(dtype, 2, 3, 2, 1000, 64) == lib.fcr_lse_bytes(2, 3, 2, 1000, 64)
+        assert lib.fcr_workspace_bytes(dtype, 2, 3, 1, 0, 64) == 0
+    assert lib.fcr_workspace_bytes(3, 2, 3, 1, 1000, 64) == lib.fcr_lse_bytes(2, 3, 1, 1000, 64)
 
 
 def _call(lib, fn, **over):
