@@ -2584,7 +2584,7 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
     return fail(FCR_E_DTYPE, "dtype must be FCR_DTYPE_F16, FCR_DTYPE_BF16 or FCR_DTYPE_F32");
   if (B < 1 || H < 1 || M < 1 || N < 1) return fail(FCR_E_SHAPE, "B, H, M, N must be >= 1");
   const int esize = elem_bytes(dtype);
-  if (D < 1 || D * esize > 64 * kMaxKStepsF32 || (D * esize) % 16 != 0)
+  if (!row_width_ok(dtype, D))
     return fail(FCR_E_SHAPE, esize == 2 ? "D must be a multiple of 8 in [8, 512]"
                                          : "D must be a multiple of 4 in [4, 256] for FCR_DTYPE_F32");
   if (M > (1 << 30) || N > (1 << 30)) return fail(FCR_E_SHAPE, "M and N must be <= 2^30");
