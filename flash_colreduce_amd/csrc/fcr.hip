@@ -2576,9 +2576,9 @@ bool row_width_ok(int dtype, int D) {
   return D >= 1 && D <= 64 * kMaxKStepsF32 / esize && (D * esize) % 16 == 0;
 }
 
-int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H, int M, int N, int D,
-                const int64_t qs[4], const int64_t ks[4], float scale, bool by_keys, bool causal,
-                int col_mode = kModeSum) {
+// The arguments of a launch over the queries or (by_keys) the keys; no HIP call.
+int check_problem(const void* q, const void* k, int dtype, int B, int H, int M, int N, int D, const int64_t qs[4],
+                  const int64_t ks[4], float scale, bool by_keys) {
   if (!q || !k || !qs || !ks) return fail(FCR_E_NULL, "null pointer argument");
   if (dtype != FCR_DTYPE_F16 && dtype != FCR_DTYPE_BF16 && dtype != FCR_DTYPE_F32)
     return fail(FCR_E_DTYPE, "dtype must be FCR_DTYPE_F16, FCR_DTYPE_BF16 or FCR_DTYPE_F32");
@@ -2596,8 +2596,16 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   const int qdims[3] = {B, H, M}, kdims[3] = {B, H, N};
   int rc = check_strides(q, qs, "q", qdims, D, esize);
   if (rc) return rc;
-  rc = check_strides(k, ks, "k", kdims, D, esize);
+  return check_strides(k, ks, "k", kdims, D, esize);
+}
+
+int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H, int M, int N, int D,
+                const int64_t qs[4], const int64_t ks[4], float scale, bool by_keys, bool causal,
+                int col_mode = kModeSum) {
+  const int rc = check_problem(q, k, dtype, B, H, M, N, D, qs, ks, scale, by_keys);
   if (rc) return rc;
+  const int esize = elem_bytes(dtype);
+  const int64_t bh = (int64_t)B * H;
   // the device is first asked (for its CU count) here, after every argument check
   const int ksteps = ksteps_of(dtype, D);
   const bool f32 = dtype == FCR_DTYPE_F32;
@@ -3412,6 +3420,10 @@ int fcr_colreduce_ws(const void* q, const void* k, void* out, void* out_max, int
   if (out_dtype != FCR_DTYPE_F16 && out_dtype != FCR_DTYPE_BF16 && out_dtype != FCR_DTYPE_F32)
     return fail(FCR_E_DTYPE, "out_dtype must be FCR_DTYPE_F16, FCR_DTYPE_BF16 or FCR_DTYPE_F32");
   if ((reinterpret_cast<uintptr_t>(ws) & 15) != 0) return fail(FCR_E_STRIDE, "the workspace must be 16-byte aligned");
+  // every argument of both launches first: the workspace's size depends on the device
+  int rc = check_problem(q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, true);
+  if (!rc) rc = check_problem(q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, false);
+  if (rc) return rc;
   const size_t need = fcr_lse_bytes(B, H, M, N, D);
   if (ws_bytes < need) {
     snprintf(g_err, sizeof(g_err), "the workspace has %zu bytes, fcr_lse_bytes asks for %zu", ws_bytes, need);

@@ -77,10 +77,13 @@ def _call(lib, fn, **over):
     if fn == "colreduce_sum_max":
         return lib.fcr_colreduce_sum_max(a["q"], a["k"], a["out"], a.get("out_max", 80), a["lse"], *common, a["causal"],
                                          None)
+    if fn == "colreduce_ws":   # no room in the workspace unless a case says so: every other error comes before that one
+        return lib.fcr_colreduce_ws(a["q"], a["k"], a["out"], a.get("out_max"), a.get("out_dtype", 0), a["lse"],
+                                    a.get("ws_bytes", 0), *common, a["red"], a["causal"], None)
     return lib.fcr_colreduce(a["q"], a["k"], a["out"], a["lse"], *common, a["red"], a["causal"], None)
 
 
-@pytest.mark.parametrize("fn", ["row_lse", "col_reduce", "colreduce", "colreduce_to", "colreduce_sum_max"])
+@pytest.mark.parametrize("fn", ["row_lse", "col_reduce", "colreduce", "colreduce_to", "colreduce_sum_max", "colreduce_ws"])
 def test_c_abi_rejects_bad_arguments_without_a_device(fn):
     """Every rejection happens before the first HIP call, so fake pointers are safe here."""
     lib = _lib.load()
@@ -102,6 +105,10 @@ def test_c_abi_rejects_bad_arguments_without_a_device(fn):
     if fn == "colreduce_to":   # takes the mean as a third reduction, and a result type
         cases += [(dict(out=None), -1), (dict(red=3), -5), (dict(red=-1), -5), (dict(out_dtype=3), -2),
                   (dict(out_dtype=-1), -2)]
+    elif fn == "colreduce_ws":
+        cases += [(dict(out=None), -1), (dict(red=3), -5), (dict(red=1, out_max=80), -5), (dict(out_dtype=3), -2),
+                  (dict(lse=52), -4), (dict(B=1 << 12, H=1 << 12, M=1), -3), (dict(M=1), -7), (dict(ws_bytes=31), -7),
+                  (dict(dtype=2, M=1, N=1000, ks=(64000, 64000, 64, 1), ws_bytes=3), -7)]
     elif fn == "colreduce_sum_max":
         cases += [(dict(out=None), -1), (dict(out_max=None), -1)]
     elif fn != "row_lse":
