@@ -3036,14 +3036,10 @@ int topk_any(const ET* scores, uint8_t* mask, float* threshold, int64_t rows, in
 
 namespace {
 size_t fcr_lse_bytes_two_kernels(int B, int H, int M, int N) {
-  // the most any row width asks for (the tile height, hence the split count, depends a little on the
-  // number of 64-byte k-steps of a row), so the size holds for every dtype and D; from five k-steps on
-  // row_blocks_per_wave gives one block for all (every call comes here: 16 widths cost the host 0.5 us)
-  int splits = 1;
-  for (int ks = 1; ks <= 5; ++ks) {
-    const int s = row_splits(B, H, M, N, ks);
-    if (s > splits) splits = s;
-  }
+  // The most any row width asks for, so the size holds for every dtype and D.  Of one problem the widths differ
+  // only in the tile height, 128 or 256 rows: four k-steps take 256 where any width does (one block costs them
+  // the most), and the higher tile has the fewer workgroups, hence the most splits.  (Every call comes here.)
+  const int splits = row_splits(B, H, M, N, 4);
   const size_t rows = (size_t)B * (size_t)H * (size_t)M;
   return rows * sizeof(float) * (splits > 1 ? 1 + (size_t)splits : 1);
 }
@@ -3270,11 +3266,11 @@ void order_end(SweepOrder* o, hipStream_t s, bool launched_it) {
 }
 
 // Both sweeps of a call, writing `out` in its final form.  ws_bytes = bytes the caller's workspace is known
-// to have (0: what fcr_lse_bytes asks for).  One query takes the path of its own where the workspace has room for
+// to have (0: what fcr_lse_bytes asks for), lse_bytes = what fcr_lse_bytes gives (if ws_bytes is known).  One query takes the path of its own where the workspace has room for
 // its scores, few queries against many keys take the single sweep.
-int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, float* ws, size_t ws_bytes, int dtype,
-               int B, int H, int M, int N, int D, const int64_t q_strides[4], const int64_t k_strides[4], float scale,
-               int mode, int causal, void* stream, void* out2 = nullptr) {
+int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, float* ws, size_t ws_bytes,
+               size_t lse_bytes, int dtype, int B, int H, int M, int N, int D, const int64_t q_strides[4],
+               const int64_t k_strides[4], float scale, int mode, int causal, void* stream, void* out2 = nullptr) {
   Params p;
   int rc = make_params(p, q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, true, causal != 0, mode);
   if (rc) return rc;
@@ -3291,7 +3287,7 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
   }
   p.stream_once = ((int64_t)p.bh_count * N * p.dgran * 16 >= (1ll << 30)) ? 1 : 0;
   if (single && M == 1 && ws_bytes != 0) {   // (the mask hides nothing from the only query)
-    const OneQueryPlan o = one_query_plan(dtype, p.bh_count, N, D, (int64_t)(fcr_lse_bytes(B, H, M, N, D) / sizeof(float)));
+    const OneQueryPlan o = one_query_plan(dtype, p.bh_count, N, D, (int64_t)(lse_bytes / sizeof(float)));
     if ((size_t)o.floats * sizeof(float) <= ws_bytes) {
       p.lse = ws;
       p.sync = fused ? reinterpret_cast<unsigned*>(ws + f.sync_at) : nullptr;   // fcr_colreduce_status looks there
@@ -3328,7 +3324,7 @@ int fcr_colreduce_sum_max(const void* q, const void* k, float* out_sum, float* o
                           int H, int M, int N, int D, const int64_t q_strides[4], const int64_t k_strides[4],
                           float scale, int causal, void* stream) {
   if (!out_sum || !out_max || !lse_ws) return fail(FCR_E_NULL, "null pointer argument");
-  return whole_call(q, k, out_sum, ResultSpec(), lse_ws, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale, kModeBoth,
+  return whole_call(q, k, out_sum, ResultSpec(), lse_ws, 0, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale, kModeBoth,
                     causal, stream, out_max);
 }
 
@@ -3338,7 +3334,7 @@ int fcr_colreduce(const void* q, const void* k, float* out, float* lse_ws, int d
   if (!out || !lse_ws) return fail(FCR_E_NULL, "null pointer argument");
   if (reduction != FCR_REDUCE_SUM && reduction != FCR_REDUCE_MAX)
     return fail(FCR_E_REDUCTION, "reduction must be FCR_REDUCE_SUM or FCR_REDUCE_MAX");
-  return whole_call(q, k, out, ResultSpec(), lse_ws, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale,
+  return whole_call(q, k, out, ResultSpec(), lse_ws, 0, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale,
                     reduction == FCR_REDUCE_MAX ? kModeMax : kModeSum, causal, stream);
 }
 
@@ -3383,7 +3379,7 @@ int fcr_colreduce_to(const void* q, const void* k, void* out, int out_dtype, flo
   ResultSpec res;
   res.fmt = out_dtype;
   res.mean = reduction == FCR_REDUCE_MEAN;
-  return whole_call(q, k, out, res, lse_ws, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale,
+  return whole_call(q, k, out, res, lse_ws, 0, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale,
                     reduction == FCR_REDUCE_MAX ? kModeMax : kModeSum, causal, stream);
 }
 
@@ -3398,7 +3394,7 @@ int fcr_colreduce_sum_max_to(const void* q, const void* k, void* out_sum, void* 
   ResultSpec res;
   res.fmt = out_dtype;
   res.mean = sum_reduction == FCR_REDUCE_MEAN;
-  return whole_call(q, k, out_sum, res, lse_ws, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale, kModeBoth, causal,
+  return whole_call(q, k, out_sum, res, lse_ws, 0, 0, dtype, B, H, M, N, D, q_strides, k_strides, scale, kModeBoth, causal,
                     stream, out_max);
 }
 
@@ -3433,8 +3429,8 @@ int fcr_colreduce_ws(const void* q, const void* k, void* out, void* out_max, int
   res.fmt = out_dtype;
   res.mean = reduction == FCR_REDUCE_MEAN;
   const int mode = out_max ? kModeBoth : reduction == FCR_REDUCE_MAX ? kModeMax : kModeSum;
-  return whole_call(q, k, out, res, static_cast<float*>(ws), ws_bytes, dtype, B, H, M, N, D, q_strides, k_strides, scale,
-                    mode, causal, stream, out_max);
+  return whole_call(q, k, out, res, static_cast<float*>(ws), ws_bytes, need, dtype, B, H, M, N, D, q_strides, k_strides,
+                    scale, mode, causal, stream, out_max);
 }
 
 int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, int B, int H, int M, int N, int D,

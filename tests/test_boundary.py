@@ -46,6 +46,32 @@ def test_version_and_sizes():
     assert lib.fcr_lse_bytes(-1, 3, 5, 7, 8) == 0 and lib.fcr_lse_bytes(1, 3, 0, 7, 8) == 0
 
 
+def test_row_sweep_scratch_covers_every_row_width():
+    """fcr_lse_bytes does not know the row width: it is the most that any number of 64-byte steps of a row asks for
+    (the tile height, hence the number of key ranges, depends on it), restated here for 256 CUs and more than 128 queries."""
+    import random
+    lib = _lib.load()
+    if torch.cuda.is_available():
+        pytest.skip("the sizes are restated for the 256 CUs that the library assumes without a device")
+    rng = random.Random(5)
+
+    def swept(m, rows):
+        rem = m % rows
+        return m // rows * rows + min((rem + 31) // 32, 4) * (rows // 4)
+
+    def splits(bh, m, n, ksteps):
+        chunks, pairs2 = (n + 63) // 64, bh * ((m + 255) // 256)
+        one = (ksteps > 4 or swept(m, 128) * (100 + 3 * ksteps) < swept(m, 256) * 100 or
+               (pairs2 < 256 and n <= 1024) or 256 <= pairs2 < 512)
+        wgs = bh * ((m + (128 if one else 256) - 1) // (128 if one else 256))
+        return 1 if wgs >= 256 or chunks < 16 else max(1, min(512 // wgs, chunks // 4, 64))
+
+    for _ in range(3000):
+        b, h, m, n = rng.randint(1, 4), rng.randint(1, 40), int(2 ** rng.uniform(7.1, 13)), int(2 ** rng.uniform(6, 18))
+        most = max(splits(b * h, m, n, ks) for ks in range(1, 17))
+        assert lib.fcr_lse_bytes(b, h, m, n, 64) == 4 * b * h * m * (1 + most if most > 1 else 1), (b, h, m, n)
+
+
 def test_workspace_size_of_one_query():
     """One query asks for its scores and key ranges behind fcr_lse_bytes, for every row width the kernels take; for
     any other width (which the call then rejects) and for more queries it is fcr_lse_bytes."""
