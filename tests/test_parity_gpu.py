@@ -1102,6 +1102,28 @@ def test_topk_narrowing(n, dtype):
         assert (mask.cpu().numpy() == want).all(), (n, k, dtype)
 
 
+@pytest.mark.parametrize("n,c", [(1100, 127), (2048, 128), (2048, 129), (4666, 126), (8192, 130), (8193, 255), (20000, 256),
+                                 (32768, 257), (32768, 600)])
+def test_topk_bins_of_many_keys(n, c):
+    """A first bin that holds c keys, on both sides of the number that is ranked at once (128, or 256 in rows of more than
+    8192 columns), with the k-th largest at its top, inside it and at its end: c equal values, c values in
+    neighbouring floats, and both kinds in one bin.  Mask and threshold."""
+    from oracle.colreduce_oracle import topk_mask_ref
+    g = torch.Generator().manual_seed(n + c)
+    base = torch.linspace(2.0, 4.0, n).repeat(3, 1)       # neighbours 2^23 / n floats apart
+    at = n // 2
+    base[:, at: at + c] = 3.0
+    steps = torch.arange(c) * 2.0 ** -22                  # neighbouring floats; a bin takes 2^13 (up to 2048 columns 2^15)
+    base[1, at: at + c] += steps
+    base[2, at: at + c] += torch.where(torch.arange(c) < c // 2, torch.zeros(c), steps)
+    rows = base[:, torch.randperm(n, generator=g)].contiguous()
+    above = int((base[0] > 3.0).sum())
+    for k in (above - 1, above + 1, above + c // 2, above + c - 1, above + c + 1):
+        mask, thr = fca.topk_keep_mask(rows.cuda(), k, return_threshold=True)
+        assert (mask.cpu().numpy() == topk_mask_ref(rows.numpy(), k)).all(), (n, c, k)
+        assert torch.equal(thr.cpu(), rows.sort(dim=1, descending=True).values[:, k - 1]), (n, c, k)
+
+
 def test_topk_on_reduced_columns():
     from oracle.colreduce_oracle import topk_mask_ref
     q, k = _inputs.config4(heads=4, n=2048)
