@@ -1889,6 +1889,7 @@ __global__ __launch_bounds__(256, 8) void one_query_scores_kernel(const Params p
 template <int MODE>
 __global__ __launch_bounds__(256) void one_query_columns_kernel(const Params p, const float* __restrict__ scores,
                                                                 int64_t pitch) {
+  __shared__ float wave_m[4], wave_l[4];
   const int tid = threadIdx.x, lane = tid & 63;
   const int bh = (int)blockIdx.x / p.tiles, tile = (int)blockIdx.x - bh * p.tiles;
   const int col0 = tile * 256 * kOneCols + tid;
@@ -1898,8 +1899,22 @@ __global__ __launch_bounds__(256) void one_query_columns_kernel(const Params p, 
   for (int i = 0; i < kOneCols; ++i) a[i] = src[min(col0 + 256 * i, p.N - 1)];
   float m = kNegInf, l = 0.f;
   const float* part = p.part + 2 * (int64_t)bh * p.splits;
-  for (int s = lane; s < p.splits; s += 64) one_query_merge(m, l, part[2 * s], part[2 * s + 1]);
+  // Few pairs have many ranges each; the four waves then take a quarter of them instead of all: 2 x 262144 x 128 bf16
+  // 33.4 -> 26.7 us per call (single sweep 31.8), 1 x 10^6 x 128 79 -> 52.
+  const bool many = p.splits > 64;
+  for (int s = many ? tid : lane; s < p.splits; s += many ? 256 : 64) one_query_merge(m, l, part[2 * s], part[2 * s + 1]);
   one_query_merge_wave(m, l);
+  if (many) {
+    if (lane == 0) {
+      wave_m[tid >> 6] = m;
+      wave_l[tid >> 6] = l;
+    }
+    __syncthreads();
+    m = wave_m[0];
+    l = wave_l[0];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) one_query_merge(m, l, wave_m[w], wave_l[w]);
+  }
   if (tile == 0 && tid == 0) p.lse[bh] = m + fast_log2(l);
   if (blockIdx.x == 0 && tid == 0 && p.sync) *p.sync = 0u;
   const float ref = (m == kNegInf) ? 0.f : m, inv = 1.0f / l;   // no score above -inf: 0 * inf, NaN sums

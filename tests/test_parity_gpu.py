@@ -466,6 +466,48 @@ def test_one_query(b, h, n, d, dtype, causal):
         torch.testing.assert_close(other, one, rtol=2e-5, atol=1e-7)
 
 
+def _one_query_ref(q, k):
+    """softmax rows of one query per pair in float64, batch entry by batch entry on the device; and their base-2 statistics."""
+    p, stat = [], []
+    for b in range(q.shape[0]):
+        s = (q[b].double() * k[b].double()).sum(-1) / math.sqrt(q.shape[3])
+        p.append(torch.softmax(s, -1))
+        stat.append(torch.logsumexp(s, -1, keepdim=True) / math.log(2))
+    return torch.stack(p), torch.stack(stat)
+
+
+@pytest.mark.parametrize("b,h,n,d,dtype", [
+    (1, 1, 16384, 64, torch.float16),    # 64 key ranges: every wave of the second launch merges all of them
+    (1, 2, 16385, 64, torch.float16),    # 65: the waves share them, the last one holds one key
+    (1, 1, 65537, 64, torch.float16),    # 257: more than one per thread
+    (1, 1100, 1025, 256, torch.float32),   # more steps than there is room for: ranges of two steps, the last one of one key
+    (8, 150, 833, 256, torch.float32),     # the same, every range whole but the last
+    (32, 1024, 70, 512, torch.float16),    # one range of three steps, the last one partial (keys shared by the batch)
+])
+def test_one_query_ranges(b, h, n, d, dtype):
+    """One query whose keys are cut into as many ranges as the merge treats differently, or into ranges of several steps
+    of a workgroup: scores that grow along the keys, so that the running maximum changes in every step."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q = torch.randn(b, h, 1, d, device="cuda", generator=g)
+    k = torch.randn(1 if n == 70 else b, h, n, d, device="cuda", generator=g)
+    k += q[:k.shape[0]] * torch.linspace(0, 8.0 / math.sqrt(d), n, device="cuda").view(1, 1, n, 1)
+    q, k = q.to(dtype), k.to(dtype).expand(b, h, n, d)
+    want, stat = _one_query_ref(q, k)
+    s, m = fca.flash_colreduce_multi(q, k, ["sum", "max"], is_causal=True, out_dtype=torch.float32)
+    for got in (s, m, fca.flash_colreduce(q, k, "sum", out_dtype=torch.float32)):
+        # products of up to 150 in base 2, 2^-24 per addition, eight or sixteen lanes' partial sums: below 1e-4 of a probability
+        torch.testing.assert_close(got.double(), want, rtol=1e-4, atol=1e-30)
+    from flash_colreduce_amd import _lib
+    from flash_colreduce_amd.flash import _DTYPES as DT
+    lib = _lib.load()
+    nbytes = lib.fcr_workspace_bytes(DT[dtype], b, h, 1, n, d)
+    ws, out = torch.full((nbytes // 4,), float("nan"), device="cuda"), torch.empty(b, h, n, device="cuda")
+    _lib.check(lib.fcr_colreduce_ws(q.data_ptr(), k.data_ptr(), out.data_ptr(), None, _lib.DTYPE_F32, ws.data_ptr(), nbytes,
+                                    DT[dtype], b, h, 1, n, d, _lib.strides4(q.stride()), _lib.strides4(k.stride()), d ** -0.5,
+                                    _lib.REDUCE_SUM, 1, torch.cuda.current_stream().cuda_stream))
+    torch.testing.assert_close(ws[: b * h].view(b, h, 1).double(), stat, rtol=0, atol=1e-4)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_one_query_non_finite(dtype):
     """One query: a NaN or +inf score makes the sums of its row NaN and its maxima 0, -inf scores count nothing (a row
