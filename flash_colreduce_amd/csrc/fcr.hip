@@ -1820,8 +1820,10 @@ __device__ __forceinline__ void granule_floats(u32x4 v, float (&f)[DT == FCR_DTY
   }
 }
 
-// Workgroup v takes keys [split * rows_wg, + rows_wg) of pair v / p.splits, split = v % p.splits.  scores: [BH, pitch].
-template <int DT, int LPR>
+// A workgroup takes keys [split * rows_wg, + rows_wg) of one pair, all ranges of a pair in a row, or with p.group > 1
+// the same range of all p.group = B batch entries of a head in a row.  scores: [BH, pitch].  ONCE: no other pair reads
+// these keys (both: see launch_one_query).
+template <int DT, int LPR, bool ONCE>
 __global__ __launch_bounds__(256, 8) void one_query_scores_kernel(const Params p, float* __restrict__ scores,
                                                                int64_t pitch, int rows_wg) {
   constexpr int E = DT == FCR_DTYPE_F32 ? 4 : 8;
@@ -1831,7 +1833,9 @@ __global__ __launch_bounds__(256, 8) void one_query_scores_kernel(const Params p
   __shared__ float wave_m[4], wave_l[4];
   const int lane = threadIdx.x & 63, g = lane & (LPR - 1), r0 = lane / LPR;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int bh = (int)blockIdx.x / p.splits, split = (int)blockIdx.x - bh * p.splits;
+  const int turn = (int)blockIdx.x / p.group, member = (int)blockIdx.x - turn * p.group;
+  const int pair = turn / p.splits, split = turn - pair * p.splits;
+  const int bh = p.group > 1 ? member * p.H + pair : pair;
   const int b = bh / p.H, h = bh - b * p.H;
   const char* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh + (int64_t)g * 16;
   const char* qb = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)g * 16;
@@ -1848,7 +1852,10 @@ __global__ __launch_bounds__(256, 8) void one_query_scores_kernel(const Params p
     for (int u = 0; u < kOneLoads; ++u) {
       const u32x4* src = reinterpret_cast<const u32x4*>(kb + (int64_t)min(row + u * kRows + r0, p.N - 1) * p.k_sr);
       v[u] = zero;
-      if (live) v[u] = __builtin_nontemporal_load(src);   // no one else reads this row
+      if (live) {
+        if constexpr (ONCE) v[u] = __builtin_nontemporal_load(src);
+        else v[u] = *src;
+      }
     }
     float done[kSel];
 #pragma unroll
@@ -1880,8 +1887,9 @@ __global__ __launch_bounds__(256, 8) void one_query_scores_kernel(const Params p
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int w = 1; w < 4; ++w) one_query_merge(m, l, wave_m[w], wave_l[w]);
-    p.part[2 * (int64_t)blockIdx.x] = m;
-    p.part[2 * (int64_t)blockIdx.x + 1] = l;
+    float* part = p.part + 2 * ((int64_t)bh * p.splits + split);
+    part[0] = m;
+    part[1] = l;
   }
 }
 
@@ -2986,18 +2994,23 @@ void launch_sweeps(int dtype, int which, const Params& p, int ksteps, bool causa
   else (long_rows ? fcr_detail::sweeps_f32_long_rows : fcr_detail::sweeps_f32)(which, p, ksteps, causal, mode, s);
 }
 
-template <int DT>
+template <int DT, bool ONCE>
 void launch_one_query_scores(const Params& p, const OneQueryPlan& o, float* scores, hipStream_t s) {
   const dim3 grid((unsigned)p.total), block(256);
   switch (o.lanes) {
-    case 1: hipLaunchKernelGGL((one_query_scores_kernel<DT, 1>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
-    case 2: hipLaunchKernelGGL((one_query_scores_kernel<DT, 2>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
-    case 4: hipLaunchKernelGGL((one_query_scores_kernel<DT, 4>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
-    case 8: hipLaunchKernelGGL((one_query_scores_kernel<DT, 8>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
-    case 16: hipLaunchKernelGGL((one_query_scores_kernel<DT, 16>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
-    case 32: hipLaunchKernelGGL((one_query_scores_kernel<DT, 32>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
-    default: hipLaunchKernelGGL((one_query_scores_kernel<DT, 64>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 1: hipLaunchKernelGGL((one_query_scores_kernel<DT, 1, ONCE>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 2: hipLaunchKernelGGL((one_query_scores_kernel<DT, 2, ONCE>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 4: hipLaunchKernelGGL((one_query_scores_kernel<DT, 4, ONCE>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 8: hipLaunchKernelGGL((one_query_scores_kernel<DT, 8, ONCE>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 16: hipLaunchKernelGGL((one_query_scores_kernel<DT, 16, ONCE>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    case 32: hipLaunchKernelGGL((one_query_scores_kernel<DT, 32, ONCE>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
+    default: hipLaunchKernelGGL((one_query_scores_kernel<DT, 64, ONCE>), grid, block, 0, s, p, scores, o.pitch, o.rows_wg); break;
   }
+}
+template <int DT>
+void launch_one_query_scores(bool once, const Params& p, const OneQueryPlan& o, float* scores, hipStream_t s) {
+  if (once) launch_one_query_scores<DT, true>(p, o, scores, s);
+  else launch_one_query_scores<DT, false>(p, o, scores, s);
 }
 
 int launch_one_query(Params& p, int dtype, const OneQueryPlan& o, float* ws, int mode, hipStream_t s) {
@@ -3005,9 +3018,20 @@ int launch_one_query(Params& p, int dtype, const OneQueryPlan& o, float* ws, int
   p.part = ws + o.part_at;
   p.splits = o.splits;
   p.total = (int)(p.bh_count * (int64_t)o.splits);
-  if (dtype == FCR_DTYPE_F16) launch_one_query_scores<FCR_DTYPE_F16>(p, o, scores, s);
-  else if (dtype == FCR_DTYPE_BF16) launch_one_query_scores<FCR_DTYPE_BF16>(p, o, scores, s);
-  else launch_one_query_scores<FCR_DTYPE_F32>(p, o, scores, s);
+  // Keys that pairs share by a stride of zero.  The heads of a batch entry follow each other and meet in the caches: no
+  // non-temporal loads (8 x 32 x 9001 x 128 bf16 81 -> 56 us, fp32 164 -> 89).  Batch entries are all heads apart.  What the
+  // eight L2s hold together still meets there (16 x 32 x 4096 bf16 63 -> 48, 64 x 8 x 16384 284 -> 138).  More than
+  // that goes range by range through the whole batch, if it has a workgroup for every XCD (16 x 32 x 6000 bf16 113 -> 70,
+  // fp32 236 -> 114; within the L2s the plain order is faster: 16 x 32 x 4096 x 64 bf16 26 against 32; 4 x 32 x 6000 bf16
+  // 27 plain and non-temporal, 35 in this order).
+  const int batch = p.bh_count / p.H;
+  const bool by_heads = p.H > 1 && p.k_sh == 0, by_batch = !by_heads && batch > 1 && p.k_sb == 0;
+  const bool fits = (int64_t)p.H * p.N * p.dgran * 16 <= (32ll << 20), beside = by_batch && !fits && batch >= 8;
+  const bool once = !by_heads && !beside && !(by_batch && fits);
+  p.group = beside ? batch : 1;
+  if (dtype == FCR_DTYPE_F16) launch_one_query_scores<FCR_DTYPE_F16>(once, p, o, scores, s);
+  else if (dtype == FCR_DTYPE_BF16) launch_one_query_scores<FCR_DTYPE_BF16>(once, p, o, scores, s);
+  else launch_one_query_scores<FCR_DTYPE_F32>(once, p, o, scores, s);
   int rc = launched("one_query_scores_kernel");
   if (rc) return rc;
   p.tiles = (p.N + 256 * kOneCols - 1) / (256 * kOneCols);

@@ -508,6 +508,28 @@ def test_one_query_ranges(b, h, n, d, dtype):
     torch.testing.assert_close(ws[: b * h].view(b, h, 1).double(), stat, rtol=0, atol=1e-4)
 
 
+@pytest.mark.parametrize("shared", ["batch", "heads", "both"])
+@pytest.mark.parametrize("b,h,n,d,dtype", [
+    (3, 5, 1025, 72, torch.bfloat16), (2, 2, 777, 256, torch.float32), (8, 1, 300, 64, torch.float16),
+    (7, 8, 16500, 128, torch.bfloat16),   # more keys than the L2s hold, fewer batch entries than XCDs
+    (8, 8, 16384, 128, torch.bfloat16),   # as many as the L2s hold
+    (8, 8, 16385, 128, torch.bfloat16), (11, 3, 30011, 256, torch.float16), (9, 8, 9001, 128, torch.float32),   # more
+])
+def test_one_query_shared_keys(b, h, n, d, dtype, shared):
+    """One query against keys that the batch, the heads or both share by a stride of zero: whatever the order of the
+    workgroups and the way the keys are loaded, the bits of the same keys held once per pair."""
+    g = torch.Generator(device="cuda").manual_seed(n + d)
+    q = torch.randn(b, h, 1, d, device="cuda", generator=g, dtype=dtype)
+    k = torch.randn(1 if shared != "heads" else b, 1 if shared != "batch" else h, n, d, device="cuda", generator=g, dtype=dtype)
+    k = k.expand(b, h, n, d)
+    whole = k.contiguous()
+    for red in REDUCTIONS:
+        got = fca.flash_colreduce(q, k, red, is_causal=True, out_dtype=torch.float32)
+        assert torch.equal(got, fca.flash_colreduce(q, whole, red, is_causal=True, out_dtype=torch.float32)), red
+    p = torch.softmax((q[-1].double() * whole[-1].double()).sum(-1) / math.sqrt(d), -1)
+    check(fca.flash_colreduce(q, k, "sum", out_dtype=torch.float32)[-1], p.cpu(), "sum", f"shared by {shared}")
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_one_query_non_finite(dtype):
     """One query: a NaN or +inf score makes the sums of its row NaN and its maxima 0, -inf scores count nothing (a row
