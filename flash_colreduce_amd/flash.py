@@ -99,6 +99,13 @@ def _ws_floats(dev_index: int, dtype: int, b: int, h: int, m: int, n: int, d: in
         return max(b * h * m, _lib.load().fcr_workspace_bytes(dtype, b, h, m, n, d) // 4)
 
 
+@functools.lru_cache(maxsize=4096)
+def _lse_floats(dev_index: int, b: int, h: int, m: int, n: int, d: int) -> int:
+    """Floats of the buffer of fcr_row_lse: the row statistics and that sweep's scratch, no room for one query's scores."""
+    with torch.cuda.device(dev_index):
+        return max(b * h * m, _lib.load().fcr_lse_bytes(b, h, m, n, d) // 4)
+
+
 def _raw_stream(dev: torch.device) -> int:
     """The current stream of `dev` as a hipStream_t value."""
     try:
@@ -173,7 +180,7 @@ def _launch(query, key, kinds, is_causal, scale):
     # the row statistics, followed by whatever scratch the row kernel wants for this shape
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     dtype = _DTYPES[q.dtype]
-    floats = _ws_floats(index, dtype, b, h, m, n, q.shape[3])
+    floats = _ws_floats(index, dtype, b, h, m, n, q.shape[3]) if kinds else _lse_floats(index, b, h, m, n, q.shape[3])
     lse = torch.empty(floats, device=dev, dtype=torch.float32)
     outs = [torch.empty((b * h, n), device=dev, dtype=torch.float32) for _ in kinds]
     if b * h * m * n == 0:

@@ -530,6 +530,18 @@ def test_one_query_shared_keys(b, h, n, d, dtype, shared):
     check(fca.flash_colreduce(q, k, "sum", out_dtype=torch.float32)[-1], p.cpu(), "sum", f"shared by {shared}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_row_lse2_of_one_query_keeps_no_score_array(dtype):
+    """The row statistics are a view of the row sweep's buffer, which has no room for the scores that one query's
+    column reduction keeps: 4 bytes per key would live as long as the (B, H, 1) result."""
+    from flash_colreduce_amd import _lib
+    b, h, n, d = 2, 3, 40000, 64
+    q, k = _inputs.randn_pair(b, h, 1, n, d, seed=8, dtype=dtype)
+    lse = fca.row_lse2(q.cuda(), k.cuda())
+    torch.testing.assert_close(lse.double().cpu(), row_lse2_ref(q, k), rtol=0, atol=3e-4)
+    assert lse.untyped_storage().nbytes() == _lib.load().fcr_lse_bytes(b, h, 1, n, d) < 4 * b * h * n
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_one_query_non_finite(dtype):
     """One query: a NaN or +inf score makes the sums of its row NaN and its maxima 0, -inf scores count nothing (a row
