@@ -326,6 +326,19 @@ def test_fp32_tiles_of_64_rows(b, h, m, n, d, causal):
     check(mx.cpu(), colreduce_ref(q, k, "max", causal), "max", "fp32 pair")
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(2, 256, 256, 64), (3, 65, 63, 72), (4, 191, 960, 128), (1, 700, 333, 256)])
+def test_fp32_tiles_of_64_rows_give_the_bits_of_taller_ones(h, m, n, d, causal):
+    """The same heads alone (64-row tiles) and among as many copies as fill the chip (128 rows or more): each row and each
+    column is added up in the same order whatever the tile."""
+    q, k = (x.cuda() for x in _inputs.randn_pair(1, h, m, n, d, seed=m + n, dtype=torch.float32))
+    copies = 512 // h
+    qs, ks = q.repeat(copies, 1, 1, 1), k.repeat(copies, 1, 1, 1)
+    assert torch.equal(fca.row_lse2(q, k, causal)[0], fca.row_lse2(qs, ks, causal)[-1])
+    for red in REDUCTIONS:
+        assert torch.equal(fca.flash_colreduce(q, k, red, causal)[0], fca.flash_colreduce(qs, ks, red, causal)[-1]), red
+
+
 @pytest.mark.parametrize("m", [100, 128, 300, 384, 600])
 def test_row_sweep_block_choice(m):
     """Query counts for which the row sweep keeps one 32-row block per wave (M <= 128 and ragged M
@@ -481,7 +494,7 @@ def _one_query_ref(q, k):
     (1, 2, 16385, 64, torch.float16),    # 65: the waves share them, the last one holds one key
     (1, 1, 65537, 64, torch.float16),    # 257: more than one per thread
     (1, 1100, 1025, 256, torch.float32),   # more steps than there is room for: ranges of two steps, the last one of one key
-    (8, 150, 833, 256, torch.float32),     # the same, every range whole but the last
+    (8, 150, 1000, 256, torch.float32),    # the same, the last range of two steps as well, its second one partial
     (32, 1024, 70, 512, torch.float16),    # one range of three steps, the last one partial (keys shared by the batch)
 ])
 def test_one_query_ranges(b, h, n, d, dtype):
@@ -540,6 +553,34 @@ def test_row_lse2_of_one_query_keeps_no_score_array(dtype):
     lse = fca.row_lse2(q.cuda(), k.cuda())
     torch.testing.assert_close(lse.double().cpu(), row_lse2_ref(q, k), rtol=0, atol=3e-4)
     assert lse.untyped_storage().nbytes() == _lib.load().fcr_lse_bytes(b, h, 1, n, d) < 4 * b * h * n
+
+
+def test_one_query_under_graph_capture():
+    """One query recorded into a HIP graph: every replay on new inputs, with eager calls between them, gives the eager bits."""
+    b, h, n, d = 3, 5, 5003, 128
+    q0, k0 = _inputs.randn_pair(b, h, 1, n, d, seed=40, dtype=torch.bfloat16)
+    qs, ks = q0.cuda(), k0.cuda()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        fca.flash_colreduce_multi(qs, ks, ["mean", "max"], True)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fca.flash_colreduce_multi(qs, ks, ["mean", "max"], True)
+    for seed in (41, 42, 43):
+        q1, k1 = _inputs.randn_pair(b, h, 1, n, d, seed=seed, dtype=torch.bfloat16)
+        qs.copy_(q1)
+        ks.copy_(k1)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [x.clone() for x in out]
+        eager = fca.flash_colreduce_multi(qs, ks, ["mean", "max"], True)
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, eager)), seed
+        # the result is rounded to bf16: half a unit of 2^-8
+        torch.testing.assert_close(got[1].float().cpu(), colreduce_ref(q1, k1, "max", True).float(), rtol=2.0 ** -8, atol=1e-7)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
@@ -1176,6 +1217,8 @@ def test_topk_narrowing(n, dtype):
         mask, thr = fca.topk_keep_mask(dev, k, return_threshold=True)
         want = topk_mask_ref(r.float().numpy(), k)
         assert (mask.cpu().numpy() == want).all(), (n, k, dtype)
+        torch.testing.assert_close(thr.cpu(), r.float().sort(dim=1, descending=True).values[:, k - 1], rtol=0, atol=0,
+                                   equal_nan=True)   # (a NaN sorts above +inf)
 
 
 @pytest.mark.parametrize("n,c", [(1100, 127), (2048, 128), (2048, 129), (4666, 126), (8192, 130), (8193, 255), (20000, 256),
