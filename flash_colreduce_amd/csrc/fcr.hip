@@ -2062,8 +2062,9 @@ __global__ __launch_bounds__(T) void topk_mask_kernel(const ET* __restrict__ sco
   // Keys that are ranked against each other, one per thread.  Ranking takes time with the square of their number, one more
   // count with VPT; rows of which one value fills the bin need no more than its minimum and maximum.  With 512 for
   // both -> now (search bit by bit), 500 equal values around the k-th: 812 rows of 4666 fp32 61 -> 21 us (42), 32 of 4666
-  // 17.2 -> 11.2 (15.3), 1024 of 8192 65 -> 24 (43), 1024 of 32768 117 -> 74 (155); bins below the limits are as before, spread
-  // scores of every type never reach them.
+  // 17.2 -> 11.2 (15.3), 1024 of 8192 65 -> 24 (43), 1024 of 32768 117 -> 74 (155).  exp(N(0, 1)) scores of every type never reach
+  // the limits; uniform ones with one near zero do: 512 rows of 16384 48 -> 36.  Just above them the count is the dearer way:
+  // 200 equal values in 1024 rows of 32768 88 -> 95.
   constexpr int kGather = VPT > 8 ? 256 : 128;
   static_assert(VPT % W == 0, "whole vectors");
   __shared__ __attribute__((aligned(16))) uint32_t hist[kBins];

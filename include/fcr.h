@@ -54,7 +54,7 @@ extern "C" {
 /* column reduction over query rows */
 #define FCR_REDUCE_SUM 0 /* also the numerator of 'mean' (flash.py:121-122) */
 #define FCR_REDUCE_MAX 1 /* flash.py:123-124 */
-#define FCR_REDUCE_MEAN 2 /* fcr_colreduce_to and fcr_colreduce_sum_max_to only: the sums divided as in flash.py:377-384 */
+#define FCR_REDUCE_MEAN 2 /* fcr_colreduce_to, _sum_max_to and _ws only: the sums divided as in flash.py:377-384 */
 
 /* argument errors */
 #define FCR_E_NULL -1      /* a required pointer is NULL */
@@ -195,14 +195,24 @@ int fcr_colreduce_to(const void* q, const void* k, void* out, int out_dtype, flo
  * fcr_colreduce_sum_max_to (out_max given; reduction then names what `out` holds, sum or mean) compute, and with
  * fcr_workspace_bytes(dtype, B, H, M, N, D) bytes by the fastest path for the problem: one query is read
  * once, without the matrix instructions, and its scores wait in the workspace (4 bytes per key) for their row's
- * sum.  With less, but at least fcr_lse_bytes, the call takes the path of the entry points above
- * (FCR_E_SCRATCH below that); results agree to rounding either way.  ws must be 16-byte aligned, its first
+ * sum (64 sequences of 32 heads and 65536 keys: 0.5 GB).  With less, but at least fcr_lse_bytes, the call takes the
+ * path of the entry points above (FCR_E_SCRATCH below that); results agree to rounding either way.  ws must be 16-byte aligned, its first
  * B*H*M floats hold the row statistics on return, its contents before the call are irrelevant.
  */
 size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D);
 int fcr_colreduce_ws(const void* q, const void* k, void* out, void* out_max, int out_dtype, void* ws, size_t ws_bytes,
                      int dtype, int B, int H, int M, int N, int D, const int64_t q_strides[4],
                      const int64_t k_strides[4], float scale, int reduction, int causal, void* stream);
+
+/*
+ * fcr_colreduce_sum_max with the tail of the reference's wrapper, as fcr_colreduce_to has it: both results
+ * leave the kernel as [B*H, N] of out_dtype, and with sum_reduction = FCR_REDUCE_MEAN (else FCR_REDUCE_SUM)
+ * the sums are divided as in flash.py:377-384.  Stands for two calls of flash_colreduce, 'sum' or 'mean' and
+ * 'max' (flash.py:311-385), bit for bit what those give up to the order of the fp32 additions.
+ */
+int fcr_colreduce_sum_max_to(const void* q, const void* k, void* out_sum, void* out_max, int out_dtype, float* lse_ws,
+                             int dtype, int B, int H, int M, int N, int D, const int64_t q_strides[4],
+                             const int64_t k_strides[4], float scale, int sum_reduction, int causal, void* stream);
 
 /*
  * fcr_colreduce without the lse_ws argument, for callers that cannot allocate device memory (code under
@@ -217,23 +227,14 @@ int fcr_colreduce_ws(const void* q, const void* k, void* out, void* out_max, int
  * a device asks the runtime for the buffer's address and should be made outside graph capture.
  * Results are bitwise those of fcr_colreduce.
  */
-/*
- * fcr_colreduce_sum_max with the tail of the reference's wrapper, as fcr_colreduce_to has it: both results
- * leave the kernel as [B*H, N] of out_dtype, and with sum_reduction = FCR_REDUCE_MEAN (else FCR_REDUCE_SUM)
- * the sums are divided as in flash.py:377-384.  Stands for two calls of flash_colreduce, 'sum' or 'mean' and
- * 'max' (flash.py:311-385), bit for bit what those give up to the order of the fp32 additions.
- */
-int fcr_colreduce_sum_max_to(const void* q, const void* k, void* out_sum, void* out_max, int out_dtype, float* lse_ws,
-                             int dtype, int B, int H, int M, int N, int D, const int64_t q_strides[4],
-                             const int64_t k_strides[4], float scale, int sum_reduction, int causal, void* stream);
-
 int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, int B, int H, int M, int N,
                          int D, const int64_t q_strides[4], const int64_t k_strides[4], float scale,
                          int reduction, int causal, void* stream);
 
 /*
  * Few queries against many keys (M <= 128, N >= 1024, 16-bit elements, rows of at most 256 bytes): the calls
- * that run both kernels (fcr_colreduce, fcr_colreduce_to, fcr_colreduce_static) then take ONE sweep that
+ * that run both kernels (fcr_colreduce, fcr_colreduce_to, their _sum_max siblings, fcr_colreduce_static and
+ * fcr_colreduce_ws, this one not for one query with the larger workspace) then take ONE sweep that
  * reads the keys once, where the reference's kernel reads them twice (flash.py:209-274).  Its workgroups
  * share a (b,h) pair and meet on counters in the workspace; a workgroup whose partners do not arrive
  * within FCR_OPT_WAIT_POLLS polls (only possible when the GPU cannot run the whole launch at once, e.g.
