@@ -1,6 +1,6 @@
 // libfcr: column reduction of softmax attention for MI355X (gfx950, CDNA4).
 //
-// Two sweeps, both built on v_mfma_f32_16x16x32_{f16,bf16} (fp32 operands: v_mfma_f32_16x16x4_f32) with
+// Two sweeps, both built on v_mfma_f32_16x16x32_{f16,bf16} (fp32 operands as two fp16 parts each) with
 // the product taken as S^T = K * Q^T (keys are MFMA rows, queries are MFMA columns).  In a 16x16
 // accumulator a lane owns ONE query (lane & 15) and 4 keys (row 4*(lane/16) + r for register r), so
 //   - everything that is per query row (softmax reference exponent, running sum, lse) is one
@@ -17,6 +17,7 @@
 //                     LDS; writes lse2[bh, i] = log2 sum_j 2^(s_ij).
 //   col_reduce_kernel a workgroup keeps 256 key rows in registers and streams query tiles (and
 //                     their lse2) through LDS; writes out[bh, j] = sum_i or max_i 2^(s_ij-lse2_i).
+//   row_lse_f32_kernel, col_reduce_f32_kernel   the same for fp32 operands, whose rows are split on the way to LDS.
 //   col_small_kernel  the same result for at most 128 query rows against many keys: queries resident
 //                     in every wave, keys streamed (HBM bound).
 //   col_fused_kernel  both sweeps in one for at most 128 query rows against many 16-bit keys: the scores of
@@ -154,16 +155,41 @@ inline int row_blocks_per_wave(int ksteps, int M, int N, int64_t bh, bool causal
   if (wgs2 < cus && N <= 1024) return 1;
   return (wgs2 >= cus && wgs2 < 2 * cus + (causal ? 1 : 0)) ? 1 : 2;
 }
-// fp32 operands that give at most one workgroup of 128 rows on every other CU: tiles of 64 rows, one 16-row group
-// per wave (NB = 0).  Such a launch lasts as long as one workgroup, whose sweep is all fp32 matrix instructions
-// (32 cycles per 16x16x4 and SIMD), and half the resident rows halve it.  With more workgroups than that the
-// halves only share the CUs.  16-bit operands spend their short sweeps on latency instead.  A row sweep of 16 chunks
-// or more is split over the idle CUs (row_splits) and keeps its tile.  Per call: 2 heads of 256 x 256 x 64 24.3 -> 18.6 us,
-// 32 of 512 x 512 x 128 72 -> 42, 16 of 900 x 900 x 64 70 -> 41, 16 of 1024 x 1024 x 256 212 -> 151, 8 of 2048 x 2048 x 128
-// 199 -> 141, 2 of 8192 x 8192 x 128 757 -> 527; just above the rule (32 heads of 1024 x 1024 x 128) 137 either way.
-inline bool half_tiles(bool f32, int64_t rows, int64_t bh) { return f32 && 2 * bh * ((rows + 127) / 128) <= chip_cus(); }
-inline bool row_half_tiles(bool f32, int M, int N, int64_t bh) { return N <= 15 * 64 && half_tiles(f32, M, bh); }
-inline int row_tile_rows(int ksteps, int M, int N, int64_t bh, bool causal) {
+// Tiles of the fp32 sweeps (row_lse_f32_kernel, col_reduce_f32_kernel): waves per workgroup (four: two workgroups share a
+// CU; eight: one) and resident 16-row groups per wave.  Two groups read a streamed fragment once for two blocks of scores,
+// eight waves share the split of a streamed row: 4 x 2 and 8 x 1 are 128 rows, 8 x 2 256, 4 x 1 64.  Per call, fp32:
+//   32 heads of 4096 x 4096 x 128   8x2 733 us, 4x2 828, 8x1 927      2 x 16 of 2048 x 2048 x 128 causal   4x2 141, 8x2 164, 8x1 160
+//   32 of 1024 x 1024 x 128         8x1 70, 4x2 75, 4x1 85, 8x2 86    32 of 3000 x 3000 x 128 causal       8x2 247, 4x2 255, 8x1 291
+//   16 of 1500 x 1500 x 96 causal   8x1 63, 4x1 76, 4x2 81, 8x2 89    32 of 512 x 512 x 128                4x1 32, 8x1 36, 4x2 40, 8x2 52
+// So: 256 rows where 128-row tiles are more than one per CU (with the mask, which wants some to level it, two), 8 x 1
+// where they are at most one, and 64 rows for short sweeps that leave every other CU without a workgroup.
+struct F32Tile {
+  int waves, groups;
+  int rows() const { return 16 * waves * groups; }
+};
+inline F32Tile f32_tile(int rows, int64_t bh, bool causal, bool short_sweep) {
+  const int64_t tiles = bh * ((rows + 127) / 128);   // of 128 rows
+  const int cus = chip_cus();
+  if (rows <= 64 || (short_sweep && 2 * tiles <= cus)) return F32Tile{4, 1};
+  if (tiles <= cus) return F32Tile{8, 1};
+  return !causal || tiles > 2 * cus ? F32Tile{8, 2} : F32Tile{4, 2};
+}
+// Sums and maxima of rows of D > 192 have no registers for two groups.  A sweep of at most 128 queries is all
+// prologue and takes four waves (32 heads of 64 x 8192 x 128 causal 66 us, with 8x2 tiles 73).
+inline F32Tile f32_col_tile(int ksteps, bool both, int M, int N, int64_t bh, bool causal) {
+  F32Tile t = f32_tile(N, bh, causal, M <= 512);
+  if (both && ksteps > 6 && t.groups == 2 && bh * ((N + 127) / 128) < (1ll << 22)) return F32Tile{8, 1};
+  if (M <= 128 && t.waves == 8) return F32Tile{4, 2};
+  return t;
+}
+// A row sweep of 16 chunks or more over fewer tiles than CUs is split over the idle CUs (row_splits), two workgroups each.
+inline F32Tile f32_row_tile(int M, int N, int64_t bh, bool causal) {
+  const F32Tile t = f32_tile(M, bh, causal, N <= 15 * 64);
+  return t.waves == 8 && t.groups == 1 && N > 15 * 64 && bh * ((M + 127) / 128) < chip_cus() ? F32Tile{4, 2} : t;
+}
+inline int f32_ksteps(int ksteps) { return (ksteps + 1) / 2; }   // k-steps of 32 d from k-steps of 64 bytes
+inline int row_tile_rows(bool f32, int ksteps, int M, int N, int64_t bh, bool causal) {
+  if (f32) return f32_row_tile(M, N, bh, causal).rows();
   return kWaves * 32 * row_blocks_per_wave(ksteps, M, N, bh, causal);
 }
 constexpr int kMaxKSteps = 8;                 // rows of up to 512 bytes: two workgroups per CU
@@ -223,7 +249,7 @@ __device__ __forceinline__ void map_group(const Params& p, int per_bh, int& bh, 
 // second workgroup of a CU is as many ranks behind the first as the chip has CUs, so the CU with the longest
 // sweep also gets the longest of the second helping.  The second helping is dealt shortest first instead,
 // and the two sweeps of every CU add up to about the same length (32 heads of 2048 x 2048 fp16: 51.4 -> 48.1 us
-// per call, 4096 x 4096: 156 -> 152, 2 x 16 heads of 2048 x 2048 x 256 bf16: 83 -> 79, fp32 D = 128: 379 -> 280).  Launches of more
+// per call, 4096 x 4096: 156 -> 152, 2 x 16 heads of 2048 x 2048 x 256 bf16: 83 -> 79).  Launches of more
 // workgroups than that fill in behind each other in any case and lose by it (40 heads of 5000: 211 -> 246 us).
 __device__ __forceinline__ int second_helping(const Params& p, int rank) {
   return (p.fill > 0 && rank >= p.fill) ? p.tiles - 1 - (rank - p.fill) : rank;
@@ -254,12 +280,9 @@ __device__ __forceinline__ void map_block_split(const Params& p, bool longest_is
 // block b has b+1 (rows) or 8-b (columns) visible sub-tiles out of 8, so every wave gets 9 of the 36
 // and the four waves reach each barrier together.  With one block per wave, wave w keeps block w
 // of four.
-// With NB = 0 a wave keeps one group, w of four.
-__host__ __device__ constexpr int wave_group_count(int nb) { return nb ? 2 * nb : 1; }
 template <int NB>
-__device__ __forceinline__ void wave_groups(int tile, int wave, int (&rows)[wave_group_count(NB)]) {
-  const int t0 = tile * (kWaves * 16 * wave_group_count(NB));
-  if constexpr (NB == 0) rows[0] = t0 + 16 * wave;
+__device__ __forceinline__ void wave_groups(int tile, int wave, int (&rows)[2 * NB]) {
+  const int t0 = tile * (kWaves * 32 * NB);
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     // blocks w, 7-w (, 8+w, 15-w): even positions count up, odd ones count down inside a run of eight
@@ -558,12 +581,12 @@ __device__ __forceinline__ void pipelined_sweep(int ta, int tb, const u32x4 (&re
 // caught by the range check.
 // a[sg][r] is the score of the lane's query against key 16*sg + 4*(lane/16) + r of the sub-step;
 // with MASK, keys whose offset 16*sg + r exceeds lim (already reduced by 4*(lane/16)) are hidden.
-template <bool MASK>
-__device__ __forceinline__ float lse_fast(const f32x4 (&a)[2], float scale2, float mref, float l, int lim) {
+template <bool MASK, int SG>
+__device__ __forceinline__ float lse_fast(const f32x4 (&a)[SG], float scale2, float mref, float l, int lim) {
   const float nm = -mref;
   float ln = l;  // one add per score and nothing else: the groups of a wave give the adder its parallelism
 #pragma unroll
-  for (int sg = 0; sg < 2; ++sg)
+  for (int sg = 0; sg < SG; ++sg)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float x = fmaf(a[sg][r], scale2, nm);
@@ -575,12 +598,12 @@ __device__ __forceinline__ float lse_fast(const f32x4 (&a)[2], float scale2, flo
 
 __device__ __forceinline__ bool lse_in_range(float l) { return (l >= 1.0f) && (l < 1.8446744e19f); }
 
-template <bool MASK>
-__device__ __forceinline__ void lse_renorm(const f32x4 (&a)[2], float scale2, float& mref, float& l, int lim) {
+template <bool MASK, int SG>
+__device__ __forceinline__ void lse_renorm(const f32x4 (&a)[SG], float scale2, float& mref, float& l, int lim) {
   const float nm = -mref;
-  float t[8];
+  float t[4 * SG];
 #pragma unroll
-  for (int sg = 0; sg < 2; ++sg)
+  for (int sg = 0; sg < SG; ++sg)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float x = fmaf(a[sg][r], scale2, nm);
@@ -589,20 +612,20 @@ __device__ __forceinline__ void lse_renorm(const f32x4 (&a)[2], float scale2, fl
     }
   float tmax = t[0];
 #pragma unroll
-  for (int i = 1; i < 8; ++i) tmax = fmaxf(tmax, t[i]);
+  for (int i = 1; i < 4 * SG; ++i) tmax = fmaxf(tmax, t[i]);
   // Nothing seen yet: the tile maximum becomes the reference (it may be far below zero, so the
   // empty sum must not be scaled: 0 * 2^(+big) is not a number).  Otherwise only ever move up.
   const bool empty = (l == 0.f);
   const float delta = empty ? ((tmax > kNegInf) ? tmax : 0.f) : fmaxf(tmax, 0.f);
   float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) s += fast_exp2(t[i] - delta);
+  for (int i = 0; i < 4 * SG; ++i) s += fast_exp2(t[i] - delta);
   l = empty ? s : l * fast_exp2(-delta) + s;
   mref += delta;
 }
 
-template <bool MASK>
-__device__ __forceinline__ void lse_update(const f32x4 (&a)[2], float scale2, float& mref, float& l, int lim) {
+template <bool MASK, int SG>
+__device__ __forceinline__ void lse_update(const f32x4 (&a)[SG], float scale2, float& mref, float& l, int lim) {
   const float ln = lse_fast<MASK>(a, scale2, mref, l, lim);
   if (__builtin_amdgcn_ballot_w64(!lse_in_range(ln)) == 0) l = ln;
   else lse_renorm<MASK>(a, scale2, mref, l, lim);
@@ -610,12 +633,12 @@ __device__ __forceinline__ void lse_update(const f32x4 (&a)[2], float scale2, fl
 
 // All groups of a fully visible sub-step; one rarely taken branch at the very end so that the
 // arithmetic above it can be scheduled against the MFMAs of the next sub-step.
-template <int NG>
-__device__ __forceinline__ void lse_update_groups(const f32x4 (&a)[NG][2], float scale2, float (&mref)[NG],
+template <int NG, int SG>
+__device__ __forceinline__ void lse_update_groups(const f32x4 (&a)[NG][SG], const float (&scale2)[NG], float (&mref)[NG],
                                                   float (&l)[NG]) {
   float ln[NG];
 #pragma unroll
-  for (int g = 0; g < NG; ++g) ln[g] = lse_fast<false>(a[g], scale2, mref[g], l[g], 0);
+  for (int g = 0; g < NG; ++g) ln[g] = lse_fast<false>(a[g], scale2[g], mref[g], l[g], 0);
   // one range check for all groups, on the smallest and the largest sum (NaN scores stay NaN on
   // either path, so they need no test of their own)
   float lo = ln[0], hi = ln[0];
@@ -630,7 +653,10 @@ __device__ __forceinline__ void lse_update_groups(const f32x4 (&a)[NG][2], float
     for (int g = 0; g < NG; ++g) l[g] = ln[g];
   } else {
 #pragma unroll
-    for (int g = 0; g < NG; ++g) lse_renorm<false>(a[g], scale2, mref[g], l[g], 0);
+    for (int g = 0; g < NG; ++g) {   // group by group: the bits of a row do not depend on what else the wave holds
+      if (__builtin_amdgcn_ballot_w64(!lse_in_range(ln[g])) == 0) l[g] = ln[g];
+      else lse_renorm<false>(a[g], scale2[g], mref[g], l[g], 0);
+    }
   }
 }
 
@@ -652,7 +678,7 @@ struct NoAux {};
 template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE>
 __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(const Params p) {
   using Rg = Ring<KS>;
-  constexpr int NG = wave_group_count(NB);
+  constexpr int NG = 2 * NB;
   constexpr int kTileRows = kWaves * 16 * NG;
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes];
   int bh, tile, split;
@@ -678,12 +704,13 @@ __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(con
   const int t_int = min(nchunks, CAUSAL ? min((tile * kTileRows + p.c + 1) / kChunk, p.N / kChunk) : p.N / kChunk);
   const int keys_end = min(p.N, nchunks * kChunk);   // nothing is fetched from here on
 
-  float mref[NG], l[NG];
+  float mref[NG], l[NG], scale2[NG];
   int last[NG];  // last key a lane's query may see, minus the lane's row offset in a group
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     mref[g] = 0.f;
     l[g] = 0.f;
+    scale2[g] = p.scale2;
     const int i = q0[g] + (lane & 15);
     last[g] = (CAUSAL ? min(p.N - 1, i + p.c) : p.N - 1) - 4 * (lane >> 4);
   }
@@ -713,7 +740,7 @@ __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(con
 
   pipelined_sweep<DT, KS, NG, false, NoAux>(
       c_begin, t_int, qf, rg, advance, stage_of, [](const char*, int) { return NoAux{}; },
-      [&](const f32x4(&a)[NG][2], NoAux) { lse_update_groups<NG>(a, p.scale2, mref, l); });
+      [&](const f32x4(&a)[NG][2], NoAux) { lse_update_groups(a, scale2, mref, l); });
 
   for (int t = max(t_int, c_begin); t < nchunks; ++t) {
     advance(t);
@@ -795,18 +822,66 @@ constexpr int kModeSum = 0, kModeMax = 1, kModeBoth = 2;
 // streamed group sg, whose lse is lse2[sg].  x = s*scale2 - lse is the base-2 log of the probability.
 // Sums add 2^x; maxima track x itself and exponentiate once at the end of the sweep (2^x is monotone),
 // so a max-only sweep has no exp.  With MASK, register r of group sg is hidden when r > lim + 16*sg.
-template <bool MASK, int MODE>
-__device__ __forceinline__ void col_update(const f32x4 (&a)[2], float scale2, const float (&lse2)[2], f32x4& csum,
+template <bool MASK, int MODE, int SG>
+__device__ __forceinline__ void col_update(const f32x4 (&a)[SG], const float (&scale2)[SG], const float (&lse2)[SG], f32x4& csum,
                                            f32x4& cmax, int lim) {
 #pragma unroll
-  for (int sg = 0; sg < 2; ++sg)
+  for (int sg = 0; sg < SG; ++sg)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float x = fmaf(a[sg][r], scale2, -lse2[sg]);
+      float x = fmaf(a[sg][r], scale2[sg], -lse2[sg]);
       if (MASK) x = (r <= lim + 16 * sg) ? x : kNegInf;
       if (MODE != kModeSum) cmax[r] = fmaxf(cmax[r], x);
       if (MODE != kModeMax) csum[r] += fast_exp2(x);
     }
+}
+
+// End of a column sweep: reduces the wave's NG groups over the 16 query lanes (a transpose through LDS, one output key per
+// lane and pass; a pass writes out four groups) and stores the columns.  Nobody uses the LDS any more.
+template <int MODE, int NG>
+__device__ __forceinline__ void col_store(const Params& p, char* smem, int bh, const int (&k0)[NG], const f32x4 (&csum)[NG],
+                                          const f32x4 (&cmax)[NG], int lane, int wave) {
+  float* red = reinterpret_cast<float*>(smem) + wave * (NG * 4 * 64);
+  const int w = lane & 15;                 // key inside its group
+  if (MODE != kModeMax) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[(g * 4 + r) * 64 + lane] = csum[g][r];
+    __syncthreads();
+#pragma unroll
+    for (int g4 = 0; g4 < NG; g4 += 4) {
+      const int grp = g4 + (lane >> 4);      // which of the wave's groups this lane writes out
+      if (grp < NG) {                        // lanes 32.. idle when a wave keeps two groups
+        const float* src = red + (grp * 4 + (w & 3)) * 64 + (w >> 2) * 16;
+        float v = 0.f;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v += src[(j + lane) & 15];
+        const int key = k0[grp] + w;
+        if (key < p.N) store_column(p, p.out, true, bh, key, v);
+      }
+    }
+  }
+  if (MODE != kModeSum) {
+    if (MODE == kModeBoth) __syncthreads();
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[(g * 4 + r) * 64 + lane] = cmax[g][r];
+    __syncthreads();
+#pragma unroll
+    for (int g4 = 0; g4 < NG; g4 += 4) {
+      const int grp = g4 + (lane >> 4);
+      if (grp < NG) {
+        const float* src = red + (grp * 4 + (w & 3)) * 64 + (w >> 2) * 16;
+        float v = kNegInf;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v = fmaxf(v, src[(j + lane) & 15]);
+        const int key = k0[grp] + w;
+        if (key < p.N) store_column(p, (MODE == kModeBoth) ? p.out2 : p.out, false, bh, key, fast_exp2(v));
+      }
+    }
+  }
 }
 
 struct LsePair {
@@ -836,7 +911,7 @@ inline int col_tile_blocks(int ksteps, int mode, int N, int64_t bh, bool causal)
 template <int DT, int KS, bool CAUSAL, int MODE, int NB>
 __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_reduce_kernel(const Params p) {
   using Rg = Ring<KS>;
-  constexpr int NG = wave_group_count(NB);
+  constexpr int NG = 2 * NB;
   constexpr int kTileRows = kWaves * 16 * NG;
   constexpr int kRed = kWaves * NG * 4 * 64 * 4;      // end-of-sweep transpose buffer
   constexpr int kSmem = (Rg::kBytes > kRed) ? Rg::kBytes : kRed;
@@ -849,6 +924,7 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
   const char* qb = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
   const char* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
   const float* lse = p.lse + (int64_t)bh * p.M;
+  const float scale2[2] = {p.scale2, p.scale2};
 
   int k0[NG];  // first key of each of this wave's groups
   wave_groups<NB>(tile, wave, k0);
@@ -931,8 +1007,8 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
           acc[1] = mma<DT>(kf[g][ks], qfrag[1][ks], acc[1]);
         }
         const bool need_mask = CAUSAL && (kg + 15 > qs + p.c);
-        if (need_mask) col_update<true, MODE>(acc, p.scale2, lq.v, csum[g], cmax[g], lim_lane + qs - kg);
-        else col_update<false, MODE>(acc, p.scale2, lq.v, csum[g], cmax[g], 0);
+        if (need_mask) col_update<true, MODE>(acc, scale2, lq.v, csum[g], cmax[g], lim_lane + qs - kg);
+        else col_update<false, MODE>(acc, scale2, lq.v, csum[g], cmax[g], 0);
       }
     }
   };
@@ -944,55 +1020,611 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
       [&](const f32x4(&a)[NG][2], const LsePair& lq) {
         // the lse values are first touched here, a sub-step after their LDS read was issued
 #pragma unroll
-        for (int g = 0; g < NG; ++g) col_update<false, MODE>(a[g], p.scale2, lq.v, csum[g], cmax[g], 0);
+        for (int g = 0; g < NG; ++g) col_update<false, MODE>(a[g], scale2, lq.v, csum[g], cmax[g], 0);
       });
 
   for (int t = nfull; t < nchunks; ++t) general_chunk(t);
 
-  // Reduce over the 16 query lanes: transpose through LDS, one output key per lane and pass; a pass
-  // writes out four of the wave's groups.
-  float* red = reinterpret_cast<float*>(smem) + wave * (NG * 4 * 64);
-  const int w = lane & 15;                 // key inside its group
   ring_sync<0>();   // every load has landed (those past the last chunk write zeros): the LDS can be reused
-  if (MODE != kModeMax) {
+  col_store<MODE, NG>(p, smem, bh, k0, csum, cmax, lane, wave);
+}
+
+// ---------------------------------------------------------------------------------------------
+// fp32 operands.  Each row is scaled by a power of two that puts its largest element at 2^14..2^15 and every element x is split
+// into two fp16 numbers, h = fp16(x) and l = fp16(x - h): 22 to 24 significant bits of x, and of elements smaller than 2^-16 of
+// the row's largest everything down to 2^-40 of that one.  A product is h h' + h l' + l h' (l l' is below 2^-24 of it), each
+// exact in fp32 and added up by v_mfma_f32_16x16x32_f16: 48 matrix cycles per 16 x 16 x 32 block where
+// v_mfma_f32_16x16x4_f32 takes 256.  Error of the scores against sums in 64 bits, relative 2-norm over N(0,1) rows (and over
+// rows whose elements spread by e^(3 N(0,1))): D = 32 8.8e-8 (8.6e-8), 64 1.1e-7 (1.1e-7), 128 1.4e-7 (1.4e-7), 256
+// 1.9e-7 (1.6e-7); the fp32 instructions, which round the running sum after every term: 1.0e-7 (1.2e-7), 1.5e-7
+// (1.5e-7), 2.0e-7 (1.9e-7), 2.9e-7 (2.5e-7).  Shorter rows have few terms to round (D = 16 8.4e-8 against 7.4e-8): below
+// D = 32 the planes hold the floats themselves and the fp32 instructions multiply them.  A row with an infinity or a
+// NaN has no scale; chunks and resident rows that hold one are multiplied on the fp32 instructions, from memory (exact_scores).
+//
+// Streamed rows are split once per workgroup on their way to LDS: global -> registers (a chunk ahead) -> two planes of a
+// stage, each laid out like a stage of Ring.  A workgroup is NW waves of NG 16-row groups (F32Tile).  What bounds the long
+// sweeps is the vector port (per 32 x 128 streamed floats and wave: the split 70 instructions in workgroups of 128 rows, 35 in
+// those of 256, scale, fma, exp2 and add of 16 scores per lane 64, 48 matrix instructions of about 10 port cycles), then package power;
+// short ones the latency of a chunk.  32 heads of 1024 x 1024 x 128: 137 -> 64 us per call, 4096 x 4096 x 128 2250 -> 730.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_row(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+struct Planes {   // eight values of a row: h and l, or (not SPLIT) the first and the last four floats
+  u32x4 p[2];
+};
+
+__device__ __forceinline__ float maximum3(float a, float b, float c) {   // a NaN wins
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
+}
+__device__ __forceinline__ uint32_t largest8(const f32x4& a, const f32x4& b) {   // bits of the largest magnitude
+  float m = maximum3(fabsf(a[0]), fabsf(a[1]), fabsf(a[2]));
+  m = maximum3(m, fabsf(a[3]), fabsf(b[0]));
+  m = maximum3(m, fabsf(b[1]), fabsf(b[2]));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_maximum(m, fabsf(b[3])));
+}
+// The power of two that a row's elements are multiplied by and the one that undoes it, from the bits of the row's largest
+// magnitude (2^126 at most: rows below 2^-112 are not brought all the way up).
+__device__ __forceinline__ void row_scale(uint32_t largest, float& up, float& down) {
+  const uint32_t e = max(largest & 0x7f800000u, 15u << 23);
+  up = __builtin_bit_cast(float, (268u << 23) - e);
+  down = __builtin_bit_cast(float, e - (14u << 23));
+}
+__device__ __forceinline__ bool has_no_scale(uint32_t largest) { return largest >= 0x7f800000u; }   // (infinity, NaN)
+
+__device__ __forceinline__ Planes split8(const f32x4& a, const f32x4& b, float up) {
+  Planes s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x2 x = (i < 2) ? (f32x2){a[2 * i], a[2 * i + 1]} : (f32x2){b[2 * i - 4], b[2 * i - 3]};
+    const f16x2 h = __builtin_convertvector((f32x2){x[0] * up, x[1] * up}, f16x2);
+    const f32x2 rest = {fmaf(x[0], up, -(float)h[0]), fmaf(x[1], up, -(float)h[1])};
+    s.p[0][i] = __builtin_bit_cast(uint32_t, h);
+    s.p[1][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, f16x2));
+  }
+  return s;
+}
+
+// Largest value over aligned groups of LANES lanes (4, 8, 16 or 32); every lane of a group ends up with it.
+template <int CTRL>
+__device__ __forceinline__ uint32_t max_dpp(uint32_t v) {
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true));
+}
+template <int LANES>
+__device__ __forceinline__ uint32_t lanes_max(uint32_t v) {
+  v = max_dpp<0xB1>(v);                        // quad_perm [1,0,3,2]
+  v = max_dpp<0x4E>(v);                        // quad_perm [2,3,0,1]
+  if (LANES >= 8) v = max_dpp<0x141>(v);       // row_half_mirror
+  if (LANES >= 16) v = max_dpp<0x140>(v);      // row_mirror
+  if (LANES >= 32) {
+    // odd rows of 16 lanes of the one register change places with even rows of the other (written out: the compiler
+    // takes the two results of __builtin_amdgcn_permlane16_swap for one)
+    uint32_t w = v;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(v), "+v"(w));
+    v = max(v, w);
+  }
+  return v;
+}
+
+// Rows of D <= 128 are streamed 32 at a time, D <= 64 64, longer ones 16: two stages take at most 32 KiB.
+constexpr int f32_chunk(int ks, int nw) { return (ks <= 2 ? 64 : ks <= 4 ? 32 : 16) * (nw / 4); }
+constexpr int f32_groups(int ks) { return ks <= 4 ? 2 : 1; }   // streamed 16-row groups per sub-step
+
+// KS: k-steps of 32 d.
+template <int KS, bool SPLIT, int NW>
+struct SplitRing {
+  static constexpr int kNumThreads = 64 * NW;
+  static constexpr int kChunkRows = f32_chunk(KS, NW);
+  static constexpr int kPitch = Ring<KS>::kPitch;            // bytes of a row in one plane
+  static constexpr int kRowGranules = kPitch / 16;           // of eight values: threads that share a row
+  static constexpr int kPlane = kChunkRows * kPitch;
+  static constexpr int kStage = 2 * kPlane;
+  static constexpr int kRowFloats = 2 * kChunkRows;          // two floats per row of a stage: its scale, and what the caller adds
+  // two stages, their row floats, a word for each: see `bad`
+  static constexpr int kBytes = 2 * kStage + 2 * kRowFloats * 4 + 16;
+  static constexpr int kPer = kChunkRows * kRowGranules / kNumThreads;   // granules per thread
+  static_assert(kPer * kNumThreads == kChunkRows * kRowGranules, "whole granules per thread");
+
+  char* smem;
+  uint32_t src[kPer];     // source byte offset inside a chunk of a granule
+  bool half[kPer];        // its second 16 bytes lie past D
+  uint32_t dst[kPer];     // where its parts go in each plane
+  uint32_t frag0;         // the lane's fragment of k-step 0 inside a 16-row group; k-step ks: ^ (ks * 64)
+  f32x4 raw[kPer][2];     // the chunk in flight
+  const char* next_ptr;
+  int rows_left, row_bytes;
+
+  __device__ __forceinline__ void init(char* lds, const char* base, int64_t row_bytes64, int row0, int nrows, int dgran,
+                                       int tid) {
+    smem = lds;
+    const int lane = tid & 63;
+    row_bytes = (int)row_bytes64;
+    next_ptr = base + (int64_t)row0 * row_bytes64;
+    rows_left = nrows - row0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int idx = i * kNumThreads + tid, row = idx / kRowGranules, c = idx % kRowGranules;
+      src[i] = (2 * c < dgran) ? (uint32_t)row * (uint32_t)row_bytes + (uint32_t)c * 32u : kPastEnd;
+      half[i] = 2 * c + 1 >= dgran;
+      dst[i] = (uint32_t)(row * kPitch + ((c ^ Ring<KS>::swz(row)) * 16));
+    }
+    // (the swizzle is an exclusive or over granule numbers, and so is adding 4 * ks to a number below 4)
+    frag0 = (uint32_t)((lane & 15) * kPitch + (((lane >> 4) ^ Ring<KS>::swz(lane & 15)) * 16));
+    if (tid < 2) bad()[tid] = -1;
+  }
+  // bad()[s]: the last chunk staged in stage s that holds a row without a scale
+  __device__ __forceinline__ int* bad() const { return reinterpret_cast<int*>(smem + 2 * kStage + 2 * kRowFloats * 4); }
+  __device__ __forceinline__ char* stage_of(int t) const { return smem + (t & 1) * kStage; }
+  __device__ __forceinline__ float* scale_of(int t) const { return reinterpret_cast<float*>(smem + 2 * kStage) + (t & 1) * kRowFloats; }
+  __device__ __forceinline__ float* extra_of(int t) const { return scale_of(t) + kChunkRows; }
+
+  // The next chunk on its way to the registers; rows past the end arrive as zeros.
+  template <int AUX = 0>
+  __device__ __forceinline__ void fetch() {
+    const int live = __builtin_amdgcn_readfirstlane(min(max(rows_left, 0), kChunkRows));
+    const __amdgpu_buffer_rsrc_t view =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(next_ptr), 0, (int)((uint32_t)live * (uint32_t)row_bytes), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      raw[i][0] = __builtin_bit_cast(f32x4, view_load16<AUX>(view, src[i]));
+      raw[i][1] = __builtin_bit_cast(f32x4, view_load16<AUX>(view, half[i] ? kPastEnd : src[i] + 16u));
+    }
+    next_ptr += (int64_t)kChunkRows * row_bytes;
+    rows_left -= kChunkRows;
+  }
+  // The chunk in the registers, number t, to its stage: granule by granule, or whole.
+  __device__ __forceinline__ void put_granule(int i, int t, int tid, uint32_t& largest) {
+    Planes s;
+    if constexpr (SPLIT) {
+      const uint32_t m = lanes_max<kRowGranules>(largest8(raw[i][0], raw[i][1]));
+      largest = max(largest, m);
+      float up, down;
+      row_scale(m, up, down);
+      s = split8(raw[i][0], raw[i][1], up);
+      scale_of(t)[(i * kNumThreads + tid) / kRowGranules] = down;   // (by every thread of the row)
+    } else {
+      s.p[0] = __builtin_bit_cast(u32x4, raw[i][0]);
+      s.p[1] = __builtin_bit_cast(u32x4, raw[i][1]);
+    }
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) *reinterpret_cast<u32x4*>(stage_of(t) + t2 * kPlane + dst[i]) = s.p[t2];
+  }
+  __device__ __forceinline__ void note(int t, uint32_t largest) {
+    if (SPLIT && has_no_scale(largest)) bad()[t & 1] = t;
+  }
+  __device__ __forceinline__ void put(int t, int tid) {
+    uint32_t largest = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) put_granule(i, t, tid, largest);
+    note(t, largest);
+  }
+  __device__ __forceinline__ bool is_bad(int t) const {
+    return SPLIT && __builtin_amdgcn_readfirstlane(bad()[t & 1]) == t;
+  }
+  // Fragment of 16-row group `group`, k-step ks, plane t2.
+  __device__ __forceinline__ u32x4 frag(const char* stage, int group, int ks, int t2) const {
+    return *reinterpret_cast<const u32x4*>(smem + (((uint32_t)(stage - smem) + frag0) ^ (uint32_t)(ks * 64)) +
+                                           group * 16 * kPitch + t2 * kPlane);
+  }
+};
+
+// The wave's resident rows as planes; down[g] undoes the scale of group g's row lane & 15.  Returns whether one of them has no scale.
+template <int KS, int NG, bool SPLIT>
+__device__ __forceinline__ bool load_resident_split(Planes (&f)[KS][NG], float (&down)[NG], const char* base, int64_t row_bytes,
+                                                    const int (&rows)[NG], int nrows, int dgran, int lane) {
+  uint32_t worst = 0;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const __amdgpu_buffer_rsrc_t view = rows_view(base, row_bytes, rows[g], nrows);
+    const uint32_t roff = (uint32_t)(lane & 15) * (uint32_t)row_bytes;
+    f32x4 x[KS][2];
+    uint32_t m = 0;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int gi = 2 * (ks * 4 + (lane >> 4));   // 16-byte granule of the row
+      x[ks][0] = __builtin_bit_cast(f32x4, view_load16(view, gi < dgran ? roff + gi * 16u : kPastEnd));
+      x[ks][1] = __builtin_bit_cast(f32x4, view_load16(view, gi + 1 < dgran ? roff + gi * 16u + 16u : kPastEnd));
+    }
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) m = max(m, largest8(x[ks][0], x[ks][1]));
+      m = max(m, (uint32_t)__shfl_xor((int)m, 16));
+      m = max(m, (uint32_t)__shfl_xor((int)m, 32));
+      worst = max(worst, m);
+      float up;
+      row_scale(m, up, down[g]);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) f[ks][g] = split8(x[ks][0], x[ks][1], up);
+    } else {
+      down[g] = 1.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2) f[ks][g].p[t2] = __builtin_bit_cast(u32x4, x[ks][t2]);
+    }
+  }
+  return SPLIT && __builtin_amdgcn_ballot_w64(has_no_scale(worst)) != 0;
+}
+
+// The same scores from the operands in memory, on the fp32 instructions.
+template <bool RESIDENT_IS_KEYS, int NG, int SG>
+__device__ __forceinline__ void exact_scores(f32x4 (&acc)[NG][SG], const char* res, int64_t res_bytes, const int (&r0)[NG],
+                                             int res_rows, const char* str, int64_t str_bytes, int s0, int str_rows,
+                                             int dgran, int lane) {
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll 1
+  for (int k0 = 0; k0 < dgran; k0 += 4) {
+    const int gi = k0 + (lane >> 4);
+    const uint32_t col = (uint32_t)min(gi, dgran - 1) * 16u;
+    u32x4 r[NG], t[SG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const u32x4 v = view_load16(rows_view(res, res_bytes, r0[g], res_rows), (uint32_t)(lane & 15) * (uint32_t)res_bytes + col);
+      r[g] = gi < dgran ? v : zero;
+    }
+#pragma unroll
+    for (int sg = 0; sg < SG; ++sg) {
+      const u32x4 v = view_load16(rows_view(str, str_bytes, s0 + 16 * sg, str_rows),
+                                  (uint32_t)(lane & 15) * (uint32_t)str_bytes + col);
+      t[sg] = gi < dgran ? v : zero;
+    }
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[(g * 4 + r) * 64 + lane] = csum[g][r];
-    __syncthreads();
+      for (int sg = 0; sg < SG; ++sg)
+        acc[g][sg] = RESIDENT_IS_KEYS ? mma<FCR_DTYPE_F32>(r[g], t[sg], acc[g][sg]) : mma<FCR_DTYPE_F32>(t[sg], r[g], acc[g][sg]);
+  }
+}
+
+// Scaled scores of sub-step `sub` (16 * SG streamed rows) of a staged chunk against the wave's resident rows; keys are the A
+// operand.  Fragments are read a k-step ahead of their matrix instructions, those of the first by the
+// caller; `between(ks)` runs behind the matrix instructions of k-step ks.
+// Matrix instructions and memory accesses keep this order, vector instructions may move across.
+template <int SG>
+struct Fragments {
+  u32x4 f[2][SG];   // per plane and group
+};
+template <int SG, int KS, bool SPLIT, int NW>
+__device__ __forceinline__ Fragments<SG> read_fragments(const SplitRing<KS, SPLIT, NW>& rg, const char* stage, int sub, int ks) {
+  Fragments<SG> x;
 #pragma unroll
-    for (int g4 = 0; g4 < NG; g4 += 4) {
-      const int grp = g4 + (lane >> 4);      // which of the wave's groups this lane writes out
-      if (grp < NG) {                        // lanes 32.. idle when a wave keeps two groups
-        const float* src = red + (grp * 4 + (w & 3)) * 64 + (w >> 2) * 16;
-        float v = 0.f;
+  for (int t2 = 1; t2 >= 0; --t2)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) v += src[(j + lane) & 15];
-        const int key = k0[grp] + w;
-        if (key < p.N) store_column(p, p.out, true, bh, key, v);
+    for (int sg = 0; sg < SG; ++sg) x.f[t2][sg] = rg.frag(stage, sub * SG + sg, ks, t2);
+  return x;
+}
+template <bool RESIDENT_IS_KEYS, bool SPLIT, int KS, int NG, int SG, int NW, class BetweenF>
+__device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes (&res)[KS][NG], const SplitRing<KS, SPLIT, NW>& rg,
+                                             const char* stage, int sub, const Fragments<SG>& first, BetweenF&& between) {
+  // products by plane: streamed l with h, h with l, h with h; or the fp32 halves
+  constexpr int kProducts = SPLIT ? 3 : 2;
+  constexpr int str_of[3] = {1, 0, 0}, res_of[3] = {SPLIT ? 0 : 1, SPLIT ? 1 : 0, 0};
+  constexpr int kType = SPLIT ? FCR_DTYPE_F16 : FCR_DTYPE_F32;
+  Fragments<SG> f[2];
+  f[0] = first;
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int sg = 0; sg < SG; ++sg) acc[g][sg] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    if (ks + 1 < KS) f[(ks + 1) & 1] = read_fragments<SG>(rg, stage, sub, ks + 1);
+    __builtin_amdgcn_sched_barrier(0x2 | 0x4 | 0x400);
+#pragma unroll
+    for (int t = 0; t < kProducts; ++t)
+#pragma unroll
+      for (int sg = 0; sg < SG; ++sg)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          const u32x4 r = res[ks][g].p[res_of[t]], s = f[ks & 1].f[str_of[t]][sg];
+          acc[g][sg] = RESIDENT_IS_KEYS ? mma<kType>(r, s, acc[g][sg]) : mma<kType>(s, r, acc[g][sg]);
+        }
+    between(ks);
+    __builtin_amdgcn_sched_barrier(0x2 | 0x4 | 0x400);
+  }
+}
+
+// A sweep over chunks [t0, t1), whose scaled scores go to `consume` a sub-step at a time, in order; those of [ta, tb) need no mask.
+// Per chunk one barrier, behind which it is staged and the other stage is free.  Under the matrix instructions of an
+// unmasked chunk run the split of the next one (fetched a chunk ago) and `consume` for the sub-step before, whose scores are kept for
+// it.  aux_of(t, sub) is what consume needs besides the scores, extra(t) what travels with a chunk; general(t, exact) does
+// a chunk that needs a mask or, `exact`, has a row without a scale.
+template <bool RESIDENT_IS_KEYS, int AUX, class Aux, bool SPLIT, int KS, int NG, int NW, class ExtraF, class AuxF, class ConsumeF,
+          class GeneralF>
+__device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, const Planes (&res)[KS][NG],
+                                            SplitRing<KS, SPLIT, NW>& rg, int tid, bool idle, bool res_bad, ExtraF&& extra,
+                                            AuxF&& aux_of, ConsumeF&& consume, GeneralF&& general) {
+  using Rg = SplitRing<KS, SPLIT, NW>;
+  constexpr int SG = f32_groups(KS), SUBS = Rg::kChunkRows / (16 * SG), STEPS = SUBS * KS, PER = Rg::kPer;
+  if (t0 >= t1) return;
+  rg.template fetch<AUX>();
+  ring_sync<63>();   // (the words at bad() are set)
+  rg.put(t0, tid);
+  extra(t0);
+  rg.template fetch<AUX>();
+  f32x4 kept[NG][SG];   // the scores not yet consumed
+  Aux kept_aux;
+  auto chunk = [&](int t, const Fragments<SG>& first, auto first_tag) {
+    constexpr bool FIRST = decltype(first_tag)::value;
+    const char* stage = rg.stage_of(t);
+    uint32_t largest = 0;
+    Fragments<SG> next = first;
+#pragma unroll
+    for (int sub = 0; sub < SUBS; ++sub) {
+      f32x4 acc[NG][SG];
+      const Aux aux = aux_of(t, sub);
+      split_scores<RESIDENT_IS_KEYS, SPLIT>(acc, res, rg, stage, sub, next, [&](int ks) {
+        const int step = sub * KS + ks;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+          if (step == max(0, (i + 1) * STEPS / (PER + 1) - 1)) rg.put_granule(i, t + 1, tid, largest);
+        if (step == STEPS - 1) {
+          extra(t + 1);
+          rg.template fetch<AUX>();
+        }
+        if (ks == KS - 1 && sub + 1 < SUBS) next = read_fragments<SG>(rg, stage, sub + 1, 0);
+      });
+      if (!FIRST || sub > 0) consume(kept, kept_aux);
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int sg = 0; sg < SG; ++sg) kept[g][sg] = acc[g][sg];
+      kept_aux = aux;
+    }
+    rg.note(t + 1, largest);
+  };
+  bool entered = false;
+  for (int t = t0; t < t1;) {
+    if (!entered) ring_sync<63>();   // waits for LDS accesses only: the fetch stays in flight
+    entered = false;
+    Fragments<SG> first = read_fragments<SG>(rg, rg.stage_of(t), 0, 0);   // (in flight while the word is looked at)
+    const bool exact = res_bad || rg.is_bad(t);
+    if (idle || exact || t < ta || t >= tb) {
+      rg.put(t + 1, tid);
+      extra(t + 1);
+      rg.template fetch<AUX>();
+      if (!idle) general(t, exact);
+      ++t;
+      continue;
+    }
+    chunk(t, first, std::true_type());
+    for (++t; t < tb; ++t) {
+      ring_sync<63>();
+      first = read_fragments<SG>(rg, rg.stage_of(t), 0, 0);
+      entered = rg.is_bad(t);
+      if (entered) break;
+      chunk(t, first, std::false_type());
+    }
+    consume(kept, kept_aux);
+  }
+}
+
+// See row_lse_kernel: the same work order, key ranges, row state and result for fp32 operands.
+template <int KS, bool CAUSAL, int NG, bool STREAM_ONCE, bool SPLIT, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p) {
+  using Rg = SplitRing<KS, SPLIT, NW>;
+  constexpr int SG = f32_groups(KS), kRows = Rg::kChunkRows, kTileRows = NW * 16 * NG;
+  __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes];
+  int bh, tile, split;
+  map_block_split(p, CAUSAL, bh, tile, split);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int b = bh / p.H, h = bh - b * p.H;
+  const char* qb = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
+  const char* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
+
+  const int kend = CAUSAL ? min(p.N, tile * kTileRows + kTileRows + p.c) : p.N;
+  const int per_split = ((p.N + kRows - 1) / kRows + p.splits - 1) / p.splits;
+  const int c_begin = split * per_split;
+  const int nchunks = min((kend + kRows - 1) / kRows, c_begin + per_split);
+  const int keys_end = min(p.N, nchunks * kRows);
+  // chunks that every query of the workgroup sees in full
+  const int t_int = min(nchunks, CAUSAL ? min((tile * kTileRows + p.c + 1) / kRows, p.N / kRows) : p.N / kRows);
+
+  int q0[NG], last[NG];
+  float mref[NG], l[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    q0[g] = tile * kTileRows + wave * 16 * NG + 16 * g;
+    mref[g] = 0.f;
+    l[g] = 0.f;
+    const int i = q0[g] + (lane & 15);
+    last[g] = (CAUSAL ? min(p.N - 1, i + p.c) : p.N - 1) - 4 * (lane >> 4);
+  }
+  Rg rg;
+  rg.init(smem, kb, p.k_sr, c_begin * kRows, keys_end, p.dgran, tid);
+  Planes qf[KS][NG];
+  float qs2[NG];   // scale2 times what undoes the scale of the lane's query
+  const bool q_bad = load_resident_split<KS, NG, SPLIT>(qf, qs2, qb, p.q_sr, q0, p.M, p.dgran, lane);
+#pragma unroll
+  for (int g = 0; g < NG; ++g) qs2[g] *= p.scale2;
+  const bool idle = q0[0] >= p.M;   // a wave whose rows all lie past M only helps staging
+
+  struct KeyScales {
+    f32x4 v[SG];   // of the lane's four keys per group
+  };
+  auto scales_at = [&](int t, int sub) {
+    KeyScales s;
+    if (SPLIT) {
+#pragma unroll
+      for (int sg = 0; sg < SG; ++sg)
+        s.v[sg] = *reinterpret_cast<const f32x4*>(rg.scale_of(t) + (sub * SG + sg) * 16 + 4 * (lane >> 4));
+    }
+    return s;
+  };
+  auto rescale = [&](f32x4(&a)[NG][SG], const KeyScales& s) {
+    if (SPLIT) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int sg = 0; sg < SG; ++sg) a[g][sg] *= s.v[sg];
+    }
+  };
+  auto general = [&](int t, bool exact) {
+    const char* stage = rg.stage_of(t);
+#pragma unroll
+    for (int sub = 0; sub < kRows / (16 * SG); ++sub) {
+      const int key0 = t * kRows + sub * 16 * SG;
+      if (key0 >= p.N || (CAUSAL && key0 > q0[NG - 1] + 15 + p.c)) continue;   // nobody sees these keys
+      f32x4 acc[NG][SG] = {};
+      if (!exact) {
+        split_scores<false, SPLIT>(acc, qf, rg, stage, sub, read_fragments<SG>(rg, stage, sub, 0), [](int) {});
+        rescale(acc, scales_at(t, sub));
+      } else {
+        exact_scores<false>(acc, qb, p.q_sr, q0, p.M, kb, p.k_sr, key0, p.N, p.dgran, lane);
+      }
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const float s2 = exact ? p.scale2 : qs2[g];
+        const bool need_mask = (key0 + 16 * SG > p.N) || (CAUSAL && key0 + 16 * SG - 1 > q0[g] + p.c);
+        if (need_mask) lse_update<true>(acc[g], s2, mref[g], l[g], last[g] - key0);
+        else lse_update<false>(acc[g], s2, mref[g], l[g], 0);
       }
     }
+  };
+  split_sweep<false, (STREAM_ONCE ? kLoadOnce : 0), KeyScales>(
+      c_begin, c_begin, t_int, nchunks, qf, rg, tid, idle, q_bad, [](int) {}, scales_at,
+      [&](f32x4(&a)[NG][SG], const KeyScales& s) {
+        rescale(a, s);
+        lse_update_groups(a, qs2, mref, l);
+      },
+      general);
+
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    float v = (l[g] == 0.f) ? kNegInf : mref[g] + fast_log2(l[g]);
+    v = lse_merge(v, __shfl_xor(v, 16));
+    v = lse_merge(v, __shfl_xor(v, 32));
+    const int i = q0[g] + lane;
+    float* out = (p.splits > 1) ? p.part + (int64_t)split * p.bh_count * p.M : p.lse;
+    if (lane < 16 && i < p.M) out[(int64_t)bh * p.M + i] = v;
   }
-  if (MODE != kModeSum) {
-    if (MODE == kModeBoth) __syncthreads();
+}
+
+// See col_reduce_kernel.
+template <int KS, bool CAUSAL, int MODE, int NG, bool SPLIT, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params p) {
+  using Rg = SplitRing<KS, SPLIT, NW>;
+  constexpr int SG = f32_groups(KS), kRows = Rg::kChunkRows, kTileRows = NW * 16 * NG;
+  constexpr int kRed = NW * NG * 4 * 64 * 4;
+  __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes > kRed ? Rg::kBytes : kRed];
+  int bh, tile;
+  map_block(p, false, bh, tile);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int b = bh / p.H, h = bh - b * p.H;
+  const char* qb = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
+  const char* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
+  const float* lse = p.lse + (int64_t)bh * p.M;
+
+  int k0[NG];
+  f32x4 csum[NG], cmax[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    k0[g] = tile * kTileRows + wave * 16 * NG + 16 * g;
+    csum[g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    cmax[g] = (f32x4){kNegInf, kNegInf, kNegInf, kNegInf};
+  }
+  const int t0 = CAUSAL ? max(0, tile * kTileRows - p.c) / kRows : 0;
+  const int nchunks = (p.M + kRows - 1) / kRows;
+  // chunks from t_int on: their queries all see every key of the tile (rows past M add 2^-inf)
+  const int t_int = CAUSAL ? max(t0, (tile * kTileRows + kTileRows - 1 - p.c + kRows - 1) / kRows) : t0;
+  const int lim_lane = (lane & 15) + p.c - 4 * (lane >> 4);
+
+  Rg rg;
+  rg.init(smem, qb, p.q_sr, t0 * kRows, p.M, p.dgran, tid);
+  Planes kf[KS][NG];
+  f32x4 ks4[NG];   // what undoes the scale of the lane's four keys per group
+  bool k_bad;
+  {
+    float down[NG];
+    k_bad = load_resident_split<KS, NG, SPLIT>(kf, down, kb, p.k_sr, k0, p.N, p.dgran, lane);
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[(g * 4 + r) * 64 + lane] = cmax[g][r];
-    __syncthreads();
+      for (int r = 0; r < 4; ++r) ks4[g][r] = SPLIT ? __shfl(down[g], 4 * (lane >> 4) + r) : 1.f;
+  }
+  const bool idle = k0[0] >= p.N;
+
+  // the lse of a chunk's queries (+inf past M: they contribute 2^-inf) travels with its rows
+  float lse_raw = 0.f;
+  auto lse_fetch = [&](int t) {
+    const int i = t * kRows + tid;
+    if (tid < kRows) lse_raw = (i < p.M) ? lse[i] : kPosInf;
+  };
+  auto extra = [&](int t) {
+    if (tid < kRows) rg.extra_of(t)[tid] = lse_raw;
+    lse_fetch(t + 1);
+  };
+  struct QueryFacts {
+    float lse[SG], s2[SG];   // of the lane's query per group: lse, scale2 times what undoes its scale
+  };
+  auto facts_at = [&](int t, int sub) {
+    QueryFacts q;
 #pragma unroll
-    for (int g4 = 0; g4 < NG; g4 += 4) {
-      const int grp = g4 + (lane >> 4);
-      if (grp < NG) {
-        const float* src = red + (grp * 4 + (w & 3)) * 64 + (w >> 2) * 16;
-        float v = kNegInf;
+    for (int sg = 0; sg < SG; ++sg) {
+      const int at = (sub * SG + sg) * 16 + (lane & 15);
+      q.lse[sg] = rg.extra_of(t)[at];
+      q.s2[sg] = SPLIT ? rg.scale_of(t)[at] * p.scale2 : p.scale2;
+    }
+    return q;
+  };
+  auto general = [&](int t, bool exact) {
+    const char* stage = rg.stage_of(t);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) v = fmaxf(v, src[(j + lane) & 15]);
-        const int key = k0[grp] + w;
-        if (key < p.N) store_column(p, (MODE == kModeBoth) ? p.out2 : p.out, false, bh, key, fast_exp2(v));
+    for (int sub = 0; sub < kRows / (16 * SG); ++sub) {
+      const int qs = t * kRows + sub * 16 * SG;
+      if (qs >= p.M || (CAUSAL && k0[0] > qs + 16 * SG - 1 + p.c)) continue;   // none of these queries sees a key of the wave
+      QueryFacts q = facts_at(t, sub);
+      f32x4 acc[NG][SG] = {};
+      if (!exact) {
+        split_scores<true, SPLIT>(acc, kf, rg, stage, sub, read_fragments<SG>(rg, stage, sub, 0), [](int) {});
+        if (SPLIT) {
+#pragma unroll
+          for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int sg = 0; sg < SG; ++sg) acc[g][sg] *= ks4[g];
+        }
+      } else {
+        exact_scores<true>(acc, kb, p.k_sr, k0, p.N, qb, p.q_sr, qs, p.M, p.dgran, lane);
+#pragma unroll
+        for (int sg = 0; sg < SG; ++sg) q.s2[sg] = p.scale2;
+      }
+      if (exact || !SPLIT) {   // a row of padding may have met a non-finite key
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int sg = 0; sg < SG; ++sg)
+            if (qs + 16 * sg + (lane & 15) >= p.M) acc[g][sg] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const bool need_mask = CAUSAL && (k0[g] + 15 > qs + p.c);
+        if (need_mask) col_update<true, MODE>(acc[g], q.s2, q.lse, csum[g], cmax[g], lim_lane + qs - k0[g]);
+        else col_update<false, MODE>(acc[g], q.s2, q.lse, csum[g], cmax[g], 0);
       }
     }
-  }
+  };
+  lse_fetch(t0);
+  split_sweep<true, 0, QueryFacts>(
+      t0, t_int, SPLIT ? nchunks : p.M / kRows, nchunks, kf, rg, tid, idle, k_bad, extra, facts_at,
+      [&](f32x4(&a)[NG][SG], const QueryFacts& q) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          if (SPLIT) {
+#pragma unroll
+            for (int sg = 0; sg < SG; ++sg) a[g][sg] *= ks4[g];
+          }
+          col_update<false, MODE>(a[g], q.s2, q.lse, csum[g], cmax[g], 0);
+        }
+      },
+      general);
+  ring_sync<63>();
+  col_store<MODE, NG>(p, smem, bh, k0, csum, cmax, lane, wave);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1172,10 +1804,6 @@ __host__ __device__ constexpr int fused_chunks(int qh, int nq = 4) { return qh =
 constexpr int kFusedSteps = 8;
 constexpr int kFusedThreads = 512;
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_row(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
 // Sum or maximum over each row of 16 lanes; every lane of the row ends up with the result.
 template <bool MAX>
 __device__ __forceinline__ float row16_reduce(float v) {
@@ -2592,10 +3220,10 @@ int head_group(int64_t bh, int64_t per_bh, bool causal) {
 }
 
 // Params::fill: see second_helping.  Only for launches of one group, whose ranks are in order over the whole
-// launch, and not for rows of more than 512 bytes, whose workgroups have a CU to themselves.
-int fill_ranks(const Params& p, bool causal) {
+// launch, and not for workgroups that have a CU to themselves.
+int fill_ranks(const Params& p, int per_cu, bool causal) {
   const int cus = chip_cus();
-  if (!causal || p.splits > 1 || p.group != p.bh_count || p.total > 2 * cus || p.dgran > 4 * kMaxKSteps) return 0;
+  if (!causal || p.splits > 1 || p.group != p.bh_count || p.total > 2 * cus || per_cu < 2) return 0;
   return (cus + p.group - 1) / p.group;
 }
 
@@ -2638,9 +3266,9 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   // the device is first asked (for its CU count) here, after every argument check
   const int ksteps = ksteps_of(dtype, D);
   const bool f32 = dtype == FCR_DTYPE_F32;
-  const bool half = by_keys ? half_tiles(f32, N, bh) : row_half_tiles(f32, M, N, bh);
-  const int trows = half ? kWaves * 16
-                         : by_keys ? kWaves * 32 * col_tile_blocks(ksteps, col_mode, N, bh, causal) : row_tile_rows(ksteps, M, N, bh, causal);
+  const int trows = !by_keys ? row_tile_rows(f32, ksteps, M, N, bh, causal)
+                    : f32    ? f32_col_tile(f32_ksteps(ksteps), col_mode == kModeBoth, M, N, bh, causal).rows()
+                             : kWaves * 32 * col_tile_blocks(ksteps, col_mode, N, bh, causal);
   const int64_t tiles = ((by_keys ? N : M) + trows - 1) / trows;
   p.q = static_cast<const char*>(q);
   p.k = static_cast<const char*>(k);
@@ -2673,10 +3301,11 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
 // Key ranges per row tile in the row kernel.  One sweep per workgroup when there is at least one
 // workgroup per CU; otherwise the keys of a tile are split so that about two per CU run, each
 // keeping at least four 64-key chunks.
-int row_splits(int B, int H, int M, int N, int ksteps) {
+int row_splits(bool f32, int B, int H, int M, int N, int ksteps) {
   const int64_t chunks = (N + kChunk - 1) / kChunk;
   if (chunks < 16) return 1;
-  const int trows = row_tile_rows(ksteps, M, N, (int64_t)B * H, false);  // same with the mask when wgs < 256
+  // (fp32 launches of at least one 128-row tile per CU are never split; the mask makes no difference below that)
+  const int trows = f32 ? 128 : row_tile_rows(false, ksteps, M, N, (int64_t)B * H, false);  // same with the mask when wgs < 256
   const int64_t wgs = (int64_t)B * H * ((M + trows - 1) / trows);
   const int cus = chip_cus();
   if (wgs >= cus) return 1;
@@ -2768,6 +3397,11 @@ int launched(const char* what) {
   return (int)e;
 }
 
+// one row tile per (b,h) and at least 1 GiB of keys: stream them past the caches
+inline bool keys_read_once(const Params& p) {
+  return p.tiles == 1 && (int64_t)p.bh_count * p.N * p.dgran * 16 >= (1ll << 30);
+}
+
 template <int DT, int KS, int NB, bool ONCE>
 void launch_lse_blocks(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(kThreads);
@@ -2777,15 +3411,10 @@ void launch_lse_blocks(const Params& p, bool causal, hipStream_t s) {
 
 template <int DT, int KS>
 void launch_lse(const Params& p, bool causal, hipStream_t s) {
-  if constexpr (DT == FCR_DTYPE_F32) {
-    if (row_half_tiles(true, p.M, p.N, p.bh_count)) return launch_lse_blocks<DT, KS, 0, false>(p, causal, s);
-  }
   if constexpr (KS <= 4) {
     if (row_blocks_per_wave(KS, p.M, p.N, p.bh_count, causal) == 2) return launch_lse_blocks<DT, KS, 2, false>(p, causal, s);
   }
-  // one row tile per (b,h) and at least 1 GiB of keys: stream them past the caches
-  const int64_t key_bytes = (int64_t)p.bh_count * p.N * p.dgran * 16;
-  if (p.tiles == 1 && key_bytes >= (1ll << 30)) return launch_lse_blocks<DT, KS, 1, true>(p, causal, s);
+  if (keys_read_once(p)) return launch_lse_blocks<DT, KS, 1, true>(p, causal, s);
   launch_lse_blocks<DT, KS, 1, false>(p, causal, s);
 }
 
@@ -2793,13 +3422,6 @@ template <int DT, int KS, int MODE>
 void launch_col_mode(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(kThreads);
   constexpr int NB = col_blocks_per_wave(KS, MODE);
-  if constexpr (DT == FCR_DTYPE_F32) {
-    if (half_tiles(true, p.N, p.bh_count)) {
-      if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 0>), grid, block, 0, s, p);
-      else hipLaunchKernelGGL((col_reduce_kernel<DT, KS, false, MODE, 0>), grid, block, 0, s, p);
-      return;
-    }
-  }
   if constexpr (NB == 2) {
     if (col_tile_blocks(KS, MODE, p.N, p.bh_count, causal) == 1) {
       if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 1>), grid, block, 0, s, p);
@@ -2809,6 +3431,46 @@ void launch_col_mode(const Params& p, bool causal, hipStream_t s) {
   }
   if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, NB>), grid, block, 0, s, p);
   else hipLaunchKernelGGL((col_reduce_kernel<DT, KS, false, MODE, NB>), grid, block, 0, s, p);
+}
+
+template <int KS, int NW, int NG, bool SPLIT>
+void launch_lse_f32_tile(const Params& p, bool causal, hipStream_t s) {
+  const dim3 grid(p.total), block(64 * NW);
+  if (keys_read_once(p)) {
+    if (causal) hipLaunchKernelGGL((row_lse_f32_kernel<KS, true, NG, true, SPLIT, NW>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((row_lse_f32_kernel<KS, false, NG, true, SPLIT, NW>), grid, block, 0, s, p);
+    return;
+  }
+  if (causal) hipLaunchKernelGGL((row_lse_f32_kernel<KS, true, NG, false, SPLIT, NW>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((row_lse_f32_kernel<KS, false, NG, false, SPLIT, NW>), grid, block, 0, s, p);
+}
+
+template <int KS, bool SPLIT = true>
+void launch_lse_f32(const Params& p, bool causal, hipStream_t s) {
+  const F32Tile t = f32_row_tile(p.M, p.N, p.bh_count, causal);
+  if (t.waves == 4) t.groups == 1 ? launch_lse_f32_tile<KS, 4, 1, SPLIT>(p, causal, s) : launch_lse_f32_tile<KS, 4, 2, SPLIT>(p, causal, s);
+  else t.groups == 1 ? launch_lse_f32_tile<KS, 8, 1, SPLIT>(p, causal, s) : launch_lse_f32_tile<KS, 8, 2, SPLIT>(p, causal, s);
+}
+
+template <int KS, int MODE, int NW, int NG, bool SPLIT>
+void launch_col_f32_tile(const Params& p, bool causal, hipStream_t s) {
+  const dim3 grid(p.total), block(64 * NW);
+  if (causal) hipLaunchKernelGGL((col_reduce_f32_kernel<KS, true, MODE, NG, SPLIT, NW>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((col_reduce_f32_kernel<KS, false, MODE, NG, SPLIT, NW>), grid, block, 0, s, p);
+}
+
+template <int KS, int MODE, bool SPLIT>
+void launch_col_f32_mode(const Params& p, bool causal, hipStream_t s) {
+  const F32Tile t = f32_col_tile(KS, MODE == kModeBoth, p.M, p.N, p.bh_count, causal);
+  if (t.waves == 4) t.groups == 1 ? launch_col_f32_tile<KS, MODE, 4, 1, SPLIT>(p, causal, s) : launch_col_f32_tile<KS, MODE, 4, 2, SPLIT>(p, causal, s);
+  else t.groups == 1 ? launch_col_f32_tile<KS, MODE, 8, 1, SPLIT>(p, causal, s) : launch_col_f32_tile<KS, MODE, 8, 2, SPLIT>(p, causal, s);
+}
+
+template <int KS, bool SPLIT = true>
+void launch_col_f32(const Params& p, bool causal, int mode, hipStream_t s) {
+  if (mode == kModeSum) launch_col_f32_mode<KS, kModeSum, SPLIT>(p, causal, s);
+  else if (mode == kModeMax) launch_col_f32_mode<KS, kModeMax, SPLIT>(p, causal, s);
+  else launch_col_f32_mode<KS, kModeBoth, SPLIT>(p, causal, s);
 }
 
 template <int DT, int KS, int MODE, int NG>
@@ -2950,14 +3612,26 @@ void fcr_detail::sweeps_bf16_single(const Params& p, int ksteps, bool causal, in
 #endif
 #if FCR_HAS(3)
 void fcr_detail::sweeps_f32(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
-  if (which == 0) { FCR_DISPATCH_KS(FCR_DTYPE_F32, ksteps, FCR_CALL_LSE) }
-  else { FCR_DISPATCH_KS(FCR_DTYPE_F32, ksteps, FCR_CALL_COL) }
+  if (p.dgran < 8) {   // D < 32
+    which == 0 ? launch_lse_f32<1, false>(p, causal, s) : launch_col_f32<1, false>(p, causal, mode, s);
+    return;
+  }
+  switch (f32_ksteps(ksteps)) {
+    case 1: which == 0 ? launch_lse_f32<1>(p, causal, s) : launch_col_f32<1>(p, causal, mode, s); break;
+    case 2: which == 0 ? launch_lse_f32<2>(p, causal, s) : launch_col_f32<2>(p, causal, mode, s); break;
+    case 3: which == 0 ? launch_lse_f32<3>(p, causal, s) : launch_col_f32<3>(p, causal, mode, s); break;
+    default: which == 0 ? launch_lse_f32<4>(p, causal, s) : launch_col_f32<4>(p, causal, mode, s); break;
+  }
 }
 #endif
 #if FCR_HAS(4)
 void fcr_detail::sweeps_f32_long_rows(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
-  if (which == 0) { FCR_DISPATCH_KS_LONG(FCR_DTYPE_F32, ksteps, FCR_CALL_LSE) }
-  else { FCR_DISPATCH_KS_LONG(FCR_DTYPE_F32, ksteps, FCR_CALL_COL) }
+  switch (f32_ksteps(ksteps)) {
+    case 5: which == 0 ? launch_lse_f32<5>(p, causal, s) : launch_col_f32<5>(p, causal, mode, s); break;
+    case 6: which == 0 ? launch_lse_f32<6>(p, causal, s) : launch_col_f32<6>(p, causal, mode, s); break;
+    case 7: which == 0 ? launch_lse_f32<7>(p, causal, s) : launch_col_f32<7>(p, causal, mode, s); break;
+    default: which == 0 ? launch_lse_f32<8>(p, causal, s) : launch_col_f32<8>(p, causal, mode, s); break;
+  }
 }
 #endif
 #if FCR_HAS(5)
@@ -3084,7 +3758,7 @@ size_t fcr_lse_bytes_two_kernels(int B, int H, int M, int N) {
   // The most any row width asks for, so the size holds for every dtype and D.  Of one problem the widths differ
   // only in the tile height, 128 or 256 rows: four k-steps take 256 where any width does (one block costs them
   // the most), and the higher tile has the fewer workgroups, hence the most splits.  (Every call comes here.)
-  const int splits = row_splits(B, H, M, N, 4);
+  const int splits = row_splits(false, B, H, M, N, 4);
   const size_t rows = (size_t)B * (size_t)H * (size_t)M;
   return rows * sizeof(float) * (splits > 1 ? 1 + (size_t)splits : 1);
 }
@@ -3123,12 +3797,12 @@ int fcr_row_lse(const void* q, const void* k, float* lse, int dtype, int B, int 
   int rc = make_params(p, q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, false, causal != 0);
   if (rc) return rc;
   p.lse = lse;
-  p.splits = row_splits(B, H, M, N, ksteps_of(dtype, D));
+  p.splits = row_splits(dtype == FCR_DTYPE_F32, B, H, M, N, ksteps_of(dtype, D));
   p.part = lse + (int64_t)B * H * M;  // only touched when splits > 1 (see fcr_lse_bytes)
   p.total *= p.splits;
-  p.group = head_group(p.bh_count, (int64_t)p.tiles * p.splits, causal != 0);
-  p.fill = fill_ranks(p, causal != 0);
   const int ksteps = ksteps_of(dtype, D);
+  p.group = head_group(p.bh_count, (int64_t)p.tiles * p.splits, causal != 0);
+  p.fill = fill_ranks(p, dtype == FCR_DTYPE_F32 ? 8 / f32_row_tile(M, N, p.bh_count, causal != 0).waves : ksteps > kMaxKSteps ? 1 : 2, causal != 0);
   hipStream_t s = static_cast<hipStream_t>(stream);
   launch_sweeps(dtype, 0, p, ksteps, causal != 0, 0, s);
   rc = launched("row_lse_kernel");
@@ -3154,7 +3828,9 @@ int col_reduce_any(const void* q, const void* k, const float* lse, void* out, vo
   int rc = make_params(p, q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, true, causal != 0, mode);
   if (rc) return rc;
   p.group = head_group(p.bh_count, p.tiles, causal != 0);
-  p.fill = fill_ranks(p, causal != 0);
+  const int ksteps = ksteps_of(dtype, D);
+  p.fill = fill_ranks(p, dtype == FCR_DTYPE_F32 ? 8 / f32_col_tile(f32_ksteps(ksteps), mode == kModeBoth, M, N, p.bh_count, causal != 0).waves : ksteps > kMaxKSteps ? 1 : 2,
+                      causal != 0);
   p.lse = const_cast<float*>(lse);
   p.out = out;
   p.out2 = out2;
@@ -3163,9 +3839,8 @@ int col_reduce_any(const void* q, const void* k, const float* lse, void* out, vo
     p.mean_from = causal ? p.c : N;
     p.inv_m = 1.0f / (float)M;
   }
-  const int ksteps = ksteps_of(dtype, D);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // (fp32 operands always take the general sweep: they are bound by the fp32 matrix rate, not by reading K)
+  // (fp32 operands always take the general sweep, which splits them)
   if (M <= kSmallRows && ksteps <= 4 && dtype != FCR_DTYPE_F32) {
     // Few queries: the sweep with all of them resident in every wave and the keys streamed, if the
     // problem fills the chip that way: 512 to 1024 workgroups (at least two per CU), each sweeping at

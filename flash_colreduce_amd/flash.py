@@ -70,9 +70,9 @@ def _device_layout(x: torch.Tensor) -> torch.Tensor:
 
 def pack_f32(x: torch.Tensor, is_key: bool, terms: int = 3) -> torch.Tensor:
     """fp32 (B,H,R,D) -> the fp16 segments of fcr_pack_f32 (include/fcr.h), for callers of the C ABI that
-    want fp32 operands multiplied on the 16-bit matrix instructions (16 times the fp32 rate) and accept
+    want fp32 operands packed once for the 16-bit kernels and accept
     fp16's range: terms = 3 gives products to about 2^-22 and needs 3 * ceil8(D) <= 256, terms = 1 is one
-    rounding to fp16.  flash_colreduce itself never comes here: it multiplies fp32 operands in fp32."""
+    rounding to fp16.  flash_colreduce itself never comes here: it keeps fp32's precision and range."""
     b, h, r, d = x.shape
     dpad = (d + 7) // 8 * 8
     src = x.contiguous()

@@ -16,7 +16,9 @@
  *     16-bit elements, a multiple of 4 in [4, 256] for fp32.  Rows must not overlap (row stride >= D).
  *     (The reference takes any strides, flash.py:292-299; a caller with other layouts makes a
  *     contiguous, zero-padded copy first -- the Python host does.)  fp32 operands are multiplied at
- *     full precision and range (the reference's tl.dot rounds them to TF32, flash.py:59,108).
+ *     fp32 precision and range (the reference's tl.dot rounds them to TF32, flash.py:59,108): from D = 32 on as two
+ *     fp16 parts of each element, scaled by row, whose scores are closer to 64-bit sums than those of the fp32 matrix
+ *     instructions; elements below 2^-16 of the largest of their row are held to 2^-40 of that one.
  *   - lse is fp32 [B*H, M] contiguous: per query row, log2(sum_j 2^(scale*log2(e)*<q_i,k_j>))
  *     over the keys the row may see.  It is the hand-over between the two kernels.  The buffer
  *     fcr_row_lse / fcr_colreduce write it to must be fcr_lse_bytes(B,H,M,N,D) long (scratch follows
@@ -49,7 +51,7 @@ extern "C" {
 /* element type of q and k */
 #define FCR_DTYPE_F16 0
 #define FCR_DTYPE_BF16 1
-#define FCR_DTYPE_F32 2 /* fp32 operands on the fp32 matrix instructions: D a multiple of 4, at most 256 */
+#define FCR_DTYPE_F32 2 /* fp32 operands: D a multiple of 4, at most 256 */
 
 /* column reduction over query rows */
 #define FCR_REDUCE_SUM 0 /* also the numerator of 'mean' (flash.py:121-122) */
@@ -148,7 +150,7 @@ int fcr_topk_mask_typed(const void* scores, int dtype, uint8_t* mask, float* thr
 
 /*
  * A faster and less exact alternative to FCR_DTYPE_F32 for fp32 operands whose values fit fp16 (the
- * 16-bit matrix instructions run at 16 times the fp32 rate): packs a contiguous fp32 [rows, D] into the fp16 [rows, terms * Dp] (Dp = D rounded up
+ * one set of fp16 numbers for the whole operand, without a scale by row): packs a contiguous fp32 [rows, D] into the fp16 [rows, terms * Dp] (Dp = D rounded up
  * to 8, zero padded) that the kernels above take with D' = terms * Dp and dtype FCR_DTYPE_F16.
  * terms = 3 writes [hi | hi | lo] for queries (is_key = 0) and [hi | lo | hi] for keys (is_key != 0),
  * hi = fp16(x), lo = fp16(x - hi): the kernels then see q.k to about 2^-22.  terms = 1 writes [hi].

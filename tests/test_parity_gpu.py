@@ -339,6 +339,73 @@ def test_fp32_tiles_of_64_rows_give_the_bits_of_taller_ones(h, m, n, d, causal):
         assert torch.equal(fca.flash_colreduce(q, k, red, causal)[0], fca.flash_colreduce(qs, ks, red, causal)[-1]), red
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(130, 257, 300, 36), (180, 300, 257, 96), (130, 257, 300, 256), (9, 511, 700, 128),
+                                     (1, 65, 33, 32), (3, 129, 1100, 28)])
+def test_fp32_split_tiles(h, m, n, d, causal):
+    """fp32 rows as two fp16 parts: tiles of 256, 128 and 64 rows with ragged ends, more than one and more than two 128-row tiles
+    per CU (which the mask treats differently), D that ends inside eight values, both sides of D = 32.  Probabilities carry
+    the error of the scores, a few 1e-7 here, and a sum that of its additions: 1e-5 as for the other fp32 tests."""
+    q, k = _inputs.randn_pair(1, h, m, n, d, seed=h + d, dtype=torch.float32)
+    s, mx = fca.flash_colreduce_multi(q.cuda(), k.cuda(), ["sum", "max"], is_causal=causal)
+    for red, pair in (("sum", s), ("mean", None), ("max", mx)):
+        want = colreduce_ref(q, k, red, causal, compute_dtype=torch.float64).float()
+        for got in (fca.flash_colreduce(q.cuda(), k.cuda(), red, is_causal=causal), pair):
+            if got is not None:
+                torch.testing.assert_close(got.cpu(), want, rtol=1e-5, atol=1e-8)
+
+
+@pytest.mark.parametrize("d", [24, 32, 128, 256])
+def test_fp32_split_rows_of_any_magnitude(d):
+    """Every row is scaled by its own power of two, from the largest float to denormal ones, and the spread inside a
+    row does not matter.  A score is off by at most 2^-23 of |q||k| per product (two parts of 2^-24 each and what is left
+    out) plus the roundings of its sum, so a log-sum-exp by at most 2^-20 of the row's largest sum of |q_d k_d|,
+    and by two units in the last place of a value between 8 and 16 (log2 of 300 keys), 2^-19, for its own rounding: a logarithm and
+    the additions that merge four partial results."""
+    m, n = 260, 300
+    g = torch.Generator().manual_seed(d)
+    q = torch.randn(1, 2, m, d, generator=g) * torch.exp(3 * torch.randn(1, 2, m, d, generator=g)) * 2.0 ** -10
+    k = torch.randn(1, 2, n, d, generator=g) * torch.exp(3 * torch.randn(1, 2, n, d, generator=g)) * 2.0 ** -10
+    k[0, 0] *= (2.0 ** (torch.arange(n) % 40 - 20).float())[:, None]
+    q[0, 1] *= (2.0 ** (torch.arange(m) % 40 - 20).float())[:, None]
+    k[0, 1, 5] = 0.0
+    k[0, 1, 6] *= 2.0 ** -130
+    for up, down in ((1.0, 1.0), (2.0 ** 70, 2.0 ** -70), (2.0 ** -80, 2.0 ** 80)):
+        qq, kk = q * up, k * down
+        got = fca.row_lse2(qq.cuda(), kk.cuda(), scale=0.1).cpu().double()
+        size = torch.matmul(qq.double().abs(), kk.double().abs().transpose(2, 3)) * (0.1 * 1.4427)
+        err = (got - row_lse2_ref(qq, kk, False, scale=0.1).double()).abs()
+        assert (err <= 2.0 ** -20 * size.amax(-1) + 2.0 ** -19).all(), (up, (err / (size.amax(-1) + 2)).max())
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(2, 200, 333, 64), (5, 130, 129, 128), (2, 300, 2100, 256), (140, 257, 130, 40), (2, 70, 99, 28)])
+def test_fp32_rows_without_a_scale(h, m, n, d, causal):
+    """Infinities: a key whose scores are -inf against every query counts for nothing, alone in its chunk, and with an
+    infinite query as well; the rest of its chunk and of its tile is as if it were not there.  A NaN query leaves NaN on the
+    columns it sees and nowhere else."""
+    q, k = _inputs.randn_pair(1, h, m, n, d, seed=m, dtype=torch.float32)
+    q, k = q.clone(), k.clone()
+    q[..., 3] = -q[..., 3].abs() - 0.1
+    dead = [0, n // 2, n - 1] if not causal else [n // 2]
+    k[:, 0, dead, 3] = float("inf")
+    keep = torch.tensor([j for j in range(n) if j not in dead])
+    c = max(n - m, 0)
+    vis = (torch.arange(m)[:, None] + c >= torch.arange(n)[None]) if causal else torch.ones(m, n, dtype=torch.bool)
+    s = (torch.matmul(q[0, 0].double(), k[0, 0, keep].double().T) * d ** -0.5).masked_fill(~vis[:, keep], -math.inf)
+    want = torch.softmax(s, -1)
+    for red in ("sum", "max"):
+        got = fca.flash_colreduce(q.cuda(), k.cuda(), red, is_causal=causal).cpu()
+        assert (got[0, 0, dead] == 0).all()
+        w = want.sum(0) if red == "sum" else want.amax(0)
+        torch.testing.assert_close(got[0, 0, keep], w.float(), rtol=1e-5, atol=1e-8)
+        other = colreduce_ref(q[:, 1:], k[:, 1:], red, causal, compute_dtype=torch.float64).float()
+        torch.testing.assert_close(got[:, 1:], other, rtol=1e-5, atol=1e-8)
+    q[0, 1, m // 2, 1] = float("nan")
+    got = fca.flash_colreduce(q.cuda(), k.cuda(), "sum", is_causal=causal).cpu()
+    assert torch.equal(torch.isnan(got[0, 1]), vis[m // 2]) and not torch.isnan(got[0, 0]).any()
+
+
 @pytest.mark.parametrize("m", [100, 128, 300, 384, 600])
 def test_row_sweep_block_choice(m):
     """Query counts for which the row sweep keeps one 32-row block per wave (M <= 128 and ragged M
