@@ -71,7 +71,7 @@ struct Params {
   int tiles;         // resident tiles per (b,h)
   int bh_count;      // B * H
   int group;         // (b,h) pairs whose workgroups are launched together (see map_block)
-  int fill;          // with the mask: tile ranks that give every CU one workgroup (see map_block), 0 = plain order
+  int fill;          // with the mask: workgroups that give every CU one (see map_group), 0 = plain order
   int stream_once;   // col_small_kernel: load the keys non-temporally
   int total;         // tiles * B * H workgroups
   // How the column kernels write a finished column (see store_column)
@@ -234,8 +234,15 @@ __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_lo
 // holds at once, so all tiles of a (b,h) run at the same time and its streamed operand comes from
 // HBM once.  Workgroups are dealt to the 8 XCDs round-robin by v, so with group a multiple of 8
 // every (b,h) stays on XCD (b,h) % 8 and that operand is shared through the XCD's L2.
+//
+// A causal launch of a few workgroups per CU, two at a time: in plain longest-first order the second workgroup of a
+// CU is as many places behind the first as the chip has CUs, so the CU with the longest sweep also gets the longest of
+// the second helping.  That helping is dealt backwards instead (p.fill; eight places at a time, which keeps the XCDs), so the
+// two sweeps of every CU add up to about the same length; what is left follows in plain order.  Host: fill_places.
 __device__ __forceinline__ void map_group(const Params& p, int per_bh, int& bh, int& r) {
-  const int v = (int)blockIdx.x;
+  int v = (int)blockIdx.x;
+  const int second = v - p.fill, dealt = (min(2 * p.fill, p.total) - p.fill) & ~7;
+  if (p.fill > 0 && second >= 0 && second < dealt) v = p.fill + (dealt - 8 - (second & ~7)) + (second & 7);
   const int per = p.group * per_bh;
   const int chunk = v / per;
   const int first = chunk * p.group;
@@ -245,20 +252,9 @@ __device__ __forceinline__ void map_group(const Params& p, int per_bh, int& bh, 
   bh = first + (w - r * g);
 }
 
-// A causal launch that is on the chip all at once, two workgroups per CU: in plain longest-first order the
-// second workgroup of a CU is as many ranks behind the first as the chip has CUs, so the CU with the longest
-// sweep also gets the longest of the second helping.  The second helping is dealt shortest first instead,
-// and the two sweeps of every CU add up to about the same length (32 heads of 2048 x 2048 fp16: 51.4 -> 48.1 us
-// per call, 4096 x 4096: 156 -> 152, 2 x 16 heads of 2048 x 2048 x 256 bf16: 83 -> 79).  Launches of more
-// workgroups than that fill in behind each other in any case and lose by it (40 heads of 5000: 211 -> 246 us).
-__device__ __forceinline__ int second_helping(const Params& p, int rank) {
-  return (p.fill > 0 && rank >= p.fill) ? p.tiles - 1 - (rank - p.fill) : rank;
-}
-
 __device__ __forceinline__ void map_block(const Params& p, bool longest_is_last_tile, int& bh, int& tile) {
   int rank;
   map_group(p, p.tiles, bh, rank);
-  rank = second_helping(p, rank);
   tile = longest_is_last_tile ? p.tiles - 1 - rank : rank;
 }
 
@@ -270,7 +266,7 @@ __device__ __forceinline__ void map_block_split(const Params& p, bool longest_is
   int r;
   map_group(p, p.tiles * p.splits, bh, r);
   const int back = r / p.tiles;   // the last key range first: with the mask it holds the diagonal, the slow part
-  const int rank = second_helping(p, r - back * p.tiles);
+  const int rank = r - back * p.tiles;
   split = p.splits - 1 - back;
   tile = longest_is_last_tile ? p.tiles - 1 - rank : rank;
 }
@@ -3219,14 +3215,6 @@ int head_group(int64_t bh, int64_t per_bh, bool causal) {
   return (int)(g < bh ? g : bh);
 }
 
-// Params::fill: see second_helping.  Only for launches of one group, whose ranks are in order over the whole
-// launch, and not for workgroups that have a CU to themselves.
-int fill_ranks(const Params& p, int per_cu, bool causal) {
-  const int cus = chip_cus();
-  if (!causal || p.splits > 1 || p.group != p.bh_count || p.total > 2 * cus || per_cu < 2) return 0;
-  return (cus + p.group - 1) / p.group;
-}
-
 // Rows the kernels take: a multiple of 16 bytes, at most 1 KiB (and no product of D that could overflow).
 bool row_width_ok(int dtype, int D) {
   const int esize = elem_bytes(dtype);
@@ -3256,6 +3244,32 @@ int check_problem(const void* q, const void* k, int dtype, int B, int H, int M, 
   return check_strides(k, ks, "k", kdims, D, esize);
 }
 
+// Rows of a launch's tiles and how many of its workgroups share a CU.
+struct TileChoice {
+  int rows, per_cu;
+};
+TileChoice tile_choice(bool f32, int ksteps, int M, int N, int64_t bh, bool by_keys, int col_mode, bool causal) {
+  if (f32) {
+    const F32Tile t = by_keys ? f32_col_tile(f32_ksteps(ksteps), col_mode == kModeBoth, M, N, bh, causal) : f32_row_tile(M, N, bh, causal);
+    return TileChoice{t.rows(), 8 / t.waves};
+  }
+  const int per_cu = ksteps > kMaxKSteps ? 1 : 2;
+  return TileChoice{by_keys ? kWaves * 32 * col_tile_blocks(ksteps, col_mode, N, bh, causal)
+                            : row_tile_rows(false, ksteps, M, N, bh, causal), per_cu};
+}
+
+// Params::fill: see map_group.  Only for launches of one group, whose places are in order of length over the whole launch, and
+// for kernels that run two workgroups per CU.  Per call, plain order and with the second helping backwards, workgroups per
+// CU in brackets: 256-row tiles, 40 heads of 3258 (2.03) 141 -> 120 us, 48 of 2929 (2.25) 133 -> 117, 32 of 5120 (2.5) 236 -> 221,
+// 32 of 5632 (2.75) 269 -> 263, but 40 of 4538 (2.81) 214 -> 216, 32 of 6656 (3.25) 339 -> 350; 128-row tiles, 12 heads of
+// 5000 (1.9) 128 -> 106, 24 of 3072, sums and maxima (2.25) 79 -> 72, 32 of 3072 x 256 (3) 155 -> 150, 8 of 16384 (4) 530 -> 514,
+// nothing lost beyond and within 1 % of it.  (All bf16 or fp16, D = 128 where none is named.)
+int fill_places(const Params& p, const TileChoice& t, bool causal) {
+  const int cus = chip_cus();
+  if (!causal || p.splits > 1 || p.group != p.bh_count || p.total <= cus || t.per_cu < 2) return 0;
+  return (int64_t)p.total * 4 <= (int64_t)cus * (t.rows > 128 ? 11 : 16) ? cus : 0;
+}
+
 int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H, int M, int N, int D,
                 const int64_t qs[4], const int64_t ks[4], float scale, bool by_keys, bool causal,
                 int col_mode = kModeSum) {
@@ -3266,9 +3280,7 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   // the device is first asked (for its CU count) here, after every argument check
   const int ksteps = ksteps_of(dtype, D);
   const bool f32 = dtype == FCR_DTYPE_F32;
-  const int trows = !by_keys ? row_tile_rows(f32, ksteps, M, N, bh, causal)
-                    : f32    ? f32_col_tile(f32_ksteps(ksteps), col_mode == kModeBoth, M, N, bh, causal).rows()
-                             : kWaves * 32 * col_tile_blocks(ksteps, col_mode, N, bh, causal);
+  const int trows = tile_choice(f32, ksteps, M, N, bh, by_keys, col_mode, causal).rows;
   const int64_t tiles = ((by_keys ? N : M) + trows - 1) / trows;
   p.q = static_cast<const char*>(q);
   p.k = static_cast<const char*>(k);
@@ -3802,7 +3814,7 @@ int fcr_row_lse(const void* q, const void* k, float* lse, int dtype, int B, int 
   p.total *= p.splits;
   const int ksteps = ksteps_of(dtype, D);
   p.group = head_group(p.bh_count, (int64_t)p.tiles * p.splits, causal != 0);
-  p.fill = fill_ranks(p, dtype == FCR_DTYPE_F32 ? 8 / f32_row_tile(M, N, p.bh_count, causal != 0).waves : ksteps > kMaxKSteps ? 1 : 2, causal != 0);
+  p.fill = fill_places(p, tile_choice(dtype == FCR_DTYPE_F32, ksteps, M, N, p.bh_count, false, 0, causal != 0), causal != 0);
   hipStream_t s = static_cast<hipStream_t>(stream);
   launch_sweeps(dtype, 0, p, ksteps, causal != 0, 0, s);
   rc = launched("row_lse_kernel");
@@ -3829,8 +3841,7 @@ int col_reduce_any(const void* q, const void* k, const float* lse, void* out, vo
   if (rc) return rc;
   p.group = head_group(p.bh_count, p.tiles, causal != 0);
   const int ksteps = ksteps_of(dtype, D);
-  p.fill = fill_ranks(p, dtype == FCR_DTYPE_F32 ? 8 / f32_col_tile(f32_ksteps(ksteps), mode == kModeBoth, M, N, p.bh_count, causal != 0).waves : ksteps > kMaxKSteps ? 1 : 2,
-                      causal != 0);
+  p.fill = fill_places(p, tile_choice(dtype == FCR_DTYPE_F32, ksteps, M, N, p.bh_count, true, mode, causal != 0), causal != 0);
   p.lse = const_cast<float*>(lse);
   p.out = out;
   p.out2 = out2;

@@ -312,6 +312,14 @@ def test_causal_launches_that_are_on_the_chip_at_once(b, h, m, n, d):
     run_all(q, k, True, what=f"{b}x{h} {m}x{n}x{d}", reductions=["sum", "max"])
 
 
+@pytest.mark.parametrize("b,h,m,n,d", [(1, 71, 1900, 1850, 16), (1, 67, 1100, 1100, 32), (5, 7, 1100, 1090, 256), (1, 33, 2048, 2050, 136)])
+def test_causal_launches_of_two_to_four_workgroups_per_cu(b, h, m, n, d):
+    """The second workgroup of every CU dealt backwards and a third helping behind it: 256-row and 128-row tiles, heads that do
+    not divide the eight dies, numbers of workgroups that are no multiple of eight."""
+    q, k = _inputs.randn_pair(b, h, m, n, d, seed=m + d)
+    run_all(q, k, True, what=f"{b}x{h} {m}x{n}x{d}", reductions=["sum", "max"])
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("b,h,m,n,d", [(1, 2, 256, 256, 64), (1, 1, 2, 65, 4), (2, 3, 65, 63, 72), (1, 4, 191, 961, 128),
                                        (1, 8, 960, 960, 132), (1, 128, 64, 128, 16), (1, 129, 64, 128, 32),
