@@ -1318,6 +1318,28 @@ def test_topk_bins_of_many_keys(n, c):
         assert torch.equal(thr.cpu(), rows.sort(dim=1, descending=True).values[:, k - 1]), (n, c, k)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [9, 2040, 2048, 2049, 8192, 8199, 16384, 16391, 32768, 32775, 65536, 65537])
+def test_topk_16_bit_rows_of_any_bits(n, dtype):
+    """16-bit rows at the edges of the workgroups that hold them, bases of every 2-byte alignment: every bit pattern (infinities,
+    NaNs, denormals, both zeros), one value in most columns, a bin of a few values, all equal to the largest key (NaN).  Mask and
+    threshold are exact."""
+    from oracle.colreduce_oracle import topk_mask_ref
+    g = torch.Generator().manual_seed(n)
+    r = torch.randint(-32768, 32768, (5, n), generator=g, dtype=torch.int32).to(torch.int16).view(dtype)
+    r[1] = torch.randn(n, generator=g).exp().to(dtype)
+    r[2] = torch.where(r[1].float() < 3, torch.ones(()), r[1].float()).to(dtype)
+    r[3] = (1 + torch.randint(0, 5, (n,), generator=g) * 2.0 ** -7).to(dtype)
+    r[3, n // 2] = float("inf")
+    r[4] = float("nan")
+    dev = r.cuda()
+    for k in (1, n // 4 + 1, n // 2, n - 1, n):
+        mask, thr = fca.topk_keep_mask(dev, k, return_threshold=True)
+        assert (mask.cpu().numpy() == topk_mask_ref(r.float().numpy(), k)).all(), (n, k)
+        kth = r.float().sort(dim=1, descending=True).values[:, k - 1]
+        torch.testing.assert_close(thr.cpu() + 0.0, kth + 0.0, rtol=0, atol=0, equal_nan=True)
+
+
 def test_topk_on_reduced_columns():
     from oracle.colreduce_oracle import topk_mask_ref
     q, k = _inputs.config4(heads=4, n=2048)
