@@ -98,6 +98,18 @@ def load():
     return _lib
 
 
+def host():
+    """The module of csrc/host.cpp (the usual call in native code), its errors raised by check()."""
+    load()
+    try:
+        from . import _host
+    except ImportError as e:
+        raise RuntimeError(f"{os.path.join(_HERE, '_host.so')} cannot be loaded ({e}): build it with "
+                           "`python -m flash_colreduce_amd.build` (there is no fallback path)") from e
+    _host.on_error(check)
+    return _host
+
+
 def strides4(values):
     return _I64x4(*[int(v) for v in values])
 

@@ -63,6 +63,29 @@ def build(verbose: bool = True, extra_flags=()) -> str:
     return LIB
 
 
+HOST_SRC = os.path.join(HERE, "csrc", "host.cpp")
+HOST_LIB = os.path.join(HERE, "_host.so")
+
+
+def build_host(verbose: bool = True) -> str:
+    """The native host path (csrc/host.cpp): a Python module on torch's C++ interface and libfcr.so next to it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    include = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include", INCLUDE]
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{d}" for d in include], HOST_SRC,
+           "-o", HOST_LIB, "-L", libs, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-L", HERE, "-lfcr",
+           "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    return HOST_LIB
+
+
 C_CHECK_SRC = os.path.join(ROOT, "tests", "c_abi", "check.c")
 C_CHECK_BIN = os.path.join(ROOT, "tests", "c_abi", "check")
 
@@ -81,4 +104,5 @@ def build_c_check(verbose: bool = True) -> str:
 
 if __name__ == "__main__":
     build(extra_flags=sys.argv[1:])
+    build_host()
     build_c_check()

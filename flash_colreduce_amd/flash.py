@@ -19,6 +19,17 @@ __all__ = ["flash_colreduce", "flash_colreduce_multi", "row_lse2", "topk_keep_ma
 _DTYPES = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16, torch.float32: _lib.DTYPE_F32}
 
 
+_native = None
+
+
+def _host():
+    """csrc/host.cpp: answers the calls that need neither a copy nor a message, and None to all others."""
+    global _native
+    if _native is None:
+        _native = _lib.host()
+    return _native
+
+
 def _validate(query: torch.Tensor, key: torch.Tensor, reduction: Optional[str]):
     # flash.py:354-364, same order and messages
     if not query.is_cuda or not key.is_cuda:
@@ -258,6 +269,10 @@ def flash_colreduce(
     dtype (flash.py:308, 377-385).  torch.float32 returns the kernel's fp32 result, with the
     mean division done in fp32.
     """
+    if query.is_cuda:
+        out = (_native or _host()).reduce(query, key, reduction, is_causal, scale, out_dtype, False)
+        if out is not None:
+            return out
     _validate(query, key, reduction)
     b, h, m, _ = query.shape
     n = key.shape[2]
@@ -292,6 +307,12 @@ def flash_colreduce_multi(
     reductions = list(reductions)
     if not reductions:
         raise ValueError("reductions must name at least one of 'sum', 'mean', 'max'.")
+    if len(reductions) == 2 and "max" in reductions and query.is_cuda:
+        other = reductions[0] if reductions[1] == "max" else reductions[1]
+        if other != "max":
+            pair = (_native or _host()).reduce(query, key, other, is_causal, scale, out_dtype, True)
+            if pair is not None:
+                return pair if reductions[1] == "max" else (pair[1], pair[0])
     _validate(query, key, reductions[0])
     for r in reductions[1:]:
         if r not in ("sum", "mean", "max"):
@@ -348,6 +369,9 @@ def topk_keep_mask(scores: torch.Tensor, k: int, return_threshold: bool = False)
     """
     if not scores.is_cuda:
         raise ValueError("scores must be on CUDA device.")
+    kept = (_native or _host()).keep(scores, k, return_threshold)
+    if kept is not None:
+        return kept
     if scores.dtype not in _DTYPES or scores.dim() < 1:
         raise ValueError(f"scores must be a float32, float16 or bfloat16 tensor with at least one dimension. "
                          f"Got {scores.dtype}.")

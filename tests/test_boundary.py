@@ -199,3 +199,17 @@ def test_naive_colreduce_matches_oracle_small(m, n, causal):
         torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-7)
     with pytest.raises(ValueError, match="Invalid reduction"):
         fca.naive_colreduce(q, k, "median")
+
+
+def test_native_host_path_leaves_the_rest_to_python():
+    """Without a device nothing is for the native path: tensors on the host, other objects, wrong counts of arguments."""
+    host = _lib.host()
+    x = torch.zeros(1, 1, 2, 8)
+    assert host.reduce(x, x, "sum", False, None, None, False) is None
+    assert host.reduce(x, None, "sum", False, None, None, False) is None
+    assert host.reduce(x, x, ["sum"], False, None, None, True) is None
+    assert host.keep(x, 1, False) is None and host.keep("x", 1, False) is None
+    with pytest.raises(TypeError):
+        host.reduce(x, x)
+    with pytest.raises(TypeError):
+        host.keep(x)

@@ -1505,6 +1505,92 @@ def test_plain_c_caller_of_the_c_abi():
     assert done.returncode == 0 and done.stdout.strip() == "ok", (done.returncode, done.stdout, done.stderr)
 
 
+class _NeverNative:
+    """Stands in for the native host path and answers nothing."""
+    def reduce(self, *a):
+        return None
+
+    def keep(self, *a):
+        return None
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_native_host_path_gives_what_the_general_one_gives(dtype, monkeypatch):
+    """Layouts, result types, scales and orders: the native path and the Python one run the same launches, so results
+    are equal bit for bit; what would need a copy, a message or another device is left to the Python one."""
+    from flash_colreduce_amd import flash as F
+    b, h, m, n, d = 2, 3, 70, 1100, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda", generator=g).to(dtype)
+
+    q, k = rand(b, h, m, d), rand(b, h, n, d)
+    qt, kt = rand(b, m, h, d).transpose(1, 2), rand(b, n, h, d).transpose(1, 2)
+    odd = rand(b, h, m, d + 3)[..., :d]                        # rows off their alignment: copied
+    cases = [(q, k, True), (qt, kt, True), (qt, k, True), (q[:1], k[:1], True), (q[:, :, :1], k, True), (q, k[:, :, 5:905], True),
+             (q, k[:1].expand(b, h, n, d), True), (q.as_strided((1, 1, 1, d), (7, 3, 5, 1)), k[:1, :1], True), (odd, k, False),
+             (q.expand(b, h, m, d)[:, :, :1].expand(b, h, m, d), k, False), (rand(b, h, m, 20)[..., :18], rand(b, h, n, 20)[..., :18], False),
+             (q.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2), k, False)]
+    calls = []
+    for x, y, native in cases:
+        assert (F._host().reduce(x, y, "sum", False, None, None, False) is not None) == native
+        for red, causal, scale, out in (("sum", True, None, None), ("mean", 1, 0.3, torch.float32), ("max", False, -0.2, torch.bfloat16)):
+            calls.append(lambda x=x, y=y, red=red, causal=causal, scale=scale, out=out: fca.flash_colreduce(x, y, red, causal, scale, out_dtype=out))
+        for reds in (["sum", "max"], ("max", "mean"), ["max", "max"], ["mean", "sum"], ["max"], ["sum", "max", "sum"]):
+            calls.append(lambda x=x, y=y, reds=reds: fca.flash_colreduce_multi(x, y, reds, is_causal=True))
+    s = rand(b, h, n)
+    for scores in (s, s[0], s[0, 0], s[:, :, ::2], s.float(), s.permute(2, 0, 1), rand(3, 1, 70000)):
+        for kk in (0, 5, scores.shape[-1], -3, True):
+            calls.append(lambda scores=scores, kk=kk: fca.topk_keep_mask(scores, kk, return_threshold=kk != 5))
+
+    def flat(r):
+        return list(r) if isinstance(r, tuple) else [r]
+
+    native = [flat(c()) for c in calls]
+    monkeypatch.setattr(F, "_native", _NeverNative())
+    for c, got in zip(calls, native):
+        want = flat(c())
+        assert len(want) == len(got)
+        for x, y in zip(got, want):
+            assert x.shape == y.shape and x.dtype == y.dtype and x.is_contiguous()
+            assert torch.equal(torch.nan_to_num(x.float(), nan=7.5), torch.nan_to_num(y.float(), nan=7.5))
+
+
+def test_native_host_path_under_capture_streams_and_modes():
+    """Allocations and launches go where torch's would: into a captured graph (replayed with other contents and eager calls between),
+    on the caller's stream, out of inference mode; a refused argument of the library raises its error."""
+    from flash_colreduce_amd import _lib
+    q, k = (x.cuda() for x in _inputs.randn_pair(1, 4, 90, 300, 64, seed=1))
+    q2, k2 = (x.cuda() for x in _inputs.randn_pair(1, 4, 90, 300, 64, seed=2))
+    want = [fca.flash_colreduce(a, c, "mean", True) for a, c in ((q, k), (q2, k2))]
+    masks = [fca.topk_keep_mask(w, 30) for w in want]
+    qs, ks = q.clone(), k.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fca.flash_colreduce(qs, ks, "mean", True)
+        mask = fca.topk_keep_mask(out, 30)
+    for i in (1, 0, 1):
+        qs.copy_((q, q2)[i])
+        ks.copy_((k, k2)[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[i]) and torch.equal(mask, masks[i])
+        assert torch.equal(fca.flash_colreduce(q, k, "mean", True), want[0])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(2_000_000)
+        late = q.clone()
+        assert torch.equal(fca.flash_colreduce(late, k, "mean", True), want[0])
+    with torch.inference_mode():
+        r = fca.flash_colreduce(q, k, "mean", True)
+        assert r.is_inference() and torch.equal(r, want[0])
+    assert not fca.flash_colreduce(q.clone().requires_grad_(), k, "mean", True).requires_grad
+    with pytest.raises(_lib.FcrError):
+        fca.flash_colreduce(q, k, "sum", scale=float("inf"))
+
+
 def test_python_errors_on_device():
     q = torch.zeros(1, 2, 4, 8, dtype=torch.float16, device="cuda")
     k = torch.zeros(1, 2, 6, 8, dtype=torch.float16, device="cuda")
