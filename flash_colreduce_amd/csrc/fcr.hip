@@ -1326,7 +1326,8 @@ __device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes 
   }
 }
 
-// A sweep over chunks [t0, t1), whose scaled scores go to `consume` a sub-step at a time, in order; those of [ta, tb) need no mask.
+// A sweep over chunks [t0, t1), the first of them fetched by the caller, whose scaled scores go to `consume` a sub-step at a time,
+// in order; those of [ta, tb) need no mask.
 // Per chunk one barrier, behind which it is staged and the other stage is free.  Under the matrix instructions of an
 // unmasked chunk run the split of the next one (fetched a chunk ago) and `consume` for the sub-step before, whose scores are kept for
 // it.  aux_of(t, sub) is what consume needs besides the scores, extra(t) what travels with a chunk; general(t, exact) does
@@ -1339,7 +1340,6 @@ __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, cons
   using Rg = SplitRing<KS, SPLIT, NW>;
   constexpr int SG = f32_groups(KS), SUBS = Rg::kChunkRows / (16 * SG), STEPS = SUBS * KS, PER = Rg::kPer;
   if (t0 >= t1) return;
-  rg.template fetch<AUX>();
   ring_sync<63>();   // (the words at bad() are set)
   rg.put(t0, tid);
   extra(t0);
@@ -1435,6 +1435,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
   }
   Rg rg;
   rg.init(smem, kb, p.k_sr, c_begin * kRows, keys_end, p.dgran, tid);
+  rg.template fetch<(STREAM_ONCE ? kLoadOnce : 0)>();   // in flight together with the resident rows
   Planes qf[KS][NG];
   float qs2[NG];   // scale2 times what undoes the scale of the lane's query
   const bool q_bad = load_resident_split<KS, NG, SPLIT>(qf, qs2, qb, p.q_sr, q0, p.M, p.dgran, lane);
@@ -1535,6 +1536,14 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
 
   Rg rg;
   rg.init(smem, qb, p.q_sr, t0 * kRows, p.M, p.dgran, tid);
+  // the lse of a chunk's queries (+inf past M: they contribute 2^-inf) travels with its rows
+  float lse_raw = 0.f;
+  auto lse_fetch = [&](int t) {
+    const int i = t * kRows + tid;
+    if (tid < kRows) lse_raw = (i < p.M) ? lse[i] : kPosInf;
+  };
+  rg.fetch();   // in flight together with the resident rows
+  lse_fetch(t0);
   Planes kf[KS][NG];
   f32x4 ks4[NG];   // what undoes the scale of the lane's four keys per group
   bool k_bad;
@@ -1548,12 +1557,6 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
   }
   const bool idle = k0[0] >= p.N;
 
-  // the lse of a chunk's queries (+inf past M: they contribute 2^-inf) travels with its rows
-  float lse_raw = 0.f;
-  auto lse_fetch = [&](int t) {
-    const int i = t * kRows + tid;
-    if (tid < kRows) lse_raw = (i < p.M) ? lse[i] : kPosInf;
-  };
   auto extra = [&](int t) {
     if (tid < kRows) rg.extra_of(t)[tid] = lse_raw;
     lse_fetch(t + 1);
@@ -1607,7 +1610,6 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
       }
     }
   };
-  lse_fetch(t0);
   split_sweep<true, 0, QueryFacts>(
       t0, t_int, SPLIT ? nchunks : p.M / kRows, nchunks, kf, rg, tid, idle, k_bad, extra, facts_at,
       [&](f32x4(&a)[NG][SG], const QueryFacts& q) {
