@@ -1837,7 +1837,10 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ 
 // NQ: groups of sixteen queries a wave holds (4; 2 for at most 32 queries: the registers then hold the scores of
 // twice as many keys per pair, and the time between two sweeps is spread over that many.  One group and four
 // times the keys was built as well and was slower than two: 1568 against 1499 us on 64 x 32 pairs of 16384 keys).
-template <int DT, int KS, bool CAUSAL, int MODE, int QH, int NQ = 4>
+// SKIP: chunks past the last key are left out instead of being computed and hidden score by score.  The team waits for its last
+// workgroup, which holds them: 6 x 40 pairs of 111 x 7284 x 128 206 -> 165 us per call, 5 x 24 of 89 x 3776 x 64 51 -> 43,
+// 7 x 24 of 100 x 15756 x 128 249 -> 237 (bf16, sums).
+template <int DT, int KS, bool CAUSAL, int MODE, int QH, int NQ, bool SKIP>
 __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Params p) {
   static_assert(NQ == 4 || (QH == 1 && NQ == 2), "fewer query groups only with one query half");
   constexpr int KG = kFusedSteps * (4 / NQ);     // steps per pair
@@ -2023,6 +2026,12 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
       if (j == 0) read_queries();   // (staged at least a whole sweep ago; the barrier above has published them)
       if (j == 1 && it + 1 < rounds) stage_queries(bh + T);   // every wave has read this pair's by now
       const char* lds = stage_of(cons_chunk + j * KH + kh);
+      if (SKIP && (c0a + j * KH + kh) * kChunk >= p.N) {
+        const float none = KEEP ? kNegInf : 0.f;
+#pragma unroll
+        for (int g = 0; g < NQ; ++g) sc[j][g] = (f32x4){none, none, none, none};
+        continue;
+      }
 #pragma unroll
       for (int g = 0; g < NQ; ++g) sc[j][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -3796,22 +3805,37 @@ bool fits_per_cu(K kernel, int threads, int want) {
   return n >= want;
 }
 
-template <int DT, int KS, int MODE, int QH, int NQ = 4>
-void launch_col_fused_mode(const Params& p, bool causal, hipStream_t s) {
+template <int DT, int KS, int MODE, int QH, int NQ, bool SKIP>
+void launch_col_fused_form(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(kFusedThreads);
   static int fits[2] = {-1, -1};   // asked once per kernel (the answer depends on its registers and LDS, not on the device of a kind)
   int f = __atomic_load_n(&fits[causal], __ATOMIC_RELAXED);
   if (f < 0) {
-    f = causal ? fits_per_cu(col_fused_kernel<DT, KS, true, MODE, QH, NQ>, kFusedThreads, 1)
-               : fits_per_cu(col_fused_kernel<DT, KS, false, MODE, QH, NQ>, kFusedThreads, 1);
+    f = causal ? fits_per_cu(col_fused_kernel<DT, KS, true, MODE, QH, NQ, SKIP>, kFusedThreads, 1)
+               : fits_per_cu(col_fused_kernel<DT, KS, false, MODE, QH, NQ, SKIP>, kFusedThreads, 1);
     __atomic_store_n(&fits[causal], f, __ATOMIC_RELAXED);
   }
   if (!f) {
     fcr_detail::fused_refused = true;
     return;
   }
-  if (causal) hipLaunchKernelGGL((col_fused_kernel<DT, KS, true, MODE, QH, NQ>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((col_fused_kernel<DT, KS, false, MODE, QH, NQ>), grid, block, 0, s, p);
+  if (causal) hipLaunchKernelGGL((col_fused_kernel<DT, KS, true, MODE, QH, NQ, SKIP>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((col_fused_kernel<DT, KS, false, MODE, QH, NQ, SKIP>), grid, block, 0, s, p);
+}
+
+// More than 64 queries: maxima gain nothing by leaving chunks out (ragged rows are hidden one by one in any case; sums and
+// maxima 323 -> 325 us), and where there is nothing to leave out the question alone costs (4 x 32 pairs of 89 x 4096 x 64
+// 40.7 -> 42.6 us, 32 of 128 x 4096 x 128 17.6 -> 17.8), so the host asks it.
+template <int DT, int KS, int MODE, int QH, int NQ>
+void launch_col_fused_mode(const Params& p, bool causal, hipStream_t s) {
+  if constexpr (QH == 2 && MODE != kModeSum) return launch_col_fused_form<DT, KS, MODE, QH, NQ, false>(p, causal, s);
+  else if constexpr (QH == 2) {
+    const int chunks = (p.N + kChunk - 1) / kChunk;
+    if (chunks % fused_chunks(QH, NQ) != 0) return launch_col_fused_form<DT, KS, MODE, QH, NQ, true>(p, causal, s);
+    launch_col_fused_form<DT, KS, MODE, QH, NQ, false>(p, causal, s);
+  } else {
+    launch_col_fused_form<DT, KS, MODE, QH, NQ, true>(p, causal, s);
+  }
 }
 
 template <int DT, int KS, int QH, int NQ>

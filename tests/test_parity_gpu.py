@@ -749,6 +749,17 @@ def test_single_sweep_rows_of_padding_meet_a_non_finite_key(m, causal):
         check(got, colreduce_ref(q, k, red, causal), red, f"padding rows m{m} {red}")
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("m,n,d", [(100, 1030, 64), (128, 1537, 128), (65, 1024 + 448, 32), (40, 1100, 128), (64, 2049, 64), (20, 2100, 128),
+                                   (2, 4100, 96)])
+def test_single_sweep_chunks_past_the_last_key(m, n, d, causal):
+    """The last workgroup of a team holds whole chunks past the last key, from one to all but one of them: left out in the
+    first sweep, and hidden in the second one (scores far from zero) and where maxima are asked for."""
+    q, k = _inputs.randn_pair(2, 3, m, n, d, seed=n)
+    run_all(q, k, causal, what=f"{m}x{n}x{d}")
+    run_all(q * 40, k, causal, what=f"{m}x{n}x{d} far from zero")
+
+
 def test_single_sweep_bounded_wait():
     """The wait for the team is bounded from the host: with a limit of zero polls a workgroup whose partners
     have not all published gives up at once, stores NaN for its columns of that pair, sets the status word
