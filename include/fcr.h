@@ -131,7 +131,7 @@ int fcr_topk_mask(const float* scores, uint8_t* mask, float* threshold, int64_t 
 
 /*
  * fcr_topk_mask with scratch memory, for long rows: with ws_bytes >= fcr_topk_bytes(rows, N) > 0 a row of
- * more than 32768 columns is spread over workgroups of 8192 columns (five launches: four digits of a
+ * more than 32768 columns is spread over workgroups of 8192 or 32768 columns (five launches: four digits of a
  * radix select, then the mask) instead of being walked by one workgroup; same result, bit for bit.
  * fcr_topk_bytes returns 0 where the scratch would not be used (N <= 32768); with ws NULL or too small
  * the call is fcr_topk_mask.  ws must be 16-byte aligned; its contents before and after are irrelevant.
@@ -143,14 +143,15 @@ int fcr_topk_mask_ws(const float* scores, uint8_t* mask, float* threshold, int64
 /*
  * The same for score rows of any FCR_DTYPE_* element type: fp16 and bf16 rows, as fcr_colreduce_to stores
  * them for 16-bit operands, are read as they are (order and ties of the stored values; threshold stays
- * fp32).  ws may be NULL (then ws_bytes is ignored); fcr_topk_bytes does not depend on the type.
+ * fp32).  ws may be NULL (then ws_bytes is ignored); fcr_topk_bytes does not depend on the type, 16-bit
+ * rows of up to 65536 columns do not read ws.
  */
 int fcr_topk_mask_typed(const void* scores, int dtype, uint8_t* mask, float* threshold, int64_t rows, int N, int k,
                         void* ws, size_t ws_bytes, void* stream);
 
 /*
- * A faster and less exact alternative to FCR_DTYPE_F32 for fp32 operands whose values fit fp16 (the
- * one set of fp16 numbers for the whole operand, without a scale by row): packs a contiguous fp32 [rows, D] into the fp16 [rows, terms * Dp] (Dp = D rounded up
+ * A less exact alternative to FCR_DTYPE_F32 for fp32 operands whose values fit fp16 (packed once, without
+ * a scale by row): packs a contiguous fp32 [rows, D] into the fp16 [rows, terms * Dp] (Dp = D rounded up
  * to 8, zero padded) that the kernels above take with D' = terms * Dp and dtype FCR_DTYPE_F16.
  * terms = 3 writes [hi | hi | lo] for queries (is_key = 0) and [hi | lo | hi] for keys (is_key != 0),
  * hi = fp16(x), lo = fp16(x - hi): the kernels then see q.k to about 2^-22.  terms = 1 writes [hi].
