@@ -2575,7 +2575,7 @@ __global__ __launch_bounds__(256) void one_query_columns_kernel(const Params p, 
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32 operands.  x = hi + lo with hi = fp16(x), lo = fp16(x - hi) carries 22 bits of x.  Packing
+// fp32 operands packed by the caller.  x = hi + lo with hi = fp16(x), lo = fp16(x - hi) carries 22 bits of x.  Packing
 // queries as [hi | hi | lo] and keys as [hi | lo | hi] along d makes the fp16 kernels compute
 // q_hi.k_hi + q_hi.k_lo + q_lo.k_hi, the product to about 2^-22 (the lo.lo term is dropped), with fp32
 // accumulation.  With terms == 1 only [hi] is written (both operands rounded to fp16).
