@@ -1072,7 +1072,9 @@ __device__ __forceinline__ void row_scale(uint32_t largest, float& up, float& do
   up = __builtin_bit_cast(float, (268u << 23) - e);
   down = __builtin_bit_cast(float, e - (14u << 23));
 }
-__device__ __forceinline__ bool has_no_scale(uint32_t largest) { return largest >= 0x7f800000u; }   // (infinity, NaN)
+// Infinities, NaNs, and rows from 2^104 on: a sum of up to 256 products of two scaled rows reaches 2^38 and is first multiplied by
+// what undoes the scale of the key, 2^(E - 14) for a row whose largest element is at 2^E, whatever the query is.
+__device__ __forceinline__ bool has_no_scale(uint32_t largest) { return largest >= (231u << 23); }
 
 __device__ __forceinline__ Planes split8(const f32x4& a, const f32x4& b, float up) {
   Planes s;

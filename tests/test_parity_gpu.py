@@ -386,6 +386,25 @@ def test_fp32_split_rows_of_any_magnitude(d):
         assert (err <= 2.0 ** -20 * size.amax(-1) + 2.0 ** -19).all(), (up, (err / (size.amax(-1) + 2)).max())
 
 
+@pytest.mark.parametrize("exponent", [-125, -120, -115, -110, -100, 88, 100, 103, 104, 106, 108, 110, 112, 115, 120, 124])
+@pytest.mark.parametrize("m,n,d", [(70, 300, 128), (300, 1100, 64), (260, 130, 256), (130, 70, 24)])
+def test_fp32_operands_near_the_ends_of_the_range(m, n, d, exponent):
+    """Finite keys and queries whose magnitudes make up for each other: the results are those of the same operands at
+    magnitude one.  A power of two changes no bit of a product; a denormal element (2^-125 N(0,1) holds some) is held to
+    2^-149, which is 2^-23 of it or more, so there the bound is the one of scores that are off by 2^-22 each."""
+    q, k = _inputs.randn_pair(1, 2, m, n, d, seed=m + d, dtype=torch.float32)
+    if exponent < 0:
+        k = (k * 2.0 ** exponent) * 2.0 ** -exponent   # the bits a denormal loses
+    else:
+        q = (q * 2.0 ** -exponent) * 2.0 ** exponent
+    big, small = k * 2.0 ** exponent, q * 2.0 ** -exponent
+    assert torch.isfinite(big).all() and torch.isfinite(small).all()
+    for red in REDUCTIONS:
+        got = fca.flash_colreduce(small.cuda(), big.cuda(), red)
+        assert torch.isfinite(got).all(), red
+        torch.testing.assert_close(got.cpu(), colreduce_ref(q, k, red, False, compute_dtype=torch.float64).float(), rtol=1e-5, atol=1e-8)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("h,m,n,d", [(2, 200, 333, 64), (5, 130, 129, 128), (2, 300, 2100, 256), (140, 257, 130, 40), (2, 70, 99, 28)])
 def test_fp32_rows_without_a_scale(h, m, n, d, causal):
