@@ -68,6 +68,7 @@ struct Params {
   int dgran;         // D / 8: valid 16-byte granules per row
   int c;             // max(N - M, 0): the causal right-alignment offset
   float scale2;      // scale * log2(e)
+  float split_most;  // fp32 operands: see SplitRing::limit
   int tiles;         // resident tiles per (b,h)
   int bh_count;      // B * H
   int group;         // (b,h) pairs whose workgroups are launched together (see map_block)
@@ -1074,7 +1075,8 @@ __device__ __forceinline__ void row_scale(uint32_t largest, float& up, float& do
 }
 // Infinities, NaNs, and rows from 2^104 on: a sum of up to 256 products of two scaled rows reaches 2^38 and is first multiplied by
 // what undoes the scale of the key, 2^(E - 14) for a row whose largest element is at 2^E, whatever the query is.
-__device__ __forceinline__ bool has_no_scale(uint32_t largest) { return largest >= (231u << 23); }
+constexpr uint32_t kNoScale = 231u << 23;
+__device__ __forceinline__ bool has_no_scale(uint32_t largest) { return largest >= kNoScale; }
 
 __device__ __forceinline__ Planes split8(const f32x4& a, const f32x4& b, float up) {
   Planes s;
@@ -1124,8 +1126,8 @@ struct SplitRing {
   static constexpr int kPlane = kChunkRows * kPitch;
   static constexpr int kStage = 2 * kPlane;
   static constexpr int kRowFloats = 2 * kChunkRows;          // two floats per row of a stage: its scale, and what the caller adds
-  // two stages, their row floats, a word for each: see `bad`
-  static constexpr int kBytes = 2 * kStage + 2 * kRowFloats * 4 + 16;
+  // two stages, their row floats, a word for each (see `bad`) and one for each wave (see `set_limit`)
+  static constexpr int kBytes = 2 * kStage + 2 * kRowFloats * 4 + 16 + 4 * NW;
   static constexpr int kPer = kChunkRows * kRowGranules / kNumThreads;   // granules per thread
   static_assert(kPer * kNumThreads == kChunkRows * kRowGranules, "whole granules per thread");
 
@@ -1137,6 +1139,7 @@ struct SplitRing {
   f32x4 raw[kPer][2];     // the chunk in flight
   const char* next_ptr;
   int rows_left, row_bytes;
+  uint32_t limit;         // bits of the magnitude from which on a streamed row is not multiplied as two parts
 
   __device__ __forceinline__ void init(char* lds, const char* base, int64_t row_bytes64, int row0, int nrows, int dgran,
                                        int tid) {
@@ -1156,7 +1159,7 @@ struct SplitRing {
     frag0 = (uint32_t)((lane & 15) * kPitch + (((lane >> 4) ^ Ring<KS>::swz(lane & 15)) * 16));
     if (tid < 2) bad()[tid] = -1;
   }
-  // bad()[s]: the last chunk staged in stage s that holds a row without a scale
+  // bad()[s]: the last chunk staged in stage s that holds a row without a scale, or one that is too large for the resident rows
   __device__ __forceinline__ int* bad() const { return reinterpret_cast<int*>(smem + 2 * kStage + 2 * kRowFloats * 4); }
   __device__ __forceinline__ char* stage_of(int t) const { return smem + (t & 1) * kStage; }
   __device__ __forceinline__ float* scale_of(int t) const { return reinterpret_cast<float*>(smem + 2 * kStage) + (t & 1) * kRowFloats; }
@@ -1193,8 +1196,25 @@ struct SplitRing {
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) *reinterpret_cast<u32x4*>(stage_of(t) + t2 * kPlane + dst[i]) = s.p[t2];
   }
+  // What an element loses that is small beside the largest of its row, up to 2^-39 of that one, is lost in a score times the
+  // largest element of the other row.  Where no channel is large in both rows the score does not grow with that product, so the
+  // product has a limit: Params::split_most = 2^17 / (scale2 sqrt(D)) puts the error, as a sum of D such terms of
+  // either sign, at 2^-22 in the exponent of 2, what the fp32 instructions lose on N(0,1) rows of D = 128 (2.0e-7 of a score
+  // of about one).  Rows of the default scale get there with elements of 300 in both; keys and queries of
+  // N(0,1) are at 2^5, keys times eight at 2^8.
+  __device__ __forceinline__ void publish(int wave, uint32_t res_largest) {
+    if (SPLIT) bad()[4 + wave] = has_no_scale(res_largest) ? 0 : (int)res_largest;   // (such a wave multiplies on the fp32 instructions anyway)
+  }
+  __device__ __forceinline__ void set_limit(float split_most) {   // behind a barrier after publish()
+    if (!SPLIT) return;
+    uint32_t x = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) x = max(x, (uint32_t)bad()[4 + w]);
+    const float y = split_most / __builtin_bit_cast(float, x);
+    limit = min(__builtin_bit_cast(uint32_t, y), kNoScale);   // (a NaN has larger bits)
+  }
   __device__ __forceinline__ void note(int t, uint32_t largest) {
-    if (SPLIT && has_no_scale(largest)) bad()[t & 1] = t;
+    if (SPLIT && largest >= limit) bad()[t & 1] = t;
   }
   __device__ __forceinline__ void put(int t, int tid) {
     uint32_t largest = 0;
@@ -1212,9 +1232,10 @@ struct SplitRing {
   }
 };
 
-// The wave's resident rows as planes; down[g] undoes the scale of group g's row lane & 15.  Returns whether one of them has no scale.
+// The wave's resident rows as planes; down[g] undoes the scale of group g's row lane & 15.  Returns the bits of their largest
+// magnitude (not SPLIT: zero).
 template <int KS, int NG, bool SPLIT>
-__device__ __forceinline__ bool load_resident_split(Planes (&f)[KS][NG], float (&down)[NG], const char* base, int64_t row_bytes,
+__device__ __forceinline__ uint32_t load_resident_split(Planes (&f)[KS][NG], float (&down)[NG], const char* base, int64_t row_bytes,
                                                     const int (&rows)[NG], int nrows, int dgran, int lane) {
   uint32_t worst = 0;
 #pragma unroll
@@ -1247,7 +1268,7 @@ __device__ __forceinline__ bool load_resident_split(Planes (&f)[KS][NG], float (
         for (int t2 = 0; t2 < 2; ++t2) f[ks][g].p[t2] = __builtin_bit_cast(u32x4, x[ks][t2]);
     }
   }
-  return SPLIT && __builtin_amdgcn_ballot_w64(has_no_scale(worst)) != 0;
+  return SPLIT ? __builtin_amdgcn_readfirstlane(lanes_max<16>(worst)) : 0u;   // (the four rows of lanes hold the same)
 }
 
 // The same scores from the operands in memory, on the fp32 instructions.
@@ -1337,15 +1358,21 @@ __device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes 
 template <bool RESIDENT_IS_KEYS, int AUX, class Aux, bool SPLIT, int KS, int NG, int NW, class ExtraF, class AuxF, class ConsumeF,
           class GeneralF>
 __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, const Planes (&res)[KS][NG],
-                                            SplitRing<KS, SPLIT, NW>& rg, int tid, bool idle, bool res_bad, ExtraF&& extra,
+                                            SplitRing<KS, SPLIT, NW>& rg, int tid, bool idle, uint32_t res_largest, float split_most, ExtraF&& extra,
                                             AuxF&& aux_of, ConsumeF&& consume, GeneralF&& general) {
   using Rg = SplitRing<KS, SPLIT, NW>;
   constexpr int SG = f32_groups(KS), SUBS = Rg::kChunkRows / (16 * SG), STEPS = SUBS * KS, PER = Rg::kPer;
   if (t0 >= t1) return;
-  ring_sync<63>();   // (the words at bad() are set)
-  rg.put(t0, tid);
+  const bool res_bad = has_no_scale(res_largest);
+  uint32_t first_largest = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) rg.put_granule(i, t0, tid, first_largest);
   extra(t0);
   rg.template fetch<AUX>();
+  rg.publish(tid >> 6, res_largest);   // (the resident rows may still be on their way up to here)
+  ring_sync<63>();                     // (the words at bad() are set)
+  rg.set_limit(split_most);
+  rg.note(t0, first_largest);
   f32x4 kept[NG][SG];   // the scores not yet consumed
   Aux kept_aux;
   auto chunk = [&](int t, const Fragments<SG>& first, auto first_tag) {
@@ -1440,7 +1467,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
   rg.template fetch<(STREAM_ONCE ? kLoadOnce : 0)>();   // in flight together with the resident rows
   Planes qf[KS][NG];
   float qs2[NG];   // scale2 times what undoes the scale of the lane's query
-  const bool q_bad = load_resident_split<KS, NG, SPLIT>(qf, qs2, qb, p.q_sr, q0, p.M, p.dgran, lane);
+  const uint32_t q_largest = load_resident_split<KS, NG, SPLIT>(qf, qs2, qb, p.q_sr, q0, p.M, p.dgran, lane);
 #pragma unroll
   for (int g = 0; g < NG; ++g) qs2[g] *= p.scale2;
   const bool idle = q0[0] >= p.M;   // a wave whose rows all lie past M only helps staging
@@ -1488,7 +1515,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
     }
   };
   split_sweep<false, (STREAM_ONCE ? kLoadOnce : 0), KeyScales>(
-      c_begin, c_begin, t_int, nchunks, qf, rg, tid, idle, q_bad, [](int) {}, scales_at,
+      c_begin, c_begin, t_int, nchunks, qf, rg, tid, idle, q_largest, p.split_most, [](int) {}, scales_at,
       [&](f32x4(&a)[NG][SG], const KeyScales& s) {
         rescale(a, s);
         lse_update_groups(a, qs2, mref, l);
@@ -1548,10 +1575,10 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
   lse_fetch(t0);
   Planes kf[KS][NG];
   f32x4 ks4[NG];   // what undoes the scale of the lane's four keys per group
-  bool k_bad;
+  uint32_t k_largest;
   {
     float down[NG];
-    k_bad = load_resident_split<KS, NG, SPLIT>(kf, down, kb, p.k_sr, k0, p.N, p.dgran, lane);
+    k_largest = load_resident_split<KS, NG, SPLIT>(kf, down, kb, p.k_sr, k0, p.N, p.dgran, lane);
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
@@ -1613,7 +1640,7 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
     }
   };
   split_sweep<true, 0, QueryFacts>(
-      t0, t_int, SPLIT ? nchunks : p.M / kRows, nchunks, kf, rg, tid, idle, k_bad, extra, facts_at,
+      t0, t_int, SPLIT ? nchunks : p.M / kRows, nchunks, kf, rg, tid, idle, k_largest, p.split_most, extra, facts_at,
       [&](f32x4(&a)[NG][SG], const QueryFacts& q) {
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
@@ -3573,6 +3600,7 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   p.dgran = D * esize / 16;
   p.c = N > M ? N - M : 0;
   p.scale2 = (float)((double)scale * 1.4426950408889634);
+  p.split_most = (float)(131072.0 / (std::fabs((double)scale * 1.4426950408889634) * std::sqrt((double)D)));
   p.tiles = (int)tiles;
   p.bh_count = (int)bh;
   p.total = (int)(bh * tiles);

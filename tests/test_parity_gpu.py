@@ -405,6 +405,26 @@ def test_fp32_operands_near_the_ends_of_the_range(m, n, d, exponent):
         torch.testing.assert_close(got.cpu(), colreduce_ref(q, k, red, False, compute_dtype=torch.float64).float(), rtol=1e-5, atol=1e-8)
 
 
+@pytest.mark.parametrize("side", ["query", "key"])
+@pytest.mark.parametrize("exponent", [6, 10, 14, 18, 22, 26, 30, 60, 90])
+@pytest.mark.parametrize("h,m,n,d", [(2, 260, 300, 128), (1, 70, 1100, 64), (140, 257, 130, 256), (2, 300, 70, 36)])
+def test_fp32_channel_that_only_one_side_uses(h, m, n, d, exponent, side):
+    """A channel of 2^exponent in the rows of one operand (in every third row, so that tiles and chunks hold both kinds),
+    zero in the other's: it takes part in no score, and the others keep their precision.  A score in the exponent of 2
+    is off by 2^-21 of its sum of |q_d k_d|, by the rounding of that sum (under 2^-21 of it for the up to 16 terms of size that it
+    has) and by 2^-20 (four times the 2^-22 that the parts of small elements may lose); log2 of up to 1100 rounds to 2^-20 at most."""
+    q, k = _inputs.randn_pair(1, h, m, n, d, seed=m + d, dtype=torch.float32)
+    q, k = q.clone(), k.clone()
+    (q if side == "query" else k)[:, :, ::3, 5] = 2.0 ** exponent
+    (k if side == "query" else q)[..., 5] = 0.0
+    size = torch.matmul(q.double().abs(), k.double().abs().transpose(2, 3)).amax(-1) * (d ** -0.5 * 1.4427)
+    err = (fca.row_lse2(q.cuda(), k.cuda()).cpu().double() - row_lse2_ref(q, k, False).double()).abs()
+    assert (err <= 2.0 ** -20 * size + 2.0 ** -20 + 2.0 ** -20).all(), err.max()
+    for red in ("sum", "max"):
+        want = colreduce_ref(q, k, red, False, compute_dtype=torch.float64).float()
+        torch.testing.assert_close(fca.flash_colreduce(q.cuda(), k.cuda(), red).cpu(), want, rtol=1e-5, atol=1e-8)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("h,m,n,d", [(2, 200, 333, 64), (5, 130, 129, 128), (2, 300, 2100, 256), (140, 257, 130, 40), (2, 70, 99, 28)])
 def test_fp32_rows_without_a_scale(h, m, n, d, causal):
