@@ -976,17 +976,18 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
   u32x4 kf[NG][KS];
   load_resident<KS, NG>(kf, kb, p.k_sr, k0, p.N, p.dgran, lane);
 
-  auto general_chunk = [&](int t) {
+  auto general_chunk = [&](int t, auto ragged_tag) {
+    constexpr bool RAGGED = decltype(ragged_tag)::value;   // rows past M are among the chunk's
     advance(t);
     const char* lds = stage_of(t);
 #pragma unroll
     for (int sub = 0; sub < kChunk / 32; ++sub) {
       const int qs = t * kChunk + sub * 32;  // first query of the sub-tile
-      if (qs >= p.M) continue;
+      if (RAGGED && qs >= p.M) continue;
       LsePair lq = aux_of(lds, sub);
       // +inf for rows past M: they contribute 2^-inf = 0
-      if (qs + (lane & 15) >= p.M) lq.v[0] = kPosInf;
-      if (qs + 16 + (lane & 15) >= p.M) lq.v[1] = kPosInf;
+      if (RAGGED && qs + (lane & 15) >= p.M) lq.v[0] = kPosInf;
+      if (RAGGED && qs + 16 + (lane & 15) >= p.M) lq.v[1] = kPosInf;
       // the sub-step's fragments once, for all groups that see it
       u32x4 qfrag[2][KS];
 #pragma unroll
@@ -1005,6 +1006,10 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
           acc[0] = mma<DT>(kf[g][ks], qfrag[0][ks], acc[0]);
           acc[1] = mma<DT>(kf[g][ks], qfrag[1][ks], acc[1]);
         }
+        if (RAGGED) {   // rows of padding, zeros, may have met a non-finite key
+          if (qs + (lane & 15) >= p.M) acc[0] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          if (qs + 16 + (lane & 15) >= p.M) acc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
         const bool need_mask = CAUSAL && (kg + 15 > qs + p.c);
         if (need_mask) col_update<true, MODE>(acc, scale2, lq.v, csum[g], cmax[g], lim_lane + qs - kg);
         else col_update<false, MODE>(acc, scale2, lq.v, csum[g], cmax[g], 0);
@@ -1012,7 +1017,7 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
     }
   };
 
-  for (int t = t0; t < t_int; ++t) general_chunk(t);
+  for (int t = t0; t < t_int; ++t) general_chunk(t, std::false_type());
 
   pipelined_sweep<DT, KS, NG, true, LsePair>(
       t_int, nfull, kf, rg, advance, stage_of, aux_of,
@@ -1022,7 +1027,7 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
         for (int g = 0; g < NG; ++g) col_update<false, MODE>(a[g], scale2, lq.v, csum[g], cmax[g], 0);
       });
 
-  for (int t = nfull; t < nchunks; ++t) general_chunk(t);
+  for (int t = nfull; t < nchunks; ++t) general_chunk(t, std::true_type());
 
   ring_sync<0>();   // every load has landed (those past the last chunk write zeros): the LDS can be reused
   col_store<MODE, NG>(p, smem, bh, k0, csum, cmax, lane, wave);
@@ -1712,10 +1717,8 @@ __global__ __launch_bounds__(kThreads, (NG <= 4 ? 3 : 2)) void col_small_kernel(
   // -lse of the lane's queries; -inf hides the rows past M
   const int qrow = 4 * (lane >> 4);
   float nlse[NG][4];
-  int rows[NG];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    rows[g] = 16 * g;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * g + qrow + r;
@@ -1723,8 +1726,19 @@ __global__ __launch_bounds__(kThreads, (NG <= 4 ? 3 : 2)) void col_small_kernel(
       nlse[g][r] = (i < p.M) ? -v : kNegInf;
     }
   }
+  // Rows past M are copies of the last one, which are as finite as that one is against every key (zeros against an infinite key
+  // would make its columns NaN).
   u32x4 qf[NG][KS];
-  load_resident<KS, NG>(qf, qb, p.q_sr, rows, p.M, p.dgran, lane);
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const char* row = qb + (int64_t)min(16 * g + (lane & 15), p.M - 1) * p.q_sr;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int gi = ks * 4 + (lane >> 4);
+      const u32x4 v = *reinterpret_cast<const u32x4*>(row + min(gi, p.dgran - 1) * 16);
+      qf[g][ks] = gi < p.dgran ? v : (u32x4){0u, 0u, 0u, 0u};
+    }
+  }
 
   void* const out_max = (MODE == kModeBoth) ? p.out2 : p.out;
   float* obuf_max = obuf + (MODE == kModeBoth ? kFlush * kChunk : 0);

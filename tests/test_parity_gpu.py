@@ -348,6 +348,36 @@ def test_fp32_tiles_of_64_rows_give_the_bits_of_taller_ones(h, m, n, d, causal):
 
 
 @pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype,h,m,n,d", [(torch.float16, 2, 70, 99, 16), (torch.bfloat16, 2, 200, 333, 64), (torch.float16, 4, 300, 2100, 256),
+                                           (torch.bfloat16, 1, 65, 130, 512), (torch.float16, 32, 70, 4096, 64), (torch.bfloat16, 64, 1, 8192, 128),
+                                           (torch.float16, 32, 33, 2048, 128), (torch.float16, 2, 128, 64, 32)])
+def test_key_that_no_query_counts_beside_rows_of_padding(dtype, h, m, n, d, causal):
+    """Keys whose scores are -inf against every query: their columns are 0 in sums and maxima, with query counts that fill no
+    tile too, in the column kernels of the two-kernel path."""
+    q, k = (x.to(dtype) for x in _inputs.randn_pair(1, h, m, n, d, seed=m + n, dtype=torch.float32))
+    q, k = q.clone(), k.clone()
+    q[..., 3] = -q[..., 3].abs() - 0.1
+    dead = [0, n // 2, n - 1] if not causal else [n // 2]   # (queries that see an infinite key only have no softmax)
+    k[:, :, dead, 3] = float("inf")
+    keep = torch.tensor([j for j in range(n) if j not in dead])
+    c = max(n - m, 0)
+    vis = (torch.arange(m)[:, None] + c >= torch.arange(n)[None]) if causal else torch.ones(m, n, dtype=torch.bool)
+    s = torch.matmul(q[0].double(), k[0][:, keep].double().transpose(1, 2).contiguous()) * d ** -0.5
+    p = torch.softmax(s.masked_fill(~vis[:, keep], -math.inf), -1)
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    try:
+        for single in (0, 1):
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, single)
+            for red, w in (("sum", p.sum(1)), ("max", p.amax(1))):
+                got = fca.flash_colreduce(q.cuda(), k.cuda(), red, is_causal=causal, out_dtype=torch.float32).cpu()
+                assert (got[0][:, dead] == 0).all(), (red, single)
+                torch.testing.assert_close(got[0][:, keep], w.float(), rtol=2e-5, atol=1e-7)
+    finally:
+        lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+
+
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("h,m,n,d", [(130, 257, 300, 36), (180, 300, 257, 96), (130, 257, 300, 256), (9, 511, 700, 128),
                                      (1, 65, 33, 32), (3, 129, 1100, 28)])
 def test_fp32_split_tiles(h, m, n, d, causal):
