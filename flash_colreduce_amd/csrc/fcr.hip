@@ -156,7 +156,18 @@ inline int row_blocks_per_wave(int ksteps, int M, int N, int64_t bh, bool causal
   if (wgs2 < cus && N <= 1024) return 1;
   return (wgs2 >= cus && wgs2 < 2 * cus + (causal ? 1 : 0)) ? 1 : 2;
 }
-// Tiles of the fp32 sweeps (row_lse_f32_kernel, col_reduce_f32_kernel): waves per workgroup (four: two workgroups share a
+// fp32 operands of D >= 32 are multiplied as two fp16 parts by kernels of their own, shorter ones on the fp32 instructions by the
+// kernels of the 16-bit types (per call, against the staging through registers that those kernels do: 8 heads of 1024 x 1024 x 16
+// 21 us against 33, 32 of 4096 x 4096 x 16 376 against 601, 2 x 16 of 2048 x 2048 x 28 causal 89 against 94).
+inline bool in_parts(int dtype, int D) { return dtype == FCR_DTYPE_F32 && D >= 32; }
+// Those on the fp32 instructions that give at most one workgroup of 128 rows on every other CU take tiles of 64 rows, one 16-row
+// group per wave (NB = 0): such a launch lasts as long as one workgroup, and half the resident rows halve its matrix instructions.
+// A row sweep of 16 chunks or more is split over the idle CUs (row_splits) and keeps its tile.
+inline bool half_tiles(int dtype, int D, int64_t rows, int64_t bh) {
+  return dtype == FCR_DTYPE_F32 && !in_parts(dtype, D) && 2 * bh * ((rows + 127) / 128) <= chip_cus();
+}
+inline bool row_half_tiles(int dtype, int D, int M, int N, int64_t bh) { return N <= 15 * 64 && half_tiles(dtype, D, M, bh); }
+// Tiles of the fp32 sweeps in parts (row_lse_f32_kernel, col_reduce_f32_kernel): waves per workgroup (four: two workgroups share a
 // CU; eight: one) and resident 16-row groups per wave.  Two groups read a streamed fragment once for two blocks of scores,
 // eight waves share the split of a streamed row: 4 x 2 and 8 x 1 are 128 rows, 8 x 2 256, 4 x 1 64.  Per call, fp32:
 //   32 heads of 4096 x 4096 x 128   8x2 733 us, 4x2 828, 8x1 927      2 x 16 of 2048 x 2048 x 128 causal   4x2 141, 8x2 164, 8x1 160
@@ -189,9 +200,12 @@ inline F32Tile f32_row_tile(int M, int N, int64_t bh, bool causal) {
   return t.waves == 8 && t.groups == 1 && N > 15 * 64 && bh * ((M + 127) / 128) < chip_cus() ? F32Tile{4, 2} : t;
 }
 inline int f32_ksteps(int ksteps) { return (ksteps + 1) / 2; }   // k-steps of 32 d from k-steps of 64 bytes
-inline int row_tile_rows(bool f32, int ksteps, int M, int N, int64_t bh, bool causal) {
-  if (f32) return f32_row_tile(M, N, bh, causal).rows();
-  return kWaves * 32 * row_blocks_per_wave(ksteps, M, N, bh, causal);
+inline int elem_bytes(int dtype) { return dtype == FCR_DTYPE_F32 ? 4 : 2; }
+inline int ksteps_of(int dtype, int D) { return (D * elem_bytes(dtype) + 63) / 64; }
+inline int row_tile_rows(int dtype, int D, int M, int N, int64_t bh, bool causal) {
+  if (in_parts(dtype, D)) return f32_row_tile(M, N, bh, causal).rows();
+  if (row_half_tiles(dtype, D, M, N, bh)) return kWaves * 16;
+  return kWaves * 32 * row_blocks_per_wave(ksteps_of(dtype, D), M, N, bh, causal);
 }
 constexpr int kMaxKSteps = 8;                 // rows of up to 512 bytes: two workgroups per CU
 constexpr int kMaxKStepsF32 = 16;             // rows of up to 1 KiB (fp32: D <= 256, 16-bit elements: D <= 512), one workgroup per CU
@@ -277,9 +291,12 @@ __device__ __forceinline__ void map_block_split(const Params& p, bool longest_is
 // block b has b+1 (rows) or 8-b (columns) visible sub-tiles out of 8, so every wave gets 9 of the 36
 // and the four waves reach each barrier together.  With one block per wave, wave w keeps block w
 // of four.
+// With NB = 0 a wave keeps one group, w of four.
+__host__ __device__ constexpr int wave_group_count(int nb) { return nb ? 2 * nb : 1; }
 template <int NB>
-__device__ __forceinline__ void wave_groups(int tile, int wave, int (&rows)[2 * NB]) {
-  const int t0 = tile * (kWaves * 32 * NB);
+__device__ __forceinline__ void wave_groups(int tile, int wave, int (&rows)[wave_group_count(NB)]) {
+  const int t0 = tile * (kWaves * 16 * wave_group_count(NB));
+  if constexpr (NB == 0) rows[0] = t0 + 16 * wave;
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     // blocks w, 7-w (, 8+w, 15-w): even positions count up, odd ones count down inside a run of eight
@@ -675,7 +692,7 @@ struct NoAux {};
 template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE>
 __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(const Params p) {
   using Rg = Ring<KS>;
-  constexpr int NG = 2 * NB;
+  constexpr int NG = wave_group_count(NB);
   constexpr int kTileRows = kWaves * 16 * NG;
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes];
   int bh, tile, split;
@@ -910,7 +927,7 @@ inline int col_tile_blocks(int ksteps, int N, int64_t bh, bool causal) {
 template <int DT, int KS, bool CAUSAL, int MODE, int NB>
 __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_reduce_kernel(const Params p) {
   using Rg = Ring<KS>;
-  constexpr int NG = 2 * NB;
+  constexpr int NG = wave_group_count(NB);
   constexpr int kTileRows = kWaves * 16 * NG;
   constexpr int kRed = kWaves * NG * 4 * 64 * 4;      // end-of-sweep transpose buffer
   constexpr int kSmem = (Rg::kBytes > kRed) ? Rg::kBytes : kRed;
@@ -1041,8 +1058,8 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 // v_mfma_f32_16x16x4_f32 takes 256.  Error of the scores against sums in 64 bits, relative 2-norm over N(0,1) rows (and over
 // rows whose elements spread by e^(3 N(0,1))): D = 32 8.8e-8 (8.6e-8), 64 1.1e-7 (1.1e-7), 128 1.4e-7 (1.4e-7), 256
 // 1.9e-7 (1.6e-7); the fp32 instructions, which round the running sum after every term: 1.0e-7 (1.2e-7), 1.5e-7
-// (1.5e-7), 2.0e-7 (1.9e-7), 2.9e-7 (2.5e-7).  Shorter rows have few terms to round (D = 16 8.4e-8 against 7.4e-8): below
-// D = 32 the planes hold the floats themselves and the fp32 instructions multiply them.  A row with an infinity or a
+// (1.5e-7), 2.0e-7 (1.9e-7), 2.9e-7 (2.5e-7).  Shorter rows have few terms to round (D = 16 8.4e-8 against 7.4e-8) and do
+// not come here (in_parts).  A row with an infinity or a
 // NaN has no scale; chunks and resident rows that hold one are multiplied on the fp32 instructions, from memory (exact_scores).
 //
 // Streamed rows are split once per workgroup on their way to LDS: global -> registers (a chunk ahead) -> two planes of a
@@ -1058,7 +1075,7 @@ __device__ __forceinline__ float dpp_row(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-struct Planes {   // eight values of a row: h and l, or (not SPLIT) the first and the last four floats
+struct Planes {   // h and l of eight values of a row
   u32x4 p[2];
 };
 
@@ -1122,7 +1139,7 @@ constexpr int f32_chunk(int ks, int nw) { return (ks <= 2 ? 64 : ks <= 4 ? 32 : 
 constexpr int f32_groups(int ks) { return ks <= 4 ? 2 : 1; }   // streamed 16-row groups per sub-step
 
 // KS: k-steps of 32 d.
-template <int KS, bool SPLIT, int NW>
+template <int KS, int NW>
 struct SplitRing {
   static constexpr int kNumThreads = 64 * NW;
   static constexpr int kChunkRows = f32_chunk(KS, NW);
@@ -1186,18 +1203,12 @@ struct SplitRing {
   }
   // The chunk in the registers, number t, to its stage: granule by granule, or whole.
   __device__ __forceinline__ void put_granule(int i, int t, int tid, uint32_t& largest) {
-    Planes s;
-    if constexpr (SPLIT) {
-      const uint32_t m = lanes_max<kRowGranules>(largest8(raw[i][0], raw[i][1]));
-      largest = max(largest, m);
-      float up, down;
-      row_scale(m, up, down);
-      s = split8(raw[i][0], raw[i][1], up);
-      scale_of(t)[(i * kNumThreads + tid) / kRowGranules] = down;   // (by every thread of the row)
-    } else {
-      s.p[0] = __builtin_bit_cast(u32x4, raw[i][0]);
-      s.p[1] = __builtin_bit_cast(u32x4, raw[i][1]);
-    }
+    const uint32_t m = lanes_max<kRowGranules>(largest8(raw[i][0], raw[i][1]));
+    largest = max(largest, m);
+    float up, down;
+    row_scale(m, up, down);
+    const Planes s = split8(raw[i][0], raw[i][1], up);
+    scale_of(t)[(i * kNumThreads + tid) / kRowGranules] = down;   // (by every thread of the row)
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) *reinterpret_cast<u32x4*>(stage_of(t) + t2 * kPlane + dst[i]) = s.p[t2];
   }
@@ -1208,10 +1219,9 @@ struct SplitRing {
   // of about one).  Rows of the default scale get there with elements of 300 in both; keys and queries of
   // N(0,1) are at 2^5, keys times eight at 2^8.
   __device__ __forceinline__ void publish(int wave, uint32_t res_largest) {
-    if (SPLIT) bad()[4 + wave] = has_no_scale(res_largest) ? 0 : (int)res_largest;   // (such a wave multiplies on the fp32 instructions anyway)
+    bad()[4 + wave] = has_no_scale(res_largest) ? 0 : (int)res_largest;   // (such a wave multiplies on the fp32 instructions anyway)
   }
   __device__ __forceinline__ void set_limit(float split_most) {   // behind a barrier after publish()
-    if (!SPLIT) return;
     uint32_t x = 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) x = max(x, (uint32_t)bad()[4 + w]);
@@ -1219,7 +1229,7 @@ struct SplitRing {
     limit = min(__builtin_bit_cast(uint32_t, y), kNoScale);   // (a NaN has larger bits)
   }
   __device__ __forceinline__ void note(int t, uint32_t largest) {
-    if (SPLIT && largest >= limit) bad()[t & 1] = t;
+    if (largest >= limit) bad()[t & 1] = t;
   }
   __device__ __forceinline__ void put(int t, int tid) {
     uint32_t largest = 0;
@@ -1228,7 +1238,7 @@ struct SplitRing {
     note(t, largest);
   }
   __device__ __forceinline__ bool is_bad(int t) const {
-    return SPLIT && __builtin_amdgcn_readfirstlane(bad()[t & 1]) == t;
+    return __builtin_amdgcn_readfirstlane(bad()[t & 1]) == t;
   }
   // Fragment of 16-row group `group`, k-step ks, plane t2.
   __device__ __forceinline__ u32x4 frag(const char* stage, int group, int ks, int t2) const {
@@ -1238,8 +1248,8 @@ struct SplitRing {
 };
 
 // The wave's resident rows as planes; down[g] undoes the scale of group g's row lane & 15.  Returns the bits of their largest
-// magnitude (not SPLIT: zero).
-template <int KS, int NG, bool SPLIT>
+// magnitude.
+template <int KS, int NG>
 __device__ __forceinline__ uint32_t load_resident_split(Planes (&f)[KS][NG], float (&down)[NG], const char* base, int64_t row_bytes,
                                                     const int (&rows)[NG], int nrows, int dgran, int lane) {
   uint32_t worst = 0;
@@ -1255,25 +1265,17 @@ __device__ __forceinline__ uint32_t load_resident_split(Planes (&f)[KS][NG], flo
       x[ks][0] = __builtin_bit_cast(f32x4, view_load16(view, gi < dgran ? roff + gi * 16u : kPastEnd));
       x[ks][1] = __builtin_bit_cast(f32x4, view_load16(view, gi + 1 < dgran ? roff + gi * 16u + 16u : kPastEnd));
     }
-    if constexpr (SPLIT) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) m = max(m, largest8(x[ks][0], x[ks][1]));
-      m = max(m, (uint32_t)__shfl_xor((int)m, 16));
-      m = max(m, (uint32_t)__shfl_xor((int)m, 32));
-      worst = max(worst, m);
-      float up;
-      row_scale(m, up, down[g]);
+    for (int ks = 0; ks < KS; ++ks) m = max(m, largest8(x[ks][0], x[ks][1]));
+    m = max(m, (uint32_t)__shfl_xor((int)m, 16));
+    m = max(m, (uint32_t)__shfl_xor((int)m, 32));
+    worst = max(worst, m);
+    float up;
+    row_scale(m, up, down[g]);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) f[ks][g] = split8(x[ks][0], x[ks][1], up);
-    } else {
-      down[g] = 1.f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) f[ks][g].p[t2] = __builtin_bit_cast(u32x4, x[ks][t2]);
-    }
+    for (int ks = 0; ks < KS; ++ks) f[ks][g] = split8(x[ks][0], x[ks][1], up);
   }
-  return SPLIT ? __builtin_amdgcn_readfirstlane(lanes_max<16>(worst)) : 0u;   // (the four rows of lanes hold the same)
+  return __builtin_amdgcn_readfirstlane(lanes_max<16>(worst));   // (the four rows of lanes hold the same)
 }
 
 // The same scores from the operands in memory, on the fp32 instructions.
@@ -1314,8 +1316,8 @@ template <int SG>
 struct Fragments {
   u32x4 f[2][SG];   // per plane and group
 };
-template <int SG, int KS, bool SPLIT, int NW>
-__device__ __forceinline__ Fragments<SG> read_fragments(const SplitRing<KS, SPLIT, NW>& rg, const char* stage, int sub, int ks) {
+template <int SG, int KS, int NW>
+__device__ __forceinline__ Fragments<SG> read_fragments(const SplitRing<KS, NW>& rg, const char* stage, int sub, int ks) {
   Fragments<SG> x;
 #pragma unroll
   for (int t2 = 1; t2 >= 0; --t2)
@@ -1323,13 +1325,13 @@ __device__ __forceinline__ Fragments<SG> read_fragments(const SplitRing<KS, SPLI
     for (int sg = 0; sg < SG; ++sg) x.f[t2][sg] = rg.frag(stage, sub * SG + sg, ks, t2);
   return x;
 }
-template <bool RESIDENT_IS_KEYS, bool SPLIT, int KS, int NG, int SG, int NW, class BetweenF>
-__device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes (&res)[KS][NG], const SplitRing<KS, SPLIT, NW>& rg,
+template <bool RESIDENT_IS_KEYS, int KS, int NG, int SG, int NW, class BetweenF>
+__device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes (&res)[KS][NG], const SplitRing<KS, NW>& rg,
                                              const char* stage, int sub, const Fragments<SG>& first, BetweenF&& between) {
-  // products by plane: streamed l with h, h with l, h with h; or the fp32 halves
-  constexpr int kProducts = SPLIT ? 3 : 2;
-  constexpr int str_of[3] = {1, 0, 0}, res_of[3] = {SPLIT ? 0 : 1, SPLIT ? 1 : 0, 0};
-  constexpr int kType = SPLIT ? FCR_DTYPE_F16 : FCR_DTYPE_F32;
+  // products by plane: streamed l with h, h with l, h with h
+  constexpr int kProducts = 3;
+  constexpr int str_of[kProducts] = {1, 0, 0}, res_of[kProducts] = {0, 1, 0};
+  constexpr int kType = FCR_DTYPE_F16;
   Fragments<SG> f[2];
   f[0] = first;
 #pragma unroll
@@ -1360,12 +1362,12 @@ __device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes 
 // unmasked chunk run the split of the next one (fetched a chunk ago) and `consume` for the sub-step before, whose scores are kept for
 // it.  aux_of(t, sub) is what consume needs besides the scores, extra(t) what travels with a chunk; general(t, exact) does
 // a chunk that needs a mask or, `exact`, has a row without a scale.
-template <bool RESIDENT_IS_KEYS, int AUX, class Aux, bool SPLIT, int KS, int NG, int NW, class ExtraF, class AuxF, class ConsumeF,
+template <bool RESIDENT_IS_KEYS, int AUX, class Aux, int KS, int NG, int NW, class ExtraF, class AuxF, class ConsumeF,
           class GeneralF>
 __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, const Planes (&res)[KS][NG],
-                                            SplitRing<KS, SPLIT, NW>& rg, int tid, bool idle, uint32_t res_largest, float split_most, ExtraF&& extra,
+                                            SplitRing<KS, NW>& rg, int tid, bool idle, uint32_t res_largest, float split_most, ExtraF&& extra,
                                             AuxF&& aux_of, ConsumeF&& consume, GeneralF&& general) {
-  using Rg = SplitRing<KS, SPLIT, NW>;
+  using Rg = SplitRing<KS, NW>;
   constexpr int SG = f32_groups(KS), SUBS = Rg::kChunkRows / (16 * SG), STEPS = SUBS * KS, PER = Rg::kPer;
   if (t0 >= t1) return;
   const bool res_bad = has_no_scale(res_largest);
@@ -1389,7 +1391,7 @@ __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, cons
     for (int sub = 0; sub < SUBS; ++sub) {
       f32x4 acc[NG][SG];
       const Aux aux = aux_of(t, sub);
-      split_scores<RESIDENT_IS_KEYS, SPLIT>(acc, res, rg, stage, sub, next, [&](int ks) {
+      split_scores<RESIDENT_IS_KEYS>(acc, res, rg, stage, sub, next, [&](int ks) {
         const int step = sub * KS + ks;
 #pragma unroll
         for (int i = 0; i < PER; ++i)
@@ -1436,9 +1438,9 @@ __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, cons
 }
 
 // See row_lse_kernel: the same work order, key ranges, row state and result for fp32 operands.
-template <int KS, bool CAUSAL, int NG, bool STREAM_ONCE, bool SPLIT, int NW>
+template <int KS, bool CAUSAL, int NG, bool STREAM_ONCE, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p) {
-  using Rg = SplitRing<KS, SPLIT, NW>;
+  using Rg = SplitRing<KS, NW>;
   constexpr int SG = f32_groups(KS), kRows = Rg::kChunkRows, kTileRows = NW * 16 * NG;
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes];
   int bh, tile, split;
@@ -1472,7 +1474,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
   rg.template fetch<(STREAM_ONCE ? kLoadOnce : 0)>();   // in flight together with the resident rows
   Planes qf[KS][NG];
   float qs2[NG];   // scale2 times what undoes the scale of the lane's query
-  const uint32_t q_largest = load_resident_split<KS, NG, SPLIT>(qf, qs2, qb, p.q_sr, q0, p.M, p.dgran, lane);
+  const uint32_t q_largest = load_resident_split<KS, NG>(qf, qs2, qb, p.q_sr, q0, p.M, p.dgran, lane);
 #pragma unroll
   for (int g = 0; g < NG; ++g) qs2[g] *= p.scale2;
   const bool idle = q0[0] >= p.M;   // a wave whose rows all lie past M only helps staging
@@ -1482,20 +1484,16 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
   };
   auto scales_at = [&](int t, int sub) {
     KeyScales s;
-    if (SPLIT) {
 #pragma unroll
-      for (int sg = 0; sg < SG; ++sg)
-        s.v[sg] = *reinterpret_cast<const f32x4*>(rg.scale_of(t) + (sub * SG + sg) * 16 + 4 * (lane >> 4));
-    }
+    for (int sg = 0; sg < SG; ++sg)
+      s.v[sg] = *reinterpret_cast<const f32x4*>(rg.scale_of(t) + (sub * SG + sg) * 16 + 4 * (lane >> 4));
     return s;
   };
   auto rescale = [&](f32x4(&a)[NG][SG], const KeyScales& s) {
-    if (SPLIT) {
 #pragma unroll
-      for (int g = 0; g < NG; ++g)
+    for (int g = 0; g < NG; ++g)
 #pragma unroll
-        for (int sg = 0; sg < SG; ++sg) a[g][sg] *= s.v[sg];
-    }
+      for (int sg = 0; sg < SG; ++sg) a[g][sg] *= s.v[sg];
   };
   auto general = [&](int t, bool exact) {
     const char* stage = rg.stage_of(t);
@@ -1505,7 +1503,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
       if (key0 >= p.N || (CAUSAL && key0 > q0[NG - 1] + 15 + p.c)) continue;   // nobody sees these keys
       f32x4 acc[NG][SG] = {};
       if (!exact) {
-        split_scores<false, SPLIT>(acc, qf, rg, stage, sub, read_fragments<SG>(rg, stage, sub, 0), [](int) {});
+        split_scores<false>(acc, qf, rg, stage, sub, read_fragments<SG>(rg, stage, sub, 0), [](int) {});
         rescale(acc, scales_at(t, sub));
       } else {
         exact_scores<false>(acc, qb, p.q_sr, q0, p.M, kb, p.k_sr, key0, p.N, p.dgran, lane);
@@ -1539,9 +1537,9 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
 }
 
 // See col_reduce_kernel.
-template <int KS, bool CAUSAL, int MODE, int NG, bool SPLIT, int NW>
+template <int KS, bool CAUSAL, int MODE, int NG, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params p) {
-  using Rg = SplitRing<KS, SPLIT, NW>;
+  using Rg = SplitRing<KS, NW>;
   constexpr int SG = f32_groups(KS), kRows = Rg::kChunkRows, kTileRows = NW * 16 * NG;
   constexpr int kRed = NW * NG * 4 * 64 * 4;
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes > kRed ? Rg::kBytes : kRed];
@@ -1583,11 +1581,11 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
   uint32_t k_largest;
   {
     float down[NG];
-    k_largest = load_resident_split<KS, NG, SPLIT>(kf, down, kb, p.k_sr, k0, p.N, p.dgran, lane);
+    k_largest = load_resident_split<KS, NG>(kf, down, kb, p.k_sr, k0, p.N, p.dgran, lane);
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) ks4[g][r] = SPLIT ? __shfl(down[g], 4 * (lane >> 4) + r) : 1.f;
+      for (int r = 0; r < 4; ++r) ks4[g][r] = __shfl(down[g], 4 * (lane >> 4) + r);
   }
   const bool idle = k0[0] >= p.N;
 
@@ -1604,7 +1602,7 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
     for (int sg = 0; sg < SG; ++sg) {
       const int at = (sub * SG + sg) * 16 + (lane & 15);
       q.lse[sg] = rg.extra_of(t)[at];
-      q.s2[sg] = SPLIT ? rg.scale_of(t)[at] * p.scale2 : p.scale2;
+      q.s2[sg] = rg.scale_of(t)[at] * p.scale2;
     }
     return q;
   };
@@ -1617,21 +1615,17 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
       QueryFacts q = facts_at(t, sub);
       f32x4 acc[NG][SG] = {};
       if (!exact) {
-        split_scores<true, SPLIT>(acc, kf, rg, stage, sub, read_fragments<SG>(rg, stage, sub, 0), [](int) {});
-        if (SPLIT) {
+        split_scores<true>(acc, kf, rg, stage, sub, read_fragments<SG>(rg, stage, sub, 0), [](int) {});
 #pragma unroll
-          for (int g = 0; g < NG; ++g)
+        for (int g = 0; g < NG; ++g)
 #pragma unroll
-            for (int sg = 0; sg < SG; ++sg) acc[g][sg] *= ks4[g];
-        }
+          for (int sg = 0; sg < SG; ++sg) acc[g][sg] *= ks4[g];
       } else {
         exact_scores<true>(acc, kb, p.k_sr, k0, p.N, qb, p.q_sr, qs, p.M, p.dgran, lane);
 #pragma unroll
         for (int sg = 0; sg < SG; ++sg) q.s2[sg] = p.scale2;
-      }
-      if (exact || !SPLIT) {   // a row of padding may have met a non-finite key
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
+        for (int g = 0; g < NG; ++g)   // a row of padding may have met a non-finite key
 #pragma unroll
           for (int sg = 0; sg < SG; ++sg)
             if (qs + 16 * sg + (lane & 15) >= p.M) acc[g][sg] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -1645,14 +1639,12 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
     }
   };
   split_sweep<true, 0, QueryFacts>(
-      t0, t_int, SPLIT ? nchunks : p.M / kRows, nchunks, kf, rg, tid, idle, k_largest, p.split_most, extra, facts_at,
+      t0, t_int, nchunks, nchunks, kf, rg, tid, idle, k_largest, p.split_most, extra, facts_at,
       [&](f32x4(&a)[NG][SG], const QueryFacts& q) {
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-          if (SPLIT) {
 #pragma unroll
-            for (int sg = 0; sg < SG; ++sg) a[g][sg] *= ks4[g];
-          }
+          for (int sg = 0; sg < SG; ++sg) a[g][sg] *= ks4[g];
           col_update<false, MODE>(a[g], q.s2, q.lse, csum[g], cmax[g], 0);
         }
       },
@@ -3493,8 +3485,6 @@ int fail(int code, const char* what) {
   return code;
 }
 
-inline int elem_bytes(int dtype) { return dtype == FCR_DTYPE_F32 ? 4 : 2; }
-inline int ksteps_of(int dtype, int D) { return (D * elem_bytes(dtype) + 63) / 64; }
 
 // dims = sizes of the batch, head and row dimensions.  The stride of a dimension of size one is never
 // used to form an address, so it may be anything (torch reports arbitrary strides there, and a slice of an
@@ -3571,14 +3561,16 @@ int check_problem(const void* q, const void* k, int dtype, int B, int H, int M, 
 struct TileChoice {
   int rows, per_cu;
 };
-TileChoice tile_choice(bool f32, int ksteps, int M, int N, int64_t bh, bool by_keys, int col_mode, bool causal) {
-  if (f32) {
+TileChoice tile_choice(int dtype, int D, int M, int N, int64_t bh, bool by_keys, int col_mode, bool causal) {
+  const int ksteps = ksteps_of(dtype, D);
+  if (in_parts(dtype, D)) {
     const F32Tile t = by_keys ? f32_col_tile(f32_ksteps(ksteps), col_mode == kModeBoth, M, N, bh, causal) : f32_row_tile(M, N, bh, causal);
     return TileChoice{t.rows(), 8 / t.waves};
   }
   const int per_cu = ksteps > kMaxKSteps ? 1 : 2;
+  if (by_keys && half_tiles(dtype, D, N, bh)) return TileChoice{kWaves * 16, per_cu};
   return TileChoice{by_keys ? kWaves * 32 * col_tile_blocks(ksteps, N, bh, causal)
-                            : row_tile_rows(false, ksteps, M, N, bh, causal), per_cu};
+                            : row_tile_rows(dtype, D, M, N, bh, causal), per_cu};
 }
 
 // Params::fill: see map_group.  Only for launches of one group, whose places are in order of length over the whole launch, and
@@ -3601,9 +3593,7 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   const int esize = elem_bytes(dtype);
   const int64_t bh = (int64_t)B * H;
   // the device is first asked (for its CU count) here, after every argument check
-  const int ksteps = ksteps_of(dtype, D);
-  const bool f32 = dtype == FCR_DTYPE_F32;
-  const int trows = tile_choice(f32, ksteps, M, N, bh, by_keys, col_mode, causal).rows;
+  const int trows = tile_choice(dtype, D, M, N, bh, by_keys, col_mode, causal).rows;
   const int64_t tiles = ((by_keys ? N : M) + trows - 1) / trows;
   p.q = static_cast<const char*>(q);
   p.k = static_cast<const char*>(k);
@@ -3637,11 +3627,11 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
 // Key ranges per row tile in the row kernel.  One sweep per workgroup when there is at least one
 // workgroup per CU; otherwise the keys of a tile are split so that about two per CU run, each
 // keeping at least four 64-key chunks.
-int row_splits(bool f32, int B, int H, int M, int N, int ksteps) {
+int row_splits(int dtype, int B, int H, int M, int N, int D) {
   const int64_t chunks = (N + kChunk - 1) / kChunk;
   if (chunks < 16) return 1;
-  // (fp32 launches of at least one 128-row tile per CU are never split; the mask makes no difference below that)
-  const int trows = f32 ? 128 : row_tile_rows(false, ksteps, M, N, (int64_t)B * H, false);  // same with the mask when wgs < 256
+  // (fp32 launches in parts of at least one 128-row tile per CU are never split; the mask makes no difference below that)
+  const int trows = in_parts(dtype, D) ? 128 : row_tile_rows(dtype, D, M, N, (int64_t)B * H, false);  // same with the mask when wgs < 256
   const int64_t wgs = (int64_t)B * H * ((M + trows - 1) / trows);
   const int cus = chip_cus();
   if (wgs >= cus) return 1;
@@ -3747,6 +3737,9 @@ void launch_lse_blocks(const Params& p, bool causal, hipStream_t s) {
 
 template <int DT, int KS>
 void launch_lse(const Params& p, bool causal, hipStream_t s) {
+  if constexpr (DT == FCR_DTYPE_F32) {
+    if (row_half_tiles(DT, p.dgran * 4, p.M, p.N, p.bh_count)) return launch_lse_blocks<DT, KS, 0, false>(p, causal, s);
+  }
   if constexpr (KS <= 4) {
     if (row_blocks_per_wave(KS, p.M, p.N, p.bh_count, causal) == 2) return launch_lse_blocks<DT, KS, 2, false>(p, causal, s);
   }
@@ -3758,6 +3751,13 @@ template <int DT, int KS, int MODE>
 void launch_col_mode(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(kThreads);
   constexpr int NB = blocks_per_wave(KS);
+  if constexpr (DT == FCR_DTYPE_F32) {
+    if (half_tiles(DT, p.dgran * 4, p.N, p.bh_count)) {
+      if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 0>), grid, block, 0, s, p);
+      else hipLaunchKernelGGL((col_reduce_kernel<DT, KS, false, MODE, 0>), grid, block, 0, s, p);
+      return;
+    }
+  }
   if constexpr (NB == 2) {
     if (col_tile_blocks(KS, p.N, p.bh_count, causal) == 1) {
       if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 1>), grid, block, 0, s, p);
@@ -3769,44 +3769,44 @@ void launch_col_mode(const Params& p, bool causal, hipStream_t s) {
   else hipLaunchKernelGGL((col_reduce_kernel<DT, KS, false, MODE, NB>), grid, block, 0, s, p);
 }
 
-template <int KS, int NW, int NG, bool SPLIT>
+template <int KS, int NW, int NG>
 void launch_lse_f32_tile(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(64 * NW);
   if (keys_read_once(p)) {
-    if (causal) hipLaunchKernelGGL((row_lse_f32_kernel<KS, true, NG, true, SPLIT, NW>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((row_lse_f32_kernel<KS, false, NG, true, SPLIT, NW>), grid, block, 0, s, p);
+    if (causal) hipLaunchKernelGGL((row_lse_f32_kernel<KS, true, NG, true, NW>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((row_lse_f32_kernel<KS, false, NG, true, NW>), grid, block, 0, s, p);
     return;
   }
-  if (causal) hipLaunchKernelGGL((row_lse_f32_kernel<KS, true, NG, false, SPLIT, NW>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((row_lse_f32_kernel<KS, false, NG, false, SPLIT, NW>), grid, block, 0, s, p);
+  if (causal) hipLaunchKernelGGL((row_lse_f32_kernel<KS, true, NG, false, NW>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((row_lse_f32_kernel<KS, false, NG, false, NW>), grid, block, 0, s, p);
 }
 
-template <int KS, bool SPLIT = true>
+template <int KS>
 void launch_lse_f32(const Params& p, bool causal, hipStream_t s) {
   const F32Tile t = f32_row_tile(p.M, p.N, p.bh_count, causal);
-  if (t.waves == 4) t.groups == 1 ? launch_lse_f32_tile<KS, 4, 1, SPLIT>(p, causal, s) : launch_lse_f32_tile<KS, 4, 2, SPLIT>(p, causal, s);
-  else t.groups == 1 ? launch_lse_f32_tile<KS, 8, 1, SPLIT>(p, causal, s) : launch_lse_f32_tile<KS, 8, 2, SPLIT>(p, causal, s);
+  if (t.waves == 4) t.groups == 1 ? launch_lse_f32_tile<KS, 4, 1>(p, causal, s) : launch_lse_f32_tile<KS, 4, 2>(p, causal, s);
+  else t.groups == 1 ? launch_lse_f32_tile<KS, 8, 1>(p, causal, s) : launch_lse_f32_tile<KS, 8, 2>(p, causal, s);
 }
 
-template <int KS, int MODE, int NW, int NG, bool SPLIT>
+template <int KS, int MODE, int NW, int NG>
 void launch_col_f32_tile(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(64 * NW);
-  if (causal) hipLaunchKernelGGL((col_reduce_f32_kernel<KS, true, MODE, NG, SPLIT, NW>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((col_reduce_f32_kernel<KS, false, MODE, NG, SPLIT, NW>), grid, block, 0, s, p);
+  if (causal) hipLaunchKernelGGL((col_reduce_f32_kernel<KS, true, MODE, NG, NW>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((col_reduce_f32_kernel<KS, false, MODE, NG, NW>), grid, block, 0, s, p);
 }
 
-template <int KS, int MODE, bool SPLIT>
+template <int KS, int MODE>
 void launch_col_f32_mode(const Params& p, bool causal, hipStream_t s) {
   const F32Tile t = f32_col_tile(KS, MODE == kModeBoth, p.M, p.N, p.bh_count, causal);
-  if (t.waves == 4) t.groups == 1 ? launch_col_f32_tile<KS, MODE, 4, 1, SPLIT>(p, causal, s) : launch_col_f32_tile<KS, MODE, 4, 2, SPLIT>(p, causal, s);
-  else t.groups == 1 ? launch_col_f32_tile<KS, MODE, 8, 1, SPLIT>(p, causal, s) : launch_col_f32_tile<KS, MODE, 8, 2, SPLIT>(p, causal, s);
+  if (t.waves == 4) t.groups == 1 ? launch_col_f32_tile<KS, MODE, 4, 1>(p, causal, s) : launch_col_f32_tile<KS, MODE, 4, 2>(p, causal, s);
+  else t.groups == 1 ? launch_col_f32_tile<KS, MODE, 8, 1>(p, causal, s) : launch_col_f32_tile<KS, MODE, 8, 2>(p, causal, s);
 }
 
-template <int KS, bool SPLIT = true>
+template <int KS>
 void launch_col_f32(const Params& p, bool causal, int mode, hipStream_t s) {
-  if (mode == kModeSum) launch_col_f32_mode<KS, kModeSum, SPLIT>(p, causal, s);
-  else if (mode == kModeMax) launch_col_f32_mode<KS, kModeMax, SPLIT>(p, causal, s);
-  else launch_col_f32_mode<KS, kModeBoth, SPLIT>(p, causal, s);
+  if (mode == kModeSum) launch_col_f32_mode<KS, kModeSum>(p, causal, s);
+  else if (mode == kModeMax) launch_col_f32_mode<KS, kModeMax>(p, causal, s);
+  else launch_col_f32_mode<KS, kModeBoth>(p, causal, s);
 }
 
 template <int DT, int KS, int MODE, int NG>
@@ -3963,8 +3963,10 @@ void fcr_detail::sweeps_bf16_single(const Params& p, int ksteps, bool causal, in
 #endif
 #if FCR_HAS(3)
 void fcr_detail::sweeps_f32(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
-  if (p.dgran < 8) {   // D < 32
-    which == 0 ? launch_lse_f32<1, false>(p, causal, s) : launch_col_f32<1, false>(p, causal, mode, s);
+  if (!in_parts(FCR_DTYPE_F32, p.dgran * 4)) {
+    constexpr int DT = FCR_DTYPE_F32;
+    if (ksteps == 1) which == 0 ? launch_lse<DT, 1>(p, causal, s) : launch_col<DT, 1>(p, causal, mode, s);
+    else which == 0 ? launch_lse<DT, 2>(p, causal, s) : launch_col<DT, 2>(p, causal, mode, s);
     return;
   }
   switch (f32_ksteps(ksteps)) {
@@ -4129,7 +4131,7 @@ size_t fcr_lse_bytes_two_kernels(int B, int H, int M, int N) {
   // The most any row width asks for, so the size holds for every dtype and D.  Of one problem the widths differ
   // only in the tile height, 128 or 256 rows: four k-steps take 256 where any width does (one block costs them
   // the most), and the higher tile has the fewer workgroups, hence the most splits.  (Every call comes here.)
-  const int splits = row_splits(false, B, H, M, N, 4);
+  const int splits = row_splits(FCR_DTYPE_F16, B, H, M, N, 128);
   const size_t rows = (size_t)B * (size_t)H * (size_t)M;
   return rows * sizeof(float) * (splits > 1 ? 1 + (size_t)splits : 1);
 }
@@ -4168,12 +4170,12 @@ int fcr_row_lse(const void* q, const void* k, float* lse, int dtype, int B, int 
   int rc = make_params(p, q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, false, causal != 0);
   if (rc) return rc;
   p.lse = lse;
-  p.splits = row_splits(dtype == FCR_DTYPE_F32, B, H, M, N, ksteps_of(dtype, D));
+  p.splits = row_splits(dtype, B, H, M, N, D);
   p.part = lse + (int64_t)B * H * M;  // only touched when splits > 1 (see fcr_lse_bytes)
   p.total *= p.splits;
   const int ksteps = ksteps_of(dtype, D);
   p.group = head_group(p.bh_count, (int64_t)p.tiles * p.splits, causal != 0);
-  p.fill = fill_places(p, tile_choice(dtype == FCR_DTYPE_F32, ksteps, M, N, p.bh_count, false, 0, causal != 0), causal != 0);
+  p.fill = fill_places(p, tile_choice(dtype, D, M, N, p.bh_count, false, 0, causal != 0), causal != 0);
   hipStream_t s = static_cast<hipStream_t>(stream);
   launch_sweeps(dtype, 0, p, ksteps, causal != 0, 0, s);
   rc = launched("row_lse_kernel");
@@ -4200,7 +4202,7 @@ int col_reduce_any(const void* q, const void* k, const float* lse, void* out, vo
   if (rc) return rc;
   p.group = head_group(p.bh_count, p.tiles, causal != 0);
   const int ksteps = ksteps_of(dtype, D);
-  p.fill = fill_places(p, tile_choice(dtype == FCR_DTYPE_F32, ksteps, M, N, p.bh_count, true, mode, causal != 0), causal != 0);
+  p.fill = fill_places(p, tile_choice(dtype, D, M, N, p.bh_count, true, mode, causal != 0), causal != 0);
   p.lse = const_cast<float*>(lse);
   p.out = out;
   p.out2 = out2;

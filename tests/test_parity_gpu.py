@@ -378,6 +378,21 @@ def test_key_that_no_query_counts_beside_rows_of_padding(dtype, h, m, n, d, caus
 
 
 @pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(2, 65, 63, 4), (3, 129, 1100, 12), (8, 960, 960, 16), (8, 961, 961, 20), (140, 130, 257, 28),
+                                     (300, 255, 70, 8), (2, 1000, 5000, 16), (40, 2000, 300, 28)])
+def test_fp32_rows_shorter_than_32(h, m, n, d, causal):
+    """D < 32 on the fp32 instructions: tiles of 64, 128 and 256 rows with ragged ends, the split row sweep, one and two k-steps.
+    At most 28 products round a score by 2^-19 of their sum of magnitudes, a few tens: 1e-5 as for the other fp32 tests."""
+    q, k = _inputs.randn_pair(1, h, m, n, d, seed=h + d, dtype=torch.float32)
+    s, mx = fca.flash_colreduce_multi(q.cuda(), k.cuda(), ["sum", "max"], is_causal=causal)
+    for red, pair in (("sum", s), ("mean", None), ("max", mx)):
+        want = colreduce_ref(q, k, red, causal, compute_dtype=torch.float64).float()
+        for got in (fca.flash_colreduce(q.cuda(), k.cuda(), red, is_causal=causal), pair):
+            if got is not None:
+                torch.testing.assert_close(got.cpu(), want, rtol=1e-5, atol=1e-8)
+
+
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("h,m,n,d", [(130, 257, 300, 36), (180, 300, 257, 96), (130, 257, 300, 256), (9, 511, 700, 128),
                                      (1, 65, 33, 32), (3, 129, 1100, 28)])
 def test_fp32_split_tiles(h, m, n, d, causal):
