@@ -162,11 +162,12 @@ inline int row_blocks_per_wave(int ksteps, int M, int N, int64_t bh, bool causal
 inline bool in_parts(int dtype, int D) { return dtype == FCR_DTYPE_F32 && D >= 32; }
 // Those on the fp32 instructions that give at most one workgroup of 128 rows on every other CU take tiles of 64 rows, one 16-row
 // group per wave (NB = 0): such a launch lasts as long as one workgroup, and half the resident rows halve its matrix instructions.
-// A row sweep of 16 chunks or more is split over the idle CUs (row_splits) and keeps its tile.
+// So do those of at most 64 rows.  A row sweep of 16 chunks or more is split over the idle CUs (row_splits) and keeps its tile if
+// it has more rows than that.
 inline bool half_tiles(int dtype, int D, int64_t rows, int64_t bh) {
-  return dtype == FCR_DTYPE_F32 && !in_parts(dtype, D) && 2 * bh * ((rows + 127) / 128) <= chip_cus();
+  return dtype == FCR_DTYPE_F32 && !in_parts(dtype, D) && (rows <= 64 || 2 * bh * ((rows + 127) / 128) <= chip_cus());
 }
-inline bool row_half_tiles(int dtype, int D, int M, int N, int64_t bh) { return N <= 15 * 64 && half_tiles(dtype, D, M, bh); }
+inline bool row_half_tiles(int dtype, int D, int M, int N, int64_t bh) { return (M <= 64 || N <= 15 * 64) && half_tiles(dtype, D, M, bh); }
 // Tiles of the fp32 sweeps in parts (row_lse_f32_kernel, col_reduce_f32_kernel): waves per workgroup (four: two workgroups share a
 // CU; eight: one) and resident 16-row groups per wave.  Two groups read a streamed fragment once for two blocks of scores,
 // eight waves share the split of a streamed row: 4 x 2 and 8 x 1 are 128 rows, 8 x 2 256, 4 x 1 64.  Per call, fp32:
@@ -1023,7 +1024,7 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
           acc[0] = mma<DT>(kf[g][ks], qfrag[0][ks], acc[0]);
           acc[1] = mma<DT>(kf[g][ks], qfrag[1][ks], acc[1]);
         }
-        if (RAGGED) {   // rows of padding, zeros, may have met a non-finite key
+        if (RAGGED && qs + 32 > p.M) {   // rows of padding, zeros, may have met a non-finite key
           if (qs + (lane & 15) >= p.M) acc[0] = (f32x4){0.f, 0.f, 0.f, 0.f};
           if (qs + 16 + (lane & 15) >= p.M) acc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
         }
@@ -1226,7 +1227,7 @@ struct SplitRing {
 #pragma unroll
     for (int w = 0; w < NW; ++w) x = max(x, (uint32_t)bad()[4 + w]);
     const float y = split_most / __builtin_bit_cast(float, x);
-    limit = min(__builtin_bit_cast(uint32_t, y), kNoScale);   // (a NaN has larger bits)
+    limit = __builtin_amdgcn_readfirstlane(min(__builtin_bit_cast(uint32_t, y), kNoScale));   // (a NaN has larger bits)
   }
   __device__ __forceinline__ void note(int t, uint32_t largest) {
     if (largest >= limit) bad()[t & 1] = t;
@@ -3738,7 +3739,10 @@ void launch_lse_blocks(const Params& p, bool causal, hipStream_t s) {
 template <int DT, int KS>
 void launch_lse(const Params& p, bool causal, hipStream_t s) {
   if constexpr (DT == FCR_DTYPE_F32) {
-    if (row_half_tiles(DT, p.dgran * 4, p.M, p.N, p.bh_count)) return launch_lse_blocks<DT, KS, 0, false>(p, causal, s);
+    if (row_half_tiles(DT, p.dgran * 4, p.M, p.N, p.bh_count)) {
+      if (keys_read_once(p)) return launch_lse_blocks<DT, KS, 0, true>(p, causal, s);
+      return launch_lse_blocks<DT, KS, 0, false>(p, causal, s);
+    }
   }
   if constexpr (KS <= 4) {
     if (row_blocks_per_wave(KS, p.M, p.N, p.bh_count, causal) == 2) return launch_lse_blocks<DT, KS, 2, false>(p, causal, s);
