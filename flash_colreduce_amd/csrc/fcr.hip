@@ -908,20 +908,26 @@ struct LsePair {
   float v[2];
 };
 
-// Blocks per wave the host asks for, whatever the sweep produces (sums and maxima together, 16-bit, one block -> two: 32 heads of
-// 32768 causal 7987 -> 7406 us per call, of 4096 268 -> 254, 48 of 2929 causal 134 -> 120).  Strictly between one and two workgroups of 256 keys per CU
+// Blocks per wave the host asks for.  Strictly between one and two workgroups of 256 keys per CU
 // leave CUs unevenly loaded, and with the mask one or two per CU are too coarse as well (the chip
 // waits for the longest sweep): those launches use 128-key tiles.
-inline int col_tile_blocks(int ksteps, int N, int64_t bh, bool causal) {
+// Sums and maxima together gain by two blocks too, but less the shorter the rows (16-bit, per call, one block against two: 32 heads of
+// 32768 x 128 causal 7987 us, 7406; of 4096 x 128 268, 253; of 4096 x 64 182, 176), and lose in rows of one k-step (256 heads of
+// 2351 x 32 394, 400; 160 of 987 x 32 53, 57) and, of two, where two blocks leave a part of a second round (160 of 1024 x 64,
+// 2.5 workgroups of 256 keys per CU, 72, 77; 44 of 4096 x 64, 2.75, 266, 264) or no more than one per CU (11 of 4096 x 64 97.5, 99.5).
+inline int col_tile_blocks(int ksteps, int mode, int N, int64_t bh, bool causal) {
   const int nb = blocks_per_wave(ksteps);
   if (nb != 2) return nb;
-  const int64_t wgs2 = bh * ((N + kWaves * 64 - 1) / (kWaves * 64));
+  const int64_t wgs2 = bh * ((N + kWaves * 64 - 1) / (kWaves * 64)), wgs1 = bh * ((N + kWaves * 32 - 1) / (kWaves * 32));
   const int cus = chip_cus();
+  if (mode == kModeBoth && ksteps == 1) return 1;
+  if (mode == kModeBoth && ksteps == 2 && !causal && (wgs2 <= cus || (wgs2 > 2 * cus && 8 * wgs2 < 22 * cus))) return 1;
   // two-block tiles only when they still give two workgroups per CU; with fewer, CUs idle or run a single
   // workgroup (32 heads of 1024 x 1024: the call takes 37 us with 128 two-block tiles, 32 us with 256 one-block tiles)
-  // (without the mask one workgroup on most CUs does better with two blocks: 16 heads of 4096 x 4096 76 -> 66 us)
+  // (without the mask one workgroup on most CUs does better with two blocks, 16 heads of 4096 x 4096 76 -> 66 us, unless the
+  // 128-key tiles are no more than the CUs either: 252 of them, 12 heads of 2661 x 2661 x 128, 60.5 us, 132 two-block ones 72.5)
   if (causal) return wgs2 <= 2 * cus ? 1 : 2;
-  if (wgs2 <= cus) return 2 * wgs2 > cus ? 2 : 1;
+  if (wgs2 <= cus) return wgs1 > cus ? 2 : 1;
   return wgs2 < 2 * cus ? 1 : 2;
 }
 
@@ -3570,7 +3576,7 @@ TileChoice tile_choice(int dtype, int D, int M, int N, int64_t bh, bool by_keys,
   }
   const int per_cu = ksteps > kMaxKSteps ? 1 : 2;
   if (by_keys && half_tiles(dtype, D, N, bh)) return TileChoice{kWaves * 16, per_cu};
-  return TileChoice{by_keys ? kWaves * 32 * col_tile_blocks(ksteps, N, bh, causal)
+  return TileChoice{by_keys ? kWaves * 32 * col_tile_blocks(ksteps, col_mode, N, bh, causal)
                             : row_tile_rows(dtype, D, M, N, bh, causal), per_cu};
 }
 
@@ -3754,7 +3760,7 @@ void launch_lse(const Params& p, bool causal, hipStream_t s) {
 template <int DT, int KS, int MODE>
 void launch_col_mode(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid(p.total), block(kThreads);
-  constexpr int NB = blocks_per_wave(KS);
+  constexpr int NB = (MODE == kModeBoth && KS == 1) ? 1 : blocks_per_wave(KS);   // (see col_tile_blocks)
   if constexpr (DT == FCR_DTYPE_F32) {
     if (half_tiles(DT, p.dgran * 4, p.N, p.bh_count)) {
       if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 0>), grid, block, 0, s, p);
@@ -3763,7 +3769,7 @@ void launch_col_mode(const Params& p, bool causal, hipStream_t s) {
     }
   }
   if constexpr (NB == 2) {
-    if (col_tile_blocks(KS, p.N, p.bh_count, causal) == 1) {
+    if (col_tile_blocks(KS, MODE, p.N, p.bh_count, causal) == 1) {
       if (causal) hipLaunchKernelGGL((col_reduce_kernel<DT, KS, true, MODE, 1>), grid, block, 0, s, p);
       else hipLaunchKernelGGL((col_reduce_kernel<DT, KS, false, MODE, 1>), grid, block, 0, s, p);
       return;

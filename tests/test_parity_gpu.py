@@ -348,6 +348,18 @@ def test_fp32_tiles_of_64_rows_give_the_bits_of_taller_ones(h, m, n, d, causal):
 
 
 @pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(129, 300, 1000, 32), (12, 547, 2661, 64), (33, 200, 2000, 64), (130, 150, 1024, 64), (176, 140, 1024, 64),
+                                     (12, 200, 2661, 128), (13, 200, 2661, 128)])
+def test_sums_and_maxima_tile_heights(h, m, n, d, causal):
+    """Both sides of the rule that gives the column tiles of sums and maxima together one or two key blocks per wave: one k-step,
+    two with at most one, about two and a half and 2.75 workgroups of 256 keys per CU, 128-key tiles that just fit the CUs."""
+    q, k = _inputs.randn_pair(1, h, m, n, d, seed=n + d)
+    s, mx = fca.flash_colreduce_multi(q.cuda(), k.cuda(), ["sum", "max"], is_causal=causal, out_dtype=torch.float32)
+    check(s, colreduce_ref(q, k, "sum", causal), "sum", "pair")
+    check(mx, colreduce_ref(q, k, "max", causal), "max", "pair")
+
+
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype,h,m,n,d", [(torch.float16, 2, 70, 99, 16), (torch.bfloat16, 2, 200, 333, 64), (torch.float16, 4, 300, 2100, 256),
                                            (torch.bfloat16, 1, 65, 130, 512), (torch.float16, 32, 70, 4096, 64), (torch.bfloat16, 64, 1, 8192, 128),
                                            (torch.float16, 32, 33, 2048, 128), (torch.float16, 2, 128, 64, 32)])
