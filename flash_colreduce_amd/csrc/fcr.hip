@@ -42,6 +42,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "f32_tiles.h"
 #include "fcr.h"
 
 // The file can be compiled whole, or in parts that are linked together (the build script does that to
@@ -168,38 +169,11 @@ inline bool half_tiles(int dtype, int D, int64_t rows, int64_t bh) {
   return dtype == FCR_DTYPE_F32 && !in_parts(dtype, D) && (rows <= 64 || 2 * bh * ((rows + 127) / 128) <= chip_cus());
 }
 inline bool row_half_tiles(int dtype, int D, int M, int N, int64_t bh) { return (M <= 64 || N <= 15 * 64) && half_tiles(dtype, D, M, bh); }
-// Tiles of the fp32 sweeps in parts (row_lse_f32_kernel, col_reduce_f32_kernel): waves per workgroup (four: two workgroups share a
-// CU; eight: one) and resident 16-row groups per wave.  Two groups read a streamed fragment once for two blocks of scores,
-// eight waves share the split of a streamed row: 4 x 2 and 8 x 1 are 128 rows, 8 x 2 256, 4 x 1 64.  Per call, fp32:
-//   32 heads of 4096 x 4096 x 128   8x2 733 us, 4x2 828, 8x1 927      2 x 16 of 2048 x 2048 x 128 causal   4x2 141, 8x2 164, 8x1 160
-//   32 of 1024 x 1024 x 128         8x1 70, 4x2 75, 4x1 85, 8x2 86    32 of 3000 x 3000 x 128 causal       8x2 247, 4x2 255, 8x1 291
-//   16 of 1500 x 1500 x 96 causal   8x1 63, 4x1 76, 4x2 81, 8x2 89    32 of 512 x 512 x 128                4x1 32, 8x1 36, 4x2 40, 8x2 52
-// So: 256 rows where 128-row tiles are more than one per CU (with the mask, which wants some to level it, two), 8 x 1
-// where they are at most one, and 64 rows for short sweeps that leave every other CU without a workgroup.
-struct F32Tile {
-  int waves, groups;
-  int rows() const { return 16 * waves * groups; }
-};
-inline F32Tile f32_tile(int rows, int64_t bh, bool causal, bool short_sweep) {
-  const int64_t tiles = bh * ((rows + 127) / 128);   // of 128 rows
-  const int cus = chip_cus();
-  if (rows <= 64 || (short_sweep && 2 * tiles <= cus)) return F32Tile{4, 1};
-  if (tiles <= cus) return F32Tile{8, 1};
-  return !causal || tiles > 2 * cus ? F32Tile{8, 2} : F32Tile{4, 2};
-}
-// Sums and maxima of rows of D > 192 have no registers for two groups.  A sweep of at most 128 queries is all
-// prologue and takes four waves (32 heads of 64 x 8192 x 128 causal 66 us, with 8x2 tiles 73).
+using fcr_tiles::F32Tile;
 inline F32Tile f32_col_tile(int ksteps, bool both, int M, int N, int64_t bh, bool causal) {
-  F32Tile t = f32_tile(N, bh, causal, M <= 512);
-  if (both && ksteps > 6 && t.groups == 2 && bh * ((N + 127) / 128) < (1ll << 22)) return F32Tile{8, 1};
-  if (M <= 128 && t.waves == 8) return F32Tile{4, 2};
-  return t;
+  return fcr_tiles::f32_col_tile(ksteps, both, M, N, bh, causal, chip_cus());
 }
-// A row sweep of 16 chunks or more over fewer tiles than CUs is split over the idle CUs (row_splits), two workgroups each.
-inline F32Tile f32_row_tile(int M, int N, int64_t bh, bool causal) {
-  const F32Tile t = f32_tile(M, bh, causal, N <= 15 * 64);
-  return t.waves == 8 && t.groups == 1 && N > 15 * 64 && bh * ((M + 127) / 128) < chip_cus() ? F32Tile{4, 2} : t;
-}
+inline F32Tile f32_row_tile(int M, int N, int64_t bh, bool causal) { return fcr_tiles::f32_row_tile(M, N, bh, causal, chip_cus()); }
 inline int f32_ksteps(int ksteps) { return (ksteps + 1) / 2; }   // k-steps of 32 d from k-steps of 64 bytes
 inline int elem_bytes(int dtype) { return dtype == FCR_DTYPE_F32 ? 4 : 2; }
 inline int ksteps_of(int dtype, int D) { return (D * elem_bytes(dtype) + 63) / 64; }
@@ -211,7 +185,7 @@ inline int row_tile_rows(int dtype, int D, int M, int N, int64_t bh, bool causal
 constexpr int kMaxKSteps = 8;                 // rows of up to 512 bytes: two workgroups per CU
 constexpr int kMaxKStepsF32 = 16;             // rows of up to 1 KiB (fp32: D <= 256, 16-bit elements: D <= 512), one workgroup per CU
 constexpr int kChunk = 64;                    // streamed rows per LDS stage (two 32-row sub-steps)
-constexpr int64_t kMaxWorkgroups = 1ll << 24; // the runtime refuses launches of 2^32 threads or more
+using fcr_tiles::kMaxWorkgroups;
 constexpr float kNegInf = -__builtin_inff();
 constexpr float kPosInf = __builtin_inff();
 
@@ -3554,7 +3528,8 @@ int check_problem(const void* q, const void* k, int dtype, int B, int H, int M, 
                                          : "D must be a multiple of 4 in [4, 256] for FCR_DTYPE_F32");
   if (M > (1 << 30) || N > (1 << 30)) return fail(FCR_E_SHAPE, "M and N must be <= 2^30");
   const int64_t bh = (int64_t)B * H;
-  // a launch may have fewer than 2^32 threads: fewer than 2^24 workgroups of 256 (the finest tiling, 128 rows)
+  // a launch may have fewer than 2^32 threads: fewer than 2^24 workgroups of 256 (the finest tiling, 128 rows; f32_tile sees to it that
+  // workgroups of 512 are half as many)
   if (bh * (((int64_t)(by_keys ? N : M) + 127) / 128) >= kMaxWorkgroups)
     return fail(FCR_E_SHAPE, "B*H*ceil(rows/128) must be below 2^24 workgroups");
   if (!isfinite(scale)) return fail(FCR_E_SCALE, "scale must be finite");

@@ -213,3 +213,39 @@ def test_native_host_path_leaves_the_rest_to_python():
         host.reduce(x, x)
     with pytest.raises(TypeError):
         host.keep(x)
+
+
+@pytest.fixture(scope="module")
+def f32_tiles(tmp_path_factory):
+    """The tile rules of the fp32 sweeps (csrc/f32_tiles.h), compiled for the host: (waves, groups) of both sweeps."""
+    import subprocess
+    where = tmp_path_factory.mktemp("tiles")
+    (where / "t.cpp").write_text('#include "f32_tiles.h"\n'
+                                 'static int code(fcr_tiles::F32Tile t) { return t.waves * 16 + t.groups; }\n'
+                                 'extern "C" int col(int ks, int both, int m, int n, long long bh, int causal, int cus) {\n'
+                                 '  return code(fcr_tiles::f32_col_tile(ks, both, m, n, bh, causal, cus)); }\n'
+                                 'extern "C" int row(int m, int n, long long bh, int causal, int cus) {\n'
+                                 '  return code(fcr_tiles::f32_row_tile(m, n, bh, causal, cus)); }\n')
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "flash_colreduce_amd", "csrc"),
+                    str(where / "t.cpp"), "-o", str(where / "t.so")], check=True)
+    lib = ctypes.CDLL(str(where / "t.so"))
+    lib.col.argtypes = [ctypes.c_int] * 4 + [ctypes.c_longlong] + [ctypes.c_int] * 2
+    lib.row.argtypes = [ctypes.c_int] * 2 + [ctypes.c_longlong] + [ctypes.c_int] * 2
+    return (lambda *a: divmod(lib.col(*a), 16)), (lambda *a: divmod(lib.row(*a), 16))
+
+
+@pytest.mark.parametrize("rows", [1, 64, 65, 128, 129, 256, 257, 300, 384, 385, 512, 513, 1000, 4097])
+def test_fp32_launches_stay_below_the_runtime_limit(f32_tiles, rows):
+    """Whatever passes the argument check (fewer than 2^24 tiles of 128 rows) is launched with fewer than 2^32 threads."""
+    col, row = f32_tiles
+    per = (rows + 127) // 128
+    for bh in {2 ** e + i for e in range(24) for i in (-1, 0, 1)} | {(2 ** 24 - 1) // per}:
+        if bh < 1 or bh * per >= 2 ** 24:
+            continue
+        for causal in (0, 1):
+            tiles = [row(rows, other, bh, causal, 256) for other in (64, 2000)]
+            tiles += [col(ks, both, other, rows, bh, causal, 256) for ks in (1, 4, 8) for both in (0, 1) for other in (5, 128, 300, 2000)]
+            for waves, groups in tiles:
+                assert (waves, groups) in ((4, 1), (4, 2), (8, 1), (8, 2))
+                height = 16 * waves * groups
+                assert bh * ((rows + height - 1) // height) * 64 * waves < 2 ** 32, (bh, causal, waves, groups)
