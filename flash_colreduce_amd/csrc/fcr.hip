@@ -4187,7 +4187,6 @@ int col_reduce_any(const void* q, const void* k, const float* lse, void* out, vo
   if (rc) return rc;
   p.group = head_group(p.bh_count, p.tiles, causal != 0);
   const int ksteps = ksteps_of(dtype, D);
-  p.fill = fill_places(p, tile_choice(dtype, D, M, N, p.bh_count, true, mode, causal != 0), causal != 0);
   p.lse = const_cast<float*>(lse);
   p.out = out;
   p.out2 = out2;
@@ -4221,6 +4220,7 @@ int col_reduce_any(const void* q, const void* k, const float* lse, void* out, vo
       return launched("col_small_kernel");
     }
   }
+  p.fill = fill_places(p, tile_choice(dtype, D, M, N, p.bh_count, true, mode, causal != 0), causal != 0);
   launch_sweeps(dtype, 1, p, ksteps, causal != 0, mode, s);
   return launched("col_reduce_kernel");
 }
