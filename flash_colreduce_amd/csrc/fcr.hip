@@ -1704,11 +1704,13 @@ __global__ __launch_bounds__(kThreads, (NG <= 4 ? 3 : 2)) void col_small_kernel(
   u32x4 qf[NG][KS];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    const char* row = qb + (int64_t)min(16 * g + (lane & 15), p.M - 1) * p.q_sr;
+    const int first = min(16 * g, (p.M - 1) & ~15);   // of the sixteen rows that are read
+    const __amdgpu_buffer_rsrc_t view = rows_view(qb, p.q_sr, first, p.M);
+    const uint32_t roff = (uint32_t)min(lane & 15, p.M - 1 - first) * (uint32_t)p.q_sr;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int gi = ks * 4 + (lane >> 4);
-      const u32x4 v = *reinterpret_cast<const u32x4*>(row + min(gi, p.dgran - 1) * 16);
+      const u32x4 v = view_load16(view, roff + (uint32_t)min(gi, p.dgran - 1) * 16u);
       qf[g][ks] = gi < p.dgran ? v : (u32x4){0u, 0u, 0u, 0u};
     }
   }
