@@ -98,14 +98,31 @@ def load():
     return _lib
 
 
+class _PythonOnly:
+    """Stands in for csrc/host.cpp where it cannot be loaded: no call is for it."""
+
+    @staticmethod
+    def reduce(*args):
+        return None
+
+    @staticmethod
+    def keep(*args):
+        return None
+
+
 def host():
-    """The module of csrc/host.cpp (the usual call in native code), its errors raised by check()."""
+    """The module of csrc/host.cpp (the usual call in native code), its errors raised by check().
+
+    It is built against one torch; where it is missing or does not load, the Python functions make every call (the same
+    kernels, 6 to 10 us more host time each) and a warning says so.  libfcr.so has no such substitute."""
     load()
     try:
         from . import _host
     except ImportError as e:
-        raise RuntimeError(f"{os.path.join(_HERE, '_host.so')} cannot be loaded ({e}): build it with "
-                           "`python -m flash_colreduce_amd.build` (there is no fallback path)") from e
+        import warnings
+        warnings.warn(f"{os.path.join(_HERE, '_host.so')} cannot be loaded ({e}): calls go through Python. Build it with "
+                      "`python -m flash_colreduce_amd.build`.", RuntimeWarning, stacklevel=3)
+        return _PythonOnly
     _host.on_error(check)
     return _host
 

@@ -104,5 +104,5 @@ def build_c_check(verbose: bool = True) -> str:
 
 if __name__ == "__main__":
     build(extra_flags=sys.argv[1:])
-    build_host()
     build_c_check()
+    build_host()

@@ -215,6 +215,19 @@ def test_native_host_path_leaves_the_rest_to_python():
         host.keep(x)
 
 
+def test_without_the_native_host_path_calls_go_through_python(monkeypatch):
+    """_host.so missing, or built against another torch: a warning, and nothing is refused."""
+    import sys
+    from flash_colreduce_amd import flash as F
+    monkeypatch.delattr(fca, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "flash_colreduce_amd._host", None)
+    monkeypatch.setattr(F, "_native", None)
+    with pytest.warns(RuntimeWarning, match="_host.so cannot be loaded"):
+        host = F._host()
+    x = torch.zeros(1, 1, 2, 8)
+    assert F._host() is host and host.reduce(x, x, "sum", False, None, None, False) is None and host.keep(x, 1, False) is None
+
+
 @pytest.fixture(scope="module")
 def f32_tiles(tmp_path_factory):
     """The tile rules of the fp32 sweeps (csrc/f32_tiles.h), compiled for the host: (waves, groups) of both sweeps."""
