@@ -60,6 +60,8 @@ def _declare(lib):
                                         c.c_void_p, c.c_size_t, c.c_void_p]
     lib.fcr_topk_bytes.restype = c.c_size_t
     lib.fcr_topk_bytes.argtypes = [c.c_int64, c.c_int]
+    lib.fcr_topk_bytes_typed.restype = c.c_size_t
+    lib.fcr_topk_bytes_typed.argtypes = [c.c_int, c.c_int64, c.c_int]
     lib.fcr_topk_mask_ws.restype = c.c_int
     lib.fcr_topk_mask_ws.argtypes = [c.c_void_p, c.c_void_p, c.c_void_p, c.c_int64, c.c_int, c.c_int, c.c_void_p,
                                      c.c_size_t, c.c_void_p]

@@ -2651,6 +2651,7 @@ __device__ __forceinline__ float key_value(uint32_t key) {
 }
 
 constexpr int kTopkThreads = 1024;
+constexpr int kTopk16Columns = 64 * kTopkThreads;   // of a 16-bit row that one workgroup selects from in one launch
 
 // Sum of v over the 64 lanes, as a wave-uniform value: butterflies inside rows of 16 lanes, then the row
 // totals are passed on to the rows behind and lane 63 holds the total.
@@ -4082,12 +4083,12 @@ int topk_any(const ET* scores, uint8_t* mask, float* threshold, int64_t rows, in
              hipStream_t s) {
   constexpr int T = kTopkThreads;
   if constexpr (sizeof(ET) == 2) {
-    // up to 65536 columns fit the registers of one workgroup, eight to a 16-byte vector
+    // up to kTopk16Columns fit the registers of one workgroup, eight to a 16-byte vector
     if (N <= 8 * 256) return launch_topk16<256, 1>(scores, mask, threshold, rows, N, k, s), 0;
     if (N <= 8 * T) return launch_topk16<T, 1>(scores, mask, threshold, rows, N, k, s), 0;
     if (N <= 16 * T) return launch_topk16<T, 2>(scores, mask, threshold, rows, N, k, s), 0;
     if (N <= 32 * T) return launch_topk16<T, 4>(scores, mask, threshold, rows, N, k, s), 0;
-    if (N <= 64 * T) return launch_topk16<T, 8>(scores, mask, threshold, rows, N, k, s), 0;
+    if (N <= kTopk16Columns) return launch_topk16<T, 8>(scores, mask, threshold, rows, N, k, s), 0;
   }
   const size_t want = fcr_topk_bytes(rows, N);
   if (ws && want != 0 && ws_bytes >= want) {
@@ -4249,6 +4250,10 @@ size_t fcr_topk_bytes(int64_t rows, int N) {
   const int parts = (N + 8 * kTopkThreads - 1) / (8 * kTopkThreads);   // the finer of the two ways to cut a row
   if (rows * parts >= (1ll << 22)) return 0;   // more workgroups of 1024 threads than one launch may have
   return 2 * topk_hist_words(rows, parts) * sizeof(uint32_t) + (size_t)rows * 4 * sizeof(TopkState);
+}
+size_t fcr_topk_bytes_typed(int dtype, int64_t rows, int N) {
+  if (dtype != FCR_DTYPE_F16 && dtype != FCR_DTYPE_BF16 && dtype != FCR_DTYPE_F32) return 0;
+  return elem_bytes(dtype) == 2 && N <= kTopk16Columns ? 0 : fcr_topk_bytes(rows, N);
 }
 
 int fcr_topk_mask_typed(const void* scores, int dtype, uint8_t* mask, float* threshold, int64_t rows, int N, int k,

@@ -149,7 +149,7 @@ PyObject* keep(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (c10::hip::current_device() != s.device().index()) Py_RETURN_NONE;
     at::Tensor mask = at::empty(s.sizes(), s.options().dtype(at::kBool)), threshold, ws;
     if (with_threshold) threshold = at::empty(s.sizes().slice(0, s.dim() - 1), s.options().dtype(at::kFloat));
-    const size_t bytes = fcr_topk_bytes(rows, (int)cols);
+    const size_t bytes = fcr_topk_bytes_typed(code, rows, (int)cols);
     if (bytes) ws = at::empty({(int64_t)bytes}, s.options().dtype(at::kByte));
     void* const stream = c10::hip::getCurrentHIPStream(s.device().index()).stream();
     const void* const sd = s.const_data_ptr();

@@ -385,7 +385,7 @@ def topk_keep_mask(scores: torch.Tensor, k: int, return_threshold: bool = False)
     thr = torch.empty(s.shape[:-1], device=s.device, dtype=torch.float32) if return_threshold else None   # always fp32
     if rows > 0 and n > 0:
         lib = _lib.load()
-        nbytes = lib.fcr_topk_bytes(rows, n)   # > 0 for long rows: scratch that lets workgroups share a row
+        nbytes = lib.fcr_topk_bytes_typed(_DTYPES[s.dtype], rows, n)   # > 0 for long rows: scratch that lets workgroups share a row
         ws = torch.empty(nbytes, device=s.device, dtype=torch.uint8) if nbytes else None
         with torch.cuda.device(s.device):
             _lib.check(lib.fcr_topk_mask_typed(s.data_ptr(), _DTYPES[s.dtype], mask.data_ptr(),

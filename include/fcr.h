@@ -143,9 +143,10 @@ int fcr_topk_mask_ws(const float* scores, uint8_t* mask, float* threshold, int64
 /*
  * The same for score rows of any FCR_DTYPE_* element type: fp16 and bf16 rows, as fcr_colreduce_to stores
  * them for 16-bit operands, are read as they are (order and ties of the stored values; threshold stays
- * fp32).  ws may be NULL (then ws_bytes is ignored); fcr_topk_bytes does not depend on the type, 16-bit
- * rows of up to 65536 columns do not read ws.
+ * fp32).  ws may be NULL (then ws_bytes is ignored).  16-bit rows of up to 65536 columns do not read ws: fcr_topk_bytes does not
+ * depend on the type, fcr_topk_bytes_typed is what a type's rows can use (0 for an unknown type).
  */
+size_t fcr_topk_bytes_typed(int dtype, int64_t rows, int N);
 int fcr_topk_mask_typed(const void* scores, int dtype, uint8_t* mask, float* threshold, int64_t rows, int N, int k,
                         void* ws, size_t ws_bytes, void* stream);
 

@@ -215,6 +215,17 @@ def test_native_host_path_leaves_the_rest_to_python():
         host.keep(x)
 
 
+def test_topk_scratch_is_what_the_type_can_use():
+    lib = _lib.load()
+    for rows in (1, 32, 1000):
+        for n in (1, 32768, 32769, 65536, 65537, 1 << 20):
+            plain = lib.fcr_topk_bytes(rows, n)
+            assert lib.fcr_topk_bytes_typed(_lib.DTYPE_F32, rows, n) == plain and (plain > 0) == (n > 32768)
+            for dtype in (_lib.DTYPE_F16, _lib.DTYPE_BF16):
+                assert lib.fcr_topk_bytes_typed(dtype, rows, n) == (plain if n > 65536 else 0)
+    assert lib.fcr_topk_bytes_typed(3, 32, 100000) == 0 and lib.fcr_topk_bytes_typed(_lib.DTYPE_F32, 0, 100000) == 0
+
+
 def test_without_the_native_host_path_calls_go_through_python(monkeypatch):
     """_host.so missing, or built against another torch: a warning, and nothing is refused."""
     import sys

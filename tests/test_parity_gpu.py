@@ -1664,6 +1664,23 @@ def test_native_host_path_gives_what_the_general_one_gives(dtype, monkeypatch):
             assert torch.equal(torch.nan_to_num(x.float(), nan=7.5), torch.nan_to_num(y.float(), nan=7.5))
 
 
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("dtype,n,scratch", [(torch.float16, 50000, False), (torch.bfloat16, 65536, False), (torch.float16, 65544, True),
+                                             (torch.float32, 50000, True)])
+def test_topk_allocates_no_scratch_that_no_kernel_reads(dtype, n, scratch, native, monkeypatch):
+    from flash_colreduce_amd import flash as F
+    if not native:
+        monkeypatch.setattr(F, "_native", _NeverNative())
+    s = torch.rand(4, n, device="cuda").to(dtype)
+    fca.topk_keep_mask(s, 100)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    mask = fca.topk_keep_mask(s, 100)
+    extra = torch.cuda.max_memory_allocated() - before
+    assert (extra > 4 * n + 4096) == scratch and mask.sum().item() == 400
+
+
 def test_native_host_path_under_capture_streams_and_modes():
     """Allocations and launches go where torch's would: into a captured graph (replayed with other contents and eager calls between),
     on the caller's stream, out of inference mode; a refused argument of the library raises its error."""
