@@ -1033,13 +1033,21 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 
 // ---------------------------------------------------------------------------------------------
 // fp32 operands.  Each row is scaled by a power of two that puts its largest element at 2^14..2^15 and every element x is split
-// into two fp16 numbers, h = fp16(x) and l = fp16(x - h): 22 to 24 significant bits of x, and of elements smaller than 2^-16 of
-// the row's largest everything down to 2^-40 of that one.  A product is h h' + h l' + l h' (l l' is below 2^-24 of it), each
+// into two fp16 numbers, h = fp16(x) and l = fp16(x - h): x to 2^-23 (one element in four loses its last bit), and elements smaller
+// than 2^-16 of the row's largest to 2^-39 of that one (see SplitRing::set_limit).  A product is h h' + h l' + l h', each
 // exact in fp32 and added up by v_mfma_f32_16x16x32_f16: 48 matrix cycles per 16 x 16 x 32 block where
-// v_mfma_f32_16x16x4_f32 takes 256.  Error of the scores against sums in 64 bits, relative 2-norm over N(0,1) rows (and over
+// v_mfma_f32_16x16x4_f32 takes 256.  What is left out, l l', is up to 2^-22 of it, so a product may be off by 2^-21 in all; the
+// rounding of the running sum, 24 times at D = 256 where the fp32 instructions round 64 times, is the larger part in sums
+// of more than about a dozen terms of like size.  Error of the scores against sums in 64 bits, relative 2-norm over N(0,1) rows (and over
 // rows whose elements spread by e^(3 N(0,1))): D = 32 8.8e-8 (8.6e-8), 64 1.1e-7 (1.1e-7), 128 1.4e-7 (1.4e-7), 256
 // 1.9e-7 (1.6e-7); the fp32 instructions, which round the running sum after every term: 1.0e-7 (1.2e-7), 1.5e-7
-// (1.5e-7), 2.0e-7 (1.9e-7), 2.9e-7 (2.5e-7).  Shorter rows have few terms to round (D = 16 8.4e-8 against 7.4e-8) and do
+// (1.5e-7), 2.0e-7 (1.9e-7), 2.9e-7 (2.5e-7).  Results over the shapes and key distributions of the timed cases (geometric mean of 40
+// calls, sums and maxima; in brackets the fp32 instructions): N(0,1) 3.19e-7 and 4.3e-7 (3.21e-7, 5.7e-7), keys with an offset
+// 3.04e-7, 4.6e-7 (3.07e-7, 6.1e-7), with sinks 5.5e-7, 1.40e-6 (5.6e-7, 1.42e-6).  Where few terms make a score the fp32 instructions are the more
+// exact: one product per score 8.3e-8 against 2.5e-8 (largest 4.8e-7, 6e-8), scores of 60 from two products each sums 2.6e-6
+// against 2.3e-7.  Giving those back was measured and costs more than it gives: l l' as a fourth product, 5 to 21 % of the time, one
+// product 7e-8, scores of 60 unchanged; three bf16 parts and six products, exact operands, 2.6e-8 and 2.2e-7, 1.35 to 1.85 times the time.
+// Rows shorter than 32 have few terms to round (D = 16 8.4e-8 against 7.4e-8) and do
 // not come here (in_parts).  A row with an infinity or a
 // NaN has no scale; chunks and resident rows that hold one are multiplied on the fp32 instructions, from memory (exact_scores).
 //

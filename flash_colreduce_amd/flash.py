@@ -83,7 +83,7 @@ def pack_f32(x: torch.Tensor, is_key: bool, terms: int = 3) -> torch.Tensor:
     """fp32 (B,H,R,D) -> the fp16 segments of fcr_pack_f32 (include/fcr.h), for callers of the C ABI that
     want fp32 operands packed once for the 16-bit kernels and accept
     fp16's range: terms = 3 gives products to about 2^-22 and needs 3 * ceil8(D) <= 256, terms = 1 is one
-    rounding to fp16.  flash_colreduce itself never comes here: it keeps fp32's precision and range."""
+    rounding to fp16.  flash_colreduce itself never comes here: it keeps fp32's range (see out of which parts in include/fcr.h)."""
     b, h, r, d = x.shape
     dpad = (d + 7) // 8 * 8
     src = x.contiguous()
@@ -261,7 +261,7 @@ def flash_colreduce(
     """Per-key sum / mean / max over queries of softmax(Q K^T * scale), shape (B, H, N).
 
     Args follow the reference (flash.py:311-352): query (B,H,M,D), key (B,H,N,D), fp16, bf16 or
-    fp32 on the GPU, rows of at most 1 KiB: D <= 512, D <= 256 for fp32 (fp32 operands are multiplied in fp32); `is_causal` applies the right-aligned mask (key j visible to query i iff
+    fp32 on the GPU, rows of at most 1 KiB: D <= 512, D <= 256 for fp32 (multiplied as two fp16 parts of each element from D = 32 on, to 2^-21 per product: include/fcr.h); `is_causal` applies the right-aligned mask (key j visible to query i iff
     j <= i + max(N-M, 0)); `scale` defaults to 1/sqrt(D).
 
     `out_dtype` (keyword only, not in the reference) selects the result dtype.  None reproduces

@@ -16,9 +16,12 @@
  *     16-bit elements, a multiple of 4 in [4, 256] for fp32.  Rows must not overlap (row stride >= D).
  *     (The reference takes any strides, flash.py:292-299; a caller with other layouts makes a
  *     contiguous, zero-padded copy first -- the Python host does.)  fp32 operands are multiplied at
- *     fp32 precision and range (the reference's tl.dot rounds them to TF32, flash.py:59,108): from D = 32 on as two
- *     fp16 parts of each element, scaled by row, whose scores are closer to 64-bit sums than those of the fp32 matrix
- *     instructions; elements below 2^-16 of the largest of their row are held to 2^-40 of that one.
+ *     fp32 range (the reference's tl.dot rounds them to TF32, flash.py:59,108), from D = 32 on as two
+ *     fp16 parts of each element, scaled by row: an element to 2^-23, a product to 2^-21.  Scores of N(0,1) operands, and results over
+ *     operands with sinks or offsets, are closer to 64-bit sums than those of the fp32 matrix instructions; scores of
+ *     few products are not (one product: 8e-8 against 2.5e-8 in the mean).  Elements below 2^-16 of the largest of their row are held to 2^-39
+ *     of that one; where that could show in a score (the largest elements of a query and a key above 300 each at the
+ *     default scale), and from 2^104 on, the fp32 instructions multiply, at about a fifth of the rate.
  *   - lse is fp32 [B*H, M] contiguous: per query row, log2(sum_j 2^(scale*log2(e)*<q_i,k_j>))
  *     over the keys the row may see.  It is the hand-over between the two kernels.  The buffer
  *     fcr_row_lse / fcr_colreduce write it to must be fcr_lse_bytes(B,H,M,N,D) long (scratch follows

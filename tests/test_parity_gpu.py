@@ -68,7 +68,7 @@ def test_config1_rounded_to_fp16():
 
 
 def test_config1_fp32():
-    """Config 1 as given: fp32 operands, multiplied on the fp32 matrix instructions.  The device result
+    """Config 1 as given: fp32 operands, multiplied as two fp16 parts (D = 64).  The device result
     is good far beyond the metric's tolerance; 1e-5 would fail with any 16-bit rounding of the operands."""
     q, k = _inputs.config1()
     qd, kd = q.cuda(), k.cuda()
@@ -85,7 +85,7 @@ def test_config1_fp32():
                                    (130, 140, 200), (300, 420, 132), (64, 1000, 256), (257, 129, 252),
                                    (40, 3000, 160)])
 def test_fp32_operands(m, n, d, causal):
-    """fp32 inputs are multiplied in fp32 for every D up to 256: held to 1e-5, which no 16-bit rounding of
+    """fp32 inputs keep their precision for every D up to 256: held to 1e-5, which no 16-bit rounding of
     the operands meets (D = 6 is zero padded to 8; rows of more than 512 bytes take the 1 KiB ring)."""
     q, k = _inputs.randn_pair(2, 2, m, n, d, seed=d, dtype=torch.float32)
     qd, kd = q.cuda(), k.cuda()
@@ -410,7 +410,8 @@ def test_fp32_rows_shorter_than_32(h, m, n, d, causal):
 def test_fp32_split_tiles(h, m, n, d, causal):
     """fp32 rows as two fp16 parts: tiles of 256, 128 and 64 rows with ragged ends, more than one and more than two 128-row tiles
     per CU (which the mask treats differently), D that ends inside eight values, both sides of D = 32.  Probabilities carry
-    the error of the scores, a few 1e-7 here, and a sum that of its additions: 1e-5 as for the other fp32 tests."""
+    the error of the scores (N(0,1) operands: 2^-21 of a sum of |q_d k_d| / sqrt(D) of ten or less, hardly ever all of it one
+    way), and a sum that of its additions: 1e-5 as for the other fp32 tests."""
     q, k = _inputs.randn_pair(1, h, m, n, d, seed=h + d, dtype=torch.float32)
     s, mx = fca.flash_colreduce_multi(q.cuda(), k.cuda(), ["sum", "max"], is_causal=causal)
     for red, pair in (("sum", s), ("mean", None), ("max", mx)):
@@ -422,10 +423,11 @@ def test_fp32_split_tiles(h, m, n, d, causal):
 
 @pytest.mark.parametrize("d", [24, 32, 128, 256])
 def test_fp32_split_rows_of_any_magnitude(d):
-    """Every row is scaled by its own power of two, from the largest float to denormal ones, and the spread inside a
-    row does not matter.  A score is off by at most 2^-23 of |q||k| per product (two parts of 2^-24 each and what is left
-    out) plus the roundings of its sum, so a log-sum-exp by at most 2^-20 of the row's largest sum of |q_d k_d|,
-    and by two units in the last place of a value between 8 and 16 (log2 of 300 keys), 2^-19, for its own rounding: a logarithm and
+    """Every row is scaled by its own power of two (test_fp32_operands_near_the_ends_of_the_range has the ends), and the spread
+    inside a row does not matter.  A score is off by at most 2^-21 of |q||k| per product (2^-23 for each operand, 2^-22 for the
+    product of the lower parts) and by the roundings of its sum, at most 2^-24 of the running sum in each of up to 24 matrix
+    instructions; signs vary, so running sums stay below a third of the sum of |q_d k_d|, which makes it 2^-21 too.  A log-sum-exp
+    is off by at most 2^-20 of the row's largest sum of |q_d k_d|, and by two units in the last place of a value between 8 and 16 (log2 of 300 keys), 2^-19, for its own rounding: a logarithm and
     the additions that merge four partial results."""
     m, n = 260, 300
     g = torch.Generator().manual_seed(d)
@@ -460,6 +462,40 @@ def test_fp32_operands_near_the_ends_of_the_range(m, n, d, exponent):
         got = fca.flash_colreduce(small.cuda(), big.cuda(), red)
         assert torch.isfinite(got).all(), red
         torch.testing.assert_close(got.cpu(), colreduce_ref(q, k, red, False, compute_dtype=torch.float64).float(), rtol=1e-5, atol=1e-8)
+
+
+@pytest.mark.parametrize("d", [16, 32, 128, 256])
+def test_fp32_scores_of_one_product(d):
+    """One non-zero product per score: 2^-21 of it at most (2^-23 for each operand, 2^-22 for the product of the lower parts; D < 32:
+    one rounding), and 2^-23 for the scale and the sum; random mantissas and those that lose the most."""
+    g = torch.Generator().manual_seed(d)
+    bh, m = 96, 70
+    q, k = torch.zeros(1, bh, m, d), torch.zeros(1, bh, 1, d)
+    at = torch.randint(0, d, (bh,), generator=g)
+    q[0, torch.arange(bh), :, at] = torch.randn(bh, m, generator=g)
+    k[0, torch.arange(bh), 0, at] = torch.randn(bh, generator=g)
+    for i, (x, y) in enumerate(((1 + 2.0 ** -11, 1 + 2.0 ** -11), (1 + 2.0 ** -11 - 2.0 ** -13,) * 2, (2 - 2.0 ** -23,) * 2,
+                                (1 + 2.0 ** -11 - 2.0 ** -23, 1 + 2.0 ** -11 + 2.0 ** -23))):
+        q[0, i, :, at[i]], k[0, i, 0, at[i]] = x, -y
+    want = (q.double() * k.double()).sum(-1) * 1.4426950408889634
+    err = (fca.row_lse2(q.cuda(), k.cuda(), scale=1.0).cpu().double() - want).abs()
+    assert (err <= (2.0 ** -21 + 2.0 ** -23) * want.abs()).all(), (err / want.abs()).max()
+
+
+@pytest.mark.parametrize("d", [16, 64, 256])
+def test_fp32_large_scores_of_two_products(d):
+    """Scores of 60 from two products each.  An exponent of 2 is off by 2^-21 of its size (as above) and 2^-23 for the roundings of
+    sum, scale and log-sum-exp, a probability by ln 2 times twice that (its own score and the row's sum)."""
+    g = torch.Generator().manual_seed(d)
+    q, k = torch.zeros(1, 4, 300, d), torch.zeros(1, 4, 500, d)
+    for at in (5, 9):
+        q[..., at] = 7 + torch.randn(1, 4, 300, generator=g).abs()
+        k[..., at] = 4 + 0.1 * torch.randn(1, 4, 500, generator=g)
+    size = (torch.matmul(q.double(), k.double().transpose(2, 3)) * 1.4427).max().item()
+    rtol = 0.6932 * 2 * (2.0 ** -21 + 2.0 ** -23) * size
+    for red in ("sum", "max"):
+        want = colreduce_ref(q, k, red, False, scale=1.0, compute_dtype=torch.float64).float()
+        torch.testing.assert_close(fca.flash_colreduce(q.cuda(), k.cuda(), red, scale=1.0).cpu(), want, rtol=rtol, atol=1e-8)
 
 
 @pytest.mark.parametrize("side", ["query", "key"])
