@@ -1214,7 +1214,7 @@ struct SplitRing {
     uint32_t x = 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) x = max(x, (uint32_t)bad()[4 + w]);
-    const float y = split_most / __builtin_bit_cast(float, x);
+    const float y = split_most * __builtin_amdgcn_rcpf(__builtin_bit_cast(float, x));   // (x = 0: infinity)
     limit = __builtin_amdgcn_readfirstlane(min(__builtin_bit_cast(uint32_t, y), kNoScale));   // (a NaN has larger bits)
   }
   __device__ __forceinline__ void note(int t, uint32_t largest) {
