@@ -17,8 +17,9 @@ constexpr int64_t kMaxWorkgroups = 1ll << 24; // of 256 threads: the runtime ref
 //   32 of 2048 x 2048 x 160         8x2 247, 4x2 313, 8x1 330         32 of 512 x 512 x 128                4x1 32, 8x1 36, 4x2 40, 8x2 52
 // So: 256 rows where 128-row tiles are more than one per CU (with the mask, which wants some to level it, two), 8 x 1
 // where they are at most that, and 64 rows for short sweeps that leave every other CU without a workgroup.  The 256-row form
-// of D > 224 that produces sums and maxima with the mask keeps 17 of its registers in memory (the others none or one) and is
-// the fastest all the same: 40 heads of 3000 x 3000 x 256 8x2 569 us, 4x2 619, 8x1 651.
+// of D > 224 that produces sums and maxima keeps 17 of its registers in memory with the mask and 8 without (other forms none or one) and is
+// the fastest all the same: 40 heads of 3000 x 3000 x 256 causal 8x2 569 us, 4x2 619, 8x1 651.  (4x2 of the same keeps 73; only launches that
+// eight waves would take past the runtime's limit come to it.)
 struct F32Tile {
   int waves, groups;
   int rows() const { return 16 * waves * groups; }
