@@ -273,3 +273,14 @@ def test_fp32_launches_stay_below_the_runtime_limit(f32_tiles, rows):
                 assert (waves, groups) in ((4, 1), (4, 2), (8, 1), (8, 2))
                 height = 16 * waves * groups
                 assert bh * ((rows + height - 1) // height) * 64 * waves < 2 ** 32, (bh, causal, waves, groups)
+
+
+def test_fp32_tiles_with_the_mask(f32_tiles):
+    """One to two 128-row tiles per CU with the mask: eight waves where the sweeps differ in length, four where most are whole or short."""
+    col, row = f32_tiles
+    for m, n, bh, waves in ((1500, 1500, 40, 8), (1000, 1400, 40, 8), (1400, 1000, 40, 8), (1000, 1900, 30, 4), (481, 2000, 20, 4), (512, 700, 60, 4)):
+        assert col(4, 0, m, n, bh, 1, 256)[0] == waves, (m, n)
+    for m, n, bh, waves in ((1500, 1500, 33, 8), (1000, 1400, 33, 8), (1000, 1900, 33, 4), (2000, 700, 24, 4)):
+        assert row(m, n, bh, 1, 256)[0] == waves, (m, n)
+    assert col(4, 0, 2000, 2000, 20, 0, 256) == (8, 2) and col(4, 0, 2000, 2000, 48, 1, 256) == (8, 2)   # no mask; three per CU
+    assert col(2, 1, 12, 15478, 2, 0, 256) == (4, 2) and col(8, 1, 128, 1024, 32, 1, 256) == (8, 1)
