@@ -1137,8 +1137,8 @@ struct SplitRing {
   static constexpr int kPlane = kChunkRows * kPitch;
   static constexpr int kStage = 2 * kPlane;
   static constexpr int kRowFloats = 2 * kChunkRows;          // two floats per row of a stage: its scale, and what the caller adds
-  // two stages, their row floats, a word for each (see `bad`) and one for each wave (see `set_limit`)
-  static constexpr int kBytes = 2 * kStage + 2 * kRowFloats * 4 + 16 + 4 * NW;
+  // two stages, their row floats, a word for each (see `bad`) and two for each wave (see `set_limit`)
+  static constexpr int kBytes = 2 * kStage + 2 * kRowFloats * 4 + 16 + 8 * NW;
   static constexpr int kPer = kChunkRows * kRowGranules / kNumThreads;   // granules per thread
   static_assert(kPer * kNumThreads == kChunkRows * kRowGranules, "whole granules per thread");
 
@@ -1207,15 +1207,21 @@ struct SplitRing {
   // either sign, at 2^-22 in the exponent of 2, what the fp32 instructions lose on N(0,1) rows of D = 128 (2.0e-7 of a score
   // of about one).  Rows of the default scale get there with elements of 300 in both; keys and queries of
   // N(0,1) are at 2^5, keys times eight at 2^8.
-  __device__ __forceinline__ void publish(int wave, uint32_t res_largest) {
+  __device__ __forceinline__ void publish(int wave, uint32_t res_largest, uint32_t first_largest) {   // first_largest: of the wave's part of the first chunk
     bad()[4 + wave] = has_no_scale(res_largest) ? 0 : (int)res_largest;   // (such a wave multiplies on the fp32 instructions anyway)
+    bad()[4 + NW + wave] = (int)first_largest;
   }
-  __device__ __forceinline__ void set_limit(float split_most) {   // behind a barrier after publish()
-    uint32_t x = 0;
+  // Behind a barrier after publish(); returns whether the first chunk holds a row that `bad` is to tell of.
+  __device__ __forceinline__ bool set_limit(float split_most) {
+    uint32_t x = 0, first = 0;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) x = max(x, (uint32_t)bad()[4 + w]);
+    for (int w = 0; w < NW; ++w) {
+      x = max(x, (uint32_t)bad()[4 + w]);
+      first = max(first, (uint32_t)bad()[4 + NW + w]);
+    }
     const float y = split_most * __builtin_amdgcn_rcpf(__builtin_bit_cast(float, x));   // (x = 0: infinity)
     limit = __builtin_amdgcn_readfirstlane(min(__builtin_bit_cast(uint32_t, y), kNoScale));   // (a NaN has larger bits)
+    return (uint32_t)__builtin_amdgcn_readfirstlane(first) >= limit;
   }
   __device__ __forceinline__ void note(int t, uint32_t largest) {
     if (largest >= limit) bad()[t & 1] = t;
@@ -1365,10 +1371,11 @@ __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, cons
   for (int i = 0; i < PER; ++i) rg.put_granule(i, t0, tid, first_largest);
   extra(t0);
   rg.template fetch<AUX>();
-  rg.publish(tid >> 6, res_largest);   // (the resident rows may still be on their way up to here)
-  ring_sync<63>();                     // (the words at bad() are set)
-  rg.set_limit(split_most);
-  rg.note(t0, first_largest);
+  first_largest = lanes_max<32>(first_largest);
+  first_largest = max((uint32_t)__builtin_amdgcn_readlane((int)first_largest, 0), (uint32_t)__builtin_amdgcn_readlane((int)first_largest, 32));
+  rg.publish(tid >> 6, res_largest, first_largest);   // (the resident rows may still be on their way up to here)
+  ring_sync<63>();   // the first chunk is staged
+  const bool first_bad = rg.set_limit(split_most);
   f32x4 kept[NG][SG];   // the scores not yet consumed
   Aux kept_aux;
   auto chunk = [&](int t, const Fragments<SG>& first, auto first_tag) {
@@ -1400,12 +1407,12 @@ __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, cons
     }
     rg.note(t + 1, largest);
   };
-  bool entered = false;
+  bool entered = true;
   for (int t = t0; t < t1;) {
     if (!entered) ring_sync<63>();   // waits for LDS accesses only: the fetch stays in flight
     entered = false;
     Fragments<SG> first = read_fragments<SG>(rg, rg.stage_of(t), 0, 0);   // (in flight while the word is looked at)
-    const bool exact = res_bad || rg.is_bad(t);
+    const bool exact = res_bad || (t == t0 ? first_bad : rg.is_bad(t));
     if (idle || exact || t < ta || t >= tb) {
       rg.put(t + 1, tid);
       extra(t + 1);
