@@ -19,10 +19,9 @@ constexpr int64_t kMaxWorkgroups = 1ll << 24; // of 256 threads: the runtime ref
 // where they are at most that, and 64 rows for short sweeps that leave every other CU without a workgroup.  Where most sweeps
 // are whole (M and N a factor of 1.5 apart) or of at most 512 streamed rows the mask leaves little to level and 4 x 2 stays (32 heads of 330 x 1294 x 224, maxima, 4x2 67,
 // 8x1 75.5; 48 of 1084 x 3477 x 80, maxima, 214, 226; 8 x 12 of 481 x 10807 x 192, sums and maxima, 1425, 1546; 40 of 512 x 900 x 64
-// 31.6, 33.2; 32 of 1000 x 1900 x 128 101, 110; but of 1000 x 1300 x 128 73.5, 67.8).  The 256-row form
-// of D > 224 that produces sums and maxima keeps 17 of its registers in memory with the mask and 8 without (other forms none or one) and is
-// the fastest all the same: 40 heads of 3000 x 3000 x 256 causal 8x2 569 us, 4x2 619, 8x1 651.  (4x2 of the same keeps 73; only launches that
-// eight waves would take past the runtime's limit come to it.)
+// 31.6, 33.2; 32 of 1000 x 1900 x 128 101, 110; but of 1000 x 1300 x 128 73.5, 67.8).  The 256-row forms
+// of D > 192 keep some registers in memory (rows up to 12, columns 1, sums and maxima 17 with the mask and 8 without) and are
+// the fastest all the same: 40 heads of 3000 x 3000 x 256 causal, sums and maxima, 8x2 569 us, 4x2 619, 8x1 651.
 struct F32Tile {
   int waves, groups;
   int rows() const { return 16 * waves * groups; }

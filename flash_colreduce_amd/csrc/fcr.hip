@@ -1371,9 +1371,11 @@ __device__ __forceinline__ void split_sweep(int t0, int ta, int tb, int t1, cons
   for (int i = 0; i < PER; ++i) rg.put_granule(i, t0, tid, first_largest);
   extra(t0);
   rg.template fetch<AUX>();
-  first_largest = lanes_max<32>(first_largest);
-  first_largest = max((uint32_t)__builtin_amdgcn_readlane((int)first_largest, 0), (uint32_t)__builtin_amdgcn_readlane((int)first_largest, 32));
-  rg.publish(tid >> 6, res_largest, first_largest);   // (the resident rows may still be on their way up to here)
+  first_largest = lanes_max<16>(first_largest);
+  uint32_t wave_largest = 0;
+#pragma unroll
+  for (int l = 0; l < 64; l += 16) wave_largest = max(wave_largest, (uint32_t)__builtin_amdgcn_readlane((int)first_largest, l));
+  rg.publish(tid >> 6, res_largest, wave_largest);   // (the resident rows may still be on their way up to here)
   ring_sync<63>();   // the first chunk is staged
   const bool first_bad = rg.set_limit(split_most);
   f32x4 kept[NG][SG];   // the scores not yet consumed
