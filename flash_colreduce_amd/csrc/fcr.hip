@@ -23,6 +23,7 @@
 //   col_fused_kernel  both sweeps in one for at most 128 query rows against many 16-bit keys: the scores of
 //                     1024 keys stay in registers while the workgroups that share a (batch, head) pair
 //                     exchange their row sums through tagged 64-bit slots, so the keys are read once.
+//   few_keys_kernel   both sweeps in one for pairs whose 16-bit keys fit the registers of a workgroup (up to 512).
 //   topk_mask_kernel  keep-mask of the k largest columns of every row of the result (one workgroup per
 //                     row; topk_spread_* kernels share a long row between workgroups).
 // where s_ij = scale * log2(e) * <q_i, k_j>.  The column kernels store the result type of the caller's choice
@@ -48,7 +49,7 @@
 // The file can be compiled whole, or in parts that are linked together (the build script does that to
 // use several cores): part 0 holds the C ABI and the small kernels, parts 1-4 the sweeps of one element
 // type each (fp16, bf16, fp32 rows up to 512 bytes, longer fp32 rows), parts 5 and 6 the sweeps over fp16 and
-// bf16 rows of more than 512 bytes, parts 7 and 8 the single sweep for fp16 and bf16.
+// bf16 rows of more than 512 bytes, parts 7 and 8 the single sweep for fp16 and bf16, parts 9 and 10 few_keys_kernel for them.
 #ifndef FCR_PART
 #define FCR_PART -1
 #endif
@@ -93,6 +94,8 @@ void sweeps_f32(int which, const Params& p, int ksteps, bool causal, int mode, h
 void sweeps_f32_long_rows(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 void sweeps_f16_single(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);    // col_fused_kernel
 void sweeps_bf16_single(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
+void sweeps_f16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s);   // few_keys_kernel
+void sweeps_bf16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s);
 void sweeps_f16_long_rows(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 void sweeps_bf16_long_rows(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 extern thread_local bool fused_refused;   // set by a launcher of col_fused_kernel that did not launch
@@ -394,24 +397,39 @@ __device__ __forceinline__ void ring_sync() {
   asm volatile("" ::: "memory");
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_row(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+// All LDS accesses of this wave done, then the workgroup's barrier.  Loads and stores to memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (7 << 4) | (0 << 8));   // vmcnt(63) expcnt(7) lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // clamp(x, 0, kChunk) on the scalar unit (written out because the compiler turns min(max()) into a
 // three-operand median that only the vector unit has, which would make everything derived from it,
 // here a buffer descriptor, a per-lane value)
+template <int CR = kChunk>
 __device__ __forceinline__ int rows_in_chunk(int rows_left) {
   int live;
-  asm("s_max_i32 %0, %1, 0\n\ts_min_i32 %0, %0, %2" : "=s"(live) : "s"(rows_left), "n"(kChunk) : "scc");
+  asm("s_max_i32 %0, %1, 0\n\ts_min_i32 %0, %0, %2" : "=s"(live) : "s"(rows_left), "n"(CR) : "scc");
   return live;
 }
 
-// LW: the waves that issue the loads (their index is what init() takes as wave_id)
-template <int KS, int NS = ring_stages(KS), int LW = kWaves>
+// LW: the waves that issue the loads (their index is what init() takes as wave_id); CR: rows of a chunk
+template <int KS, int NS = ring_stages(KS), int LW = kWaves, int CR = kChunk>
 struct Ring {
   static constexpr int kN = NS;
   static constexpr int kPitch = KS <= 1 ? 64 : KS == 2 ? 128 : KS <= 4 ? 256 : KS <= 8 ? 512 : 1024;   // LDS row pitch
   static constexpr int kRowsPerLoad = 1024 / kPitch;                 // rows one wave-wide load covers
-  static constexpr int kPer = kChunk / (LW * kRowsPerLoad);          // loads per loading wave and chunk
-  static constexpr int kRows = kChunk * kPitch;                      // bytes of rows in a stage
-  static constexpr int kStage = kRows + kChunk * 4;                  // rows + 64 floats
+  static constexpr int kPer = CR / (LW * kRowsPerLoad);              // loads per loading wave and chunk
+  static_assert(kPer * LW * kRowsPerLoad == CR, "whole loads");
+  static constexpr int kRows = CR * kPitch;                          // bytes of rows in a stage
+  static constexpr int kStage = kRows + CR * 4;                      // rows + a float for each
   static constexpr int kBytes = kN * kStage;
   static constexpr int kSwz = kPitch < 256 ? kPitch : 256;
   static __host__ __device__ constexpr int swz(int row) { return 2 * ((row * kSwz / 256) & (kSwz / 32 - 1)); }
@@ -447,22 +465,22 @@ struct Ring {
     rows_left = nrows - row0;
     row_bytes32 = (uint32_t)row_bytes;
   }
-  // The next kChunk rows into `stage`.
+  // The next CR rows into `stage`.
   template <int AUX = 0>
   __device__ __forceinline__ void issue_next(char* stage) {
-    const int live = rows_in_chunk(rows_left);   // the view covers this chunk's rows only
+    const int live = rows_in_chunk<CR>(rows_left);   // the view covers this chunk's rows only
     const __amdgpu_buffer_rsrc_t view = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(next_ptr), 0, (int)((uint32_t)live * row_bytes32), 0x00020000);
 #pragma unroll
     for (int i = 0; i < kPer; ++i) dma16<AUX>(view, voff[i], stage + (wave * kPer + i) * 1024);
-    next_ptr += (int64_t)kChunk * row_bytes32;
-    rows_left -= kChunk;
+    next_ptr += (int64_t)CR * row_bytes32;
+    rows_left -= CR;
   }
-  // kChunk rows from `ptr` on into `stage`, of which the first `rows` (clamped to [0, kChunk]) exist;
+  // CR rows from `ptr` on into `stage`, of which the first `rows` (clamped to [0, CR]) exist;
   // for sweeps that do not walk one operand front to back.
   template <int AUX = 0>
   __device__ __forceinline__ void issue_at(char* stage, const char* ptr, int rows) {
-    const int live = rows_in_chunk(rows);
+    const int live = rows_in_chunk<CR>(rows);
     const __amdgpu_buffer_rsrc_t view = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(ptr), 0, (int)((uint32_t)live * row_bytes32), 0x00020000);
 #pragma unroll
@@ -1032,6 +1050,497 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 }
 
 // ---------------------------------------------------------------------------------------------
+// Both sweeps in one for a pair whose keys all fit the registers of one workgroup: every wave keeps 16 * NG keys (groups w, w + NW,
+// w + 2 NW, .., which levels the mask), the queries stream through the ring 16 * SQ at a time, and a workgroup that sees a query
+// sees all of its keys, so a score is formed once and its row's sum is a matter of the workgroup.  Per chunk and behind one barrier:
+// the waves' sums of the rows of the chunk before are added up, and what was kept of its scores, times the reciprocal, goes
+// to the columns; the chunk's own scores become 2^score (maxima keep the score itself), each wave's sum per row goes to LDS.
+// Sums are of 2^score itself.  One outside [2^-20, 2^100), which a NaN, an infinity, a row without a visible key and scores far from
+// zero all end in, is not used: the workgroup forms the chunk's scores again, row maximum first (`exact`; every wave reads the same
+// sums and so comes to the same conclusion).  A 2^score below 2^-126 counts as 0, a probability of 2^-106 at most.
+// The accumulators of hidden keys, those past N and those behind the mask, start at -inf.
+// The queries of a pair are dealt chunk by chunk to p.splits workgroups, which leave fp32 columns behind each other for
+// merge_columns_kernel (p.out, p.out2: [splits, BH, N]); one workgroup per pair stores the final form.
+// Bound by the vector port, then by the chain through one barrier per chunk (32 queries against 512 keys of 128: 2560 cycles of
+// port work on two waves per SIMD, 2810 taken; of 64: 1960, 2350), and where a CU gets one workgroup by reading its keys first (6000 of
+// 28000 cycles for 512 keys of 64).  Scores formed and exponentiated once take 30 port cycles per 64 of D = 128 where the two sweeps
+// take 52.  Per call, two kernels -> this one, fp16 sums: 512 pairs of 512 x 512 x 128 79.5 -> 53.5 us, of 256 x 256 34.7 -> 19.4, of
+// 100 x 100 18.5 -> 7.6; 128 pairs of 512 x 512 x 64 18.9 -> 15.0, 2 pairs 14.1 -> 8.3; 8 pairs of 8192 x 512 x 128 86 -> 19.
+// More than 512 keys of 64 were built with eight groups per wave and sixteen queries per chunk, and with 64 queries per chunk: both
+// keep registers in memory in some forms and gave up to 1.3 times on 1024 keys without a mask, nothing or less with one.
+__device__ __forceinline__ void swap_halves(float& a, float& b) {   // upper half of a with the lower half of b
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void swap_rows(float& a, float& b) {     // odd rows of 16 lanes of a with the even rows of b
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+// Sums (maxima) over the four rows of lanes.  One value: in every lane.  Two: the first in the lower half, the second in the upper.
+template <bool MAX>
+__device__ __forceinline__ float lane_rows_reduce(const float (&v)[1]) {
+  float a = v[0], b = v[0];
+  swap_halves(a, b);
+  a = MAX ? fmaxf(a, b) : a + b;
+  b = a;
+  swap_rows(a, b);
+  return MAX ? fmaxf(a, b) : a + b;
+}
+template <bool MAX>
+__device__ __forceinline__ float lane_rows_reduce(const float (&v)[2]) {
+  float a = v[0], b = v[1];
+  swap_halves(a, b);
+  a = MAX ? fmaxf(a, b) : a + b;
+  b = a;
+  swap_rows(a, b);
+  return MAX ? fmaxf(a, b) : a + b;
+}
+
+// Sum (maximum) of each of 16 values over the 16 lanes of a row: lane l of a row ends up with value l, v[l / 4][l % 4].
+template <bool MAX>
+__device__ __forceinline__ float lanes16_scatter(const f32x4 (&v)[4], int lane) {
+  auto join = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+  float x[8], y[4], z[2];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {   // lanes 8.. keep the upper half of the values, of the mirrored lanes as well
+    const float lo = v[j >> 2][j & 3], hi = v[2 + (j >> 2)][j & 3];
+    x[j] = join((lane & 8) ? hi : lo, dpp_row<0x140>((lane & 8) ? lo : hi));
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[j] = join((lane & 4) ? x[j + 4] : x[j], dpp_row<0x141>((lane & 4) ? x[j] : x[j + 4]));
+#pragma unroll
+  for (int j = 0; j < 2; ++j) z[j] = join((lane & 2) ? y[j + 2] : y[j], dpp_row<0x4E>((lane & 2) ? y[j] : y[j + 2]));
+  return join((lane & 1) ? z[1] : z[0], dpp_row<0xB1>((lane & 1) ? z[0] : z[1]));
+}
+
+// 16-row groups of keys per wave where there are more than 256 keys: eight while their fragments leave room for what is added up.
+// 16-row groups of keys per wave where there are more than 128 keys: what leaves room for a chunk's scores beside their fragments.
+constexpr int few_keys_groups(int ks) { return ks > 4 ? 2 : 4; }
+constexpr int few_keys_queries(int ks) { return ks > 4 ? 1 : 2; }   // streamed 16-row groups per chunk
+
+template <int DT, int KS, bool CAUSAL, int MODE, int NG, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
+  constexpr int SQ = few_keys_queries(KS), CR = 16 * SQ;
+  static_assert(!CAUSAL || 16 * NW > CR + 14, "a chunk's diagonal meets one group of a wave");
+  constexpr int kLoads = CR * Ring<KS>::kPitch / 1024;
+  constexpr int LW = kLoads < NW ? kLoads : NW;
+  constexpr int NS = 8;
+  using Rg = Ring<KS, NS, LW, CR>;
+  constexpr int kSums = CR * NW;
+  __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes + 4 * kSums * 4];
+  float* const sums = reinterpret_cast<float*>(smem + Rg::kBytes);   // two sets by parity of the chunk, [query][wave]
+  float* const redo = sums + 2 * kSums;                              // maxima and sums of a chunk that is done again
+  // grid: heads, batch, splits
+  const int split = (int)blockIdx.z, S = p.splits, bh = (int)blockIdx.y * p.H + (int)blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const char* qb = p.q + (int64_t)blockIdx.y * p.q_sb + (int64_t)blockIdx.x * p.q_sh;
+  const char* kb = p.k + (int64_t)blockIdx.y * p.k_sb + (int64_t)blockIdx.x * p.k_sh;
+
+  int k0[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) k0[g] = 16 * (wave + NW * g);
+  // of this workgroup: split, split + S, ..  (uniform, which a division hides from the compiler)
+  const int chunks = S == 1 ? (p.M + CR - 1) / CR : __builtin_amdgcn_readfirstlane(((p.M + CR - 1) / CR - split + S - 1) / S);
+  Rg rg;
+  rg.init(p.q_sr, p.dgran, lane, wave);
+  rg.start(qb, p.q_sr, split * CR, p.M);
+  auto stage_of = [&](int i) { return smem + ((uint32_t)i % NS) * Rg::kStage; };
+  auto first_row = [&](int i) { return (split + i * S) * CR; };
+  const int64_t step = (int64_t)(S - 1) * CR * p.q_sr;
+  auto issue = [&](int i) __attribute__((always_inline)) {   // in order: the cursor walks over the workgroup's chunks
+    if (wave >= LW) return;
+    rg.issue_next(stage_of(i));
+    rg.next_ptr += step;
+    rg.rows_left -= (S - 1) * CR;
+  };
+  // The stage of the chunk before the current one is not refilled yet: it may be done again.
+#pragma unroll
+  for (int i = 0; i < NS - 2; ++i) issue(i);
+  // The keys through one view (the host checks that the workgroup's rows end below 2 GiB; granules past D come from past that).
+  u32x4 kf[NG][KS];
+  {
+    const __amdgpu_buffer_rsrc_t view = rows_view(kb, p.k_sr, 0, p.N);
+    uint32_t off[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int gi = ks * 4 + (lane >> 4);
+      off[ks] = gi < p.dgran ? (uint32_t)(16 * wave + (lane & 15)) * (uint32_t)p.k_sr + (uint32_t)gi * 16u : 0x80000000u;
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[g][ks] = view_load16(view, off[ks] + (uint32_t)(16 * NW * g) * (uint32_t)p.k_sr);
+  }
+
+  const int live_all = max(0, min(NG, (p.N - 16 * wave + 16 * NW - 1) / (16 * NW)));   // groups with keys
+  const float hidden = p.scale2 < 0.f ? kPosInf : kNegInf;   // (times a scale of 0: a NaN, and the chunk is done again)
+  f32x4 csum[NG], cmax[NG];   // the set a MODE does not use is never touched and costs no registers
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    csum[g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    cmax[g] = (f32x4){kNegInf, kNegInf, kNegInf, kNegInf};
+  }
+
+  // groups that some query of a chunk sees; only the last of them can need a mask (they are 16 * NW keys apart)
+  auto live_groups = [&](int q0) __attribute__((always_inline)) {
+    if (!CAUSAL) return live_all;
+    const int last = q0 + CR - 1 + p.c - 16 * wave;
+    return last < 0 ? 0 : min(live_all, last / (16 * NW) + 1);
+  };
+  // first chunk from which on every query sees every key of the wave, and all of its groups are whole
+  int i_full = 1 << 30;
+  if (k0[NG - 1] + 16 <= p.N) {
+    const int row = CAUSAL ? max(0, k0[NG - 1] + 15 - p.c) : 0;   // first row that sees the wave's last key
+    i_full = CAUSAL ? __builtin_amdgcn_readfirstlane(max(0, ((row + CR - 1) / CR - split + S - 1) / S)) : 0;
+  }
+  // a wave's sums (maxima) per row, over its lanes
+  auto write_partials = [&](float* set, const float (&v)[SQ], auto max_tag) __attribute__((always_inline)) {
+    constexpr bool MAX = decltype(max_tag)::value;
+    if constexpr (SQ == 1) {
+      const float x = lane_rows_reduce<MAX>(v);
+      if (lane < 16) set[lane * NW + wave] = x;
+    } else {
+      const float x = lane_rows_reduce<MAX>(v);
+      if ((lane & 16) == 0) set[((lane >> 5) * 16 + (lane & 15)) * NW + wave] = x;
+    }
+  };
+  auto read_partials = [&](const float* set, float (&w)[SQ][NW]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq)
+#pragma unroll
+      for (int i = 0; i < NW; i += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(set + (16 * sq + (lane & 15)) * NW + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[sq][i + e] = x[e];
+      }
+  };
+  auto add_up = [&](const float (&w)[SQ][NW], float (&l)[SQ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {
+      l[sq] = (w[sq][0] + w[sq][1]) + (w[sq][2] + w[sq][3]);
+#pragma unroll
+      for (int v = 4; v < NW; v += 4) l[sq] += (w[sq][v] + w[sq][v + 1]) + (w[sq][v + 2] + w[sq][v + 3]);
+    }
+  };
+
+  u32x4 f[SQ][KS];   // fragments of the chunk that comes next
+  auto read_fragments = [&](int i) __attribute__((always_inline)) {
+    const char* stage = stage_of(i);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq) f[sq][ks] = rg.frag(stage, 0, sq, ks);
+  };
+  // 2^score of a group, into the row sums; s is what adding it up needs of it
+  auto exponents = [&](const f32x4(&t)[SQ], f32x4(&s)[SQ], float (&part)[SQ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = t[sq][r] * p.scale2, e = fast_exp2(x);
+        part[sq] += e;
+        s[sq][r] = MODE == kModeSum ? e : x;
+      }
+  };
+
+  // log2 of a row sum, the exponent apart: rounded once at the size of the result
+  auto row_lse = [](float l) __attribute__((always_inline)) { return (float)__builtin_amdgcn_frexp_expf(l) + fast_log2(__builtin_amdgcn_frexp_mantf(l)); };
+  auto store_lse = [&](int q0, const float (&lse)[SQ]) __attribute__((always_inline)) {
+    float v = lse[0];
+#pragma unroll
+    for (int sq = 1; sq < SQ; ++sq) v = lane >> 4 == sq ? lse[sq] : v;
+    if (lane < CR && q0 + lane < p.M) p.lse[(int64_t)bh * p.M + q0 + lane] = v;
+  };
+  // Chunk i once more, for rows whose sum of 2^score is unusable: row maximum first.
+  auto exact = [&](int i) __attribute__((always_inline)) {
+    const char* stage = stage_of(i);
+    const int q0 = first_row(i), live = live_groups(q0);
+    f32x4 x[NG][SQ];
+    float part[SQ], w[SQ][NW], ref[SQ], lse[SQ], l[SQ];
+    int lane_again = lane;   // opaque: what follows from it is not to be kept in registers from chunk to chunk
+    asm volatile("" : "+v"(lane_again));
+    auto seen = [&](int g, int sq, int r) __attribute__((always_inline)) {
+      const int key = k0[g] + 4 * (lane_again >> 4) + r, q = q0 + 16 * sq + (lane_again & 15);
+      return key < p.N && q < p.M && (!CAUSAL || key <= q + p.c);
+    };
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) part[sq] = kNegInf;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g >= live) continue;
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) acc = mma<DT>(kf[g][ks], rg.frag(stage, 0, sq, ks), acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          x[g][sq][r] = seen(g, sq, r) ? acc[r] * p.scale2 : kNegInf;
+          part[sq] = fmaxf(part[sq], x[g][sq][r]);
+        }
+      }
+    }
+    write_partials(redo, part, std::true_type());
+    lds_barrier();
+    read_partials(redo, w);
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {
+      float m = w[sq][0];
+#pragma unroll
+      for (int v = 1; v < NW; ++v) m = fmaxf(m, w[sq][v]);
+      ref[sq] = m == kNegInf ? 0.f : m;   // no visible key: any finite reference
+      part[sq] = 0.f;
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g >= live) continue;
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)   // (+inf - inf is a NaN, as the row kernel's lse then is)
+          part[sq] += seen(g, sq, r) ? fast_exp2(x[g][sq][r] - ref[sq]) : 0.f;
+    }
+    write_partials(redo + kSums, part, std::false_type());
+    lds_barrier();
+    read_partials(redo + kSums, w);
+    add_up(w, l);
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) lse[sq] = l[sq] == 0.f ? kNegInf : ref[sq] + fast_log2(l[sq]);
+    if (wave == 0) store_lse(q0, lse);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g >= live) continue;
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float y = seen(g, sq, r) ? x[g][sq][r] - lse[sq] : kNegInf;
+          if (MODE != kModeMax) csum[g][r] += fast_exp2(y);
+          if (MODE != kModeSum) cmax[g][r] = fmaxf(cmax[g][r], y);
+        }
+    }
+  };
+
+  constexpr float kNothing = MODE == kModeSum ? 0.f : kNegInf;
+  f32x4 s[NG][SQ];   // of the chunk whose columns are added up next: 2^score, or (maxima) the scaled score
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) s[g][sq] = (f32x4){kNothing, kNothing, kNothing, kNothing};
+  // per row of that chunk: the reciprocal of its sum, or its lse; such that rows past M, and a chunk before the first, add nothing
+  float fact[SQ];
+#pragma unroll
+  for (int sq = 0; sq < SQ; ++sq) fact[sq] = MODE == kModeSum ? 0.f : kPosInf;
+  auto add_group = [&](int g) __attribute__((always_inline)) {
+    if constexpr (MODE == kModeSum) {
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) csum[g][r] = fmaf(s[g][sq][r], fact[sq], csum[g][r]);
+    } else {
+      float one[SQ];
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq) one[sq] = 1.f;
+      col_update<false, MODE>(s[g], one, fact, csum[g], cmax[g], 0);
+    }
+  };
+  constexpr int GP = SQ == 1 ? 2 : 1, NBT = NG / GP;   // groups side by side: two independent chains of matrix instructions
+  f32x4 t[2][GP][SQ];
+  auto scores = [&](int bt, auto init) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < GP; ++e) init(k0[bt * GP + e], t[bt & 1][e]);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int e = 0; e < GP; ++e)
+#pragma unroll
+        for (int sq = 0; sq < SQ; ++sq) t[bt & 1][e][sq] = mma<DT>(kf[bt * GP + e][ks], f[sq][ks], t[bt & 1][e][sq]);
+  };
+  auto visible = [](int, f32x4(&c)[SQ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) c[sq] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  };
+  auto enter = [&](int i) __attribute__((always_inline)) {
+    ring_sync<(NS - 4) * Rg::kPer>();   // chunk i + 1 is there, the sums of chunk i - 1 are
+    issue(i + NS - 2);
+    if (i == 0) read_fragments(0);
+  };
+  // What the rows of chunk i contribute with, into `fact`; whether a row's sum is unusable (the same in every wave).
+  auto row_facts = [&](int i, float (&l)[SQ]) __attribute__((always_inline)) {
+    const int q0 = first_row(i);
+    float w[SQ][NW];
+    read_partials(sums + (i & 1) * kSums, w);
+    add_up(w, l);
+    bool good = true;
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {
+      good = good && l[sq] >= 9.5367432e-7f && l[sq] < 1.2676506e30f;
+      const bool row = q0 + 16 * sq + (lane & 15) < p.M;
+      if (MODE == kModeSum) fact[sq] = row ? __builtin_amdgcn_rcpf(l[sq]) : 0.f;
+      else fact[sq] = row ? row_lse(l[sq]) : kPosInf;
+    }
+    return __builtin_amdgcn_ballot_w64(!good) != 0;
+  };
+  auto lse_of = [&](int i, const float (&l)[SQ]) __attribute__((always_inline)) {
+    if (wave != 0) return;
+    float lse[SQ];
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) lse[sq] = row_lse(l[sq]);
+    store_lse(first_row(i), lse);
+  };
+  int batches = 0;   // of GP groups, in use in the chunk whose columns are added up next
+  auto add_batches = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int bt = 0; bt < NBT; ++bt)
+      if (bt < batches) {
+#pragma unroll
+        for (int e = 0; e < GP; ++e) add_group(bt * GP + e);
+      }
+  };
+
+  int i = 0;
+  // chunks that some key of the wave is hidden from, and the one behind them (whose predecessor's groups are not all in use)
+#pragma unroll 1
+  for (; i < chunks && i_full > 0 && i <= i_full; ++i) {
+    enter(i);
+    const int q0 = first_row(i), live = live_groups(q0), in_use = (live + GP - 1) / GP;
+    int lane_again = lane;
+    asm volatile("" : "+v"(lane_again));
+    // the last batch holds what is hidden: the diagonal, keys past N, a group that nobody sees
+    auto masked = [&](int key0, f32x4(&c)[SQ]) __attribute__((always_inline)) {
+      const int key = key0 + 4 * (lane_again >> 4);
+      int lim = p.N - 1 - key;
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq) {
+        if (CAUSAL) lim = min(p.N - 1 - key, q0 + 16 * sq + (lane_again & 15) + p.c - key);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[sq][r] = r <= lim ? 0.f : hidden;
+      }
+    };
+    auto batch = [&](int bt) __attribute__((always_inline)) {
+      if (bt + 1 < in_use) scores(bt, visible);
+      else if (bt < in_use) scores(bt, masked);
+    };
+    batch(0);
+    if (NBT > 1) batch(1);
+    if (i > 0) {
+      float l[SQ];
+      if (row_facts(i - 1, l)) {
+        exact(i - 1);
+      } else {
+        add_batches();
+        lse_of(i - 1, l);
+      }
+    }
+    float part[SQ];
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) part[sq] = 0.f;
+#pragma unroll
+    for (int bt = 0; bt < NBT; ++bt) {
+      if (bt < in_use) {
+#pragma unroll
+        for (int e = 0; e < GP; ++e) exponents(t[bt & 1][e], s[bt * GP + e], part);
+      } else {
+#pragma unroll
+        for (int e = 0; e < GP; ++e)
+#pragma unroll
+          for (int sq = 0; sq < SQ; ++sq) s[bt * GP + e][sq] = (f32x4){kNothing, kNothing, kNothing, kNothing};
+      }
+      if (bt + 2 < NBT) batch(bt + 2);
+    }
+    read_fragments(i + 1);
+    write_partials(sums + (i & 1) * kSums, part, std::false_type());
+    batches = in_use;
+  }
+  // The others, without branches but for rows whose sums are unusable: the columns of chunk i - 1 are added up, and the exponents of
+  // each group of chunk i taken, under the matrix instructions of the groups behind it.
+#pragma unroll 1
+  for (; i < chunks; ++i) {
+    enter(i);
+    scores(0, visible);
+    if (NBT > 1) scores(1, visible);
+    float l[SQ];
+    bool bad = i == 0;
+    if (i > 0) {
+      bad = row_facts(i - 1, l);
+      if (bad) exact(i - 1);
+    }
+    if (!bad) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) add_group(g);
+      lse_of(i - 1, l);
+    }
+    float part[SQ];
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) part[sq] = 0.f;
+#pragma unroll
+    for (int bt = 0; bt < NBT; ++bt) {
+#pragma unroll
+      for (int e = 0; e < GP; ++e) exponents(t[bt & 1][e], s[bt * GP + e], part);
+      if (bt + 2 < NBT) scores(bt + 2, visible);
+      if (bt + 3 == NBT || (NBT < 3 && bt == 0)) read_fragments(i + 1);
+    }
+    write_partials(sums + (i & 1) * kSums, part, std::false_type());
+  }
+  ring_sync<0>();   // (and the loads past the last chunk have written their zeros)
+  float l[SQ];
+  if (row_facts(chunks - 1, l)) {
+    exact(chunks - 1);
+  } else {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) add_group(g);
+    lse_of(chunks - 1, l);
+  }
+
+  // Columns: a reduce-scatter over the 16 query lanes, 16 values (four groups) at a time; lane l ends up with group (l & 15) / 4,
+  // key 4 * (l / 16) + (l & 3) of it.
+  Params mine = p;
+  if (S > 1) {
+    const int64_t at = (int64_t)split * p.bh_count * p.N * 4;
+    mine.out = static_cast<char*>(p.out) + at;
+    mine.out2 = static_cast<char*>(p.out2) + at;
+  }
+  const int r = lane & 3;
+#pragma unroll
+  for (int g4 = 0; g4 < NG; g4 += 4) {
+    const int grp = g4 + ((lane & 15) >> 2);
+    const int key = 16 * (wave + NW * grp) + 4 * (lane >> 4) + r;
+    f32x4 c4[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) c4[g] = g4 + g < NG ? csum[(g4 + g) % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
+    const float sum = MODE != kModeMax ? lanes16_scatter<false>(c4, lane) : 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) c4[g] = g4 + g < NG ? cmax[(g4 + g) % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
+    const float most = MODE != kModeSum ? lanes16_scatter<true>(c4, lane) : 0.f;
+    if (grp < NG && key < p.N) {
+      if (MODE != kModeMax) store_column(mine, mine.out, true, bh, key, sum);
+      if (MODE != kModeSum) store_column(mine, MODE == kModeBoth ? mine.out2 : mine.out, false, bh, key, fast_exp2(most));
+    }
+  }
+}
+
+// out = the sums or maxima of p.splits columns that lie BH * N apart at p.part (both: maxima p.splits * BH * N behind the sums).
+template <int MODE>
+__global__ __launch_bounds__(256) void merge_columns_kernel(const Params p) {
+  const int64_t n = (int64_t)p.bh_count * p.N, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (at >= n) return;
+  const int bh = (int)(at / p.N), key = (int)(at - (int64_t)bh * p.N);
+  const float* src = p.part + at;
+  if (MODE != kModeMax) {
+    float v = 0.f;
+#pragma unroll 8
+    for (int s = 0; s < p.splits; ++s) v += src[s * n];
+    store_column(p, p.out, true, bh, key, v);
+  }
+  if (MODE != kModeSum) {
+    if (MODE == kModeBoth) src += p.splits * n;
+    float v = 0.f;   // (maxima of probabilities)
+#pragma unroll 8
+    for (int s = 0; s < p.splits; ++s) v = fmaxf(v, src[s * n]);
+    store_column(p, MODE == kModeBoth ? p.out2 : p.out, false, bh, key, v);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // fp32 operands.  Each row is scaled by a power of two that puts its largest element at 2^14..2^15 and every element x is split
 // into two fp16 numbers, h = fp16(x) and l = fp16(x - h): x to 2^-23 (one element in four loses its last bit), and elements smaller
 // than 2^-16 of the row's largest to 2^-39 of that one (see SplitRing::set_limit).  A product is h h' + h l' + l h', each
@@ -1058,11 +1567,6 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 // short ones the latency of a chunk.  32 heads of 1024 x 1024 x 128: 137 -> 64 us per call, 4096 x 4096 x 128 2250 -> 730.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_row(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
 
 struct Planes {   // h and l of eight values of a row
   u32x4 p[2];
@@ -1851,14 +2355,6 @@ __device__ __forceinline__ float row16_reduce(float v) {
   o = dpp_row<0x140>(v);         // row_mirror
   v = MAX ? fmaxf(v, o) : v + o;
   return v;
-}
-
-// All LDS accesses of this wave done, then the workgroup's barrier.  Loads and stores to memory stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (7 << 4) | (0 << 8));   // vmcnt(63) expcnt(7) lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ w, int n) {
@@ -3718,6 +4214,49 @@ OneQueryPlan one_query_plan(int dtype, int64_t bh, int N, int D, int64_t base_fl
   return o;
 }
 
+// The path for pairs whose keys fit the registers of a workgroup (few_keys_kernel): up to 512 16-bit keys of 128, 256 of 256.  It won
+// 190 of 200 shapes of 2 to 512 pairs, 2 to 8192 queries and 64 to 512 keys against the two kernels, by 1.05 to 2.4 times (6.8 where
+// few keys meet thousands of queries).  Not taken, with the mask and more than 256 keys (eight waves, one workgroup per CU, whose half of
+// the triangle is paid for with whole chunks): where two or three workgroups share a pair (128 pairs of 512 x 512 x 128 19.5 us, 23.0
+// here) and in several rounds of short rows (512 pairs of 300 x 300 x 64 26.8, 28.3); nor there, mask or not, for sums and maxima
+// together unless at least four share a pair (128 pairs of 512 x 512 x 128 23.9, 27.7; 512 of 300 x 300 x 64 36.5, 37.7).
+// form -1: the other paths.
+struct FewKeysPlan {
+  int form;          // keys of a workgroup: 128 << form
+  int splits;        // workgroups per pair
+  int64_t part_at, floats;   // where the columns of the splits start and the workspace ends, in floats
+};
+FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool both, bool causal, int64_t base_floats) {
+  FewKeysPlan o;
+  o.form = -1;
+  o.splits = 1;
+  o.part_at = o.floats = base_floats;
+  const int ks = ksteps_of(dtype, D);
+  const int64_t bh = (int64_t)B * H;
+  if (dtype == FCR_DTYPE_F32 || ks > kMaxKSteps || M < 2 || B > 65535 || bh >= kMaxWorkgroups / 2) return o;   // (the grid's limits)
+  const int groups = few_keys_groups(ks), most = groups == 4 ? 2 : 1;
+  int form = 0;
+  while (form <= most && N > (128 << form)) ++form;
+  if (form > most) return o;
+  o.form = form;
+  const int waves = form == most ? 8 : 4;
+  const int rows = 16 * few_keys_queries(ks);
+  const int64_t chunks = ((int64_t)M + rows - 1) / rows;
+  int64_t s = (waves == 8 ? 1 : 2) * (int64_t)chip_cus() / bh;
+  if (s > chunks) s = chunks;
+  if (s < 1) s = 1;
+  if (N > 256 && s < 4 && (both || (causal && (s > 1 || (ks <= 2 && bh > chip_cus()))))) {
+    o.form = -1;
+    return o;
+  }
+  o.splits = (int)s;
+  if (s > 1) {
+    o.part_at = (base_floats + 63) / 64 * 64;
+    o.floats = o.part_at + (both ? 2 : 1) * s * bh * N;
+  }
+  return o;
+}
+
 int launched(const char* what) {
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) return 0;
@@ -3904,6 +4443,31 @@ void launch_col(const Params& p, bool causal, int mode, hipStream_t s) {
   else launch_col_mode<DT, KS, kModeBoth>(p, causal, s);
 }
 
+template <int DT, int KS, int MODE, int NG, int NW>
+void launch_few_keys_form(const Params& p, bool causal, hipStream_t s) {
+  const dim3 grid((unsigned)p.H, (unsigned)(p.bh_count / p.H), (unsigned)p.splits), block(64 * NW);
+  if (causal) hipLaunchKernelGGL((few_keys_kernel<DT, KS, true, MODE, NG, NW>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((few_keys_kernel<DT, KS, false, MODE, NG, NW>), grid, block, 0, s, p);
+}
+
+template <int DT, int KS, int MODE>
+void launch_few_keys_mode(const Params& p, bool causal, int form, hipStream_t s) {
+  if (form == 0) return launch_few_keys_form<DT, KS, MODE, 2, 4>(p, causal, s);
+  if constexpr (few_keys_groups(KS) == 2) {
+    launch_few_keys_form<DT, KS, MODE, 2, 8>(p, causal, s);
+  } else {
+    if (form == 1) launch_few_keys_form<DT, KS, MODE, 4, 4>(p, causal, s);
+    else launch_few_keys_form<DT, KS, MODE, 4, 8>(p, causal, s);
+  }
+}
+
+template <int DT, int KS>
+void launch_few_keys(const Params& p, bool causal, int mode, int form, hipStream_t s) {
+  if (mode == kModeSum) launch_few_keys_mode<DT, KS, kModeSum>(p, causal, form, s);
+  else if (mode == kModeMax) launch_few_keys_mode<DT, KS, kModeMax>(p, causal, form, s);
+  else launch_few_keys_mode<DT, KS, kModeBoth>(p, causal, form, s);
+}
+
 #define FCR_DISPATCH_KS(DT, ksteps, CALL)                  \
   switch (ksteps) {                                        \
     case 1: CALL(DT, 1); break;                            \
@@ -3944,6 +4508,7 @@ void launch_col(const Params& p, bool causal, int mode, hipStream_t s) {
 #define FCR_CALL_COL(DT, KS) launch_col<DT, KS>(p, causal, mode, s)
 #define FCR_CALL_COL_SMALL(DT, KS) launch_col_small<DT, KS>(p, causal, mode, s)
 #define FCR_CALL_COL_FUSED(DT, KS) launch_col_fused<DT, KS>(p, causal, mode, s)
+#define FCR_CALL_FEW_KEYS(DT, KS) launch_few_keys<DT, KS>(p, causal, mode, form, s)
 #define FCR_SWEEPS_16BIT(NAME, DT)                                                                       \
   void fcr_detail::NAME(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s) { \
     if (which == 0) { FCR_DISPATCH_KS(DT, ksteps, FCR_CALL_LSE) }                                        \
@@ -3964,6 +4529,16 @@ void fcr_detail::sweeps_f16_single(const Params& p, int ksteps, bool causal, int
 #if FCR_HAS(8)
 void fcr_detail::sweeps_bf16_single(const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
   FCR_DISPATCH_KS4(FCR_DTYPE_BF16, ksteps, FCR_CALL_COL_FUSED)
+}
+#endif
+#if FCR_HAS(9)
+void fcr_detail::sweeps_f16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s) {
+  FCR_DISPATCH_KS(FCR_DTYPE_F16, ksteps, FCR_CALL_FEW_KEYS)
+}
+#endif
+#if FCR_HAS(10)
+void fcr_detail::sweeps_bf16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s) {
+  FCR_DISPATCH_KS(FCR_DTYPE_BF16, ksteps, FCR_CALL_FEW_KEYS)
 }
 #endif
 #if FCR_HAS(3)
@@ -4008,6 +4583,7 @@ void fcr_detail::sweeps_bf16_long_rows(int which, const Params& p, int ksteps, b
 #undef FCR_CALL_COL
 #undef FCR_CALL_COL_SMALL
 #undef FCR_CALL_COL_FUSED
+#undef FCR_CALL_FEW_KEYS
 
 #if FCR_HAS(0)
 namespace {
@@ -4073,6 +4649,28 @@ int launch_one_query(Params& p, int dtype, const OneQueryPlan& o, float* ws, int
   else if (mode == kModeMax) hipLaunchKernelGGL(one_query_columns_kernel<kModeMax>, grid, block, 0, s, p, scores, o.pitch);
   else hipLaunchKernelGGL(one_query_columns_kernel<kModeBoth>, grid, block, 0, s, p, scores, o.pitch);
   return launched("one_query_columns_kernel");
+}
+
+int launch_few_keys(Params& p, int dtype, int ksteps, const FewKeysPlan& o, float* ws, int mode, bool causal, hipStream_t s) {
+  p.lse = ws;
+  Params sweep = p;
+  sweep.splits = o.splits;
+  if (o.splits > 1) {
+    sweep.out = ws + o.part_at;
+    sweep.out2 = ws + o.part_at + (mode == kModeBoth ? (int64_t)o.splits * p.bh_count * p.N : 0);
+    sweep.out_fmt = FCR_DTYPE_F32;
+    sweep.mean_from = -1;
+  }
+  (dtype == FCR_DTYPE_F16 ? fcr_detail::sweeps_f16_few_keys : fcr_detail::sweeps_bf16_few_keys)(sweep, ksteps, causal, mode, o.form, s);
+  const int rc = launched("few_keys_kernel");
+  if (rc || o.splits == 1) return rc;
+  p.part = ws + o.part_at;
+  p.splits = o.splits;
+  const dim3 grid((unsigned)((p.bh_count * (int64_t)p.N + 255) / 256)), block(256);
+  if (mode == kModeSum) hipLaunchKernelGGL(merge_columns_kernel<kModeSum>, grid, block, 0, s, p);
+  else if (mode == kModeMax) hipLaunchKernelGGL(merge_columns_kernel<kModeMax>, grid, block, 0, s, p);
+  else hipLaunchKernelGGL(merge_columns_kernel<kModeBoth>, grid, block, 0, s, p);
+  return launched("merge_columns_kernel");
 }
 
 template <int VPT, typename ET>
@@ -4395,6 +4993,12 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
       return launch_one_query(p, dtype, o, ws, mode, static_cast<hipStream_t>(stream));
     }
   }
+  if (single && ws_bytes != 0) {
+    const FewKeysPlan o = few_keys_plan(dtype, B, H, M, N, D, mode == kModeBoth, causal != 0, (int64_t)(lse_bytes / sizeof(float)));
+    // (the keys of a pair are read through one view: all rows of a workgroup below 2 GiB)
+    if (o.form >= 0 && (size_t)o.floats * sizeof(float) <= ws_bytes && ((int64_t)128 << o.form) * p.k_sr <= 0x7fffffff)
+      return launch_few_keys(p, dtype, ksteps, o, ws, mode, causal != 0, static_cast<hipStream_t>(stream));
+  }
   if (single && fused) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     p.lse = ws;
@@ -4504,6 +5108,11 @@ size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D) {
   if (base == 0 || (dtype != FCR_DTYPE_F16 && dtype != FCR_DTYPE_BF16 && dtype != FCR_DTYPE_F32)) return base;
   if (M == 1 && row_width_ok(dtype, D))   // (a row the call rejects has no plan: no power of two of 64 lanes or less)
     return (size_t)one_query_plan(dtype, (int64_t)B * H, N, D, (int64_t)(base / sizeof(float))).floats * sizeof(float);
+  if (row_width_ok(dtype, D)) {
+    const int64_t floats = (int64_t)(base / sizeof(float));
+    const FewKeysPlan one = few_keys_plan(dtype, B, H, M, N, D, false, false, floats), both = few_keys_plan(dtype, B, H, M, N, D, true, false, floats);
+    return (size_t)(one.floats > both.floats ? one.floats : both.floats) * sizeof(float);
+  }
   return base;
 }
 

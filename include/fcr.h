@@ -72,7 +72,7 @@ extern "C" {
 #define FCR_E_WAIT -8      /* fcr_colreduce_status: a workgroup of the single sweep gave up waiting for its team */
 
 /* fcr_set_option */
-#define FCR_OPT_SINGLE_SWEEP 0 /* 0: few queries against many keys, or one query, take the two kernels as well (default 1) */
+#define FCR_OPT_SINGLE_SWEEP 0 /* 0: few queries against many keys, one query and few keys take the two kernels as well (default 1) */
 #define FCR_OPT_WAIT_POLLS 1   /* polls of a team's slots after which a workgroup gives up (default 2^20) */
 
 /* size of the built-in scratch buffer of fcr_colreduce_static, per GPU */
@@ -202,7 +202,9 @@ int fcr_colreduce_to(const void* q, const void* k, void* out, int out_dtype, flo
  * fcr_colreduce_sum_max_to (out_max given; reduction then names what `out` holds, sum or mean) compute, and with
  * fcr_workspace_bytes(dtype, B, H, M, N, D) bytes by the fastest path for the problem: one query is read
  * once, without the matrix instructions, and its scores wait in the workspace (4 bytes per key) for their row's
- * sum (64 sequences of 32 heads and 65536 keys: 0.5 GB).  With less, but at least fcr_lse_bytes, the call takes the
+ * sum (64 sequences of 32 heads and 65536 keys: 0.5 GB); 16-bit keys that fit the registers of a workgroup (at most
+ * 512, or 256 in rows of more than 256 bytes) form each score once, and where several workgroups share a pair their columns
+ * wait in the workspace for a second launch.  With less, but at least fcr_lse_bytes, the call takes the
  * path of the entry points above (FCR_E_SCRATCH below that); results agree to rounding either way.  ws must be 16-byte aligned, its first
  * B*H*M floats hold the row statistics on return, its contents before the call are irrelevant.
  */

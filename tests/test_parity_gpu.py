@@ -1547,6 +1547,123 @@ def test_random_decode_shapes_and_fp32_against_oracle():
             check(got, colreduce_ref(q, k, red, causal, scale=scale), red, what)
 
 
+def _columns_f64(q, k, causal, scale=None):
+    """Column sums and maxima in 64 bits on the device (q, k: (B,H,.,D) on the GPU)."""
+    q, k = q.double(), k.double()
+    m, n = q.shape[2], k.shape[2]
+    s = torch.matmul(q, k.transpose(-1, -2).contiguous()) * (q.shape[3] ** -0.5 if scale is None else scale)
+    if causal:
+        hidden = torch.arange(n, device=q.device)[None] > torch.arange(m, device=q.device)[:, None] + max(n - m, 0)
+        s = s.masked_fill(hidden, float("-inf"))
+    p = s.softmax(-1)
+    return p.sum(2), p.amax(2)
+
+
+def _rel(got, want):
+    return ((got.double() - want).norm() / want.norm()).item()
+
+
+# keys around what a wave's groups and the forms hold (16, 128, 256, 512), one more than the most; queries around a chunk (16, 32)
+# and a split; pairs that share workgroups (few) and that do not
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d,dtype", [
+    (1, 2, 1, 8, torch.float16), (3, 31, 15, 64, torch.bfloat16), (2, 33, 129, 128, torch.float16), (130, 64, 128, 72, torch.bfloat16),
+    (300, 17, 127, 128, torch.float16), (5, 300, 256, 128, torch.float16), (260, 70, 250, 96, torch.bfloat16), (2, 257, 257, 64, torch.float16),
+    (20, 512, 512, 128, torch.bfloat16), (140, 100, 511, 128, torch.float16), (70, 320, 300, 40, torch.float16), (300, 40, 512, 32, torch.float16),
+    (2, 5000, 200, 128, torch.float16), (3, 100, 256, 256, torch.bfloat16), (260, 33, 130, 192, torch.float16), (4, 65, 257, 256, torch.float16),
+    (4, 90, 513, 128, torch.float16), (64, 1, 200, 128, torch.float16), (300, 15, 16, 136, torch.bfloat16)])
+def test_few_keys(h, m, n, d, dtype, causal):
+    """Pairs whose keys fit a workgroup's registers: sums, maxima, both at once and the row statistics, against 64 bits.  A score of
+    magnitude 2^4 is rounded to 2^-20, so a probability is good to 2^-19 and a few 1e-6 in the norm; 1e-5 leaves room for
+    the order of the sums."""
+    g = torch.Generator(device="cuda").manual_seed(h + m + n)
+    q, k = (torch.randn(2, h, r, d, device="cuda", generator=g).to(dtype) for r in (m, n))
+    sums, most = _columns_f64(q, k, causal)
+    got = fca.flash_colreduce(q, k, "sum", causal, out_dtype=torch.float32)
+    assert torch.isfinite(got).all() and _rel(got, sums) <= 1e-5
+    mx = fca.flash_colreduce(q, k, "max", causal, out_dtype=torch.float32)
+    assert _rel(mx, most) <= 1e-5
+    s2, m2 = fca.flash_colreduce_multi(q, k, ["sum", "max"], causal, out_dtype=torch.float32)
+    assert _rel(s2, sums) <= 1e-5 and _rel(m2, most) <= 1e-5
+    ws = torch.empty(_lib_workspace(q, k), device="cuda")
+    out = torch.empty(2 * h, n, device="cuda")
+    _ws_call(q, k, out, ws, causal)
+    torch.testing.assert_close(ws[: 2 * h * m].view(2, h, m), fca.row_lse2(q, k, causal), rtol=1e-5, atol=1e-5)
+    assert torch.equal(out.view(2, h, n), got)
+
+
+def _lib_workspace(q, k):
+    from flash_colreduce_amd import _lib
+    b, h, m, d = q.shape
+    return _lib.load().fcr_workspace_bytes({torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}[q.dtype], b, h, m, k.shape[2], d) // 4
+
+
+def _ws_call(q, k, out, ws, causal, scale=None):
+    from flash_colreduce_amd import _lib
+    b, h, m, d = q.shape
+    code = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}[q.dtype]
+    _lib.check(_lib.load().fcr_colreduce_ws(
+        q.data_ptr(), k.data_ptr(), out.data_ptr(), None, _lib.DTYPE_F32, ws.data_ptr(), 4 * ws.numel(), code, b, h, m, k.shape[2], d,
+        _lib.strides4(q.stride()), _lib.strides4(k.stride()), d ** -0.5 if scale is None else scale, _lib.REDUCE_SUM, int(causal),
+        torch.cuda.current_stream().cuda_stream))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(2, 100, 100, 64), (3, 70, 300, 128), (300, 40, 200, 128), (2, 65, 250, 256)])
+def test_few_keys_scores_that_the_plain_sums_do_not_take(h, m, n, d, causal):
+    """Against the two kernels where 2^score leaves the range of a sum, scales of any sign, layouts, rows and keys that are not finite:
+    the same columns are NaN, the others agree to what scores of magnitude 2^9 (2^-15 each) leave."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(h + n)
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda", generator=g)
+
+    q, k = rand(1, h, m, d), rand(1, h, n, d)
+    far_q, far_k, jump = q.clone(), k.clone(), k.clone()
+    far_q[:, :, m // 2:] *= 40
+    far_k[:, :, ::3] -= 6 * q[:, :, :1]
+    jump[:, :, n // 2] *= 60
+    bad_q, bad_k, low_k = q.clone(), k.clone(), k.clone()
+    bad_q[:, 0, m // 3, 0] = float("nan")
+    bad_q[:, -1, m - 1, 1] = float("inf")
+    bad_k[:, 0, n // 2, 0] = float("inf")
+    low_k[:, :, 1:, :] = 0
+    low_k[:, :, 0, 0] = float("-inf")
+    cases = [(q, k, None), (far_q, k, None), (q, far_k, None), (q, jump, None), (bad_q, k, None), (q, bad_k, None), (q.abs(), low_k, None),
+             (q, k, 0.0), (q, k, -0.3), (q.transpose(2, 1).contiguous().transpose(2, 1), k[:, :1].expand(1, h, n, d), None),
+             (q, torch.nn.functional.pad(k, (0, 8))[..., :d], None)]
+    for at, (x, y, scale) in enumerate(cases):
+        x, y = x.half(), y.half() if at != 9 else k[:, :1].half().expand(1, h, n, d)
+        for red in ("sum", "max"):
+            got = {}
+            for option in (1, 0):
+                lib.fcr_set_option(0, option)
+                try:
+                    got[option] = fca.flash_colreduce(x, y, red, causal, scale, out_dtype=torch.float32)
+                finally:
+                    lib.fcr_set_option(0, 1)
+            assert torch.equal(got[1].isnan(), got[0].isnan()), (at, red)
+            torch.testing.assert_close(got[1], got[0], rtol=2e-4, atol=1e-6, equal_nan=True, msg=lambda t: f"case {at} {red}: {t}")
+
+
+def test_few_keys_under_graph_capture():
+    """Shared pairs (two launches) in a captured graph, replayed with other contents and eager calls between."""
+    q, k = (torch.randn(1, 4, r, 64, device="cuda").half() for r in (300, 200))
+    fca.flash_colreduce(q, k, "mean", True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fca.flash_colreduce(q, k, "mean", True)
+    for _ in range(4):
+        q.copy_(torch.randn(q.shape, device="cuda"))
+        k.copy_(torch.randn(k.shape, device="cuda"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, fca.flash_colreduce(q, k, "mean", True))
+
+
 def test_hip_graph_capture_and_replay():
     """The whole call (torch allocations, both kernels, cast) captured in a graph and replayed with
     new contents in the static inputs; every replay must equal the eager result for those contents."""
