@@ -1112,6 +1112,26 @@ __device__ __forceinline__ float lanes16_scatter(const f32x4 (&v)[4], int lane) 
 }
 
 // 16-row groups of keys per wave where there are more than 256 keys: eight while their fragments leave room for what is added up.
+// Sum (maximum) of each of 8 values over the four rows of lanes: row rho of lanes ends up with values 2 rho and 2 rho + 1 in v[0], v[1].
+template <bool MAX>
+__device__ __forceinline__ void lane_rows_scatter(float (&v)[8]) {
+  float y[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = v[j], b = v[j + 4];
+    swap_halves(a, b);
+    y[j] = MAX ? fmaxf(a, b) : a + b;
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    float a = y[j], b = y[j + 2];
+    swap_rows(a, b);
+    v[j] = MAX ? fmaxf(a, b) : a + b;
+  }
+}
+// log2 of a row sum, the exponent apart: rounded once at the size of the result.
+__device__ __forceinline__ float log2_of_sum(float l) { return (float)__builtin_amdgcn_frexp_expf(l) + fast_log2(__builtin_amdgcn_frexp_mantf(l)); }
+
 // 16-row groups of keys per wave where there are more than 128 keys: what leaves room for a chunk's scores beside their fragments.
 constexpr int few_keys_groups(int ks) { return ks > 4 ? 2 : 4; }
 constexpr int few_keys_queries(int ks) { return ks > 4 ? 1 : 2; }   // streamed 16-row groups per chunk
@@ -1242,8 +1262,6 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
       }
   };
 
-  // log2 of a row sum, the exponent apart: rounded once at the size of the result
-  auto row_lse = [](float l) __attribute__((always_inline)) { return (float)__builtin_amdgcn_frexp_expf(l) + fast_log2(__builtin_amdgcn_frexp_mantf(l)); };
   auto store_lse = [&](int q0, const float (&lse)[SQ]) __attribute__((always_inline)) {
     float v = lse[0];
 #pragma unroll
@@ -1376,7 +1394,7 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
       good = good && l[sq] >= 9.5367432e-7f && l[sq] < 1.2676506e30f;
       const bool row = q0 + 16 * sq + (lane & 15) < p.M;
       if (MODE == kModeSum) fact[sq] = row ? __builtin_amdgcn_rcpf(l[sq]) : 0.f;
-      else fact[sq] = row ? row_lse(l[sq]) : kPosInf;
+      else fact[sq] = row ? log2_of_sum(l[sq]) : kPosInf;
     }
     return __builtin_amdgcn_ballot_w64(!good) != 0;
   };
@@ -1384,7 +1402,7 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     if (wave != 0) return;
     float lse[SQ];
 #pragma unroll
-    for (int sq = 0; sq < SQ; ++sq) lse[sq] = row_lse(l[sq]);
+    for (int sq = 0; sq < SQ; ++sq) lse[sq] = log2_of_sum(l[sq]);
     store_lse(first_row(i), lse);
   };
   int batches = 0;   // of GP groups, in use in the chunk whose columns are added up next
@@ -2313,16 +2331,15 @@ __global__ __launch_bounds__(kThreads, (NG <= 4 ? 3 : 2)) void col_small_kernel(
 // Per pair a workgroup
 //   1. streams its keys through the LDS ring and computes their scores, which STAY IN REGISTERS (16 per
 //      lane and step): for column sums as 2^score, otherwise (maxima) as the scaled scores themselves;
-//   2. sums 2^score per row, turns the sums into the log-sum-exp of every row over its own keys and
-//      publishes the 64 or 128 values.  A sum outside [2^-60, 2^100) (scores far from zero, a row that
-//      sees none of these keys, a NaN) is not trusted: the scores are then reduced the exact way, row
-//      maximum first -- from the registers if they hold scores, else after a second sweep over the same
-//      keys that keeps the scores;
-//   3. reads the values the other workgroups of its team have published for this pair and merges them
-//      into the rows' lse (every workgroup of the team does this merge for itself);
-//   4. turns what it kept into probabilities (2^score * 2^-lse: one multiply-add per score), reduces them
-//      down the rows and stores its columns.
-// The grid is teams * splits workgroups and never more than one per CU, so every workgroup of a team is
+//   2. sums 2^score per row over its own keys and publishes the 32, 64 or 128 sums.  A sum outside [2^-60, 2^100)
+//      (scores far from zero, a row that sees none of these keys, a NaN) is not trusted: the scores are then
+//      reduced the exact way, row maximum first -- from the registers if they hold scores, else after a second sweep
+//      over the same keys that keeps the scores -- and the log2 of the sum is published;
+//   3. reads what the other workgroups of its team have published for this pair and adds it up (every workgroup of the
+//      team does this for itself; a log2 among the values turns the addition into a merge);
+//   4. turns what it kept into probabilities (2^score times the reciprocal of the sum: one multiply-add per score),
+//      reduces them down the rows and leaves its columns in LDS, from where they go to memory under the next sweep.
+// The grid is teams * splits workgroups and never more than the CUs hold at once (one of eight waves, two of four), so every workgroup of a team is
 // running when its partners wait for it; team t takes pairs t, t + teams, t + 2 teams, ..  The first keys
 // of the next pair stream into the ring while a workgroup does steps 2-4, and the next pair's queries are
 // staged in LDS a whole sweep ahead.  A wait is bounded: after p.spin_limit polls the workgroup gives up,
@@ -2341,7 +2358,7 @@ __global__ __launch_bounds__(kThreads, (NG <= 4 ? 3 : 2)) void col_small_kernel(
 // groups of sixteen queries (nq) instead of four
 __host__ __device__ constexpr int fused_chunks(int qh, int nq = 4) { return qh == 1 ? 16 * (4 / nq) : 8; }
 constexpr int kFusedSteps = 8;
-constexpr int kFusedThreads = 512;
+constexpr unsigned kIsLog = 0x80000000u;   // of a slot's round number: the value is a log2
 
 // Sum or maximum over each row of 16 lanes; every lane of the row ends up with the result.
 template <bool MAX>
@@ -2371,27 +2388,38 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ 
 // SKIP: chunks past the last key are left out instead of being computed and hidden score by score.  The team waits for its last
 // workgroup, which holds them: 6 x 40 pairs of 111 x 7284 x 128 206 -> 165 us per call, 5 x 24 of 89 x 3776 x 64 51 -> 43,
 // 7 x 24 of 100 x 15756 x 128 249 -> 237 (bf16, sums).
-template <int DT, int KS, bool CAUSAL, int MODE, int QH, int NQ, bool SKIP>
-__global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Params p) {
+// NW: waves.  Four (a step is one chunk, and a pair's keys are shared by twice the workgroups) leave room for two
+// workgroups on a CU, of different teams or key ranges: one streams while the other exchanges its row sums.  For at most 32 queries
+// (NQ = 2): 512 pairs of 32 x 16384 x 128 411 -> 369 us, 347 with the shorter exchange below.  With 64 they
+// lose, 397 -> 412: every workgroup reads a word per row of every other one of its team, 0.27 GB beside 2.1 GB of keys.
+// The time between two sweeps, 64 queries and 1024 keys, in cycles: row sums 3000 -> 2600, the team's values 2300 -> 1800, their
+// merge 2200 -> 1900 (sums instead of logarithms), columns 3600 -> 1100 (no question per step), their way to memory 1500 -> 0.
+template <int DT, int KS, bool CAUSAL, int MODE, int QH, int NQ, bool SKIP, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
   static_assert(NQ == 4 || (QH == 1 && NQ == 2), "fewer query groups only with one query half");
+  static_assert(NW == 8 || (NW == 4 && QH == 1), "four waves hold one query half");
   constexpr int KG = kFusedSteps * (4 / NQ);     // steps per pair
-  constexpr int KH = 3 - QH;                     // chunks per step
-  constexpr int NS = (QH == 1) ? 8 : 6;          // ring stages (chunks): 130 KiB or 98 KiB for 256-byte rows
+  constexpr int KH = NW == 4 ? 1 : 3 - QH;       // chunks per step
+  // ring stages (chunks): 130 KiB or 98 KiB for 256-byte rows, 49 with four waves
+  constexpr int NS = NW == 4 ? (KS <= 2 ? 6 : 3) : (QH == 1) ? 8 : 6;
   using Rg = Ring<KS, NS>;                       // four loads of 1 KiB per loading wave and chunk for 256-byte rows
   constexpr int kQBytes = QH * Rg::kRows;        // the queries of a pair, staged like a chunk of keys per 64 rows
-  constexpr int kNumThreads = kFusedThreads;
+  constexpr int kNumThreads = 64 * NW;
   constexpr int kRowsWg = 16 * NQ * QH;          // query rows a workgroup holds
   constexpr int kItemKeys = KG * KH * kChunk;    // keys of a workgroup per pair
   constexpr int kBatchKeys = kFusedSteps * KH * kChunk;   // finished columns leave eight steps at a time
   constexpr int kBatches = KG / kFusedSteps;
   constexpr int kRes = (MODE == kModeBoth) ? 2 : 1;
   constexpr int kObufFloats = QH * kRes * kBatchKeys;
-  constexpr int kRedFloats = 8 * 64;
+  constexpr int kRedFloats = NW * 64;
   // waves per row that share the merge of the team's partial values (half of them when two results are
   // buffered for 1024 keys: the LDS is full)
-  constexpr int kMergeWaves = (8 / QH) / ((kRes == 2 && QH == 1) ? 2 : 1);
-  constexpr int kBatch = 4 * QH;                 // slots a lane fetches together: one round trip for teams of up to 32
+  constexpr int kMergeWaves = (NW / QH) / ((kRes == 2 && QH == 1 && NW == 8) ? 2 : 1);
+  constexpr int kBatch = 4 * QH * (8 / NW);                 // slots a lane fetches together: one round trip for teams of up to 32
   constexpr int kMrgFloats = kMergeWaves * kRowsWg * 2;
+  // Column sums: the row sums are taken as the scores come, while the sweep waits for memory, or, where that costs sixteen registers
+  // too many, after it.
+  constexpr bool kSumsInSweep = QH == 1 && NQ == 4;
   constexpr int kAhead = NS / KH - 1;            // steps in flight in front of the one being computed
   constexpr int kInFlight = (NS / KH - 2) * Rg::kPer;   // loads a loading wave may have outstanding when a step starts
   // (one LDS object: see col_small_kernel)
@@ -2409,7 +2437,7 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
   const int qh = (QH == 2) ? (wave >> 2) : 0;    // which 64 queries
   const int kh = (KH == 2) ? (wave >> 2) : 0;    // which chunk of a step
   const int wq = wave & 3;                       // which 16 keys of the chunk
-  const bool loader = (KH == 2) || (wave < 4);
+  const bool loader = (KH == 2) || (wave < 4);   // (four waves: all)
   const int S = p.splits, T = p.teams;
   const int team = (int)blockIdx.x / S, split = (int)blockIdx.x - team * S;
   const int c0 = split * (KG * KH);              // first chunk of this workgroup's keys
@@ -2425,7 +2453,7 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
   Rg rg;
   rg.init(p.k_sr, p.dgran, lane0, 0);   // (for the fragment offsets; the loads are issued below)
   const bool once = p.stream_once != 0;
-  auto stage_of = [&](int c) { return smem + ((uint32_t)c % NS) * Rg::kStage; };   // NS is a power of two
+  auto stage_of = [&](int c) { return smem + ((uint32_t)c % NS) * Rg::kStage; };
   // The loaders walk the workgroup's stream of chunks with a running address: KG * KH chunks of one pair,
   // then the same range of keys of the next pair of the team.  Chunk number c goes to stage c % NS.
   const int64_t chunk_bytes = (int64_t)kChunk * p.k_sr;
@@ -2524,7 +2552,34 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
   // the query exists and may see the key: 16g + r in [first, mlim).
   const int mlim0 = p.M - 64 * qh - qrow0;
   const bool ragged_rows = p.M < 16 * NQ * (qh + 1);
-  constexpr int kRowWaves = 8 / QH;   // row tid (tid < kRowsWg) is held by all eight waves, or by 0-3 / 4-7 for rows below / from 64
+  constexpr int kRowWaves = NW / QH;   // row tid (tid < kRowsWg) is held by all waves, or by 0-3 / 4-7 for rows below / from 64
+
+  // Columns of batch bt of pair bh from their buffer to memory (all waves have passed a barrier since they wrote them).
+  bool waiting = false, met = true;   // the last batch of the pair before is still in the buffer; its team was met
+  auto store_columns = [&](int bh, int bt, bool met) __attribute__((always_inline)) {
+    void* const out_max = (MODE == kModeBoth) ? p.out2 : p.out;
+    const float poison = __builtin_nanf("");
+    const int bkey0 = key0 + bt * kBatchKeys;
+    int tid_here = threadIdx.x;
+    asm volatile("" : "+v"(tid_here));
+#pragma unroll
+    for (int r = 0; r < kBatchKeys / kNumThreads; ++r) {
+      const int i = tid_here + r * kNumThreads;
+      if (bkey0 + i < keys_end) {
+        if (MODE != kModeMax) {
+          float v = obuf[i];
+          if (QH == 2) v += obuf[kRes * kBatchKeys + i];
+          store_column(p, p.out, true, bh, bkey0 + i, met ? v : poison);
+        }
+        if (MODE != kModeSum) {
+          const float* om = obuf + (MODE == kModeBoth ? kBatchKeys : 0);
+          float v = om[i];
+          if (QH == 2) v = fmaxf(v, om[kRes * kBatchKeys + i]);
+          store_column(p, out_max, false, bh, bkey0 + i, met ? v : poison);
+        }
+      }
+    }
+  };
 
   for (int it = 0; it < rounds; ++it) {
     const int bh = team + it * T;
@@ -2533,7 +2588,22 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
     // the scores are gone by the time it shows, and the keys of the pair are streamed once more.
     f32x4 sc[KG][NQ];
     f32x4 rs[NQ];   // per row (register) and key (lane): sum of 2^score over the steps
-    float my_lse = kNegInf;   // of row tid over this workgroup's keys, for tid < kRowsWg
+    float my_lse = kNegInf;   // of row tid over this workgroup's keys, for tid < kRowsWg (where the plain sums are not usable)
+    // A partial value and the number of its round travel as ONE 64-bit word, so a word that carries this round's number carries this
+    // round's value: nobody waits for a store to complete and there is no counter.  The slots start at zero (round
+    // numbers start at 1).  The value is the row's sum of 2^score, or, with the top bit set, its log2.
+    unsigned long long* const slots =
+        reinterpret_cast<unsigned long long*>(p.part) + ((int64_t)(team * 2 + (it & 1)) * S) * kRowsWg;
+    const unsigned round_no = (unsigned)it + 1u;
+    // A row is published once, whatever becomes of the others: the team adds up the same values.
+    bool published = false;
+    auto publish = [&](int row, unsigned kind, float v) __attribute__((always_inline)) {
+      if (published) return;
+      published = true;
+      __hip_atomic_store(slots + (int64_t)split * kRowsWg + row,
+                         ((unsigned long long)(round_no | kind) << 32) | __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    };
     // Steps 1 and the first half of 2, in two forms (KEEP: the registers end up holding the scores).  Returns
     // whether some row's sum of 2^score is unusable.
     auto sweep = [&](auto keep_tag) -> bool {
@@ -2556,11 +2626,18 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
       issue_step();
       if (j == 0) read_queries();   // (staged at least a whole sweep ago; the barrier above has published them)
       if (j == 1 && it + 1 < rounds) stage_queries(bh + T);   // every wave has read this pair's by now
+      if (j == 1 && waiting) {   // the columns of the pair before, under the loads of this one (the barriers above have published them)
+        store_columns(bh - T, kBatches - 1, met);
+        waiting = false;
+      }
       const char* lds = stage_of(cons_chunk + j * KH + kh);
       if (SKIP && (c0a + j * KH + kh) * kChunk >= p.N) {
         const float none = KEEP ? kNegInf : 0.f;
 #pragma unroll
-        for (int g = 0; g < NQ; ++g) sc[j][g] = (f32x4){none, none, none, none};
+        for (int g = 0; g < NQ; ++g) {
+          sc[j][g] = (f32x4){none, none, none, none};
+          if (kSumsInSweep && !KEEP && j == 1) rs[g] = sc[0][g];
+        }
         continue;
       }
 #pragma unroll
@@ -2597,16 +2674,20 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
         for (int g = 0; g < NQ; ++g)
 #pragma unroll
           for (int r = 0; r < 4; ++r) rs[g][r] += fast_exp2(sc[j][g][r]);
-      } else {   // (the row sums are taken after the loop: sixteen registers less while the queries are held)
+      } else {
 #pragma unroll
         for (int g = 0; g < NQ; ++g)
 #pragma unroll
           for (int r = 0; r < 4; ++r) sc[j][g][r] = fast_exp2(sc[j][g][r]);
+        if (kSumsInSweep && j > 0) {
+#pragma unroll
+          for (int g = 0; g < NQ; ++g) rs[g] = (j == 1) ? sc[0][g] + sc[1][g] : rs[g] + sc[j][g];
+        }
       }
     }
     cons_chunk += KG * KH;
     }
-    if (!KEEP) {
+    if (!KEEP && !kSumsInSweep) {
 #pragma unroll
       for (int g = 0; g < NQ; ++g) {
         rs[g] = sc[0][g];
@@ -2625,24 +2706,26 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
     // 2. log-sum-exp of every row over this workgroup's keys.  The sums of 2^x were taken as the scores
     // came; they are good unless a sum left fp32's comfortable range (or a row saw no key at all), and then
     // the scores, still in registers, are reduced again the exact way: row maximum first.
+    {
+      f32x4 all[4];
 #pragma unroll
-    for (int g = 0; g < NQ; ++g) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) rs[g][r] = row16_reduce<false>(rs[g][r]);
-      if ((lane & 15) == 0) *reinterpret_cast<f32x4*>(red + wave * 64 + 16 * g + qrow) = rs[g];
+      for (int g = 0; g < 4; ++g) all[g] = g < NQ ? rs[g % NQ] : (f32x4){0.f, 0.f, 0.f, 0.f};
+      const float v = lanes16_scatter<false>(all, lane);   // row 16 * ((lane & 15) / 4) + qrow + (lane & 3)
+      const int g = (lane & 15) >> 2;
+      if (g < NQ) red[wave * 64 + 16 * g + qrow + (lane & 3)] = v;
     }
     lds_barrier();
     if (tid < kRowsWg) {
       float l = 0.f;
 #pragma unroll
       for (int w = 0; w < kRowWaves; ++w) l += red_row[64 * w];
-      my_lse = fast_log2(l);
       // 2^-60 <= l < 2^100: terms flushed to zero are far below the sum's last bit, and 2^score times 2^-lse
       // (the lse of all keys is at least this one) neither overflows nor loses anything above 2^-26
       const bool good = (l >= 8.6736174e-19f) && (l < 1.2676506e30f);
       if (!good && tid < p.M) flag[0] = 1;   // (written by whoever finds a bad row; thread 0 resets it below)
       if (!KEEP && tid >= p.M && !(l < kPosInf)) flag[0] = 1;   // a row of zeros met a non-finite key
       if (tid == 0) flag[1] = 1;
+      if (good || tid >= p.M) publish(tid, 0u, good ? l : 1.f);   // (rows that do not exist: anything finite)
     }
     lds_barrier();
     return flag[0] != 0;   // uniform over the workgroup
@@ -2714,24 +2797,17 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
         my_lse = (my_max == kNegInf) ? kNegInf : my_max + fast_log2(l);
       }
     }
-    // 3. meet the team.  A partial value and the number of its round travel as ONE 64-bit word, so a word
-    // that carries this round's number carries this round's value: nobody waits for a store to complete
-    // and there is no counter.  The slots start at zero (round numbers start at 1).
-    unsigned long long* const slots =
-        reinterpret_cast<unsigned long long*>(p.part) + ((int64_t)(team * 2 + (it & 1)) * S) * kRowsWg;
-    const unsigned round_no = (unsigned)it + 1u;
-    if (tid < kRowsWg)
-      __hip_atomic_store(slots + (int64_t)split * kRowsWg + tid,
-                         ((unsigned long long)round_no << 32) | __builtin_bit_cast(unsigned, my_lse), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+    // 3. meet the team.
+    if (bad_sum && tid < kRowsWg) publish(tid, kIsLog, my_lse);
     // All waves share the team's slots: lane = row, the waves of a row take every kMergeWaves-th slot, poll
     // until it carries this round, and fold the values into (max, sum).  (The keys a wave has in flight
     // for the next pair return before these loads do; they were requested during the last steps above.)
+    // Plain sums are added up; where one is a log2 all are taken as such, as (max, sum) pairs.
     if (wave / QH < kMergeWaves) {
       const int rgroup = wave % QH, sub = wave / QH;
       const bool row_here = 64 * rgroup + lane < kRowsWg;   // (fewer than 64 rows per workgroup with NQ < 4)
       const unsigned long long* mine = slots + 64 * rgroup + lane;
-      float m = kNegInf, acc = 0.f;
+      float m = 0.f, acc = 0.f;
       bool nan = false, ok = true;
       int polls = 0;
       for (int s0 = sub; s0 < S; s0 += kMergeWaves * kBatch) {
@@ -2742,10 +2818,10 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
           for (int i = 0; i < kBatch; ++i) {
             const int sidx = s0 + i * kMergeWaves;
             w[i] = (sidx < S && row_here) ? __hip_atomic_load(mine + (int64_t)sidx * kRowsWg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                              : (((unsigned long long)round_no << 32) | 0xff800000u);   // -inf: adds nothing
+                              : ((unsigned long long)round_no << 32);   // a sum of 0
           }
 #pragma unroll
-          for (int i = 0; i < kBatch; ++i) all = all && ((unsigned)(w[i] >> 32) == round_no);
+          for (int i = 0; i < kBatch; ++i) all = all && (((unsigned)(w[i] >> 32) & ~kIsLog) == round_no);
           if (all) break;
           if (++polls > spin_limit) {
             ok = false;
@@ -2757,11 +2833,23 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
         float v[kBatch];
 #pragma unroll
         for (int i = 0; i < kBatch; ++i) v[i] = __builtin_bit_cast(float, (unsigned)w[i]);
+        bool logs = false;
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) logs = logs || (int)(w[i] >> 32) < 0;
+        if (__builtin_amdgcn_ballot_w64(logs || m != 0.f) == 0) {
+#pragma unroll
+          for (int i = 0; i < kBatch; ++i) acc += v[i];
+          continue;
+        }
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i)
+          if ((int)(w[i] >> 32) >= 0) v[i] = fast_log2(v[i]);   // (0: -inf, adds nothing)
         float bm = v[0];
 #pragma unroll
         for (int i = 1; i < kBatch; ++i) bm = fmaxf(bm, v[i]);
 #pragma unroll
         for (int i = 0; i < kBatch; ++i) nan = nan || (v[i] != v[i]);
+        if (acc == 0.f) m = kNegInf;   // nothing yet
         const float nm = fmaxf(m, bm);
         if (nm > kNegInf) {
           acc *= fast_exp2(m - nm);   // m = -inf: acc is 0 and stays 0
@@ -2789,25 +2877,38 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
         mv[w] = ma.x;
         av[w] = ma.y;
       }
-      float m = kNegInf;
-      bool nan = false;
+      bool plain = true;
 #pragma unroll
-      for (int w = 0; w < kMergeWaves; ++w) {
-        nan = nan || (mv[w] != mv[w]);
-        m = fmaxf(m, mv[w]);
+      for (int w = 0; w < kMergeWaves; ++w) plain = plain && mv[w] == 0.f;
+      float lse, factor;
+      if (__builtin_amdgcn_ballot_w64(!plain) == 0) {
+        float sum = av[0];
+#pragma unroll
+        for (int w = 1; w < kMergeWaves; ++w) sum += av[w];
+        lse = log2_of_sum(sum);
+        factor = __builtin_amdgcn_rcpf(sum);
+      } else {
+        float m = kNegInf;
+        bool nan = false;
+#pragma unroll
+        for (int w = 0; w < kMergeWaves; ++w) {
+          nan = nan || (mv[w] != mv[w]);
+          m = fmaxf(m, av[w] == 0.f ? kNegInf : mv[w]);   // (a wave without a slot has nothing to say)
+        }
+        const float ref = (m > kNegInf) ? m : 0.f;
+        float acc = 0.f;
+#pragma unroll
+        for (int w = 0; w < kMergeWaves; ++w) acc += av[w] == 0.f ? 0.f : av[w] * fast_exp2(mv[w] - ref);
+        lse = nan ? __builtin_nanf("") : ((m > kNegInf) ? m + fast_log2(acc) : kNegInf);
+        factor = lse != kNegInf ? fast_exp2(-lse) : 0.f;
       }
-      const float ref = (m > kNegInf) ? m : 0.f;   // 2^(-inf - ref) = 0 times a finite sum: no branches
-      float acc = 0.f;
-#pragma unroll
-      for (int w = 0; w < kMergeWaves; ++w) acc = fmaf(av[w], fast_exp2(mv[w] - ref), acc);
-      const float lse = nan ? __builtin_nanf("") : ((m > kNegInf) ? m + fast_log2(acc) : kNegInf);
       // what step 4 adds to a score, or multiplies 2^score by (nothing for rows that do not exist)
       // (a NaN lse stays a NaN factor: the row's visible columns become NaN, as in the other kernels)
-      rowv[tid] = keep_scores ? -lse : ((tid < p.M && lse != kNegInf) ? fast_exp2(-lse) : 0.f);
+      rowv[tid] = keep_scores ? -lse : (tid < p.M ? factor : 0.f);
       if (split == 0 && tid < p.M) p.lse[(int64_t)bh * p.M + tid] = lse;   // (not meaningful if the team was not met)
     }
     lds_barrier();
-    const bool met = flag[1] != 0;
+    met = flag[1] != 0;
     if (tid == 0) flag[0] = 0;
     if (!met) spin_limit = min(spin_limit, 64);   // the call has failed: later waits of this workgroup are short
     // 4. probabilities, reduced down the rows
@@ -2818,9 +2919,22 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
     float* const omax = osum + (MODE == kModeBoth ? kBatchKeys : 0);
     int c0b = c0;
     asm volatile("" : "+s"(c0b));
-#pragma unroll
-    for (int bt = 0; bt < kBatches; ++bt) {   // eight steps at a time through the column buffer
+    auto columns = [&](auto batch_tag) __attribute__((always_inline)) {   // eight steps at a time through the column buffer
+    constexpr int bt = decltype(batch_tag)::value;
     float vs[kFusedSteps], vm[kFusedSteps];   // per step: the lane's key, reduced over the lane's queries
+    const int kend = (c0b + (bt + 1) * kFusedSteps * KH) * kChunk;   // of the batch's keys
+    if (MODE == kModeSum && !keep_scores && kend <= p.N && (!CAUSAL || kend - 1 <= p.c + 64 * qh)) {
+      // the usual case, without a question per step: 3000 -> 1100 cycles on 1024 keys and 64 queries
+#pragma unroll
+      for (int jj = 0; jj < kFusedSteps; ++jj) {
+        f32x4 part = sc[bt * kFusedSteps + jj][0] * nl[0];
+#pragma unroll
+        for (int g = 1; g < NQ; ++g)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) part[r] = fmaf(sc[bt * kFusedSteps + jj][g][r], nl[g][r], part[r]);
+        vs[jj] = (part[0] + part[1]) + (part[2] + part[3]);
+      }
+    } else {
 #pragma unroll
     for (int jj = 0; jj < kFusedSteps; ++jj) {
       const int j = bt * kFusedSteps + jj;
@@ -2871,57 +2985,33 @@ __global__ __launch_bounds__(kFusedThreads, 2) void col_fused_kernel(const Param
       vs[jj] = (part[0] + part[1]) + (part[2] + part[3]);
       vm[jj] = vmax;
     }
-    // the four lane groups hold different queries of the same key: two exchanges, all steps at once
+    }
+    // the four rows of lanes hold different queries of the same key: a reduce-scatter, after which row rho of lanes has
+    // steps 2 rho and 2 rho + 1
+    const int at = ((lane >> 4) * 2 * KH + kh) * kChunk + 16 * wq + (lane & 15);
     if (MODE != kModeMax) {
-      float o[kFusedSteps];
-#pragma unroll
-      for (int j = 0; j < kFusedSteps; ++j) o[j] = __shfl_xor(vs[j], 16);
-#pragma unroll
-      for (int j = 0; j < kFusedSteps; ++j) vs[j] += o[j];
-#pragma unroll
-      for (int j = 0; j < kFusedSteps; ++j) o[j] = __shfl_xor(vs[j], 32);
-      if (lane < 16) {
-#pragma unroll
-        for (int j = 0; j < kFusedSteps; ++j) osum[(j * KH + kh) * kChunk + 16 * wq + lane] = vs[j] + o[j];
-      }
+      lane_rows_scatter<false>(vs);
+      osum[at] = vs[0];
+      osum[at + KH * kChunk] = vs[1];
     }
     if (MODE != kModeSum) {
-      float o[kFusedSteps];
-#pragma unroll
-      for (int j = 0; j < kFusedSteps; ++j) o[j] = __shfl_xor(vm[j], 16);
-#pragma unroll
-      for (int j = 0; j < kFusedSteps; ++j) vm[j] = fmaxf(vm[j], o[j]);
-#pragma unroll
-      for (int j = 0; j < kFusedSteps; ++j) o[j] = __shfl_xor(vm[j], 32);
-      if (lane < 16) {
-#pragma unroll
-        for (int j = 0; j < kFusedSteps; ++j) omax[(j * KH + kh) * kChunk + 16 * wq + lane] = fast_exp2(fmaxf(vm[j], o[j]));
-      }
+      lane_rows_scatter<true>(vm);
+      omax[at] = fast_exp2(vm[0]);
+      omax[at + KH * kChunk] = fast_exp2(vm[1]);
     }
-    lds_barrier();
-    void* const out_max = (MODE == kModeBoth) ? p.out2 : p.out;
-    const float poison = __builtin_nanf("");
-    const int bkey0 = key0 + bt * kBatchKeys;
-    for (int i = tid; i < kBatchKeys; i += kNumThreads) {
-      if (bkey0 + i < keys_end) {
-        if (MODE != kModeMax) {
-          float v = obuf[i];
-          if (QH == 2) v += obuf[kRes * kBatchKeys + i];
-          store_column(p, p.out, true, bh, bkey0 + i, met ? v : poison);
-        }
-        if (MODE != kModeSum) {
-          const float* om = obuf + (MODE == kModeBoth ? kBatchKeys : 0);
-          float v = om[i];
-          if (QH == 2) v = fmaxf(v, om[kRes * kBatchKeys + i]);
-          store_column(p, out_max, false, bh, bkey0 + i, met ? v : poison);
-        }
-      }
+    if (bt + 1 < kBatches) {   // the next batch writes the buffer again
+      lds_barrier();
+      store_columns(bh, bt, met);
+      lds_barrier();
     }
-    if (bt + 1 < kBatches) lds_barrier();   // the next batch writes the buffer again
-    }
+    };
+    columns(std::integral_constant<int, 0>());
+    if constexpr (kBatches == 2) columns(std::integral_constant<int, 1>());
+    waiting = true;
     // the next writers of obuf, red, rowv and flag are behind the ring barriers of the next pair
   }
   ring_sync<0>();   // the loads past the last chunk write their zeros before the LDS is given back
+  if (waiting) store_columns(team + (rounds - 1) * T, kBatches - 1, met);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -4184,6 +4274,24 @@ bool fused_shape(int64_t bh, int M, int N, FusedPlan& f) {
   return true;
 }
 
+// The single sweep in workgroups of four waves, two per CU, for at most 64 queries in several rounds, where the caller's workspace
+// has room for their slots (they follow the status word of the form above).
+struct FusedPairPlan {
+  int nq, splits, teams;   // teams 0: not this form
+  int64_t part_at, floats;
+};
+FusedPairPlan fused_pair_plan(int64_t bh, int M, int N, const FusedPlan& f) {
+  FusedPairPlan o{f.nq, 0, 0, f.sync_at + 32, f.floats};
+  if (f.qh != 1 || f.nq != 2 || bh <= f.teams) return o;
+  const int cap = 2 * chip_cus();
+  const int64_t nchunks = ((int64_t)N + kChunk - 1) / kChunk, chunks = kFusedSteps * (4 / o.nq), splits = (nchunks + chunks - 1) / chunks;
+  if (splits > cap) return o;
+  o.splits = (int)splits;
+  o.teams = (int)((cap / splits) < bh ? cap / splits : bh);
+  o.floats = o.part_at + 2 * (2ll * o.teams * o.splits * 64);
+  return o;
+}
+
 // The path for one query (one_query_*_kernel): sizes of its launches and its scratch, which lies behind everything
 // fcr_lse_bytes asks for.  Any element type and any number of keys.
 struct OneQueryPlan {
@@ -4386,54 +4494,55 @@ bool fits_per_cu(K kernel, int threads, int want) {
   return n >= want;
 }
 
-template <int DT, int KS, int MODE, int QH, int NQ, bool SKIP>
+template <int DT, int KS, int MODE, int QH, int NQ, bool SKIP, int NW>
 void launch_col_fused_form(const Params& p, bool causal, hipStream_t s) {
-  const dim3 grid(p.total), block(kFusedThreads);
+  const dim3 grid(p.total), block(64 * NW);
   static int fits[2] = {-1, -1};   // asked once per kernel (the answer depends on its registers and LDS, not on the device of a kind)
   int f = __atomic_load_n(&fits[causal], __ATOMIC_RELAXED);
   if (f < 0) {
-    f = causal ? fits_per_cu(col_fused_kernel<DT, KS, true, MODE, QH, NQ, SKIP>, kFusedThreads, 1)
-               : fits_per_cu(col_fused_kernel<DT, KS, false, MODE, QH, NQ, SKIP>, kFusedThreads, 1);
+    f = causal ? fits_per_cu(col_fused_kernel<DT, KS, true, MODE, QH, NQ, SKIP, NW>, 64 * NW, 8 / NW)
+               : fits_per_cu(col_fused_kernel<DT, KS, false, MODE, QH, NQ, SKIP, NW>, 64 * NW, 8 / NW);
     __atomic_store_n(&fits[causal], f, __ATOMIC_RELAXED);
   }
   if (!f) {
     fcr_detail::fused_refused = true;
     return;
   }
-  if (causal) hipLaunchKernelGGL((col_fused_kernel<DT, KS, true, MODE, QH, NQ, SKIP>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((col_fused_kernel<DT, KS, false, MODE, QH, NQ, SKIP>), grid, block, 0, s, p);
+  if (causal) hipLaunchKernelGGL((col_fused_kernel<DT, KS, true, MODE, QH, NQ, SKIP, NW>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((col_fused_kernel<DT, KS, false, MODE, QH, NQ, SKIP, NW>), grid, block, 0, s, p);
 }
 
 // More than 64 queries: maxima gain nothing by leaving chunks out (ragged rows are hidden one by one in any case; sums and
 // maxima 323 -> 325 us), and where there is nothing to leave out the question alone costs (4 x 32 pairs of 89 x 4096 x 64
 // 40.7 -> 42.6 us, 32 of 128 x 4096 x 128 17.6 -> 17.8), so the host asks it.
-template <int DT, int KS, int MODE, int QH, int NQ>
+template <int DT, int KS, int MODE, int QH, int NQ, int NW>
 void launch_col_fused_mode(const Params& p, bool causal, hipStream_t s) {
-  if constexpr (QH == 2 && MODE != kModeSum) return launch_col_fused_form<DT, KS, MODE, QH, NQ, false>(p, causal, s);
+  if constexpr (QH == 2 && MODE != kModeSum) return launch_col_fused_form<DT, KS, MODE, QH, NQ, false, NW>(p, causal, s);
   else if constexpr (QH == 2) {
     const int chunks = (p.N + kChunk - 1) / kChunk;
-    if (chunks % fused_chunks(QH, NQ) != 0) return launch_col_fused_form<DT, KS, MODE, QH, NQ, true>(p, causal, s);
-    launch_col_fused_form<DT, KS, MODE, QH, NQ, false>(p, causal, s);
+    if (chunks % fused_chunks(QH, NQ) != 0) return launch_col_fused_form<DT, KS, MODE, QH, NQ, true, NW>(p, causal, s);
+    launch_col_fused_form<DT, KS, MODE, QH, NQ, false, NW>(p, causal, s);
   } else {
-    launch_col_fused_form<DT, KS, MODE, QH, NQ, true>(p, causal, s);
+    launch_col_fused_form<DT, KS, MODE, QH, NQ, true, NW>(p, causal, s);
   }
 }
 
-template <int DT, int KS, int QH, int NQ>
+template <int DT, int KS, int QH, int NQ, int NW>
 void launch_col_fused_groups(const Params& p, bool causal, int m, hipStream_t s) {
-  if (m == kModeSum) launch_col_fused_mode<DT, KS, kModeSum, QH, NQ>(p, causal, s);
-  else if (m == kModeMax) launch_col_fused_mode<DT, KS, kModeMax, QH, NQ>(p, causal, s);
-  else launch_col_fused_mode<DT, KS, kModeBoth, QH, NQ>(p, causal, s);
+  if (m == kModeSum) launch_col_fused_mode<DT, KS, kModeSum, QH, NQ, NW>(p, causal, s);
+  else if (m == kModeMax) launch_col_fused_mode<DT, KS, kModeMax, QH, NQ, NW>(p, causal, s);
+  else launch_col_fused_mode<DT, KS, kModeBoth, QH, NQ, NW>(p, causal, s);
 }
 
 // mode: kModeSum, kModeMax or kModeBoth, + 4 for more than 64 queries, + 8 for two groups of sixteen queries
-// per wave
+// per wave, + 16 for four waves
 template <int DT, int KS>
 void launch_col_fused(const Params& p, bool causal, int mode, hipStream_t s) {
   const int m = mode & 3;
-  if (mode & 4) launch_col_fused_groups<DT, KS, 2, 4>(p, causal, m, s);
-  else if (mode & 8) launch_col_fused_groups<DT, KS, 1, 2>(p, causal, m, s);
-  else launch_col_fused_groups<DT, KS, 1, 4>(p, causal, m, s);
+  if (mode & 4) launch_col_fused_groups<DT, KS, 2, 4, 8>(p, causal, m, s);
+  else if (mode & 16) (mode & 8) ? launch_col_fused_groups<DT, KS, 1, 2, 4>(p, causal, m, s) : launch_col_fused_groups<DT, KS, 1, 4, 4>(p, causal, m, s);
+  else if (mode & 8) launch_col_fused_groups<DT, KS, 1, 2, 8>(p, causal, m, s);
+  else launch_col_fused_groups<DT, KS, 1, 4, 8>(p, causal, m, s);
 }
 
 template <int DT, int KS>
@@ -5006,14 +5115,23 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
     p.sync = reinterpret_cast<unsigned*>(ws + f.sync_at);
     p.splits = f.splits;
     p.teams = f.teams;
-    p.total = f.teams * f.splits;
+    unsigned* zero = reinterpret_cast<unsigned*>(p.part);   // the slots and the status word start at zero
+    int words = (int)(f.floats - f.part_at), form = (f.qh == 2 ? 4 : 0) | (f.nq == 2 ? 8 : 0);
+    const FusedPairPlan two = fused_pair_plan(p.bh_count, M, N, f);
+    if (two.teams > 0 && (size_t)two.floats * sizeof(float) <= ws_bytes) {
+      p.part = ws + two.part_at;
+      p.splits = two.splits;
+      p.teams = two.teams;
+      zero = p.sync;
+      words = (int)(two.floats - f.sync_at);
+      form = 16 | (two.nq == 2 ? 8 : 0);
+    }
+    p.total = p.teams * p.splits;
     const long long polls = __atomic_load_n(&g_wait_polls, __ATOMIC_RELAXED);
     p.spin_limit = polls > 0x7fffffffll ? 0x7fffffff : (int)polls;
-    const int words = (int)(f.floats - f.part_at);   // the slots and the error word start at zero
     fcr_detail::fused_refused = false;
     SweepOrder* const order = order_begin(s);
-    launch_sweeps(dtype, 3, p, ksteps, causal != 0, mode | (f.qh == 2 ? 4 : 0) | (f.nq == 2 ? 8 : 0), s,
-                  reinterpret_cast<unsigned*>(p.part), words);
+    launch_sweeps(dtype, 3, p, ksteps, causal != 0, mode | form, s, zero, words);
     const int lrc = fcr_detail::fused_refused ? 0 : launched("col_fused_kernel");
     order_end(order, s, !fcr_detail::fused_refused && lrc == 0);
     if (!fcr_detail::fused_refused) return lrc;
@@ -5111,7 +5229,13 @@ size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D) {
   if (row_width_ok(dtype, D)) {
     const int64_t floats = (int64_t)(base / sizeof(float));
     const FewKeysPlan one = few_keys_plan(dtype, B, H, M, N, D, false, false, floats), both = few_keys_plan(dtype, B, H, M, N, D, true, false, floats);
-    return (size_t)(one.floats > both.floats ? one.floats : both.floats) * sizeof(float);
+    int64_t most = one.floats > both.floats ? one.floats : both.floats;
+    FusedPlan f;
+    if (dtype != FCR_DTYPE_F32 && ksteps_of(dtype, D) <= 4 && fused_shape((int64_t)B * H, M, N, f)) {
+      const FusedPairPlan two = fused_pair_plan((int64_t)B * H, M, N, f);
+      if (two.floats > most) most = two.floats;
+    }
+    return (size_t)most * sizeof(float);
   }
   return base;
 }

@@ -920,6 +920,58 @@ def test_single_sweep_bounded_wait():
     assert lib.fcr_set_option(7, 1) == -3 and lib.fcr_set_option(_lib.OPT_WAIT_POLLS, -1) == -3
 
 
+# pairs in several rounds, so that at most 32 queries take the workgroups of four waves (two per CU): one team member, several and many,
+# keys that fill no step, no batch and no chunk, both edges of the query groups
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d,dtype", [(300, 20, 1100, 64, torch.float16), (60, 32, 5001, 128, torch.bfloat16), (520, 2, 1024, 40, torch.float16),
+                                           (20, 17, 20000, 96, torch.float16), (60, 33, 5001, 128, torch.float16), (150, 31, 2049, 128, torch.bfloat16)])
+def test_single_sweep_in_rounds(h, m, n, d, dtype, causal):
+    """Against 64 bits (see test_few_keys for the bound), then scores far from zero, NaN rows and infinite keys against the two kernels."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(h + n)
+    q, k = (torch.randn(2, h, r, d, device="cuda", generator=g).to(dtype) for r in (m, n))
+    sums, most = _columns_f64(q, k, causal)
+    assert _rel(fca.flash_colreduce(q, k, "sum", causal, out_dtype=torch.float32), sums) <= 1e-5
+    s2, m2 = fca.flash_colreduce_multi(q, k, ["sum", "max"], causal, out_dtype=torch.float32)
+    assert _rel(s2, sums) <= 1e-5 and _rel(m2, most) <= 1e-5
+    q[0, 1] *= 30
+    k[0, 2, n // 2] *= 60
+    q[1, 3, m - 1, 0] = float("nan")
+    k[1, 4, n // 3, 0] = float("inf")
+    for red in ("sum", "max"):
+        got = {}
+        for option in (1, 0):
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+            try:
+                got[option] = fca.flash_colreduce(q, k, red, causal, out_dtype=torch.float32)
+            finally:
+                lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+        assert torch.equal(got[1].isnan(), got[0].isnan()), red
+        torch.testing.assert_close(got[1], got[0], rtol=2e-4, atol=1e-6, equal_nan=True)   # scores of 2^9: 2^-15 each
+
+
+def test_single_sweep_in_rounds_bounded_wait():
+    """As test_single_sweep_bounded_wait, in workgroups of four waves."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    q, k = (torch.randn(2, 60, r, 64, device="cuda").half() for r in (30, 8192))
+    ws, out = torch.empty(_lib_workspace(q, k), device="cuda"), torch.empty(120, 8192, device="cuda")
+    assert 4 * ws.numel() > lib.fcr_lse_bytes(2, 60, 30, 8192, 64)
+    want, _ = _columns_f64(q, k, True)
+    want = want.view(120, 8192)
+    for polls in (0, 1 << 20):
+        assert lib.fcr_set_option(_lib.OPT_WAIT_POLLS, polls) == 0
+        try:
+            _ws_call(q, k, out, ws, True)
+            status = lib.fcr_colreduce_status(ws.data_ptr(), _lib.DTYPE_F16, 2, 60, 30, 8192, 64, torch.cuda.current_stream().cuda_stream)
+        finally:
+            assert lib.fcr_set_option(_lib.OPT_WAIT_POLLS, 1 << 20) == 0
+        gave_up = torch.isnan(out)
+        assert status == (_lib.E_WAIT if gave_up.any() else 0) and not (polls and status)
+        torch.testing.assert_close(out[~gave_up], want[~gave_up].float(), rtol=1e-4, atol=1e-6)
+
+
 def test_single_sweeps_on_two_streams_are_chained():
     """A single sweep expects the whole chip (its workgroups wait for each other), so the library chains the
     single sweeps that a process issues on different streams with an event: calls issued alternately on two
