@@ -3580,30 +3580,64 @@ __global__ __launch_bounds__(T) void topk16_mask_kernel(const ET* __restrict__ s
   hist[2 * tid] = (u32x4){0u, 0u, 0u, 0u};
   hist[2 * tid + 1] = (u32x4){0u, 0u, 0u, 0u};
   if (tid < 64) fine[tid] = 0u;
+  u16x2 most = both(0);   // as unsigned numbers: above infinity where there is a sign or a NaN
 #pragma unroll
   for (int j = 0; j < W4; ++j)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) mag = __builtin_elementwise_max(mag, pk(u[j][e] & 0x7fff7fffu));
-  const bool any_nan = __builtin_amdgcn_ballot_w64(mag[0] > kInf || mag[1] > kInf) != 0;
+    for (int e = 0; e < 4; ++e) most = __builtin_elementwise_max(most, pk(u[j][e]));
   u16x2 hi = both(0), lo1 = both(0xffff);   // largest key, smallest key - 1 (where 0, no key, is the largest)
+  if (__builtin_amdgcn_ballot_w64(most[0] > kInf || most[1] > kInf) == 0) {
+    // Neither, which is what column sums, means and maxima are: such a number and the top bit is its key, three
+    // instructions per pair where the general case takes twelve (a call with 32 rows of 32768 fp16 11.6 -> 9.9 us, 640 rows 34 -> 28.5, 32 of
+    // 60000 20.6 -> 17.3; 8192 columns and fewer 0-5 %).
+    u16x2 least = both(0x7fff);
 #pragma unroll
-  for (int j = 0; j < W4; ++j) {
-    const int col = (j * T + tid) * 8;
+    for (int j = 0; j < W4; ++j) {
+      const int col = (j * T + tid) * 8;
+      if (__builtin_amdgcn_ballot_w64(col + 8 > N) == 0) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t x = u[j][e];
-      uint32_t key = order_pair(x);
-      if (any_nan) {
-        const u16x2 over = __builtin_elementwise_min(__builtin_elementwise_sub_sat(pk(x & 0x7fff7fffu), both(kInf)), both(1));
-        key |= word(both(0) - over);
+        for (int e = 0; e < 4; ++e) {
+          least = __builtin_elementwise_min(least, pk(u[j][e]));
+          u[j][e] ^= 0x80008000u;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint32_t key = u[j][e] ^ 0x80008000u;
+          if (col + 2 * e >= N) key = 0u;
+          else if (col + 2 * e + 1 >= N) key &= 0xffffu;
+          u[j][e] = key;
+          lo1 = __builtin_elementwise_min(lo1, pk(key) - both(1));
+        }
       }
-      if (col + 8 > N) {   // (the last vectors of the row)
-        if (col + 2 * e >= N) key = 0u;
-        else if (col + 2 * e + 1 >= N) key &= 0xffffu;
+    }
+    if (tid * 8 < N) hi = pk(word(most) ^ 0x80008000u);
+    lo1 = __builtin_elementwise_min(lo1, pk(word(least) ^ 0x80008000u) - both(1));
+  } else {
+#pragma unroll
+    for (int j = 0; j < W4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mag = __builtin_elementwise_max(mag, pk(u[j][e] & 0x7fff7fffu));
+    const bool any_nan = __builtin_amdgcn_ballot_w64(mag[0] > kInf || mag[1] > kInf) != 0;
+#pragma unroll
+    for (int j = 0; j < W4; ++j) {
+      const int col = (j * T + tid) * 8;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t x = u[j][e];
+        uint32_t key = order_pair(x);
+        if (any_nan) {
+          const u16x2 over = __builtin_elementwise_min(__builtin_elementwise_sub_sat(pk(x & 0x7fff7fffu), both(kInf)), both(1));
+          key |= word(both(0) - over);
+        }
+        if (col + 8 > N) {   // (the last vectors of the row)
+          if (col + 2 * e >= N) key = 0u;
+          else if (col + 2 * e + 1 >= N) key &= 0xffffu;
+        }
+        u[j][e] = key;
+        hi = __builtin_elementwise_max(hi, pk(key));
+        lo1 = __builtin_elementwise_min(lo1, pk(key) - both(1));
       }
-      u[j][e] = key;
-      hi = __builtin_elementwise_max(hi, pk(key));
-      lo1 = __builtin_elementwise_min(lo1, pk(key) - both(1));
     }
   }
   auto equals = [](const uint32_t(&v)[4], uint32_t x) {   // how many of eight 16-bit numbers are x

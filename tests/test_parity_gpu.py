@@ -1535,6 +1535,28 @@ def test_topk_16_bit_rows_of_any_bits(n, dtype):
         torch.testing.assert_close(thr.cpu() + 0.0, kth + 0.0, rtol=0, atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 17, 511, 513, 2050, 8193, 20011])
+def test_topk_16_bit_rows_without_signs(n, dtype):
+    """Waves whose columns are all at least zero take their keys from the bits: such rows, all zeros, denormals and infinities, and
+    rows of which one wave alone holds a negative number, a negative zero or a NaN.  Exact."""
+    from oracle.colreduce_oracle import topk_mask_ref
+    g = torch.Generator().manual_seed(n)
+    r = torch.rand(7, n, generator=g).mul(4).exp().to(dtype)
+    r[1] = 0
+    r[2] = torch.randint(0, 40, (n,), generator=g, dtype=torch.int32).to(torch.int16).view(dtype)
+    r[3, n // 2] = float("inf")
+    r[4, n - 1] = -1
+    r[5, 0] = -0.0
+    r[6, n // 3] = float("nan")
+    dev = r.cuda()
+    for k in sorted({1, (n + 3) // 4, n}):
+        mask, thr = fca.topk_keep_mask(dev, k, return_threshold=True)
+        assert (mask.cpu().numpy() == topk_mask_ref(r.float().numpy(), k)).all(), (n, k)
+        kth = r.float().sort(dim=1, descending=True).values[:, k - 1]
+        torch.testing.assert_close(thr.cpu() + 0.0, kth + 0.0, rtol=0, atol=0, equal_nan=True)
+
+
 def test_topk_on_reduced_columns():
     from oracle.colreduce_oracle import topk_mask_ref
     q, k = _inputs.config4(heads=4, n=2048)
