@@ -4394,7 +4394,12 @@ FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool bot
   int64_t s = (waves == 8 ? 1 : 2) * (int64_t)chip_cus() / bh;
   if (s > chunks) s = chunks;
   if (s < 1) s = 1;
-  if (N > 256 && s < 4 && (both || (causal && (s > 1 || (ks <= 2 && bh > chip_cus()))))) {
+  // A few chunks go to one workgroup, whose launch is then the only one: 2 pairs of 64 x 64 x 128 8.8 -> 5.0 us per call, of 128 x 128 8.8 -> 6.1,
+  // of 160 x 160 8.9 -> 8.4, but of 200 x 200 8.9 -> 11.0; rows of 512 bytes 100 x 100 8.8 -> 8.3, 128 x 128 8.7 -> 9.1; more than 256 keys
+  // 96 x 500 x 64 8.9 -> 7.8, 128 x 500 x 128 10.4 -> 11.2.
+  if (chunks <= (form == 2 ? 3 : ks > 4 ? 7 : 5)) {
+    s = 1;
+  } else if (N > 256 && s < 4 && (both || (causal && (s > 1 || (ks <= 2 && bh > chip_cus()))))) {
     o.form = -1;
     return o;
   }
