@@ -3202,6 +3202,92 @@ __global__ __launch_bounds__(256) void one_query_columns_kernel(const Params p, 
   }
 }
 
+// The whole of it in one launch, a workgroup per pair, whose raw products wait in LDS (one_query_alone has where and why).  A CU
+// alone has 16 waves with eight to sixteen loads of 1 KiB in flight and reads about 70 bytes per ns; with a workgroup on every CU the
+// memory is the limit again.
+constexpr int kOnePairThreads = 1024;
+constexpr int kOnePairKeys = 8192;   // 32 KiB of products
+
+template <int DT, int LPR>
+__global__ __launch_bounds__(kOnePairThreads) void one_query_pair_kernel(const Params p, int mode) {
+  constexpr int E = DT == FCR_DTYPE_F32 ? 4 : 8;
+  constexpr int kRows = 64 / LPR;                               // key rows per load
+  constexpr int kSel = kOneLoads > LPR ? kOneLoads / LPR : 1;   // finished scores per lane and step
+  constexpr int kStep = kOneLoads * kRows;                      // key rows per wave and step
+  constexpr int kW = kOnePairThreads / 64;
+  __shared__ float scores[kOnePairKeys];
+  __shared__ float wave_m[kW], wave_l[kW];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane & (LPR - 1), r0 = lane / LPR;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bh = (int)blockIdx.x, b = bh / p.H, h = bh - b * p.H;
+  const char* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh + (int64_t)g * 16;
+  const char* qb = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)g * 16;
+  const bool live = g < p.dgran;   // the lanes past the end of a row neither load nor count
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  float qf[E];
+  granule_floats<DT>(live ? *reinterpret_cast<const u32x4*>(qb) : zero, qf);
+  float m = kNegInf, l = 0.f;
+  auto load = [&](u32x4(&v)[kOneLoads], int row) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kOneLoads; ++u) {
+      v[u] = zero;
+      if (live) v[u] = *reinterpret_cast<const u32x4*>(kb + (int64_t)min(row + u * kRows + r0, p.N - 1) * p.k_sr);
+    }
+  };
+  auto take = [&](const u32x4(&v)[kOneLoads], int row) __attribute__((always_inline)) {
+    float done[kSel];
+#pragma unroll
+    for (int i = 0; i < kSel; ++i) done[i] = 0.f;
+#pragma unroll
+    for (int u = 0; u < kOneLoads; ++u) {
+      float f[E], s = 0.f;
+      granule_floats<DT>(v[u], f);
+#pragma unroll
+      for (int e = 0; e < E; ++e) s = fmaf(f[e], qf[e], s);
+      s = group_sum<LPR>(s);
+      if (g == (u & (LPR - 1))) done[u / LPR] = s;   // lane g of a group keeps load g's row (and every LPR-th after it)
+    }
+#pragma unroll
+    for (int i = 0; i < kSel; ++i) {
+      const int r = row + (i * LPR + g) * kRows + r0;
+      if (i * LPR + g < kOneLoads && r < p.N) {
+        scores[r] = done[i];
+        one_query_merge(m, l, done[i] * p.scale2, 1.f);
+      }
+    }
+  };
+  // a step ahead: the next keys are on their way while these are multiplied
+  constexpr int kPass = kW * kStep;
+  u32x4 va[kOneLoads], vb[kOneLoads];
+  int row = wave * kStep;
+  if (row < p.N) load(va, row);
+  for (; row < p.N; row += 2 * kPass) {
+    if (row + kPass < p.N) load(vb, row + kPass);
+    take(va, row);
+    if (row + kPass >= p.N) break;
+    if (row + 2 * kPass < p.N) load(va, row + 2 * kPass);
+    take(vb, row + kPass);
+  }
+  one_query_merge_wave(m, l);
+  if (lane == 0) {
+    wave_m[wave] = m;
+    wave_l[wave] = l;
+  }
+  __syncthreads();
+  m = wave_m[0];
+  l = wave_l[0];
+#pragma unroll
+  for (int w = 1; w < kW; ++w) one_query_merge(m, l, wave_m[w], wave_l[w]);
+  if (tid == 0) p.lse[bh] = m + fast_log2(l);
+  if (bh == 0 && tid == 0 && p.sync) *p.sync = 0u;
+  const float ref = (m == kNegInf) ? 0.f : m, inv = 1.0f / l;   // as one_query_columns_kernel
+  for (int key = tid; key < p.N; key += kOnePairThreads) {
+    const float v = fast_exp2(fmaf(scores[key], p.scale2, -ref)) * inv;
+    if (mode != kModeMax) store_column(p, p.out, true, bh, key, v);
+    if (mode != kModeSum) store_column(p, mode == kModeBoth ? p.out2 : p.out, false, bh, key, fmaxf(v, 0.f));   // drops a NaN
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // fp32 operands packed by the caller.  x = hi + lo with hi = fp16(x), lo = fp16(x - hi) carries 22 bits of x.  Packing
 // queries as [hi | hi | lo] and keys as [hi | lo | hi] along d makes the fp16 kernels compute
@@ -4777,7 +4863,37 @@ void launch_one_query_scores(bool once, const Params& p, const OneQueryPlan& o, 
   else launch_one_query_scores<DT, false>(p, o, scores, s);
 }
 
+// Keys that a workgroup reads while the second launch of the other way would still be on its way to the device, 256 KiB, or, where
+// the pairs are a workgroup for at least every other CU and no second round, 1 MiB.  Per call, two launches and one, bf16 keys of 128:
+// 8 pairs of 512 9.2 -> 5.7 us, of 1024 9.5 -> 7.5, but of 2048 9.5, 11.0; 256 of 64 9.0 -> 5.6, of 512 9.5 -> 6.0, of 1024 14.7 both, of 2048
+// 24.8 -> 23.4, of 4096 46.6 -> 42.7, but of 8192 91.5, 95.5; 640 pairs of 512 17.2, 20.6, of 2048 58.1, 66.8.
+inline bool one_query_alone(const Params& p) {
+  const int cus = chip_cus();
+  const int64_t most = 2 * (int64_t)p.bh_count >= cus ? 1 << 20 : 256 << 10;
+  return p.bh_count <= cus && p.N <= kOnePairKeys && (int64_t)p.N * p.dgran * 16 <= most;
+}
+
+template <int DT>
+void launch_one_query_pair(const Params& p, int lanes, int mode, hipStream_t s) {
+  const dim3 grid((unsigned)p.bh_count), block(kOnePairThreads);
+  switch (lanes) {
+    case 1: hipLaunchKernelGGL((one_query_pair_kernel<DT, 1>), grid, block, 0, s, p, mode); break;
+    case 2: hipLaunchKernelGGL((one_query_pair_kernel<DT, 2>), grid, block, 0, s, p, mode); break;
+    case 4: hipLaunchKernelGGL((one_query_pair_kernel<DT, 4>), grid, block, 0, s, p, mode); break;
+    case 8: hipLaunchKernelGGL((one_query_pair_kernel<DT, 8>), grid, block, 0, s, p, mode); break;
+    case 16: hipLaunchKernelGGL((one_query_pair_kernel<DT, 16>), grid, block, 0, s, p, mode); break;
+    case 32: hipLaunchKernelGGL((one_query_pair_kernel<DT, 32>), grid, block, 0, s, p, mode); break;
+    default: hipLaunchKernelGGL((one_query_pair_kernel<DT, 64>), grid, block, 0, s, p, mode); break;
+  }
+}
+
 int launch_one_query(Params& p, int dtype, const OneQueryPlan& o, float* ws, int mode, hipStream_t s) {
+  if (one_query_alone(p)) {
+    if (dtype == FCR_DTYPE_F16) launch_one_query_pair<FCR_DTYPE_F16>(p, o.lanes, mode, s);
+    else if (dtype == FCR_DTYPE_BF16) launch_one_query_pair<FCR_DTYPE_BF16>(p, o.lanes, mode, s);
+    else launch_one_query_pair<FCR_DTYPE_F32>(p, o.lanes, mode, s);
+    return launched("one_query_pair_kernel");
+  }
   float* const scores = ws + o.scores_at;
   p.part = ws + o.part_at;
   p.splits = o.splits;

@@ -750,6 +750,27 @@ def test_one_query_shared_keys(b, h, n, d, dtype, shared):
     check(fca.flash_colreduce(q, k, "sum", out_dtype=torch.float32)[-1], p.cpu(), "sum", f"shared by {shared}")
 
 
+# one launch and two: the largest number of keys of either limit and one more, the most pairs and one more, every number of lanes per row
+@pytest.mark.parametrize("b,h,n,d,dtype", [(1, 8, 1024, 128, torch.bfloat16), (1, 8, 1025, 128, torch.bfloat16), (1, 130, 4096, 128, torch.float16),
+                                           (1, 130, 4097, 128, torch.float16), (4, 64, 500, 64, torch.float16), (1, 257, 500, 64, torch.float16),
+                                           (1, 3, 8192, 8, torch.float16), (1, 3, 8193, 8, torch.float16), (2, 2, 33, 16, torch.bfloat16),
+                                           (1, 5, 255, 256, torch.float32), (1, 5, 1, 72, torch.bfloat16), (2, 70, 700, 40, torch.float32),
+                                           (1, 2, 513, 512, torch.float16)])
+def test_one_query_in_one_launch(b, h, n, d, dtype):
+    """Against 64 bits: a probability is good to the rounding of its score (2^4: 2^-20) and of the sum."""
+    g = torch.Generator(device="cuda").manual_seed(n + d)
+    q, k = (torch.randn(b, h, r, d, device="cuda", generator=g).to(dtype) for r in (1, n))
+    want, _ = _columns_f64(q, k, False)
+    for causal in (False, True):
+        for red in REDUCTIONS:
+            assert _rel(fca.flash_colreduce(q, k, red, causal, out_dtype=torch.float32), want) <= 1e-5
+    s, m = fca.flash_colreduce_multi(q, k, ["sum", "max"], out_dtype=torch.float32)
+    assert torch.equal(s, m)
+    k[0, 1 % h, n // 2, 0] = float("nan")
+    s = fca.flash_colreduce(q, k, "sum", out_dtype=torch.float32)
+    assert s[0, 1 % h].isnan().all() and s.isnan().sum().item() == n
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_row_lse2_of_one_query_keeps_no_score_array(dtype):
     """The row statistics are a view of the row sweep's buffer, which has no room for the scores that one query's
