@@ -3065,6 +3065,17 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// one_query_merge over each aligned group of LPR lanes: the maximum first, then every sum is scaled once and the scaled ones
+// are added pairwise.
+template <int LPR>
+__device__ __forceinline__ void one_query_join(float& m, float& l) {
+  float mx = m;
+#pragma unroll
+  for (int d = 1; d < LPR; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+  l = group_sum<LPR>(l * fast_exp2(m - ((mx == kNegInf) ? 0.f : mx)));
+  m = mx;
+}
+
 // The elements of a 16-byte granule as floats.
 template <int DT>
 __device__ __forceinline__ void granule_floats(u32x4 v, float (&f)[DT == FCR_DTYPE_F32 ? 4 : 8]) {
@@ -3268,16 +3279,16 @@ __global__ __launch_bounds__(kOnePairThreads) void one_query_pair_kernel(const P
     if (row + 2 * kPass < p.N) load(va, row + 2 * kPass);
     take(vb, row + kPass);
   }
-  one_query_merge_wave(m, l);
+  // Merging the waves one after the other rescales and rounds the sum fifteen times.
+  one_query_join<64>(m, l);
   if (lane == 0) {
     wave_m[wave] = m;
     wave_l[wave] = l;
   }
   __syncthreads();
-  m = wave_m[0];
-  l = wave_l[0];
-#pragma unroll
-  for (int w = 1; w < kW; ++w) one_query_merge(m, l, wave_m[w], wave_l[w]);
+  m = wave_m[lane & (kW - 1)];
+  l = wave_l[lane & (kW - 1)];
+  one_query_join<kW>(m, l);
   if (tid == 0) p.lse[bh] = m + fast_log2(l);
   if (bh == 0 && tid == 0 && p.sync) *p.sync = 0u;
   const float ref = (m == kNegInf) ? 0.f : m, inv = 1.0f / l;   // as one_query_columns_kernel
