@@ -4876,8 +4876,8 @@ void launch_one_query_scores(bool once, const Params& p, const OneQueryPlan& o, 
 
 // Keys that a workgroup reads while the second launch of the other way would still be on its way to the device, 256 KiB, or, where
 // the pairs are a workgroup for at least every other CU and no second round, 1 MiB.  Per call, two launches and one, bf16 keys of 128:
-// 8 pairs of 512 9.2 -> 5.7 us, of 1024 9.5 -> 7.5, but of 2048 9.5, 11.0; 256 of 64 9.0 -> 5.6, of 512 9.5 -> 6.0, of 1024 14.7 both, of 2048
-// 24.8 -> 23.4, of 4096 46.6 -> 42.7, but of 8192 91.5, 95.5; 640 pairs of 512 17.2, 20.6, of 2048 58.1, 66.8.
+// 8 pairs of 512 8.1 -> 5.2 us, of 1024 8.5 -> 6.4, but of 2048 9.5, 11.0; 256 of 64 9.0 -> 5.6, of 512 9.5 -> 5.1, of 1024 14.7 both, of 2048
+// 24.8 -> 22.4, of 4096 46.6 -> 42.6, but of 8192 91.5, 95.5 (1024 and 64 of 256, and the losing ones, with a merge of the waves 0.5-1 us longer); 640 pairs of 512 17.2, 20.6, of 2048 58.1, 66.8.
 inline bool one_query_alone(const Params& p) {
   const int cus = chip_cus();
   const int64_t most = 2 * (int64_t)p.bh_count >= cus ? 1 << 20 : 256 << 10;
