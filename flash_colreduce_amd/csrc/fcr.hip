@@ -1056,8 +1056,10 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 // the waves' sums of the rows of the chunk before are added up, and what was kept of its scores, times the reciprocal, goes
 // to the columns; the chunk's own scores become 2^score (maxima keep the score itself), each wave's sum per row goes to LDS.
 // Sums are of 2^score itself.  One outside [2^-20, 2^100), which a NaN, an infinity, a row without a visible key and scores far from
-// zero all end in, is not used: the workgroup forms the chunk's scores again, row maximum first (`exact`; every wave reads the same
-// sums and so comes to the same conclusion).  A 2^score below 2^-126 counts as 0, a probability of 2^-106 at most.
+// zero all end in, is not used: the workgroup forms that chunk again, and the rest of its chunks once, row maximum first (`exact`; every
+// wave reads the same sums and so comes to the same conclusion).  Where every score is that far off, the two kernels -> this one, fp16
+// sums: 512 pairs of 512 x 512 x 128 81 -> 79 us, with the mask 77 -> 77, of 256 x 256 x 64 21 -> 18 and 18.4 -> 20.1 (the worst), 8 pairs of 8192 x
+// 512 x 128 88 -> 38; with every chunk formed both ways they took 145, 145, 31, 31 and 44.  A 2^score below 2^-126 counts as 0, a probability of 2^-106 at most.
 // The accumulators of hidden keys, those past N and those behind the mask, start at -inf.
 // The queries of a pair are dealt chunk by chunk to p.splits workgroups, which leave fp32 columns behind each other for
 // merge_columns_kernel (p.out, p.out2: [splits, BH, N]); one workgroup per pair stores the final form.
@@ -1212,14 +1214,11 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     const int row = CAUSAL ? max(0, k0[NG - 1] + 15 - p.c) : 0;   // first row that sees the wave's last key
     i_full = CAUSAL ? __builtin_amdgcn_readfirstlane(max(0, ((row + CR - 1) / CR - split + S - 1) / S)) : 0;
   }
-  // a wave's sums (maxima) per row, over its lanes
-  auto write_partials = [&](float* set, const float (&v)[SQ], auto max_tag) __attribute__((always_inline)) {
-    constexpr bool MAX = decltype(max_tag)::value;
+  // a wave's sums (maxima) per row, reduced over its lanes
+  auto write_reduced = [&](float* set, float x) __attribute__((always_inline)) {
     if constexpr (SQ == 1) {
-      const float x = lane_rows_reduce<MAX>(v);
       if (lane < 16) set[lane * NW + wave] = x;
     } else {
-      const float x = lane_rows_reduce<MAX>(v);
       if ((lane & 16) == 0) set[((lane >> 5) * 16 + (lane & 15)) * NW + wave] = x;
     }
   };
@@ -1268,87 +1267,117 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     for (int sq = 1; sq < SQ; ++sq) v = lane >> 4 == sq ? lse[sq] : v;
     if (lane < CR && q0 + lane < p.M) p.lse[(int64_t)bh * p.M + q0 + lane] = v;
   };
-  // Chunk i once more, for rows whose sum of 2^score is unusable: row maximum first.  Scaling a product and taking a maximum or the lse
-  // off rounds once, as in the two kernels: with two roundings the errors of such rows were up to 1.04 of theirs, now 0.98 at most.
-  auto exact = [&](int i) __attribute__((always_inline)) {
-    const char* stage = stage_of(i);
-    const int q0 = first_row(i), live = live_groups(q0);
-    f32x4 x[NG][SQ];
-    float part[SQ], w[SQ][NW], ref[SQ], lse[SQ], l[SQ];
+  // Chunk i for rows whose sums of 2^score are unusable: every wave takes its own maximum of a row first, and behind one barrier the
+  // waves' sums are brought to a common one.  Scaling a product and taking a maximum or the lse off rounds once, as in the two
+  // kernels.  Keys come with the sign of the scale, up = |scale|.
+  const float up = fabsf(p.scale2);
+  auto exact = [&](int i, auto masked_tag, auto barrier) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_tag)::value;   // some key is hidden from some row: of the last live group, or all from rows past M
+    const int q0 = first_row(i), live = MASKED ? live_groups(q0) : NG;
+    const bool tail = q0 + CR > p.M;
     int lane_again = lane;   // opaque: what follows from it is not to be kept in registers from chunk to chunk
     asm volatile("" : "+v"(lane_again));
-    auto seen = [&](int g, int sq, int r) __attribute__((always_inline)) {
-      const int key = k0[g] + 4 * (lane_again >> 4) + r, q = q0 + 16 * sq + (lane_again & 15);
-      return key < p.N && q < p.M && (!CAUSAL || key <= q + p.c);
-    };
+    // body(g, sq, seen) for every group in use; seen(r) is a question only in groups that are hidden in part, and there if it has to be
+    auto groups = [&](bool ask, auto body) __attribute__((always_inline)) {
 #pragma unroll
-    for (int sq = 0; sq < SQ; ++sq) part[sq] = kNegInf;
+      for (int g = 0; g < NG; ++g) {
+        if (g >= live) continue;
+        if (!MASKED || !ask || (g + 1 < live && !tail)) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      if (g >= live) continue;
+          for (int sq = 0; sq < SQ; ++sq) body(g, sq, [](int) { return true; });
+        } else {
 #pragma unroll
-      for (int sq = 0; sq < SQ; ++sq) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) acc = mma<DT>(kf[g][ks], rg.frag(stage, 0, sq, ks), acc);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          x[g][sq][r] = acc[r];
-          part[sq] = fmaxf(part[sq], seen(g, sq, r) ? acc[r] * p.scale2 : kNegInf);
+          for (int sq = 0; sq < SQ; ++sq) {
+            const int key = k0[g] + 4 * (lane_again >> 4), q = q0 + 16 * sq + (lane_again & 15);
+            const int lim = q >= p.M ? -1 : CAUSAL ? min(p.N - 1 - key, q + p.c - key) : p.N - 1 - key;
+            body(g, sq, [lim](int r) { return r <= lim; });
+          }
         }
       }
+    };
+    read_fragments(i);
+    f32x4 x[NG][SQ];   // products, hidden ones -inf; later (sums) 2^score relative to the wave's maximum
+    float most[SQ], part[SQ], factor[SQ], lse[SQ];
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) most[sq] = kNegInf, part[sq] = 0.f;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g >= live) continue;
+#pragma unroll
+      for (int sq = 0; sq < SQ; ++sq) x[g][sq] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int sq = 0; sq < SQ; ++sq) x[g][sq] = mma<DT>(kf[g][ks], f[sq][ks], x[g][sq]);
     }
-    write_partials(redo, part, std::true_type());
-    lds_barrier();
-    read_partials(redo, w);
+    groups(true, [&](int g, int sq, auto seen) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[g][sq][r] = seen(r) ? x[g][sq][r] : kNegInf;
+        most[sq] = fmaxf(most[sq], x[g][sq][r]);
+      }
+    });
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {   // the largest score; -inf if the row sees none of the wave's keys
+      const float m[1] = {most[sq] == kNegInf ? kNegInf : most[sq] * up};
+      most[sq] = lane_rows_reduce<true>(m);
+    }
+    groups(up == 0.f, [&](int g, int sq, auto seen) __attribute__((always_inline)) {   // (-inf times 0 is a NaN)
+      const float ref = most[sq] == kNegInf ? 0.f : most[sq];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {   // (+inf - inf is a NaN, as the row kernel's lse then is)
+        const float e = seen(r) ? fast_exp2(fmaf(x[g][sq][r], up, -ref)) : 0.f;
+        part[sq] += e;
+        if (MODE == kModeSum) x[g][sq][r] = e;
+      }
+    });
+    float* const set_m = redo + (i & 1) * kSums;
+    float* const set_l = sums + (i & 1) * kSums;
+    write_reduced(set_m, SQ == 1 || lane < 32 ? most[0] : most[SQ - 1]);
+    write_reduced(set_l, lane_rows_reduce<false>(part));
+    barrier();
+    // Each row of lanes takes its share of the waves.
+    constexpr int PW = NW / 4;
+    bool odd = up == 0.f;
 #pragma unroll
     for (int sq = 0; sq < SQ; ++sq) {
-      float m = w[sq][0];
+      const int at = (16 * sq + (lane & 15)) * NW + PW * (lane >> 4);
+      float wm[PW], wl[PW], m[1], l[1] = {0.f};
 #pragma unroll
-      for (int v = 1; v < NW; ++v) m = fmaxf(m, w[sq][v]);
-      ref[sq] = m == kNegInf ? 0.f : m;   // no visible key: any finite reference
-      part[sq] = 0.f;
+      for (int v = 0; v < PW; ++v) wm[v] = set_m[at + v], wl[v] = set_l[at + v];
+      m[0] = wm[0];
+#pragma unroll
+      for (int v = 1; v < PW; ++v) m[0] = fmaxf(m[0], wm[v]);
+      m[0] = lane_rows_reduce<true>(m);
+      const float ref = m[0] == kNegInf ? 0.f : m[0];
+#pragma unroll
+      for (int v = 0; v < PW; ++v) l[0] = fmaf(wl[v], fast_exp2(wm[v] - ref), l[0]);   // (a wave without a key: 0 times 0)
+      l[0] = lane_rows_reduce<false>(l);
+      lse[sq] = l[0] == 0.f ? kNegInf : ref + fast_log2(l[0]);
+      factor[sq] = (most[sq] == kNegInf ? 0.f : fast_exp2(most[sq] - ref)) * __builtin_amdgcn_rcpf(l[0]);
     }
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      if (g >= live) continue;
-#pragma unroll
-      for (int sq = 0; sq < SQ; ++sq)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)   // (+inf - inf is a NaN, as the row kernel's lse then is)
-          part[sq] += seen(g, sq, r) ? fast_exp2(fmaf(x[g][sq][r], p.scale2, -ref[sq])) : 0.f;
-    }
-    write_partials(redo + kSums, part, std::false_type());
-    lds_barrier();
-    read_partials(redo + kSums, w);
-    add_up(w, l);
-#pragma unroll
-    for (int sq = 0; sq < SQ; ++sq) lse[sq] = l[sq] == 0.f ? kNegInf : ref[sq] + fast_log2(l[sq]);
     if (wave == 0) store_lse(q0, lse);
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      if (g >= live) continue;
-#pragma unroll
-      for (int sq = 0; sq < SQ; ++sq)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float y = seen(g, sq, r) ? fmaf(x[g][sq][r], p.scale2, -lse[sq]) : kNegInf;
-          if (MODE != kModeMax) csum[g][r] += fast_exp2(y);
-          if (MODE != kModeSum) cmax[g][r] = fmaxf(cmax[g][r], y);
-        }
+    for (int sq = 0; sq < SQ; ++sq) {
+      if (MASKED && q0 + 16 * sq + (lane & 15) >= p.M) factor[sq] = 0.f, lse[sq] = kPosInf;
+      odd = odd || !(MODE == kModeSum ? factor[sq] < kPosInf : lse[sq] > kNegInf);   // a NaN, or a row whose scores are all -inf
     }
+    groups(__builtin_amdgcn_ballot_w64(odd) != 0, [&](int g, int sq, auto seen) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (MODE == kModeSum) {
+          csum[g][r] = seen(r) ? fmaf(x[g][sq][r], factor[sq], csum[g][r]) : csum[g][r];
+        } else {
+          const float y = seen(r) ? fmaf(x[g][sq][r], up, -lse[sq]) : kNegInf;
+          if (MODE == kModeBoth) csum[g][r] += fast_exp2(y);
+          cmax[g][r] = fmaxf(cmax[g][r], y);
+        }
+      }
+    });
   };
 
-  constexpr float kNothing = MODE == kModeSum ? 0.f : kNegInf;
   f32x4 s[NG][SQ];   // of the chunk whose columns are added up next: 2^score, or (maxima) the scaled score
-#pragma unroll
-  for (int g = 0; g < NG; ++g)
-#pragma unroll
-    for (int sq = 0; sq < SQ; ++sq) s[g][sq] = (f32x4){kNothing, kNothing, kNothing, kNothing};
-  // per row of that chunk: the reciprocal of its sum, or its lse; such that rows past M, and a chunk before the first, add nothing
-  float fact[SQ];
-#pragma unroll
-  for (int sq = 0; sq < SQ; ++sq) fact[sq] = MODE == kModeSum ? 0.f : kPosInf;
+  float fact[SQ];    // per row of that chunk: the reciprocal of its sum, or its lse; such that rows past M add nothing
   auto add_group = [&](int g) __attribute__((always_inline)) {
     if constexpr (MODE == kModeSum) {
 #pragma unroll
@@ -1378,10 +1407,9 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
 #pragma unroll
     for (int sq = 0; sq < SQ; ++sq) c[sq] = (f32x4){0.f, 0.f, 0.f, 0.f};
   };
-  auto enter = [&](int i) __attribute__((always_inline)) {
+  auto arrive = [&](int i) __attribute__((always_inline)) {
     ring_sync<(NS - 4) * Rg::kPer>();   // chunk i + 1 is there, the sums of chunk i - 1 are
     issue(i + NS - 2);
-    if (i == 0) read_fragments(0);
   };
   // What the rows of chunk i contribute with, into `fact`; whether a row's sum is unusable (the same in every wave).
   auto row_facts = [&](int i, float (&l)[SQ]) __attribute__((always_inline)) {
@@ -1416,11 +1444,12 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
       }
   };
 
-  int i = 0;
-  // chunks that some key of the wave is hidden from, and the one behind them (whose predecessor's groups are not all in use)
-#pragma unroll 1
-  for (; i < chunks && i_full > 0 && i <= i_full; ++i) {
-    enter(i);
+  // Chunk i: its scores and their exponents, and, unless it is the first of a run, the columns of the chunk before between the two.
+  // Returns without the exponents if a row of that one is unusable (the same in every wave).
+  // A chunk that some key of the wave is hidden from, or the one behind them (whose predecessor's groups are not all in use):
+  auto some_hidden = [&](int i) __attribute__((always_inline)) {
+    arrive(i);
+    if (__builtin_expect(i == 0, 0)) read_fragments(0);
     const int q0 = first_row(i), live = live_groups(q0), in_use = (live + GP - 1) / GP;
     int lane_again = lane;
     asm volatile("" : "+v"(lane_again));
@@ -1441,14 +1470,11 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     };
     batch(0);
     if (NBT > 1) batch(1);
-    if (i > 0) {
+    if (__builtin_expect(i > 0, 1)) {
       float l[SQ];
-      if (row_facts(i - 1, l)) {
-        exact(i - 1);
-      } else {
-        add_batches();
-        lse_of(i - 1, l);
-      }
+      if (__builtin_expect(row_facts(i - 1, l), 0)) return false;
+      add_batches();
+      lse_of(i - 1, l);
     }
     float part[SQ];
 #pragma unroll
@@ -1458,32 +1484,24 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
       if (bt < in_use) {
 #pragma unroll
         for (int e = 0; e < GP; ++e) exponents(t[bt & 1][e], s[bt * GP + e], part);
-      } else {
-#pragma unroll
-        for (int e = 0; e < GP; ++e)
-#pragma unroll
-          for (int sq = 0; sq < SQ; ++sq) s[bt * GP + e][sq] = (f32x4){kNothing, kNothing, kNothing, kNothing};
       }
       if (bt + 2 < NBT) batch(bt + 2);
     }
     read_fragments(i + 1);
-    write_partials(sums + (i & 1) * kSums, part, std::false_type());
+    write_reduced(sums + (i & 1) * kSums, lane_rows_reduce<false>(part));
     batches = in_use;
-  }
-  // The others, without branches but for rows whose sums are unusable: the columns of chunk i - 1 are added up, and the exponents of
-  // each group of chunk i taken, under the matrix instructions of the groups behind it.
-#pragma unroll 1
-  for (; i < chunks; ++i) {
-    enter(i);
+    return true;
+  };
+  // The others, without branches but for such rows: the columns of chunk i - 1 are added up, and the exponents of each group of chunk i
+  // taken, under the matrix instructions of the groups behind it.
+  auto all_visible = [&](int i) __attribute__((always_inline)) {
+    arrive(i);
+    if (__builtin_expect(i == 0, 0)) read_fragments(0);
     scores(0, visible);
     if (NBT > 1) scores(1, visible);
-    float l[SQ];
-    bool bad = i == 0;
-    if (i > 0) {
-      bad = row_facts(i - 1, l);
-      if (bad) exact(i - 1);
-    }
-    if (!bad) {
+    if (__builtin_expect(i > 0, 1)) {
+      float l[SQ];
+      if (__builtin_expect(row_facts(i - 1, l), 0)) return false;
 #pragma unroll
       for (int g = 0; g < NG; ++g) add_group(g);
       lse_of(i - 1, l);
@@ -1498,43 +1516,87 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
       if (bt + 2 < NBT) scores(bt + 2, visible);
       if (bt + 3 == NBT || (NBT < 3 && bt == 0)) read_fragments(i + 1);
     }
-    write_partials(sums + (i & 1) * kSums, part, std::false_type());
-  }
-  ring_sync<0>();   // (and the loads past the last chunk have written their zeros)
-  float l[SQ];
-  if (row_facts(chunks - 1, l)) {
-    exact(chunks - 1);
-  } else {
-#pragma unroll
-    for (int g = 0; g < NG; ++g) add_group(g);
-    lse_of(chunks - 1, l);
-  }
+    write_reduced(sums + (i & 1) * kSums, lane_rows_reduce<false>(part));
+    return true;
+  };
 
+  constexpr int kCalm = 2;
   // Columns: a reduce-scatter over the 16 query lanes, 16 values (four groups) at a time; lane l ends up with group (l & 15) / 4,
   // key 4 * (l / 16) + (l & 3) of it.
-  Params mine = p;
-  if (S > 1) {
-    const int64_t at = (int64_t)split * p.bh_count * p.N * 4;
-    mine.out = static_cast<char*>(p.out) + at;
-    mine.out2 = static_cast<char*>(p.out2) + at;
+  auto store_columns = [&]() __attribute__((always_inline)) {
+    Params mine = p;
+    if (S > 1) {
+      const int64_t at = (int64_t)split * p.bh_count * p.N * 4;
+      mine.out = static_cast<char*>(p.out) + at;
+      mine.out2 = static_cast<char*>(p.out2) + at;
+    }
+    const int r = lane & 3;
+#pragma unroll
+    for (int g4 = 0; g4 < NG; g4 += 4) {
+      const int grp = g4 + ((lane & 15) >> 2);
+      const int key = 16 * (wave + NW * grp) + 4 * (lane >> 4) + r;
+      f32x4 c4[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) c4[g] = g4 + g < NG ? csum[(g4 + g) % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
+      const float sum = MODE != kModeMax ? lanes16_scatter<false>(c4, lane) : 0.f;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) c4[g] = g4 + g < NG ? cmax[(g4 + g) % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
+      const float most = MODE != kModeSum ? lanes16_scatter<true>(c4, lane) : 0.f;
+      if (grp < NG && key < p.N) {
+        if (MODE != kModeMax) store_column(mine, mine.out, true, bh, key, sum);
+        if (MODE != kModeSum) store_column(mine, MODE == kModeBoth ? mine.out2 : mine.out, false, bh, key, fast_exp2(most));
+      }
+    }
+  };
+
+  int i = 0;
+  bool usable = true;
+#pragma unroll 1
+  for (; i < chunks && i_full > 0 && i <= i_full; ++i) {
+    usable = some_hidden(i);
+    if (__builtin_expect(!usable, 0)) break;
   }
-  const int r = lane & 3;
-#pragma unroll
-  for (int g4 = 0; g4 < NG; g4 += 4) {
-    const int grp = g4 + ((lane & 15) >> 2);
-    const int key = 16 * (wave + NW * grp) + 4 * (lane >> 4) + r;
-    f32x4 c4[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) c4[g] = g4 + g < NG ? csum[(g4 + g) % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
-    const float sum = MODE != kModeMax ? lanes16_scatter<false>(c4, lane) : 0.f;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) c4[g] = g4 + g < NG ? cmax[(g4 + g) % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
-    const float most = MODE != kModeSum ? lanes16_scatter<true>(c4, lane) : 0.f;
-    if (grp < NG && key < p.N) {
-      if (MODE != kModeMax) store_column(mine, mine.out, true, bh, key, sum);
-      if (MODE != kModeSum) store_column(mine, MODE == kModeBoth ? mine.out2 : mine.out, false, bh, key, fast_exp2(most));
+  if (__builtin_expect(usable, 1)) {
+#pragma unroll 1
+    for (; i < chunks; ++i) {
+      usable = all_visible(i);
+      if (__builtin_expect(!usable, 0)) break;
+      batches = NBT;
     }
   }
+  if (__builtin_expect(usable, 1)) {
+    ring_sync<0>();   // (and the loads past the last chunk have written their zeros)
+    float l[SQ];
+    usable = !row_facts(chunks - 1, l);
+    if (__builtin_expect(usable, 1)) {
+      add_batches();
+      lse_of(chunks - 1, l);
+      store_columns();
+      return;
+    }
+  }
+  // Chunk i - 1 has such a row.  It and all that follow are done the other way at once, formed once, behind one barrier each, the one that
+  // the next chunk is there after.  (Back to the usual way after a few chunks without one was built; the loops above then keep
+  // less in registers and lose 2-6 %.)
+  lds_barrier();   // (everybody has read the plain sums, whose place is used again)
+  if (p.scale2 < 0.f) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[g][ks] ^= (u32x4){0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+  }
+  int at = i - 1;
+  auto next_is_there = [&]() __attribute__((always_inline)) {
+    if (at < i && i < chunks) lds_barrier();   // chunk i has been waited for
+    else if (at + 1 < chunks) arrive(at + 1);
+    else ring_sync<0>();
+  };
+#pragma unroll 1
+  do {
+    if (at < i_full || first_row(at) + CR > p.M) exact(at, std::true_type(), next_is_there);
+    else exact(at, std::false_type(), next_is_there);
+  } while (++at < chunks);
+  store_columns();
 }
 
 // out = the sums or maxima of p.splits columns that lie BH * N apart at p.part (both: maxima p.splits * BH * N behind the sums).

@@ -1783,6 +1783,35 @@ def test_few_keys_far_scores_round_once(dtype, level):
     assert all(now <= 1.003 * two for now, two in zip(err[1], err[0])), err
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d,scale", [(2, 100, 100, 64, None), (300, 97, 130, 128, None), (3, 300, 256, 96, -0.1), (300, 70, 512, 64, None),
+                                           (2, 1000, 300, 128, None), (2, 65, 250, 256, None), (260, 49, 120, 192, -0.07)])
+def test_few_keys_from_a_far_row_on(h, m, n, d, scale, causal):
+    """Rows whose scores lie around -30, which the plain sums do not take, from the first row on, from one inside a chunk, from the first of a chunk,
+    in the last row only and in one row alone: what is left of a workgroup's chunks is then formed the other way.  Scores of magnitude
+    2^6 are rounded to 2^-18, those of products of 30 * sqrt(d) in fp32 sums to about the same: 2e-5 in the norm holds both."""
+    g = torch.Generator(device="cuda").manual_seed(h + m + d)
+    q0, k = (torch.randn(1, h, r, d, device="cuda", generator=g) for r in (m, n))
+    o = torch.randn(1, h, 1, d, device="cuda", generator=g)
+    o *= (30 / (d ** -0.5 if scale is None else -scale)) ** 0.5 / o.norm(dim=-1, keepdim=True)
+    if scale is not None:
+        k = -k
+    k = k - o if scale is None else k + o
+    k = k.half()
+    for rows in (slice(0, m), slice(m // 2, m), slice(m // 3, m // 3 + 1), slice(32, 64), slice(m - 1, m)):
+        q = q0.clone()
+        q[:, :, rows] += o if scale is None else -o
+        q = q.half()
+        sums, most = _columns_f64(q, k, causal, scale)
+        got = [fca.flash_colreduce(q, k, red, causal, scale, out_dtype=torch.float32) for red in ("sum", "max")]
+        both = fca.flash_colreduce_multi(q, k, ["sum", "max"], causal, scale, out_dtype=torch.float32)
+        for x, want in ((got[0], sums), (got[1], most), (both[0], sums), (both[1], most)):
+            assert _rel(x, want) <= 2e-5, rows
+        ws, out = torch.empty(_lib_workspace(q, k), device="cuda"), torch.empty(h, n, device="cuda")
+        _ws_call(q, k, out, ws, causal, scale)
+        torch.testing.assert_close(ws[: h * m].view(1, h, m), fca.row_lse2(q, k, causal, scale), rtol=1e-5, atol=1e-5)
+
+
 def test_few_keys_under_graph_capture():
     """Shared pairs (two launches) in a captured graph, replayed with other contents and eager calls between."""
     q, k = (torch.randn(1, 4, r, 64, device="cuda").half() for r in (300, 200))
