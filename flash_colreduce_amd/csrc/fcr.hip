@@ -1055,11 +1055,13 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 // sees all of its keys, so a score is formed once and its row's sum is a matter of the workgroup.  Per chunk and behind one barrier:
 // the waves' sums of the rows of the chunk before are added up, and what was kept of its scores, times the reciprocal, goes
 // to the columns; the chunk's own scores become 2^score (maxima keep the score itself), each wave's sum per row goes to LDS.
-// Sums are of 2^score itself.  One outside [2^-20, 2^100), which a NaN, an infinity, a row without a visible key and scores far from
+// Sums are of 2^score itself.  One outside [1, 2^100), which a NaN, an infinity, a row without a visible key and scores far from
 // zero all end in, is not used: the workgroup forms that chunk again, and the rest of its chunks once, row maximum first (`exact`; every
 // wave reads the same sums and so comes to the same conclusion).  Where every score is that far off, the two kernels -> this one, fp16
 // sums: 512 pairs of 512 x 512 x 128 81 -> 79 us, with the mask 77 -> 77, of 256 x 256 x 64 21 -> 18 and 18.4 -> 20.1 (the worst), 8 pairs of 8192 x
-// 512 x 128 88 -> 38; with every chunk formed both ways they took 145, 145, 31, 31 and 44.  A 2^score below 2^-126 counts as 0, a probability of 2^-106 at most.
+// 512 x 128 88 -> 38; with every chunk formed both ways they took 145, 145, 31, 31 and 44.
+// A 2^score below 2^-126 is 0, which is a probability below 2^-126 if the row's sum is 1 or more.  So sums below 1 are good only in chunks
+// whose first row sees less than 64 keys, where they are common, and there a wave that finds such a 2^score makes its sum a NaN.
 // The accumulators of hidden keys, those past N and those behind the mask, start at -inf.
 // The queries of a pair are dealt chunk by chunk to p.splits workgroups, which leave fp32 columns behind each other for
 // merge_columns_kernel (p.out, p.out2: [splits, BH, N]); one workgroup per pair stores the final form.
@@ -1411,6 +1413,30 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     ring_sync<(NS - 4) * Rg::kPer>();   // chunk i + 1 is there, the sums of chunk i - 1 are
     issue(i + NS - 2);
   };
+  // some row of chunk i sees less than 64 keys
+  auto few_seen = [&](int i) __attribute__((always_inline)) { return (CAUSAL ? first_row(i) + p.c + 1 : p.N) < 64; };
+  // The wave's sums of chunk i to LDS.  (A minimum per score, of numbers that are not negative, in the first chunk behind the mask: 0.1 to 0.15 us
+  // of a call.  In every chunk it cost 2-4 %.)
+  auto write_sums = [&](int i, int live, const float (&v)[SQ]) __attribute__((always_inline)) {
+    float x = lane_rows_reduce<false>(v);
+    if (MODE == kModeSum && __builtin_expect(few_seen(i) && live > 0 && __builtin_amdgcn_ballot_w64(x < 1.f) != 0, 0)) {
+      uint32_t smallest = 0x3f800000u;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        if (g >= live) continue;
+        const int key = k0[g] + 4 * (lane >> 4);
+#pragma unroll
+        for (int sq = 0; sq < SQ; ++sq) {
+          int lim = p.N - 1 - key;
+          if (CAUSAL) lim = min(lim, first_row(i) + 16 * sq + (lane & 15) + p.c - key);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) smallest = min(smallest, r <= lim ? __builtin_bit_cast(uint32_t, s[g][sq][r]) : 0x3f800000u);
+        }
+      }
+      if (__builtin_amdgcn_ballot_w64(smallest < 0x00800000u) != 0) x = __builtin_nanf("");
+    }
+    write_reduced(sums + (i & 1) * kSums, x);
+  };
   // What the rows of chunk i contribute with, into `fact`; whether a row's sum is unusable (the same in every wave).
   auto row_facts = [&](int i, float (&l)[SQ]) __attribute__((always_inline)) {
     const int q0 = first_row(i);
@@ -1418,9 +1444,10 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     read_partials(sums + (i & 1) * kSums, w);
     add_up(w, l);
     bool good = true;
+    const float least = MODE != kModeSum || few_seen(i) ? 9.5367432e-7f : 1.f;   // (maxima take a logarithm off the score)
 #pragma unroll
     for (int sq = 0; sq < SQ; ++sq) {
-      good = good && l[sq] >= 9.5367432e-7f && l[sq] < 1.2676506e30f;
+      good = good && l[sq] >= least && l[sq] < 1.2676506e30f;
       const bool row = q0 + 16 * sq + (lane & 15) < p.M;
       if (MODE == kModeSum) fact[sq] = row ? __builtin_amdgcn_rcpf(l[sq]) : 0.f;
       else fact[sq] = row ? log2_of_sum(l[sq]) : kPosInf;
@@ -1488,7 +1515,7 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
       if (bt + 2 < NBT) batch(bt + 2);
     }
     read_fragments(i + 1);
-    write_reduced(sums + (i & 1) * kSums, lane_rows_reduce<false>(part));
+    write_sums(i, live, part);
     batches = in_use;
     return true;
   };
@@ -1516,7 +1543,7 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
       if (bt + 2 < NBT) scores(bt + 2, visible);
       if (bt + 3 == NBT || (NBT < 3 && bt == 0)) read_fragments(i + 1);
     }
-    write_reduced(sums + (i & 1) * kSums, lane_rows_reduce<false>(part));
+    write_reduced(sums + (i & 1) * kSums, lane_rows_reduce<false>(part));   // (a wave's last key is past the 64th: no few_seen chunk)
     return true;
   };
 

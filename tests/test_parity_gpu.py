@@ -1812,6 +1812,27 @@ def test_few_keys_from_a_far_row_on(h, m, n, d, scale, causal):
         torch.testing.assert_close(ws[: h * m].view(1, h, m), fca.row_lse2(q, k, causal, scale), rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("m,n,d", [(40, 40, 64), (20, 200, 128), (33, 250, 256), (16, 500, 64)])
+def test_few_keys_small_probabilities_of_small_sums(m, n, d, causal):
+    """Rows whose sum of 2^score is between 2^-20 and 1 with keys whose 2^score fp32 cannot hold, though their probabilities of 2^-118 to
+    2^-126 it can: bf16 and fp32 results keep them, as the two kernels do.  The exponents are integers here and the sums short, so a
+    probability is good to the rounding of an lse of magnitude 2^3 and of a score of 2^7 (2^-18 together)."""
+    q = torch.zeros(1, 3, m, d, device="cuda", dtype=torch.float16)
+    k = torch.zeros(1, 3, n, d, device="cuda", dtype=torch.float16)
+    q[..., 0] = 1
+    k[..., 0] = -math.floor(math.log2(n)) - 4        # 2^-4 to 2^-3 in a row that sees every key
+    k[:, :, 1::7, 0] = -126 - torch.arange(1, 4, device="cuda").repeat(n)[: len(range(1, n, 7))].half()
+    want, most = _columns_f64(q, k, causal, math.log(2))
+    assert ((want > 0) & (want < 2.0 ** -110)).any()
+    got = fca.flash_colreduce(q, k, "sum", causal, math.log(2), out_dtype=torch.float32)
+    two = fca.flash_colreduce_multi(q, k, ["sum", "max"], causal, math.log(2), out_dtype=torch.float32)
+    for x, y in ((got, want), (two[0], want), (two[1], most)):
+        assert ((x.double() - y).abs() <= 2.0 ** -17 * y).all(), ((x.double() - y) / y).abs().max()
+    low = fca.flash_colreduce(q.bfloat16(), k.bfloat16(), "sum", causal, math.log(2))
+    assert ((low.double() - want).abs() <= 2.0 ** -8 * want).all()
+
+
 def test_few_keys_under_graph_capture():
     """Shared pairs (two launches) in a captured graph, replayed with other contents and eager calls between."""
     q, k = (torch.randn(1, 4, r, 64, device="cuda").half() for r in (300, 200))
