@@ -1414,7 +1414,7 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     issue(i + NS - 2);
   };
   // some row of chunk i sees less than 64 keys
-  auto few_seen = [&](int i) __attribute__((always_inline)) { return (CAUSAL ? first_row(i) + p.c + 1 : p.N) < 64; };
+  auto few_seen = [&](int i) __attribute__((always_inline)) { return (CAUSAL ? min(p.N, first_row(i) + p.c + 1) : p.N) < 64; };
   // The wave's sums of chunk i to LDS.  (A minimum per score, of numbers that are not negative, in the first chunk behind the mask: 0.1 to 0.15 us
   // of a call.  In every chunk it cost 2-4 %.)
   auto write_sums = [&](int i, int live, const float (&v)[SQ]) __attribute__((always_inline)) {
