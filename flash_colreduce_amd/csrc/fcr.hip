@@ -4550,19 +4550,21 @@ OneQueryPlan one_query_plan(int dtype, int64_t bh, int N, int D, int64_t base_fl
   return o;
 }
 
-// The path for pairs whose keys fit the registers of a workgroup (few_keys_kernel): up to 512 16-bit keys of 128, 256 of 256.  It won
-// 190 of 200 shapes of 2 to 512 pairs, 2 to 8192 queries and 64 to 512 keys against the two kernels, by 1.05 to 2.4 times (6.8 where
-// few keys meet thousands of queries).  Not taken, with the mask and more than 256 keys (eight waves, one workgroup per CU, whose half of
-// the triangle is paid for with whole chunks): where two or three workgroups share a pair (128 pairs of 512 x 512 x 128 19.5 us, 23.0
-// here) and in several rounds of short rows (512 pairs of 300 x 300 x 64 26.8, 28.3); nor there, mask or not, for sums and maxima
-// together unless at least four share a pair (128 pairs of 512 x 512 x 128 23.9, 27.7; 512 of 300 x 300 x 64 36.5, 37.7).
+// The path for pairs whose keys fit the registers of a workgroup (few_keys_kernel): up to 512 16-bit keys of 128, 256 of 256.  Against
+// the two kernels, 11000 shapes of 1 to 1500 pairs, 2 to 8192 queries, 2 to 512 keys, all reductions, with and without the mask: 0.56 of their
+// time where one launch does (below), 0.74 elsewhere.  Not taken for more than 128 keys where no two workgroups share a pair, sixteen chunks
+// or more are done one behind the other (48 with at most 256 keys) and neither the pairs fill the chip nor the keys the registers (`filled`):
+// two kernels -> here, 300 pairs of 5970 x 384 x 64, maxima, 262 -> 458 us, 257 of 4715 x 141 x 8 82 -> 153, 300 of 1831 x 400 x 96, both, 140 -> 205;
+// nor for more than 256 keys of 64 bytes in such calls, whose time is the vector port's in both (1024 pairs of 2172 x 428 x 8, maxima, 215 -> 315).
+// What that leaves out (526 shapes) takes 1.15 times as long here; of the others 2 % lose 3 % or more, most of them rows of 64 bytes against at
+// most 128 keys.
 // form -1: the other paths.
 struct FewKeysPlan {
   int form;          // keys of a workgroup: 128 << form
   int splits;        // workgroups per pair
   int64_t part_at, floats;   // where the columns of the splits start and the workspace ends, in floats
 };
-FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool both, bool causal, int64_t base_floats) {
+FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool both, int64_t base_floats) {
   FewKeysPlan o;
   o.form = -1;
   o.splits = 1;
@@ -4578,17 +4580,27 @@ FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool bot
   const int waves = form == most ? 8 : 4;
   const int rows = 16 * few_keys_queries(ks);
   const int64_t chunks = ((int64_t)M + rows - 1) / rows;
-  int64_t s = (waves == 8 ? 1 : 2) * (int64_t)chip_cus() / bh;
+  const int64_t places = (waves == 8 ? 1 : 2) * (int64_t)chip_cus();
+  int64_t s = places / bh;
   if (s > chunks) s = chunks;
   if (s < 1) s = 1;
   // A few chunks go to one workgroup, whose launch is then the only one: 2 pairs of 64 x 64 x 128 8.8 -> 5.0 us per call, of 128 x 128 8.8 -> 6.1,
   // of 160 x 160 8.9 -> 8.4, but of 200 x 200 8.9 -> 11.0; rows of 512 bytes 100 x 100 8.8 -> 8.3, 128 x 128 8.7 -> 9.1; more than 256 keys
-  // 96 x 500 x 64 8.9 -> 7.8, 128 x 500 x 128 10.4 -> 11.2.
+  // 96 x 500 x 64 8.9 -> 7.8, 128 x 500 x 128 10.4 -> 11.2.  (3840 shapes of all reductions, masks and up to 1500 pairs: two were slower.)
   if (chunks <= (form == 2 ? 3 : ks > 4 ? 7 : 5)) {
     s = 1;
-  } else if (N > 256 && s < 4 && (both || (causal && (s > 1 || (ks <= 2 && bh > chip_cus()))))) {
-    o.form = -1;
-    return o;
+  } else if (s == 1) {
+    // chunks one behind the other, and the share of the chip's workgroups and of their keys that is there
+    const int64_t rounds = (bh + places - 1) / places, steps = rounds * chunks;
+    const double filled = (double)bh / (double)(rounds * places) * N / (128 << form);
+    const bool many = steps >= 48;
+    double least = 0.0;
+    if (form == 2) least = steps < 16 ? 0.0 : ks == 1 ? 2.0 : ks == 2 ? (many ? 0.7 : 0.6) : many ? 0.5 : 0.4;
+    else if (form == 1 && many) least = ks == 1 ? 0.6 : ks > 4 ? 0.45 : 0.0;
+    if (filled < least) {
+      o.form = -1;
+      return o;
+    }
   }
   o.splits = (int)s;
   if (s > 1) {
@@ -5366,7 +5378,7 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
     }
   }
   if (single && ws_bytes != 0) {
-    const FewKeysPlan o = few_keys_plan(dtype, B, H, M, N, D, mode == kModeBoth, causal != 0, (int64_t)(lse_bytes / sizeof(float)));
+    const FewKeysPlan o = few_keys_plan(dtype, B, H, M, N, D, mode == kModeBoth, (int64_t)(lse_bytes / sizeof(float)));
     // (the keys of a pair are read through one view: all rows of a workgroup below 2 GiB)
     if (o.form >= 0 && (size_t)o.floats * sizeof(float) <= ws_bytes && ((int64_t)128 << o.form) * p.k_sr <= 0x7fffffff)
       return launch_few_keys(p, dtype, ksteps, o, ws, mode, causal != 0, static_cast<hipStream_t>(stream));
@@ -5491,8 +5503,7 @@ size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D) {
     return (size_t)one_query_plan(dtype, (int64_t)B * H, N, D, (int64_t)(base / sizeof(float))).floats * sizeof(float);
   if (row_width_ok(dtype, D)) {
     const int64_t floats = (int64_t)(base / sizeof(float));
-    const FewKeysPlan one = few_keys_plan(dtype, B, H, M, N, D, false, false, floats), both = few_keys_plan(dtype, B, H, M, N, D, true, false, floats);
-    int64_t most = one.floats > both.floats ? one.floats : both.floats;
+    int64_t most = few_keys_plan(dtype, B, H, M, N, D, true, floats).floats;   // (one result takes half of it)
     FusedPlan f;
     if (dtype != FCR_DTYPE_F32 && ksteps_of(dtype, D) <= 4 && fused_shape((int64_t)B * H, M, N, f)) {
       const FusedPairPlan two = fused_pair_plan((int64_t)B * H, M, N, f);

@@ -1681,7 +1681,10 @@ def _rel(got, want):
     (300, 17, 127, 128, torch.float16), (5, 300, 256, 128, torch.float16), (260, 70, 250, 96, torch.bfloat16), (2, 257, 257, 64, torch.float16),
     (20, 512, 512, 128, torch.bfloat16), (140, 100, 511, 128, torch.float16), (70, 320, 300, 40, torch.float16), (300, 40, 512, 32, torch.float16),
     (2, 5000, 200, 128, torch.float16), (3, 100, 256, 256, torch.bfloat16), (260, 33, 130, 192, torch.float16), (4, 65, 257, 256, torch.float16),
-    (4, 90, 513, 128, torch.float16), (64, 1, 200, 128, torch.float16), (300, 15, 16, 136, torch.bfloat16)])
+    (4, 90, 513, 128, torch.float16), (64, 1, 200, 128, torch.float16), (300, 15, 16, 136, torch.bfloat16),
+    # long calls on both sides of the line that leaves them to the two kernels
+    (150, 255, 300, 64, torch.float16), (150, 257, 300, 64, torch.float16), (256, 500, 500, 64, torch.bfloat16), (70, 520, 300, 32, torch.float16),
+    (160, 1500, 141, 8, torch.float16), (160, 1537, 141, 8, torch.bfloat16), (150, 790, 400, 96, torch.float16), (70, 1000, 3, 64, torch.float16)])
 def test_few_keys(h, m, n, d, dtype, causal):
     """Pairs whose keys fit a workgroup's registers: sums, maxima, both at once and the row statistics, against 64 bits.  A score of
     magnitude 2^4 is rounded to 2^-20, so a probability is good to 2^-19 and a few 1e-6 in the norm; 1e-5 leaves room for
