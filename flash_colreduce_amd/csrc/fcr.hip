@@ -4977,13 +4977,18 @@ void launch_one_query_scores(bool once, const Params& p, const OneQueryPlan& o, 
 }
 
 // Keys that a workgroup reads while the second launch of the other way would still be on its way to the device, 256 KiB, or, where
-// the pairs are a workgroup for at least every other CU and no second round, 1 MiB.  Per call, two launches and one, bf16 keys of 128:
-// 8 pairs of 512 8.1 -> 5.2 us, of 1024 8.5 -> 6.4, but of 2048 9.5, 11.0; 256 of 64 9.0 -> 5.6, of 512 9.5 -> 5.1, of 1024 14.7 both, of 2048
-// 24.8 -> 22.4, of 4096 46.6 -> 42.6, but of 8192 91.5, 95.5 (1024 and 64 of 256, and the losing ones, with a merge of the waves 0.5-1 us longer); 640 pairs of 512 17.2, 20.6, of 2048 58.1, 66.8.
-inline bool one_query_alone(const Params& p) {
+// the pairs are a workgroup for at least every other CU and no second round, 1 MiB.  us per call, two launches and one, bf16 keys of 128,
+// calls queued behind each other: 8 pairs of 512 6.7, 4.8, of 1024 7.0, 6.5, but of 2048 7.0, 10.1; 100 of 1024 10.3, 6.8; 256 of 64 6.5, 3.7, of
+// 512 10.4, 5.3, of 1024 15.5, 13.7, of 2048 25.1, 21.9, of 4096 46.4, 41.1, but of 8192 91.0, 94.5; 640 pairs of 512 17.8, 18.6.
+// A load spans `lanes` granules whatever the row holds of them, and a few pairs wait for nothing but their loads: there rows of 17
+// granules in 32 lanes count as 32 (keys of 136: 1 pair of 764 6.5, 8.1, 4 of 938 7.0, 9.4, 24 of 960 7.8, 9.6; of 320: 4 of 377 6.8, 8.8).
+inline bool one_query_alone(const Params& p, int lanes) {
   const int cus = chip_cus();
-  const int64_t most = 2 * (int64_t)p.bh_count >= cus ? 1 << 20 : 256 << 10;
-  return p.bh_count <= cus && p.N <= kOnePairKeys && (int64_t)p.N * p.dgran * 16 <= most;
+  if (p.bh_count > cus || p.N > kOnePairKeys) return false;
+  const int64_t bytes = (int64_t)p.N * p.dgran * 16, loaded = (int64_t)p.N * lanes * 16;
+  if (2 * (int64_t)p.bh_count >= cus) return bytes <= 1 << 20;
+  const int64_t most = 16 * (int64_t)p.bh_count < cus ? 256 << 10 : 4 * (int64_t)p.bh_count < cus ? 384 << 10 : 512 << 10;
+  return bytes <= 256 << 10 && loaded <= most;
 }
 
 template <int DT>
@@ -5001,7 +5006,7 @@ void launch_one_query_pair(const Params& p, int lanes, int mode, hipStream_t s) 
 }
 
 int launch_one_query(Params& p, int dtype, const OneQueryPlan& o, float* ws, int mode, hipStream_t s) {
-  if (one_query_alone(p)) {
+  if (one_query_alone(p, o.lanes)) {
     if (dtype == FCR_DTYPE_F16) launch_one_query_pair<FCR_DTYPE_F16>(p, o.lanes, mode, s);
     else if (dtype == FCR_DTYPE_BF16) launch_one_query_pair<FCR_DTYPE_BF16>(p, o.lanes, mode, s);
     else launch_one_query_pair<FCR_DTYPE_F32>(p, o.lanes, mode, s);

@@ -755,7 +755,10 @@ def test_one_query_shared_keys(b, h, n, d, dtype, shared):
                                            (1, 130, 4097, 128, torch.float16), (4, 64, 500, 64, torch.float16), (1, 257, 500, 64, torch.float16),
                                            (1, 3, 8192, 8, torch.float16), (1, 3, 8193, 8, torch.float16), (2, 2, 33, 16, torch.bfloat16),
                                            (1, 5, 255, 256, torch.float32), (1, 5, 1, 72, torch.bfloat16), (2, 70, 700, 40, torch.float32),
-                                           (1, 2, 513, 512, torch.float16)])
+                                           (1, 2, 513, 512, torch.float16),
+                                           # rows that fill half of their lanes: few pairs, more, and a quarter of the chip's
+                                           (1, 4, 512, 136, torch.float16), (1, 4, 513, 136, torch.float16), (1, 20, 768, 136, torch.bfloat16),
+                                           (1, 20, 769, 136, torch.bfloat16), (1, 64, 963, 136, torch.float16), (1, 64, 964, 136, torch.float16)])
 def test_one_query_in_one_launch(b, h, n, d, dtype):
     """Against 64 bits: a probability is good to the rounding of its score (2^4: 2^-20) and of the sum."""
     g = torch.Generator(device="cuda").manual_seed(n + d)
