@@ -2476,7 +2476,7 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ 
   if (i == 0) *one = 0u;
 }
 
-// Eight waves, one workgroup per CU, eight steps per workgroup and pair.  Up to 64 queries (QH = 1, KH = 2):
+// Eight waves, one workgroup per CU, or four, two per CU; eight steps per workgroup and pair (sixteen with two query groups).  Up to 64 queries (QH = 1, KH = 2):
 // a step is two chunks of 64 keys, waves 0-3 take (and load) the first, waves 4-7 the second.  Up to 128
 // queries (QH = 2, KH = 1): a step is one chunk, waves 4-7 hold queries 64-127, waves 0-3 load.
 // NQ: groups of sixteen queries a wave holds (4; 2 for at most 32 queries: the registers then hold the scores of
@@ -2494,7 +2494,7 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ 
 template <int DT, int KS, bool CAUSAL, int MODE, int QH, int NQ, bool SKIP, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
   static_assert(NQ == 4 || (QH == 1 && NQ == 2), "fewer query groups only with one query half");
-  static_assert(NW == 8 || (NW == 4 && QH == 1), "four waves hold one query half");
+  static_assert(NW == 8 || (NW == 4 && NQ == 2), "four waves hold two query groups");
   constexpr int KG = kFusedSteps * (4 / NQ);     // steps per pair
   constexpr int KH = NW == 4 ? 1 : 3 - QH;       // chunks per step
   // ring stages (chunks): 130 KiB or 98 KiB for 256-byte rows, 49 with four waves
@@ -4502,21 +4502,27 @@ bool fused_shape(int64_t bh, int M, int N, FusedPlan& f) {
   return true;
 }
 
-// The single sweep in workgroups of four waves, two per CU, for at most 64 queries in several rounds, where the caller's workspace
-// has room for their slots (they follow the status word of the form above).
+// The single sweep in workgroups of four waves, two per CU, for at most 32 queries in several rounds, where the caller's workspace
+// has room for their slots (they follow the status word of the form above).  The rule, over 1500 shapes of 2 to 32 queries, 1024 to 65536
+// keys and 4 to 1000 pairs in several rounds of eight waves, us per call of eight waves and of four: where eight waves keep four query groups
+// four waves won everywhere (484 shapes, 0.81: 300 pairs of 32 x 2045 x 32, maxima, 35.9, 22.1; 128 of 32 x 5001 x 128, both, 51.7, 41.4; 300 of 2 x 1024 x 128
+// 26.0, 21.6).  Where those keep two groups the rounds are the same, and what decides is the time between two sweeps against that of
+// the loads: rows of more than 128 bytes 0.96 (512 pairs of 32 x 16384 x 128 is one of them), of 128 bytes 1.00, of 64 bytes 1.04 (64 of
+// 31 x 15509 x 32 25.0, 28.6; 128 of 16 x 7672 x 32 23.9, 27.0); of 128 bytes and one eight-wave workgroup per pair, which exchanges nothing,
+// 1.05 (444 of 17 x 1313 x 64 25.8, 29.0).  The last two keep eight waves.
 struct FusedPairPlan {
-  int nq, splits, teams;   // teams 0: not this form
+  int splits, teams;   // teams 0: not this form
   int64_t part_at, floats;
 };
-FusedPairPlan fused_pair_plan(int64_t bh, int M, int N, const FusedPlan& f) {
-  FusedPairPlan o{f.nq, 0, 0, f.sync_at + 32, f.floats};
-  if (f.qh != 1 || f.nq != 2 || bh <= f.teams) return o;
+FusedPairPlan fused_pair_plan(int64_t bh, int M, int N, int ksteps, const FusedPlan& f) {
+  FusedPairPlan o{0, 0, f.sync_at + 32, f.floats};
+  if (M > 32 || bh <= f.teams || (f.nq == 2 && ksteps <= 2 && (ksteps == 1 || f.splits == 1))) return o;
   const int cap = 2 * chip_cus();
-  const int64_t nchunks = ((int64_t)N + kChunk - 1) / kChunk, chunks = kFusedSteps * (4 / o.nq), splits = (nchunks + chunks - 1) / chunks;
+  const int64_t nchunks = ((int64_t)N + kChunk - 1) / kChunk, chunks = kFusedSteps * 2, splits = (nchunks + chunks - 1) / chunks;
   if (splits > cap) return o;
   o.splits = (int)splits;
   o.teams = (int)((cap / splits) < bh ? cap / splits : bh);
-  o.floats = o.part_at + 2 * (2ll * o.teams * o.splits * 64);
+  o.floats = o.part_at + 2 * (2ll * o.teams * o.splits * 32);
   return o;
 }
 
@@ -4780,12 +4786,12 @@ void launch_col_fused_groups(const Params& p, bool causal, int m, hipStream_t s)
 }
 
 // mode: kModeSum, kModeMax or kModeBoth, + 4 for more than 64 queries, + 8 for two groups of sixteen queries
-// per wave, + 16 for four waves
+// per wave, + 16 for that in four waves
 template <int DT, int KS>
 void launch_col_fused(const Params& p, bool causal, int mode, hipStream_t s) {
   const int m = mode & 3;
   if (mode & 4) launch_col_fused_groups<DT, KS, 2, 4, 8>(p, causal, m, s);
-  else if (mode & 16) (mode & 8) ? launch_col_fused_groups<DT, KS, 1, 2, 4>(p, causal, m, s) : launch_col_fused_groups<DT, KS, 1, 4, 4>(p, causal, m, s);
+  else if (mode & 16) launch_col_fused_groups<DT, KS, 1, 2, 4>(p, causal, m, s);
   else if (mode & 8) launch_col_fused_groups<DT, KS, 1, 2, 8>(p, causal, m, s);
   else launch_col_fused_groups<DT, KS, 1, 4, 8>(p, causal, m, s);
 }
@@ -5300,7 +5306,7 @@ int fcr_pack_f32(const float* src, void* dst, int64_t rows, int D, int terms, in
 }
 
 namespace {
-// A single sweep expects the whole chip: its workgroups wait for each other, one per CU.  Two of them issued on
+// A single sweep expects the whole chip: its workgroups wait for each other, one of eight waves or two of four per CU.  Two of them issued on
 // different streams could be dispatched side by side, each holding CUs the other needs, until their bounded
 // waits run out.  So inside a process they are chained: a single sweep on another stream than the one before
 // first waits (on the GPU; the host never blocks) for an event recorded at the end of that stream.  Calls that
@@ -5396,13 +5402,13 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
     p.splits = f.splits;
     p.teams = f.teams;
     int form = (f.qh == 2 ? 4 : 0) | (f.nq == 2 ? 8 : 0), rows = f.qh == 2 ? 128 : 16 * f.nq;
-    const FusedPairPlan two = fused_pair_plan(p.bh_count, M, N, f);
+    const FusedPairPlan two = fused_pair_plan(p.bh_count, M, N, ksteps, f);
     if (two.teams > 0 && (size_t)two.floats * sizeof(float) <= ws_bytes) {
       p.part = ws + two.part_at;
       p.splits = two.splits;
       p.teams = two.teams;
-      form = 16 | (two.nq == 2 ? 8 : 0);
-      rows = 16 * two.nq;
+      form = 16;
+      rows = 32;
     }
     // the slots that the launch polls (one set of them for one round) and the status word start at zero
     const int words = (p.bh_count > p.teams ? 2 : 1) * p.teams * p.splits * rows * 2;
@@ -5511,7 +5517,7 @@ size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D) {
     int64_t most = few_keys_plan(dtype, B, H, M, N, D, true, floats).floats;   // (one result takes half of it)
     FusedPlan f;
     if (dtype != FCR_DTYPE_F32 && ksteps_of(dtype, D) <= 4 && fused_shape((int64_t)B * H, M, N, f)) {
-      const FusedPairPlan two = fused_pair_plan((int64_t)B * H, M, N, f);
+      const FusedPairPlan two = fused_pair_plan((int64_t)B * H, M, N, ksteps_of(dtype, D), f);
       if (two.floats > most) most = two.floats;
     }
     return (size_t)most * sizeof(float);

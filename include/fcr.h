@@ -250,7 +250,7 @@ int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, in
  * under a CU mask) stores NaN columns for that pair, sets a word in the workspace and goes on.
  * fcr_colreduce_status waits for the stream and returns FCR_E_WAIT if that happened in the last call that
  * used lse_ws with these sizes, 0 otherwise (also for problems that do not take the single sweep).
- * A single sweep fills the chip, one workgroup per CU, and two of them dispatched side by side would
+ * A single sweep fills the chip, one or two workgroups per CU, and two of them dispatched side by side would
  * starve each other until their waits run out.  Inside a process the library prevents that: a single
  * sweep issued on another stream than the previous one is made to wait on the GPU (an event recorded on
  * that stream, hipStreamWaitEvent on the new one; the host does not block, calls that stay on one stream

@@ -959,15 +959,21 @@ def test_single_sweep_bounded_wait():
     assert lib.fcr_set_option(7, 1) == -3 and lib.fcr_set_option(_lib.OPT_WAIT_POLLS, -1) == -3
 
 
-# pairs in several rounds, so that at most 32 queries take the workgroups of four waves (two per CU): one team member, several and many,
-# keys that fill no step, no batch and no chunk, both edges of the query groups
+# pairs in several rounds: at most 32 queries in workgroups of four waves (two per CU) where they are faster on 256 CUs (`four`), else of eight;
+# one workgroup per team (1024 keys), several and many, keys that fill no step, no batch and no chunk, both edges of the query groups
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("h,m,n,d,dtype", [(300, 20, 1100, 64, torch.float16), (60, 32, 5001, 128, torch.bfloat16), (520, 2, 1024, 40, torch.float16),
-                                           (20, 17, 20000, 96, torch.float16), (60, 33, 5001, 128, torch.float16), (150, 31, 2049, 128, torch.bfloat16)])
-def test_single_sweep_in_rounds(h, m, n, d, dtype, causal):
+@pytest.mark.parametrize("h,m,n,d,dtype,four", [
+    (300, 20, 1100, 64, torch.float16, False), (60, 32, 5001, 128, torch.bfloat16, True), (520, 2, 1024, 40, torch.float16, True),
+    (20, 17, 20000, 96, torch.float16, True), (60, 33, 5001, 128, torch.float16, False), (150, 31, 2049, 128, torch.bfloat16, True),
+    (128, 32, 8192, 128, torch.bfloat16, True), (128, 2, 4100, 96, torch.float16, True), (64, 16, 8191, 128, torch.float16, True),
+    (150, 17, 2048, 32, torch.bfloat16, True), (10, 31, 33000, 64, torch.float16, True), (32, 9, 16384, 32, torch.bfloat16, False)])
+def test_single_sweep_in_rounds(h, m, n, d, dtype, four, causal):
     """Against 64 bits (see test_few_keys for the bound), then scores far from zero, NaN rows and infinite keys against the two kernels."""
     from flash_colreduce_amd import _lib
     lib = _lib.load()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:   # the slots of that form need room behind what every form needs
+        code = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}[dtype]
+        assert (lib.fcr_workspace_bytes(code, 2, h, m, n, d) > lib.fcr_lse_bytes(2, h, m, n, d)) == four
     g = torch.Generator(device="cuda").manual_seed(h + n)
     q, k = (torch.randn(2, h, r, d, device="cuda", generator=g).to(dtype) for r in (m, n))
     sums, most = _columns_f64(q, k, causal)
