@@ -2464,14 +2464,14 @@ __device__ __forceinline__ float row16_reduce(float v) {
   return v;
 }
 
-// n words from w on (16-byte aligned), and the word at `one`.  A launch of its own in front of every single sweep: 16 bytes per
+// n words from w on, and the word at `one`.  (A workspace of one of the calls without a size may start at any multiple of 8 bytes.)  A launch of its own in front of every single sweep: 16 bytes per
 // thread, and of a launch of one round one of the two sets of slots (32 pairs of 128 x 4096 x 128 17.8 -> 17.4 us per call).
 __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ w, int n, unsigned* __restrict__ one) {
   const int i = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4;
-  if (i + 4 <= n) {
+  if ((reinterpret_cast<uintptr_t>(w) & 15) == 0 && i + 4 <= n) {
     *reinterpret_cast<u32x4*>(w + i) = (u32x4){0u, 0u, 0u, 0u};
   } else {
-    for (int j = i; j < n; ++j) w[j] = 0u;
+    for (int j = i; j < n && j < i + 4; ++j) w[j] = 0u;
   }
   if (i == 0) *one = 0u;
 }

@@ -25,7 +25,8 @@
  *   - lse is fp32 [B*H, M] contiguous: per query row, log2(sum_j 2^(scale*log2(e)*<q_i,k_j>))
  *     over the keys the row may see.  It is the hand-over between the two kernels.  The buffer
  *     fcr_row_lse / fcr_colreduce write it to must be fcr_lse_bytes(B,H,M,N,D) long (scratch follows
- *     the result); fcr_col_reduce only reads the first B*H*M floats.
+ *     the result) and 8-byte aligned (the single sweep's slots are 64-bit words; fcr_colreduce_ws asks for 16);
+ *     fcr_col_reduce only reads the first B*H*M floats.
  *   - out is fp32 [B*H, N] contiguous and is fully overwritten (no zero-fill needed, unlike the
  *     atomically accumulated buffer at flash.py:286).
  *   - causal != 0 applies the right-aligned mask: key j takes part in row i iff

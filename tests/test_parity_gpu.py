@@ -931,6 +931,28 @@ def test_single_sweep_chunks_past_the_last_key(m, n, d, causal):
     run_all(q * 40, k, causal, what=f"{m}x{n}x{d} far from zero")
 
 
+@pytest.mark.parametrize("m,n", [(60, 3000), (7, 1030)])
+def test_single_sweep_in_a_workspace_of_8_byte_alignment(m, n):
+    """The calls without a size take a workspace at any multiple of 8 bytes: the slots are cleared there too, to their last word and no further."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    h, d = 5, 64
+    q, k = (torch.randn(1, h, r, d, device="cuda").half() for r in (m, n))
+    want, _ = _columns_f64(q, k, True)
+    size = lib.fcr_lse_bytes(1, h, m, n, d) // 4
+    for start in (2, 4):
+        ws = torch.full((size + 8,), 1.0, device="cuda")
+        lse = ws[start : start + size]
+        assert lse.data_ptr() % 16 == 8 * (start % 4 == 2)
+        out = torch.empty(1, h, n, device="cuda")
+        _lib.check(lib.fcr_colreduce(q.data_ptr(), k.data_ptr(), out.data_ptr(), lse.data_ptr(), _lib.DTYPE_F16, 1, h, m, n, d,
+                                     _lib.strides4(q.stride()), _lib.strides4(k.stride()), d ** -0.5, _lib.REDUCE_SUM, 1,
+                                     torch.cuda.current_stream().cuda_stream))
+        assert lib.fcr_colreduce_status(lse.data_ptr(), _lib.DTYPE_F16, 1, h, m, n, d, None) == 0
+        assert _rel(out, want) <= 1e-5
+        assert (ws[:start] == 1).all() and (ws[start + size :] == 1).all()
+
+
 def test_single_sweep_bounded_wait():
     """The wait for the team is bounded from the host: with a limit of zero polls a workgroup whose partners
     have not all published gives up at once, stores NaN for its columns of that pair, sets the status word
