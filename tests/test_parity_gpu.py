@@ -1777,9 +1777,16 @@ def test_few_keys_scores_that_the_plain_sums_do_not_take(h, m, n, d, causal):
     low_k[:, :, 0, 0] = float("-inf")
     cases = [(q, k, None), (far_q, k, None), (q, far_k, None), (q, jump, None), (bad_q, k, None), (q, bad_k, None), (q.abs(), low_k, None),
              (q, k, 0.0), (q, k, -0.3), (q.transpose(2, 1).contiguous().transpose(2, 1), k[:, :1].expand(1, h, n, d), None),
-             (q, torch.nn.functional.pad(k, (0, 8))[..., :d], None)]
+             (q, k, None), (q, k, None)]
     for at, (x, y, scale) in enumerate(cases):
-        x, y = x.half(), y.half() if at != 9 else k[:, :1].half().expand(1, h, n, d)
+        x, y = x.half(), y.half()
+        if at == 9:      # keys that the heads share by a stride of zero (a conversion would make each head its own)
+            y = k[:, :1].half().expand(1, h, n, d)
+        elif at == 10:   # padded key rows
+            y = torch.nn.functional.pad(y, (0, 8))[..., :d]
+        elif at == 11:   # token-major keys
+            y = y.transpose(1, 2).contiguous().transpose(1, 2)
+        assert y.stride(2) == {10: d + 8, 11: h * d}.get(at, d)
         for red in ("sum", "max"):
             got = {}
             for option in (1, 0):
