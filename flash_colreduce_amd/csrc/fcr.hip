@@ -1115,7 +1115,6 @@ __device__ __forceinline__ float lanes16_scatter(const f32x4 (&v)[4], int lane) 
   return join((lane & 1) ? z[1] : z[0], dpp_row<0xB1>((lane & 1) ? z[0] : z[1]));
 }
 
-// 16-row groups of keys per wave where there are more than 256 keys: eight while their fragments leave room for what is added up.
 // Sum (maximum) of each of 8 values over the four rows of lanes: row rho of lanes ends up with values 2 rho and 2 rho + 1 in v[0], v[1].
 template <bool MAX>
 __device__ __forceinline__ void lane_rows_scatter(float (&v)[8]) {
