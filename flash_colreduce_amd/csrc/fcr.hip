@@ -1436,14 +1436,15 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     }
     write_reduced(sums + (i & 1) * kSums, x);
   };
-  // What the rows of chunk i contribute with, into `fact`; whether a row's sum is unusable (the same in every wave).
-  auto row_facts = [&](int i, float (&l)[SQ]) __attribute__((always_inline)) {
+  // What the rows of chunk i contribute with, into `fact`; whether a row's sum is unusable (the same in every wave).  all_seen: no row sees
+  // less than 64 keys.
+  auto row_facts = [&](int i, float (&l)[SQ], bool all_seen = false) __attribute__((always_inline)) {
     const int q0 = first_row(i);
     float w[SQ][NW];
     read_partials(sums + (i & 1) * kSums, w);
     add_up(w, l);
     bool good = true;
-    const float least = MODE != kModeSum || few_seen(i) ? 9.5367432e-7f : 1.f;   // (maxima take a logarithm off the score)
+    const float least = MODE != kModeSum || (!all_seen && few_seen(i)) ? 9.5367432e-7f : 1.f;   // (maxima take a logarithm off the score)
 #pragma unroll
     for (int sq = 0; sq < SQ; ++sq) {
       good = good && l[sq] >= least && l[sq] < 1.2676506e30f;
@@ -1527,7 +1528,7 @@ __global__ __launch_bounds__(64 * NW, 2) void few_keys_kernel(const Params p) {
     if (NBT > 1) scores(1, visible);
     if (__builtin_expect(i > 0, 1)) {
       float l[SQ];
-      if (__builtin_expect(row_facts(i - 1, l), 0)) return false;
+      if (__builtin_expect(row_facts(i - 1, l, !CAUSAL), 0)) return false;
 #pragma unroll
       for (int g = 0; g < NG; ++g) add_group(g);
       lse_of(i - 1, l);
