@@ -31,6 +31,8 @@
  *     atomically accumulated buffer at flash.py:286).
  *   - causal != 0 applies the right-aligned mask: key j takes part in row i iff
  *     j <= i + max(N-M, 0)   (flash.py:22-27, 198-207; naive.py:20-24).
+ *   - A call is reproducible bit for bit.  The last bits of a (batch, head) pair's sums may differ between calls with different
+ *     numbers of pairs, which decide how the pairs' rows or keys are dealt to workgroups, and between entry points.
  *   - stream is a hipStream_t (NULL = the default stream).  Launches are asynchronous.
  *   - Return value: 0 on success; negative FCR_E_* for a rejected argument (nothing was
  *     launched); positive = the hipError_t of a failed launch.  fcr_last_error() returns a
@@ -206,7 +208,8 @@ int fcr_colreduce_to(const void* q, const void* k, void* out, int out_dtype, flo
  * sum (64 sequences of 32 heads and 65536 keys: 0.5 GB); 16-bit keys that fit the registers of a workgroup (at most
  * 512, or 256 in rows of more than 256 bytes) form each score once, and where several workgroups share a pair their columns
  * wait in the workspace for a second launch.  With less, but at least fcr_lse_bytes, the call takes the
- * path of the entry points above (FCR_E_SCRATCH below that); results agree to rounding either way.  ws must be 16-byte aligned, its first
+ * path of the entry points above, as it does for long calls of few keys that would fill neither the chip nor a workgroup's
+ * registers (FCR_E_SCRATCH below that); results agree to rounding either way.  ws must be 16-byte aligned, its first
  * B*H*M floats hold the row statistics on return, its contents before the call are irrelevant.
  */
 size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D);
