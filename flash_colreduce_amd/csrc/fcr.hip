@@ -18,6 +18,7 @@
 //   col_reduce_kernel a workgroup keeps 256 key rows in registers and streams query tiles (and
 //                     their lse2) through LDS; writes out[bh, j] = sum_i or max_i 2^(s_ij-lse2_i).
 //   row_lse_f32_kernel, col_reduce_f32_kernel   the same for fp32 operands, whose rows are split on the way to LDS.
+//   both_sweeps_kernel  both in one launch: column sweeps start where row sweeps leave a CU and wait for the lse they need.
 //   col_small_kernel  the same result for at most 128 query rows against many keys: queries resident
 //                     in every wave, keys streamed (HBM bound).
 //   col_fused_kernel  both sweeps in one for at most 128 query rows against many 16-bit keys: the scores of
@@ -31,7 +32,7 @@
 // into a swizzled ring of LDS stages (buffer loads with the LDS as destination).  Nothing of size M*N
 // is written anywhere and nothing in global memory is updated by read-modify-write atomics: one workgroup
 // owns its output rows / columns (col_fused_kernel hands its partial row values to its team with atomic
-// 64-bit stores and loads, value and round number in one word).
+// 64-bit stores and loads, value and round number in one word; both_sweeps_kernel its lse, word by word, to column sweeps).
 //
 // Replaces the Triton kernel of the reference (flash_colreduce/flash.py:11-274).
 
@@ -49,7 +50,8 @@
 // The file can be compiled whole, or in parts that are linked together (the build script does that to
 // use several cores): part 0 holds the C ABI and the small kernels, parts 1-4 the sweeps of one element
 // type each (fp16, bf16, fp32 rows up to 512 bytes, longer fp32 rows), parts 5 and 6 the sweeps over fp16 and
-// bf16 rows of more than 512 bytes, parts 7 and 8 the single sweep for fp16 and bf16, parts 9 and 10 few_keys_kernel for them.
+// bf16 rows of more than 512 bytes, parts 7 and 8 the single sweep for fp16 and bf16, parts 9 and 10 few_keys_kernel for them,
+// parts 11 and 12 both_sweeps_kernel.
 #ifndef FCR_PART
 #define FCR_PART -1
 #endif
@@ -85,6 +87,9 @@ struct Params {
   int teams;
   unsigned* sync;    // error word; zero at launch, like the slots at `part`
   int spin_limit;    // polls of the counter after which a wait gives up
+  // both_sweeps_kernel: `tiles`, `group`, `fill` and `total` are of the row sweeps
+  int col_tiles, col_group;
+  int row_blocks, col_blocks;
 };
 // which: 0 = row statistics, 1 = column sweep, 2 = column sweep for few queries, 3 = both sweeps in one for few
 // queries, mode + 4 for more than 64 of them (2 and 3: 16-bit types only)
@@ -96,6 +101,8 @@ void sweeps_f16_single(const Params& p, int ksteps, bool causal, int mode, hipSt
 void sweeps_bf16_single(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 void sweeps_f16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s);   // few_keys_kernel
 void sweeps_bf16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s);
+void sweeps_f16_both(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);   // both_sweeps_kernel
+void sweeps_bf16_both(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 void sweeps_f16_long_rows(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 void sweeps_bf16_long_rows(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 extern thread_local bool fused_refused;   // set by a launcher of col_fused_kernel that did not launch
@@ -232,8 +239,7 @@ __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_lo
 // CU is as many places behind the first as the chip has CUs, so the CU with the longest sweep also gets the longest of
 // the second helping.  That helping is dealt backwards instead (p.fill; eight places at a time, which keeps the XCDs), so the
 // two sweeps of every CU add up to about the same length; what is left follows in plain order.  Host: fill_places.
-__device__ __forceinline__ void map_group(const Params& p, int per_bh, int& bh, int& r) {
-  int v = (int)blockIdx.x;
+__device__ __forceinline__ void map_group(const Params& p, int v, int per_bh, int& bh, int& r) {
   const int second = v - p.fill, dealt = (min(2 * p.fill, p.total) - p.fill) & ~7;
   if (p.fill > 0 && second >= 0 && second < dealt) v = p.fill + (dealt - 8 - (second & ~7)) + (second & 7);
   const int per = p.group * per_bh;
@@ -245,19 +251,19 @@ __device__ __forceinline__ void map_group(const Params& p, int per_bh, int& bh, 
   bh = first + (w - r * g);
 }
 
-__device__ __forceinline__ void map_block(const Params& p, bool longest_is_last_tile, int& bh, int& tile) {
+__device__ __forceinline__ void map_block(const Params& p, int v, bool longest_is_last_tile, int& bh, int& tile) {
   int rank;
-  map_group(p, p.tiles, bh, rank);
+  map_group(p, v, p.tiles, bh, rank);
   tile = longest_is_last_tile ? p.tiles - 1 - rank : rank;
 }
 
 // Row kernel with the keys of a tile split over several workgroups (few query rows, many keys):
 // inside a group the order is (b,h), then the tile, then the key range: the tiles that stream the
 // same keys start next to each other on the same XCD and share them through its L2.
-__device__ __forceinline__ void map_block_split(const Params& p, bool longest_is_last_tile, int& bh, int& tile,
+__device__ __forceinline__ void map_block_split(const Params& p, int v, bool longest_is_last_tile, int& bh, int& tile,
                                                 int& split) {
   int r;
-  map_group(p, p.tiles * p.splits, bh, r);
+  map_group(p, v, p.tiles * p.splits, bh, r);
   const int back = r / p.tiles;   // the last key range first: with the mask it holds the diagonal, the slow part
   const int rank = r - back * p.tiles;
   split = p.splits - 1 - back;
@@ -346,9 +352,11 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t view, uint32_t byte
   __builtin_amdgcn_raw_ptr_buffer_load_lds(view, (__attribute__((address_space(3))) void*)lds_wave_base, 16,
                                            (int)byte_off, 0, 0, AUX);
 }
+constexpr int kFromMemory = 16;   // sc1: past the caches of the workgroup's die, as atomic loads at device scope are done
+template <int AUX = 0>
 __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t view, uint32_t byte_off, char* lds_wave_base) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(view, (__attribute__((address_space(3))) void*)lds_wave_base, 4,
-                                           (int)byte_off, 0, 0, 0);
+                                           (int)byte_off, 0, 0, AUX);
 }
 
 // Waits until at most N of this wave's loads are outstanding and all its LDS reads have returned, then
@@ -535,7 +543,7 @@ __device__ __forceinline__ void mma_groups(f32x4 (&n)[NG][2], u32x4 (&f)[2][KS],
 //     MFMA(s1 of t)   || VALU of s0 of t   || fragments <- s0 of t+1
 //     MFMA(s0 of t+1) || VALU of s1 of t   || fragments <- s1 of t+1
 // Every LDS read is issued a sub-step before its use.
-// aux_of(stage, sub) reads what the consumer needs per sub-step besides the scores (the column
+// aux_of(t, stage, sub) reads what the consumer needs per sub-step besides the scores (the column
 // kernel: lse of the lane's queries); it travels with the fragments so that it too is read before
 // the barrier that lets the stage be refilled.
 template <int DT, int KS, int NG, bool RESIDENT_IS_KEYS, class Aux, class RingT, class AdvF, class StageF,
@@ -555,20 +563,20 @@ __device__ __forceinline__ void pipelined_sweep(int ta, int tb, const u32x4 (&re
       f[0][ks] = rg.frag(lds, 0, 0, ks);
       f[1][ks] = rg.frag(lds, 0, 1, ks);
     }
-    ap = aux_of(lds, 0);
+    ap = aux_of(ta, lds, 0);
     mma_groups<DT, KS, NG, RESIDENT_IS_KEYS, true>(pa, f, res, rg, lds, 1);
-    af = aux_of(lds, 1);
+    af = aux_of(ta, lds, 1);
   }
   for (int t = ta; t + 1 < tb; ++t) {
     advance(t + 1);
     const char* nxt = stage_of(t + 1);
     an = af;
     mma_groups<DT, KS, NG, RESIDENT_IS_KEYS, true>(pb, f, res, rg, nxt, 0);
-    af = aux_of(nxt, 0);
+    af = aux_of(t + 1, nxt, 0);
     consume(pa, ap);
     ap = af;
     mma_groups<DT, KS, NG, RESIDENT_IS_KEYS, true>(pa, f, res, rg, nxt, 1);
-    af = aux_of(nxt, 1);
+    af = aux_of(t + 1, nxt, 1);
     consume(pb, an);
   }
   mma_groups<DT, KS, NG, RESIDENT_IS_KEYS, false>(pb, f, res, rg, nullptr, 0);
@@ -682,14 +690,14 @@ struct NoAux {};
 // and so many keys that none of them survives in a cache until the column kernel: they are loaded
 // non-temporally (7.0 instead of 6.2 TB/s on 34 GB of keys).  With several row tiles, or few keys, the
 // default policy is the faster one.
-template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE>
-__global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(const Params p) {
+// TELL: column sweeps of the same launch wait for the values (both_sweeps_kernel).
+template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE, bool TELL>
+__device__ __forceinline__ void row_sweep(const Params& p, char* smem, int v) {
   using Rg = Ring<KS>;
   constexpr int NG = wave_group_count(NB);
   constexpr int kTileRows = kWaves * 16 * NG;
-  __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes];
   int bh, tile, split;
-  map_block_split(p, CAUSAL, bh, tile, split);
+  map_block_split(p, v, CAUSAL, bh, tile, split);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, keeps the row views scalar
   const int b = bh / p.H, h = bh - b * p.H;
@@ -746,7 +754,7 @@ __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(con
   load_resident<KS, NG>(qf, qb, p.q_sr, q0, p.M, p.dgran, lane);
 
   pipelined_sweep<DT, KS, NG, false, NoAux>(
-      c_begin, t_int, qf, rg, advance, stage_of, [](const char*, int) { return NoAux{}; },
+      c_begin, t_int, qf, rg, advance, stage_of, [](int, const char*, int) { return NoAux{}; },
       [&](const f32x4(&a)[NG][2], NoAux) { lse_update_groups(a, scale2, mref, l); });
 
   for (int t = max(t_int, c_begin); t < nchunks; ++t) {
@@ -788,8 +796,18 @@ __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(con
     v = lse_merge(v, __shfl_xor(v, 32));
     const int i = q0[g] + lane;
     float* dst = (p.splits > 1) ? p.part + (int64_t)split * p.bh_count * p.M : p.lse;
-    if (lane < 16 && i < p.M) dst[(int64_t)bh * p.M + i] = v;
+    if (lane < 16 && i < p.M) {
+      if (TELL) __hip_atomic_store(reinterpret_cast<uint32_t*>(dst) + (int64_t)bh * p.M + i, v != v ? 0x7fc00000u : __builtin_bit_cast(uint32_t, v),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else dst[(int64_t)bh * p.M + i] = v;
+    }
   }
+}
+
+template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE>
+__global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(const Params p) {
+  __shared__ __attribute__((aligned(1024))) char smem[Ring<KS>::kBytes];
+  row_sweep<DT, KS, CAUSAL, NB, STREAM_ONCE, false>(p, smem, (int)blockIdx.x);
 }
 
 // lse[r] = log2 sum_s 2^part[s][r] over the key ranges of a split row sweep.  One thread per row; the
@@ -850,9 +868,10 @@ __device__ __forceinline__ void col_update(const f32x4 (&a)[SG], const float (&s
 
 // End of a column sweep: reduces the wave's NG groups over the 16 query lanes (a transpose through LDS, one output key per
 // lane and pass; a pass writes out four groups) and stores the columns.  Nobody uses the LDS any more.
+// nans: NaN in their place.
 template <int MODE, int NG>
 __device__ __forceinline__ void col_store(const Params& p, char* smem, int bh, const int (&k0)[NG], const f32x4 (&csum)[NG],
-                                          const f32x4 (&cmax)[NG], int lane, int wave) {
+                                          const f32x4 (&cmax)[NG], int lane, int wave, bool nans = false) {
   float* red = reinterpret_cast<float*>(smem) + wave * (NG * 4 * 64);
   const int w = lane & 15;                 // key inside its group
   if (MODE != kModeMax) {
@@ -870,7 +889,7 @@ __device__ __forceinline__ void col_store(const Params& p, char* smem, int bh, c
 #pragma unroll
         for (int j = 0; j < 16; ++j) v += src[(j + lane) & 15];
         const int key = k0[grp] + w;
-        if (key < p.N) store_column(p, p.out, true, bh, key, v);
+        if (key < p.N) store_column(p, p.out, true, bh, key, nans ? __builtin_nanf("") : v);
       }
     }
   }
@@ -890,7 +909,7 @@ __device__ __forceinline__ void col_store(const Params& p, char* smem, int bh, c
 #pragma unroll
         for (int j = 0; j < 16; ++j) v = fmaxf(v, src[(j + lane) & 15]);
         const int key = k0[grp] + w;
-        if (key < p.N) store_column(p, (MODE == kModeBoth) ? p.out2 : p.out, false, bh, key, fast_exp2(v));
+        if (key < p.N) store_column(p, (MODE == kModeBoth) ? p.out2 : p.out, false, bh, key, nans ? __builtin_nanf("") : fast_exp2(v));
       }
     }
   }
@@ -923,16 +942,23 @@ inline int col_tile_blocks(int ksteps, int mode, int N, int64_t bh, bool causal)
   return wgs2 < 2 * cus ? 1 : 2;
 }
 
-template <int DT, int KS, bool CAUSAL, int MODE, int NB>
-__global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_reduce_kernel(const Params p) {
+// FOLLOW: row sweeps of the same launch may not have stored the lse of the streamed rows yet (both_sweeps_kernel).
+constexpr uint32_t kNotYet = 0xffffffffu;   // an lse that is still to come: no row sweep stores this NaN
+constexpr int kLseSlots = 8;                // of 64 rows each
+template <int KS, int NB, bool FOLLOW>
+__host__ __device__ constexpr int col_sweep_bytes() {
+  const int red = kWaves * wave_group_count(NB) * 4 * 64 * 4;      // end-of-sweep transpose buffer
+  const int ring = Ring<KS>::kBytes + (FOLLOW ? kLseSlots * kChunk * 4 : 0);
+  return ring > red ? ring : red;
+}
+template <int DT, int KS, bool CAUSAL, int MODE, int NB, bool FOLLOW>
+__device__ __forceinline__ void col_sweep(const Params& p, char* smem, int v) {
   using Rg = Ring<KS>;
+  static_assert(!FOLLOW || Rg::kN + 1 <= kLseSlots, "a slot for every chunk whose lse is read or on its way");
   constexpr int NG = wave_group_count(NB);
   constexpr int kTileRows = kWaves * 16 * NG;
-  constexpr int kRed = kWaves * NG * 4 * 64 * 4;      // end-of-sweep transpose buffer
-  constexpr int kSmem = (Rg::kBytes > kRed) ? Rg::kBytes : kRed;
-  __shared__ __attribute__((aligned(1024))) char smem[kSmem];
   int bh, tile;
-  map_block(p, false, bh, tile);
+  map_block(p, v, false, bh, tile);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, keeps the row views scalar
   const int b = bh / p.H, h = bh - b * p.H;
@@ -968,23 +994,54 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
   auto stage_of = [&](int t) { return smem + ((uint32_t)t % Rg::kN) * Rg::kStage; };
   rg.start(qb, p.q_sr, t0 * kChunk, p.M);
   const float* lse_next = lse + t0 * kChunk;   // walks along with the ring's cursor
+  int lse_left = p.M - t0 * kChunk;            // (FOLLOW: the lse is ahead of the rows)
+  auto lse_slot = [&](int t) { return smem + Rg::kBytes + (t & (kLseSlots - 1)) * (kChunk * 4); };   // (FOLLOW)
+  auto issue_lse = [&](char* to, int live) {
+    const __amdgpu_buffer_rsrc_t view = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(lse_next), 0, live * 4, 0x00020000);
+    dma4<(FOLLOW ? kFromMemory : 0)>(view, (uint32_t)lane * 4u, to);   // every wave writes the same 64 values: no branch
+    lse_next += kChunk;
+    lse_left -= kChunk;
+  };
+  // FOLLOW: the lse is requested a chunk ahead of its rows, into slots of its own, so that a wave can look at it a chunk before its use
+  // (`word`: of the chunk that comes next, the lane's row).
+  uint32_t word = 0;
+  bool given_up = false;
   auto issue = [&](int t) {
     char* stage = stage_of(t);
-    const int live = rows_in_chunk(rg.rows_left);
+    const int live = rows_in_chunk(FOLLOW ? lse_left : rg.rows_left);
     rg.issue_next(stage);
-    const __amdgpu_buffer_rsrc_t view = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(lse_next), 0, live * 4, 0x00020000);
-    dma4(view, (uint32_t)lane * 4u, stage + Rg::kRows);   // every wave writes the same 64 values: no branch
-    lse_next += kChunk;
+    issue_lse(FOLLOW ? lse_slot(t + 1) : stage + Rg::kRows, live);
+  };
+  auto wait_for = [&](int t) {   // every wave by itself: the slot then holds the same values whoever wrote last
+    const int i = t * kChunk + lane;
+    const uint32_t* at = reinterpret_cast<const uint32_t*>(lse) + (i < p.M ? i : p.M - 1);
+    int polls = 0;
+    uint32_t x = kNotYet;
+    for (;;) {
+      x = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__builtin_amdgcn_ballot_w64(x == kNotYet) == 0) break;
+      if (given_up || ++polls > p.spin_limit) {
+        given_up = true;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(8);
+    }
+    reinterpret_cast<uint32_t*>(lse_slot(t))[lane] = x;
   };
   auto advance = [&](int t) {
     ring_sync<(Rg::kN - 2) * (Rg::kPer + 1)>();
+    if constexpr (FOLLOW) {
+      if (t == t0) word = reinterpret_cast<const uint32_t*>(lse_slot(t))[lane];
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(word == kNotYet) != 0, 0)) wait_for(t);
+      word = reinterpret_cast<const uint32_t*>(lse_slot(t + 1))[lane];
+    }
     issue(t + Rg::kN - 1);
   };
-  auto aux_of = [&](const char* lds, int sub) {
-    const float* v = reinterpret_cast<const float*>(lds + Rg::kRows) + sub * 32 + (lane & 15);
+  auto aux_of = [&](int t, const char* lds, int sub) {
+    const float* v = reinterpret_cast<const float*>(FOLLOW ? lse_slot(t) : lds + Rg::kRows) + sub * 32 + (lane & 15);
     return LsePair{{v[0], v[16]}};
   };
+  if (FOLLOW) issue_lse(lse_slot(t0), rows_in_chunk(lse_left));
   // The first chunks of the streamed operand are requested before the resident one, so that all of
   // them are in flight together.
 #pragma unroll
@@ -1000,7 +1057,7 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
     for (int sub = 0; sub < kChunk / 32; ++sub) {
       const int qs = t * kChunk + sub * 32;  // first query of the sub-tile
       if (RAGGED && qs >= p.M) continue;
-      LsePair lq = aux_of(lds, sub);
+      LsePair lq = aux_of(t, lds, sub);
       // +inf for rows past M: they contribute 2^-inf = 0
       if (RAGGED && qs + (lane & 15) >= p.M) lq.v[0] = kPosInf;
       if (RAGGED && qs + 16 + (lane & 15) >= p.M) lq.v[1] = kPosInf;
@@ -1046,8 +1103,43 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
   for (int t = nfull; t < nchunks; ++t) general_chunk(t, std::true_type());
 
   ring_sync<0>();   // every load has landed (those past the last chunk write zeros): the LDS can be reused
-  col_store<MODE, NG>(p, smem, bh, k0, csum, cmax, lane, wave);
+  col_store<MODE, NG>(p, smem, bh, k0, csum, cmax, lane, wave, given_up);
 }
+
+template <int DT, int KS, bool CAUSAL, int MODE, int NB>
+__global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_reduce_kernel(const Params p) {
+  __shared__ __attribute__((aligned(1024))) char smem[col_sweep_bytes<KS, NB, false>()];
+  col_sweep<DT, KS, CAUSAL, MODE, NB, false>(p, smem, (int)blockIdx.x);
+}
+
+// Both sweeps in one launch: workgroups [0, p.total) take row tiles as row_lse_kernel does, those from the next multiple of eight on
+// (which keeps the XCDs) column tiles as col_reduce_kernel.  The row statistics start as kNotYet (fill_words_kernel), a row sweep stores its rows' values with
+// device scope, and a column sweep takes a chunk of queries once their values are there: every word says so by itself, so there are
+// no flags, no order between words and no fences.  Workgroups are dispatched in order, on every XCD the row tiles first, and a row tile
+// waits for nobody: whatever a column sweep waits for is running or done.  Should that not hold the wait ends after p.spin_limit polls and
+// the columns become NaN.
+// What it is for: a launch that waits for its longest or last sweeps keeps CUs idle at its end, and here only the second one does.  With
+// the mask, the first column tile needs only the rows of the first row tile at first, which end early, and follows the row sweeps chunk
+// by chunk.  A column sweep looks at a chunk's values a chunk ahead, one LDS read and one branch per chunk, within 1 % of a sweep of its
+// own (32 heads of 8192 x 8192 x 128 467 -> 472 us, where nothing is gained).  When a CU holds two workgroups the older one runs at nearly its
+// full speed and the younger one on what is left (1.15 us and 3.3 per chunk of 64 rows against 1.05 alone), so the order of
+// dispatch decides what ends together: see map_group, and both_plan for what was measured.
+template <int DT, int KS, bool CAUSAL, int MODE, int NBR, int NBC>
+__global__ __launch_bounds__(kThreads, 2) void both_sweeps_kernel(const Params p) {
+  constexpr int kCols = col_sweep_bytes<KS, NBC, true>();
+  __shared__ __attribute__((aligned(1024))) char smem[kCols > Ring<KS>::kBytes ? kCols : Ring<KS>::kBytes];
+  const int v = (int)blockIdx.x, rows = (p.total + 7) & ~7;
+  if (v < rows) {
+    if (v < p.total) row_sweep<DT, KS, CAUSAL, NBR, false, true>(p, smem, v);
+    return;
+  }
+  Params c = p;
+  c.tiles = p.col_tiles;
+  c.group = p.col_group;
+  c.fill = 0;
+  col_sweep<DT, KS, CAUSAL, MODE, NBC, true>(c, smem, v - rows);
+}
+
 
 // ---------------------------------------------------------------------------------------------
 // Both sweeps in one for a pair whose keys all fit the registers of one workgroup: every wave keeps 16 * NG keys (groups w, w + NW,
@@ -2054,7 +2146,7 @@ __global__ __launch_bounds__(64 * NW, 2) void row_lse_f32_kernel(const Params p)
   constexpr int SG = f32_groups(KS), kRows = Rg::kChunkRows, kTileRows = NW * 16 * NG;
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes];
   int bh, tile, split;
-  map_block_split(p, CAUSAL, bh, tile, split);
+  map_block_split(p, (int)blockIdx.x, CAUSAL, bh, tile, split);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = bh / p.H, h = bh - b * p.H;
@@ -2154,7 +2246,7 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
   constexpr int kRed = NW * NG * 4 * 64 * 4;
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes > kRed ? Rg::kBytes : kRed];
   int bh, tile;
-  map_block(p, false, bh, tile);
+  map_block(p, (int)blockIdx.x, false, bh, tile);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = bh / p.H, h = bh - b * p.H;
@@ -2289,7 +2381,7 @@ __global__ __launch_bounds__(kThreads, (NG <= 4 ? 3 : 2)) void col_small_kernel(
   __shared__ __attribute__((aligned(1024))) char smem[Rg::kBytes + kObufBytes];
   float* const obuf = reinterpret_cast<float*>(smem + Rg::kBytes);
   int bh, split;
-  map_group(p, p.splits, bh, split);
+  map_group(p, (int)blockIdx.x, p.splits, bh, split);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = bh / p.H, h = bh - b * p.H;
@@ -2466,6 +2558,14 @@ __device__ __forceinline__ float row16_reduce(float v) {
 
 // n words from w on, and the word at `one`.  (A workspace of one of the calls without a size may start at any multiple of 8 bytes.)  A launch of its own in front of every single sweep: 16 bytes per
 // thread, and of a launch of one round one of the two sets of slots (32 pairs of 128 x 4096 x 128 17.8 -> 17.4 us per call).
+__global__ __launch_bounds__(256) void fill_words_kernel(unsigned* __restrict__ w, int64_t n, unsigned value) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + (int)threadIdx.x) * 4;
+  if ((reinterpret_cast<uintptr_t>(w) & 15) == 0 && i + 4 <= n) {
+    *reinterpret_cast<u32x4*>(w + i) = (u32x4){value, value, value, value};
+  } else {
+    for (int64_t j = i; j < n && j < i + 4; ++j) w[j] = value;
+  }
+}
 __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ w, int n, unsigned* __restrict__ one) {
   const int i = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4;
   if ((reinterpret_cast<uintptr_t>(w) & 15) == 0 && i + 4 <= n) {
@@ -4437,6 +4537,7 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   p.teams = 0;
   p.sync = nullptr;
   p.spin_limit = 0;
+  p.col_tiles = p.col_group = p.row_blocks = p.col_blocks = 0;
   return 0;
 }
 
@@ -4613,6 +4714,52 @@ FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool bot
     o.part_at = (base_floats + 63) / 64 * 64;
     o.floats = o.part_at + (both ? 2 : 1) * s * bh * N;
   }
+  return o;
+}
+
+// Both sweeps in one launch (both_sweeps_kernel): 32-row blocks per wave of its row and its column tiles; row_blocks 0: two launches.
+// The column sweeps start where row sweeps leave a CU, so a launch that does not fill its last round no longer costs a round twice, and
+// where the mask gives row tiles that end early the column sweeps follow them.  us per call, two launches -> one, against 256-row tiles per CU (`rows`), of
+// 480 shapes of 4 to 512 pairs, 530 to 9000 queries, fp16 and bf16, all reductions:
+//   With the mask and as many keys as queries, rows of more than 128 bytes: up to 0.9 both tiles have 128 rows (18 pairs of 2240 x 128 55.5 -> 41,
+//   11 of 4078 x 128 103 -> 67, 4 of 570 x 128 18.9 -> 16.6), up to 1.9 the column tiles (27 of 2240 65 -> 54, 37 of 2810 106 -> 92), and from 2.65 on
+//   neither (155 of 1538 151 -> 133, 43 of 6338 514 -> 447).  In between two launches, each with its second helping dealt
+//   backwards (map_group), are as fast (48 of 2929 118 -> 120, 25 of 5834 212 -> 220, 32 of 4954 199 -> 197), and so are they for a few rounds of long sweeps, whose
+//   last round is a small part (32 of 8192 468 -> 472, of 16384 1798 -> 1810).  Rows of 129 to 192 bytes lose between 1.0 and 1.3 as well (60 of 1045 x 80 27.3 -> 29.5).
+//   Rows of up to 128 bytes: 128-row tiles, four workgroups to a CU; two launches between 1.1 and 2.6 (10 of 8777 x 64 138 -> 148, 61 of 2304 68 -> 75; but 259 of
+//   626 41 -> 34, 206 of 1100 77 -> 60).  Rows of more than 256 bytes: 128-row tiles, always (10 of 1895 x 256 54 -> 41, 32 of 2048 79 -> 68, 77 of 4305 692 -> 675).
+//   Without the mask, or with many more keys than queries, no column can start before the rows of its pair end: there have to be row
+//   tiles for every CU (24 of 2893 x 128 144 -> 121, 48 of 2929 244 -> 207, 61 of 2223 174 -> 143, 18 of 7902 x 64 449 -> 355; but 17 of 2873 x 128 88 -> 89, 5 of 3039 50 -> 64;
+//   with 128 queries per 1000 keys 68 of 1090 x 8104 318 -> 334).
+struct BothPlan {
+  int row_blocks = 0, col_blocks = 0;
+};
+BothPlan both_plan(int dtype, int ksteps, int64_t bh, int M, int N, bool causal) {
+  BothPlan o;
+  // (a wait is bounded by polls, a microsecond or more each: row sweeps of up to 2^20 keys take a tenth of the default bound)
+  if (dtype == FCR_DTYPE_F32 || ksteps > kMaxKSteps || M <= kSmallRows || M > (1 << 20) || N > (1 << 20)) return o;
+  const int cus = chip_cus();
+  const int64_t tiles = bh * ((M + 127) / 128), cols = bh * ((N + 127) / 128);   // of 128 rows
+  if (tiles + cols >= kMaxWorkgroups / 2) return o;
+  const double small = (double)tiles / cus, rows = (double)(bh * ((M + 255) / 256)) / cus;
+  const bool longer = 2 * (int64_t)N > 3 * (int64_t)M, level = causal && !longer;   // level: the column sweeps can follow the row sweeps
+  int nr = 1, nc = 1;
+  if (ksteps > 4) {
+    if (!level && small < 1.05) return o;
+  } else if (ksteps <= 2) {
+    if (level ? rows >= 1.1 && (rows < 2.7 || N >= 10000) : longer ? rows < 1.1 : small < 1.02 || (small >= 1.5 && rows < 1.1)) return o;
+  } else if (level) {
+    if (rows >= 1.85 && (rows < 2.1 ? N > 8500 : rows < 2.65 || N >= 8000)) return o;
+    if (ksteps == 3 && rows >= 1.0 && rows < 1.3) return o;
+    nr = rows >= 0.9 ? 2 : 1;
+    nc = rows >= 1.9 ? 2 : 1;
+  } else {
+    if (longer ? rows < 1.85 : small < 1.02 || (small >= 1.5 && rows < 1.0)) return o;
+    nr = rows >= 1.5 ? 2 : 1;
+    nc = rows >= 1.85 ? 2 : 1;
+  }
+  o.row_blocks = nr;
+  o.col_blocks = nc;
   return o;
 }
 
@@ -4828,6 +4975,27 @@ void launch_few_keys(const Params& p, bool causal, int mode, int form, hipStream
   else launch_few_keys_mode<DT, KS, kModeBoth>(p, causal, form, s);
 }
 
+template <int DT, int KS, int MODE, int NBR, int NBC>
+void launch_both_tiles(const Params& p, bool causal, hipStream_t s) {
+  const dim3 grid((unsigned)(((p.total + 7) & ~7) + p.bh_count * p.col_tiles)), block(kThreads);
+  if (causal) hipLaunchKernelGGL((both_sweeps_kernel<DT, KS, true, MODE, NBR, NBC>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((both_sweeps_kernel<DT, KS, false, MODE, NBR, NBC>), grid, block, 0, s, p);
+}
+template <int DT, int KS, int MODE>
+void launch_both_mode(const Params& p, bool causal, hipStream_t s) {
+  if constexpr (KS == 3 || KS == 4) {
+    if (p.row_blocks == 2 && p.col_blocks == 2) return launch_both_tiles<DT, KS, MODE, 2, 2>(p, causal, s);
+    if (p.row_blocks == 2) return launch_both_tiles<DT, KS, MODE, 2, 1>(p, causal, s);
+  }
+  launch_both_tiles<DT, KS, MODE, 1, 1>(p, causal, s);
+}
+template <int DT, int KS>
+void launch_both(const Params& p, bool causal, int mode, hipStream_t s) {
+  if (mode == kModeSum) launch_both_mode<DT, KS, kModeSum>(p, causal, s);
+  else if (mode == kModeMax) launch_both_mode<DT, KS, kModeMax>(p, causal, s);
+  else launch_both_mode<DT, KS, kModeBoth>(p, causal, s);
+}
+
 #define FCR_DISPATCH_KS(DT, ksteps, CALL)                  \
   switch (ksteps) {                                        \
     case 1: CALL(DT, 1); break;                            \
@@ -4901,6 +5069,17 @@ void fcr_detail::sweeps_bf16_few_keys(const Params& p, int ksteps, bool causal, 
   FCR_DISPATCH_KS(FCR_DTYPE_BF16, ksteps, FCR_CALL_FEW_KEYS)
 }
 #endif
+#define FCR_CALL_BOTH(DT, KS) launch_both<DT, KS>(p, causal, mode, s)
+#if FCR_HAS(11)
+void fcr_detail::sweeps_f16_both(const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
+  FCR_DISPATCH_KS(FCR_DTYPE_F16, ksteps, FCR_CALL_BOTH)
+}
+#endif
+#if FCR_HAS(12)
+void fcr_detail::sweeps_bf16_both(const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
+  FCR_DISPATCH_KS(FCR_DTYPE_BF16, ksteps, FCR_CALL_BOTH)
+}
+#endif
 #if FCR_HAS(3)
 void fcr_detail::sweeps_f32(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
   if (!in_parts(FCR_DTYPE_F32, p.dgran * 4)) {
@@ -4947,6 +5126,9 @@ void fcr_detail::sweeps_bf16_long_rows(int which, const Params& p, int ksteps, b
 
 #if FCR_HAS(0)
 namespace {
+int g_single_sweep = 1;
+long long g_wait_polls = 1ll << 20;
+
 // sweeps of the element type `dtype`
 void launch_sweeps(int dtype, int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s,
                    unsigned* zero = nullptr, int zero_words = 0) {
@@ -5046,6 +5228,27 @@ int launch_one_query(Params& p, int dtype, const OneQueryPlan& o, float* ws, int
   return launched("one_query_columns_kernel");
 }
 
+int launch_both(Params& p, int dtype, int ksteps, const BothPlan& o, float* ws, int mode, bool causal, hipStream_t s) {
+  p.lse = ws;
+  p.row_blocks = o.row_blocks;
+  p.col_blocks = o.col_blocks;
+  const int row_rows = kWaves * 32 * o.row_blocks, col_rows = kWaves * 32 * o.col_blocks;
+  p.tiles = (p.M + row_rows - 1) / row_rows;
+  p.col_tiles = (p.N + col_rows - 1) / col_rows;
+  p.total = p.bh_count * p.tiles;
+  p.group = head_group(p.bh_count, p.tiles, causal);
+  p.col_group = head_group(p.bh_count, p.col_tiles, causal);
+  p.fill = fill_places(p, TileChoice{row_rows, 2}, causal);
+  const long long polls = __atomic_load_n(&g_wait_polls, __ATOMIC_RELAXED);
+  p.spin_limit = polls > 0x7fffffffll ? 0x7fffffff : (int)polls;
+  const int64_t words = (int64_t)p.bh_count * p.M;
+  hipLaunchKernelGGL(fill_words_kernel, dim3((unsigned)((words + 1023) / 1024)), dim3(256), 0, s, reinterpret_cast<unsigned*>(ws), words, kNotYet);
+  const int rc = launched("fill_words_kernel");
+  if (rc) return rc;
+  (dtype == FCR_DTYPE_F16 ? fcr_detail::sweeps_f16_both : fcr_detail::sweeps_bf16_both)(p, ksteps, causal, mode, s);
+  return launched("both_sweeps_kernel");
+}
+
 int launch_few_keys(Params& p, int dtype, int ksteps, const FewKeysPlan& o, float* ws, int mode, bool causal, hipStream_t s) {
   p.lse = ws;
   Params sweep = p;
@@ -5135,8 +5338,6 @@ size_t fcr_lse_bytes_two_kernels(int B, int H, int M, int N) {
 }
 
 // process-wide switches (fcr_set_option)
-int g_single_sweep = 1;
-long long g_wait_polls = 1ll << 20;
 }  // namespace
 thread_local bool fcr_detail::fused_refused = false;
 
@@ -5421,6 +5622,10 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
     const int lrc = fcr_detail::fused_refused ? 0 : launched("col_fused_kernel");
     order_end(order, s, !fcr_detail::fused_refused && lrc == 0);
     if (!fcr_detail::fused_refused) return lrc;
+  }
+  if (single) {
+    const BothPlan o = both_plan(dtype, ksteps, p.bh_count, M, N, causal != 0);
+    if (o.row_blocks > 0) return launch_both(p, dtype, ksteps, o, ws, mode, causal != 0, static_cast<hipStream_t>(stream));
   }
   rc = fcr_row_lse(q, k, ws, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream);
   if (rc) return rc;

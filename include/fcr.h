@@ -75,8 +75,8 @@ extern "C" {
 #define FCR_E_WAIT -8      /* fcr_colreduce_status: a workgroup of the single sweep gave up waiting for its team */
 
 /* fcr_set_option */
-#define FCR_OPT_SINGLE_SWEEP 0 /* 0: few queries against many keys, one query and few keys take the two kernels as well (default 1) */
-#define FCR_OPT_WAIT_POLLS 1   /* polls of a team's slots after which a workgroup gives up (default 2^20) */
+#define FCR_OPT_SINGLE_SWEEP 0 /* 0: every call takes the two kernels, in two launches (default 1) */
+#define FCR_OPT_WAIT_POLLS 1   /* polls, of a team's slots or of the row statistics, after which a workgroup gives up (default 2^20) */
 
 /* size of the built-in scratch buffer of fcr_colreduce_static, per GPU */
 #define FCR_STATIC_SCRATCH_BYTES (16u << 20)
@@ -169,7 +169,9 @@ int fcr_topk_mask_typed(const void* scores, int dtype, uint8_t* mask, float* thr
 int fcr_pack_f32(const float* src, void* dst, int64_t rows, int D, int terms, int is_key, void* stream);
 
 /*
- * Both kernels back to back on one stream: the whole of _flash_colreduce (flash.py:277-308)
+ * Both kernels on one stream, back to back or, where that is the faster way, in one launch whose column sweeps wait for the
+ * row statistics they need (16-bit operands; a wait ends after FCR_OPT_WAIT_POLLS polls, with NaN columns, which takes a GPU
+ * that does not dispatch the workgroups of a launch in order): the whole of _flash_colreduce (flash.py:277-308)
  * except the final cast to the input dtype, which stays with the host.  lse_ws is scratch of
  * fcr_lse_bytes(B,H,M,N,D) bytes whose first B*H*M floats hold the row statistics on return.
  */
@@ -267,7 +269,7 @@ int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, in
 int fcr_colreduce_status(const float* lse_ws, int dtype, int B, int H, int M, int N, int D, void* stream);
 
 /*
- * Process-wide switches (FCR_OPT_*), read by every later call: the single sweep on or off (results agree
+ * Process-wide switches (FCR_OPT_*), read by every later call: every path but the two launches on or off (results agree
  * to rounding either way) and the bound on its waits.  For tests and comparisons; returns 0 or FCR_E_SHAPE.
  */
 int fcr_set_option(int option, long long value);

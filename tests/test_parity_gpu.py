@@ -2115,3 +2115,95 @@ def test_python_errors_on_device():
     torch.testing.assert_close(out, torch.full((1, 2, 6), 1 / 6, device="cuda"))
     assert fca.flash_colreduce(q[:, :, :0], k, "sum").shape == (1, 2, 6)
     assert fca.flash_colreduce(q, k[:, :, :0], "sum").shape == (1, 2, 0)
+
+
+@pytest.mark.parametrize("h,m,n,d,dtype,causal", [
+    (3, 700, 700, 128, torch.float16, True), (2, 900, 640, 128, torch.bfloat16, True), (3, 600, 850, 128, torch.float16, True),
+    (1, 513, 513, 104, torch.float16, True), (60, 1000, 1000, 128, torch.bfloat16, True), (240, 520, 520, 128, torch.float16, True),
+    (5, 1101, 1101, 64, torch.float16, True), (270, 520, 521, 48, torch.bfloat16, True), (4, 640, 640, 24, torch.float16, True),
+    (9, 777, 777, 96, torch.bfloat16, True), (100, 1000, 1000, 80, torch.float16, True), (3, 530, 530, 256, torch.float16, True),
+    (2, 1200, 1200, 200, torch.bfloat16, True), (1, 641, 600, 136, torch.float16, True),
+    (130, 600, 600, 128, torch.float16, False), (250, 530, 530, 128, torch.bfloat16, False), (100, 530, 540, 128, torch.float16, False),
+    (130, 600, 600, 64, torch.bfloat16, False), (130, 576, 600, 160, torch.float16, False), (240, 600, 1500, 72, torch.float16, False)])
+def test_both_sweeps_in_one_launch(h, m, n, d, dtype, causal):
+    """Every tile size of the launch that holds both sweeps, ragged tiles and chunks, more and fewer keys than queries: sums, maxima,
+    both and the row statistics, against 64 bits (see test_few_keys for the bound) and, where the row sweep of the two launches is not
+    split, bit for bit against those."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(h + m + n)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g).to(dtype) for r in (m, n))
+    sums, most = _columns_f64(q, k, causal)
+    got = {}
+    for option in (1, 0):
+        lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+        try:
+            one = [fca.flash_colreduce(q, k, red, causal, out_dtype=torch.float32) for red in ("sum", "max")]
+            pair = fca.flash_colreduce_multi(q, k, ["sum", "max"], causal, out_dtype=torch.float32)
+            ws, out = torch.empty(_lib_workspace(q, k), device="cuda"), torch.empty(h, n, device="cuda")
+            _ws_call(q, k, out, ws, causal)
+            got[option] = [*one, *pair, ws[: h * m].clone(), out.view(1, h, n)]
+        finally:
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+    for x, want in zip(got[1], (sums, most, sums, most, None, sums)):
+        assert want is None or (torch.isfinite(x).all() and _rel(x, want) <= 1e-5)
+    same = h * ((m + 255) // 256) >= 256 and m > 256   # no row sweep of these is split
+    for x, y in zip(got[1], got[0]):
+        assert torch.equal(x, y) if same else torch.allclose(x, y, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("h,m,n,d", [(3, 700, 700, 128), (60, 1000, 1000, 128), (5, 1100, 1100, 64), (2, 600, 600, 256)])
+def test_both_sweeps_in_one_launch_special_rows(h, m, n, d):
+    """Rows and keys that are not finite, scores of exactly zero (an lse of 0 for the row that sees one key), scales of any sign:
+    NaN in the same columns as with two launches, the others the same to rounding."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(h + n)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g).half() for r in (m, n))
+    bad_q, bad_k, zero = q.clone(), k.clone(), torch.zeros_like(q)
+    bad_q[:, 0, m // 3, 0] = float("nan")
+    bad_q[:, -1, m - 1, 1] = float("inf")
+    bad_k[:, 0, n // 2, 0] = float("-inf")
+    for x, y, scale in ((bad_q, k, None), (q, bad_k, None), (zero, k, None), (q, k, 0.0), (q, k, -0.3)):
+        for red in ("sum", "max"):
+            got = {}
+            for option in (1, 0):
+                lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+                try:
+                    got[option] = fca.flash_colreduce(x, y, red, True, scale, out_dtype=torch.float32)
+                finally:
+                    lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+            torch.testing.assert_close(got[1], got[0], rtol=1e-4, atol=1e-6, equal_nan=True)
+
+
+@pytest.mark.parametrize("reduction", ["sum", "max", "pair"])
+def test_both_sweeps_wait_is_bounded(reduction):
+    """With no polls allowed the column sweeps, which all start beside the row sweeps here, give up: the kernel ends, the
+    columns are NaN, and the next call is right."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    q, k = (x.cuda() for x in _inputs.randn_pair(1, 4, 1200, 1200, 128, seed=5, dtype=torch.float16))
+    call = lambda: (fca.flash_colreduce_multi(q, k, ["sum", "max"], True) if reduction == "pair" else [fca.flash_colreduce(q, k, reduction, True)])
+    want = call()
+    lib.fcr_set_option(_lib.OPT_WAIT_POLLS, 0)
+    try:
+        assert all(x.isnan().any() for x in call())
+    finally:
+        lib.fcr_set_option(_lib.OPT_WAIT_POLLS, 1 << 20)
+    for x, y in zip(call(), want):
+        assert torch.isfinite(x).all() and torch.equal(x, y)
+
+
+def test_both_sweeps_under_graph_capture():
+    """The fill, the row sweeps and the column sweeps are kernels of one graph: replays on new operands, with eager calls and
+    synchronizations between them, give the eager result."""
+    q, k = (x.cuda() for x in _inputs.randn_pair(2, 6, 900, 900, 128, seed=3, dtype=torch.bfloat16))
+    fca.flash_colreduce(q, k, "sum", True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fca.flash_colreduce(q, k, "sum", True)
+    for step in range(4):
+        q.copy_(torch.randn_like(q))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, fca.flash_colreduce(q, k, "sum", True)), step
