@@ -51,7 +51,7 @@
 // use several cores): part 0 holds the C ABI and the small kernels, parts 1-4 the sweeps of one element
 // type each (fp16, bf16, fp32 rows up to 512 bytes, longer fp32 rows), parts 5 and 6 the sweeps over fp16 and
 // bf16 rows of more than 512 bytes, parts 7 and 8 the single sweep for fp16 and bf16, parts 9 and 10 few_keys_kernel for them,
-// parts 11 and 12 both_sweeps_kernel.
+// parts 11 and 12 both_sweeps_kernel, part 13 few_keys_f32_kernel.
 #ifndef FCR_PART
 #define FCR_PART -1
 #endif
@@ -90,6 +90,7 @@ struct Params {
   // both_sweeps_kernel: `tiles`, `group`, `fill` and `total` are of the row sweeps
   int col_tiles, col_group;
   int row_blocks, col_blocks;
+  int parts;         // few_keys_f32_kernel: ranges of a pair's queries whose columns are added up apart
 };
 // which: 0 = row statistics, 1 = column sweep, 2 = column sweep for few queries, 3 = both sweeps in one for few
 // queries, mode + 4 for more than 64 of them (2 and 3: 16-bit types only)
@@ -101,6 +102,7 @@ void sweeps_f16_single(const Params& p, int ksteps, bool causal, int mode, hipSt
 void sweeps_bf16_single(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 void sweeps_f16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s);   // few_keys_kernel
 void sweeps_bf16_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s);
+void sweeps_f32_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s);    // few_keys_f32_kernel
 void sweeps_f16_both(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);   // both_sweeps_kernel
 void sweeps_bf16_both(const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
 void sweeps_f16_long_rows(int which, const Params& p, int ksteps, bool causal, int mode, hipStream_t s);
@@ -1831,11 +1833,11 @@ __device__ __forceinline__ uint32_t lanes_max(uint32_t v) {
 constexpr int f32_chunk(int ks, int nw) { return (ks <= 2 ? 64 : ks <= 4 ? 32 : 16) * (nw / 4); }
 constexpr int f32_groups(int ks) { return ks <= 4 ? 2 : 1; }   // streamed 16-row groups per sub-step
 
-// KS: k-steps of 32 d.
-template <int KS, int NW>
+// KS: k-steps of 32 d; CR: rows of a chunk.
+template <int KS, int NW, int CR = f32_chunk(KS, NW)>
 struct SplitRing {
   static constexpr int kNumThreads = 64 * NW;
-  static constexpr int kChunkRows = f32_chunk(KS, NW);
+  static constexpr int kChunkRows = CR;
   static constexpr int kPitch = Ring<KS>::kPitch;            // bytes of a row in one plane
   static constexpr int kRowGranules = kPitch / 16;           // of eight values: threads that share a row
   static constexpr int kPlane = kChunkRows * kPitch;
@@ -1843,8 +1845,10 @@ struct SplitRing {
   static constexpr int kRowFloats = 2 * kChunkRows;          // two floats per row of a stage: its scale, and what the caller adds
   // two stages, their row floats, a word for each (see `bad`) and two for each wave (see `set_limit`)
   static constexpr int kBytes = 2 * kStage + 2 * kRowFloats * 4 + 16 + 8 * NW;
-  static constexpr int kPer = kChunkRows * kRowGranules / kNumThreads;   // granules per thread
-  static_assert(kPer * kNumThreads == kChunkRows * kRowGranules, "whole granules per thread");
+  static constexpr int kGranules = kChunkRows * kRowGranules;
+  static constexpr bool kAll = kGranules >= kNumThreads;                // every thread stages; else the first kGranules of them, whole waves
+  static constexpr int kPer = kAll ? kGranules / kNumThreads : 1;        // granules per staging thread
+  static_assert(kAll ? kPer * kNumThreads == kGranules : kGranules % 64 == 0, "whole granules per thread, whole waves");
 
   char* smem;
   uint32_t src[kPer];     // source byte offset inside a chunk of a granule
@@ -1882,8 +1886,8 @@ struct SplitRing {
 
   // The next chunk on its way to the registers; rows past the end arrive as zeros.
   template <int AUX = 0>
-  __device__ __forceinline__ void fetch() {
-    const int live = __builtin_amdgcn_readfirstlane(min(max(rows_left, 0), kChunkRows));
+  __device__ __forceinline__ void fetch(bool staging = true) {   // staging: of the waves that stage (see kAll)
+    const int live = __builtin_amdgcn_readfirstlane(staging ? min(max(rows_left, 0), kChunkRows) : 0);
     const __amdgpu_buffer_rsrc_t view =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(next_ptr), 0, (int)((uint32_t)live * (uint32_t)row_bytes), 0x00020000);
 #pragma unroll
@@ -2015,8 +2019,8 @@ template <int SG>
 struct Fragments {
   u32x4 f[2][SG];   // per plane and group
 };
-template <int SG, int KS, int NW>
-__device__ __forceinline__ Fragments<SG> read_fragments(const SplitRing<KS, NW>& rg, const char* stage, int sub, int ks) {
+template <int SG, int KS, int NW, int CR>
+__device__ __forceinline__ Fragments<SG> read_fragments(const SplitRing<KS, NW, CR>& rg, const char* stage, int sub, int ks) {
   Fragments<SG> x;
 #pragma unroll
   for (int t2 = 1; t2 >= 0; --t2)
@@ -2024,8 +2028,8 @@ __device__ __forceinline__ Fragments<SG> read_fragments(const SplitRing<KS, NW>&
     for (int sg = 0; sg < SG; ++sg) x.f[t2][sg] = rg.frag(stage, sub * SG + sg, ks, t2);
   return x;
 }
-template <bool RESIDENT_IS_KEYS, int KS, int NG, int SG, int NW, class BetweenF>
-__device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes (&res)[KS][NG], const SplitRing<KS, NW>& rg,
+template <bool RESIDENT_IS_KEYS, int KS, int NG, int SG, int NW, int CR, class BetweenF>
+__device__ __forceinline__ void split_scores(f32x4 (&acc)[NG][SG], const Planes (&res)[KS][NG], const SplitRing<KS, NW, CR>& rg,
                                              const char* stage, int sub, const Fragments<SG>& first, BetweenF&& between) {
   // products by plane: streamed l with h, h with l, h with h
   constexpr int kProducts = 3;
@@ -2353,6 +2357,336 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
       general);
   ring_sync<63>();
   col_store<MODE, NG>(p, smem, bh, k0, csum, cmax, lane, wave);
+}
+
+// ---------------------------------------------------------------------------------------------
+// few_keys_kernel for fp32 operands: the same work order, groups of keys, splits and columns, and the parts, limits and exact chunks of
+// the fp32 sweeps.  A row's maximum comes first in every chunk: every wave takes its own, its 2^score and their sum are relative to that, and
+// behind the barrier of the next chunk the waves' (maximum, sum) are merged, so no scores need another form.  Forming a score
+// is three matrix instructions per k-step and the split of its row, which the maximum adds little to.  At most 256 keys: two groups per
+// wave are what the registers hold in parts beside a chunk's scores (four groups of D <= 64 and 16 queries per chunk were built: 256 pairs of 512 x
+// 512 x 64 77 -> 63 us, with the mask 60 -> 67, and some forms kept registers in memory).  Bound by the chain of a chunk, barrier, merge,
+// products, maximum, exponents, sum, on two waves per SIMD: 4700 cycles per chunk of 32 queries against 256 keys of 128, of which 1540 are
+// matrix and 3000 port cycles.  Per call, two kernels -> this one: see few_keys_f32_plan.
+
+template <int KS, bool CAUSAL, int MODE, int NG, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void few_keys_f32_kernel(const Params p) {
+  constexpr int SQ = f32_groups(KS), CR = 16 * SQ;
+  using Rg = SplitRing<KS, NW, CR>;
+  constexpr int kSums = CR * NW;
+  constexpr int kSetsAt = (Rg::kBytes + 15) & ~15;
+  __shared__ __attribute__((aligned(1024))) char smem[kSetsAt + 4 * kSums * 4];
+  float* const sets = reinterpret_cast<float*>(smem + kSetsAt);   // by parity of the chunk: maxima, then sums, [query][wave]
+  const int split = (int)blockIdx.z, S = p.splits, bh = (int)blockIdx.y * p.H + (int)blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const char* qb = p.q + (int64_t)blockIdx.y * p.q_sb + (int64_t)blockIdx.x * p.q_sh;
+  const char* kb = p.k + (int64_t)blockIdx.y * p.k_sb + (int64_t)blockIdx.x * p.k_sh;
+  const bool staging = Rg::kAll || wave * 64 < Rg::kGranules;
+  // The chunks of a pair are dealt in p.parts ranges of L, the last one shorter perhaps, and a workgroup takes ranges split, split + S, ..
+  const int all = (p.M + CR - 1) / CR, L = __builtin_amdgcn_readfirstlane((all + p.parts - 1) / p.parts);
+  const int ranges = __builtin_amdgcn_readfirstlane((p.parts - split + S - 1) / S);
+  const int chunks = min(ranges * L, all - (split + (ranges - 1) * S) * L + (ranges - 1) * L);   // of this workgroup
+
+  Rg rg;
+  rg.init(smem, qb, p.q_sr, split * L * CR, p.M, p.dgran, tid);
+  int fetched = 0;   // of a range
+  auto fetch = [&]() __attribute__((always_inline)) {   // in order: the cursor walks over the workgroup's chunks
+    rg.fetch(staging);
+    if (++fetched == L) {
+      fetched = 0;
+      rg.next_ptr += (int64_t)(S - 1) * L * CR * p.q_sr;
+      rg.rows_left -= (S - 1) * L * CR;
+    }
+  };
+  uint32_t largest = 0;
+  auto put = [&](int i) __attribute__((always_inline)) {
+    if (!staging) return;
+#pragma unroll
+    for (int j = 0; j < Rg::kPer; ++j) rg.put_granule(j, i, tid, largest);
+  };
+  fetch();   // in flight together with the keys
+  int k0[NG];
+  f32x4 csum[NG], cmax[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    k0[g] = 16 * (wave + NW * g);
+    csum[g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    cmax[g] = (f32x4){kNegInf, kNegInf, kNegInf, kNegInf};
+  }
+  Planes kf[KS][NG];
+  f32x4 ks4[NG];   // what undoes the scale of the lane's four keys per group, with the sign of the scale
+  const float sign = p.scale2 < 0.f ? -1.f : 1.f, up = fabsf(p.scale2);
+  uint32_t k_largest;
+  {
+    float down[NG];
+    k_largest = load_resident_split<KS, NG>(kf, down, kb, p.k_sr, k0, p.N, p.dgran, lane);
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ks4[g][r] = sign * __shfl(down[g], 4 * (lane >> 4) + r);
+  }
+  const bool res_bad = has_no_scale(k_largest);
+
+  const int live_all = max(0, min(NG, (p.N - 16 * wave + 16 * NW - 1) / (16 * NW)));   // groups with keys
+  auto live_groups = [&](int q0) __attribute__((always_inline)) {   // those that some query of a chunk sees
+    if (!CAUSAL) return live_all;
+    const int last = q0 + CR - 1 + p.c - 16 * wave;
+    return last < 0 ? 0 : min(live_all, last / (16 * NW) + 1);
+  };
+  // first row from which on every query sees every key of the wave, and all of its groups are whole
+  const int full_row = k0[NG - 1] + 16 > p.N ? 0x7fffffff : CAUSAL ? max(0, k0[NG - 1] + 15 - p.c) : 0;
+
+  // Of the chunk whose columns are added up next: its products (sums: 2^score relative to the wave's maximum), the maximum per row, what
+  // its queries' products are scaled by, and whether some key is hidden from some row of it (or a row is padding).
+  f32x4 x[NG][SQ];
+  float most[SQ], s2[SQ];
+  bool some_hidden = false, no_scale = false;   // no_scale: some s2 is 0, which makes a NaN of a hidden product (-inf)
+  int live = 0, kept_row = 0;
+  // body(g, sq, seen) for every group in use; seen(r) is a question only in groups that are hidden in part, and there if it has to be
+  auto groups = [&](auto masked_tag, bool ask, int lane_again, auto body) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_tag)::value;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (MASKED && g >= live) continue;
+      if (!MASKED || !ask || (g + 1 < live && kept_row + CR <= p.M)) {
+#pragma unroll
+        for (int sq = 0; sq < SQ; ++sq) body(g, sq, [](int) { return true; });
+      } else {
+#pragma unroll
+        for (int sq = 0; sq < SQ; ++sq) {
+          const int key = k0[g] + 4 * (lane_again >> 4), q = kept_row + 16 * sq + (lane_again & 15);
+          const int lim = q >= p.M ? -1 : CAUSAL ? min(p.N - 1 - key, q + p.c - key) : p.N - 1 - key;
+          body(g, sq, [lim](int r) { return r <= lim; });
+        }
+      }
+    }
+  };
+  // The (maximum, sum) that the waves left of the rows of chunk i: each row of lanes takes its share of the waves.
+  constexpr int PW = NW / 4;
+  float wm[SQ][PW], wl[SQ][PW];
+  auto read_partials = [&](int i) __attribute__((always_inline)) {
+    const float* const set = sets + (i & 1) * 2 * kSums;
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq)
+#pragma unroll
+      for (int v = 0; v < PW; ++v) {
+        const int at = (16 * sq + (lane & 15)) * NW + PW * (lane >> 4) + v;
+        wm[sq][v] = set[at];
+        wl[sq][v] = set[kSums + at];
+      }
+  };
+  // Columns of the kept chunk, whose partials have been read.
+  auto columns = [&](auto masked_tag) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_tag)::value;
+    int lane_again = lane;   // opaque: what follows from it is not to be kept in registers from chunk to chunk
+    asm volatile("" : "+v"(lane_again));
+    float factor[SQ], lse[SQ];
+    bool odd = no_scale;
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {
+      float m[1] = {wm[sq][0]}, l[1] = {0.f};
+#pragma unroll
+      for (int v = 1; v < PW; ++v) m[0] = fmaxf(m[0], wm[sq][v]);
+      m[0] = lane_rows_reduce<true>(m);
+      const float ref = m[0] == kNegInf ? 0.f : m[0];
+#pragma unroll
+      for (int v = 0; v < PW; ++v) l[0] = fmaf(wl[sq][v], fast_exp2(wm[sq][v] - ref), l[0]);   // (a wave without a key: 0 times 0)
+      l[0] = lane_rows_reduce<false>(l);
+      lse[sq] = l[0] == 0.f ? kNegInf : ref + fast_log2(l[0]);
+      factor[sq] = (most[sq] == kNegInf ? 0.f : fast_exp2(most[sq] - ref)) * __builtin_amdgcn_rcpf(l[0]);
+    }
+    if (wave == 0) {
+      float v = lse[0];
+#pragma unroll
+      for (int sq = 1; sq < SQ; ++sq) v = lane_again >> 4 == sq ? lse[sq] : v;
+      if (lane_again < CR && kept_row + lane_again < p.M) p.lse[(int64_t)bh * p.M + kept_row + lane_again] = v;
+    }
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {
+      if (MASKED && kept_row + 16 * sq + (lane_again & 15) >= p.M) factor[sq] = 0.f, lse[sq] = kPosInf;
+      odd = odd || !(MODE == kModeSum ? factor[sq] < kPosInf : lse[sq] > kNegInf);   // a NaN, or a row whose scores are all -inf
+    }
+    groups(masked_tag, MASKED && __builtin_amdgcn_ballot_w64(odd) != 0, lane_again, [&](int g, int sq, auto seen) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (MODE == kModeSum) {
+          csum[g][r] = seen(r) ? fmaf(x[g][sq][r], factor[sq], csum[g][r]) : csum[g][r];
+        } else {
+          const float y = seen(r) ? fmaf(x[g][sq][r], s2[sq], -lse[sq]) : kNegInf;
+          if (MODE == kModeBoth) csum[g][r] += fast_exp2(y);
+          cmax[g][r] = fmaxf(cmax[g][r], y);
+        }
+      }
+    });
+  };
+  // The products of chunk i, whose groups in use are `live`, become the kept ones.
+  auto exponents = [&](int i, f32x4(&acc)[NG][SQ], bool exact, auto masked_tag) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_tag)::value;
+    int lane_again = lane;
+    asm volatile("" : "+v"(lane_again));
+    float part[SQ];
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {
+      s2[sq] = MASKED && exact ? up : up * rg.scale_of(i)[16 * sq + (lane_again & 15)];
+      most[sq] = kNegInf;
+      part[sq] = 0.f;
+    }
+    if (MASKED) no_scale = __builtin_amdgcn_ballot_w64(s2[0] == 0.f || s2[SQ - 1] == 0.f) != 0;   // (a scale of 0, or rows so small, padding too)
+    groups(masked_tag, MASKED, lane_again, [&](int g, int sq, auto seen) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float y = acc[g][sq][r] * (MASKED && exact ? sign : ks4[g][r]);
+        x[g][sq][r] = seen(r) ? y : kNegInf;
+        most[sq] = fmaxf(most[sq], x[g][sq][r]);
+      }
+    });
+#pragma unroll
+    for (int sq = 0; sq < SQ; ++sq) {   // the largest score; -inf if the row sees none of the wave's keys
+      const float m[1] = {most[sq] == kNegInf ? kNegInf : most[sq] * s2[sq]};
+      most[sq] = lane_rows_reduce<true>(m);
+    }
+    groups(masked_tag, MASKED && no_scale, lane_again, [&](int g, int sq, auto seen) __attribute__((always_inline)) {
+      const float ref = most[sq] == kNegInf ? 0.f : most[sq];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {   // (+inf - inf is a NaN, as the row kernel's lse then is)
+        const float e = seen(r) ? fast_exp2(fmaf(x[g][sq][r], s2[sq], -ref)) : 0.f;
+        part[sq] += e;
+        if (MODE == kModeSum) x[g][sq][r] = e;
+      }
+    });
+    float* const set_m = sets + (i & 1) * 2 * kSums;
+    auto write_reduced = [&](float* set, float v) __attribute__((always_inline)) {
+      if constexpr (SQ == 1) {
+        if (lane_again < 16) set[lane_again * NW + wave] = v;
+      } else {
+        if ((lane_again & 16) == 0) set[((lane_again >> 5) * 16 + (lane_again & 15)) * NW + wave] = v;
+      }
+    };
+    write_reduced(set_m, SQ == 1 || lane_again < 32 ? most[0] : most[SQ - 1]);
+    write_reduced(set_m + kSums, lane_rows_reduce<false>(part));
+  };
+
+  put(0);
+  fetch();
+  {
+    const uint32_t first = lanes_max<16>(largest);
+    uint32_t wave_largest = 0;
+#pragma unroll
+    for (int l = 0; l < 64; l += 16) wave_largest = max(wave_largest, (uint32_t)__builtin_amdgcn_readlane((int)first, l));
+    rg.publish(wave, k_largest, wave_largest);
+  }
+  ring_sync<63>();   // the first chunk is staged (waits for LDS accesses only: the fetch stays in flight)
+  const bool first_bad = rg.set_limit(p.split_most);
+  // the products of the first G groups, the keys in parts
+  auto products = [&](f32x4(&acc)[NG][SQ], const char* stage, auto groups_tag, auto between) __attribute__((always_inline)) {
+    constexpr int G = decltype(groups_tag)::value;
+    if constexpr (G == NG) {
+      split_scores<true>(acc, kf, rg, stage, 0, read_fragments<SQ>(rg, stage, 0, 0), between);
+    } else {
+      Planes keys[KS][G];
+      f32x4 part[G][SQ];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int g = 0; g < G; ++g) keys[ks][g] = kf[ks][g];
+      split_scores<true>(part, keys, rg, stage, 0, read_fragments<SQ>(rg, stage, 0, 0), between);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int sq = 0; sq < SQ; ++sq) acc[g][sq] = part[g][sq];
+    }
+  };
+  // The columns of a range: a reduce-scatter over the 16 query lanes; lane l ends up with key 4 * (l / 16) + (l & 3) of group (l & 15) / 4.
+  const int col_grp = (lane & 15) >> 2, col_key = 16 * (wave + NW * col_grp) + 4 * (lane >> 4) + (lane & 3);
+  const bool col_mine = col_grp < NG && col_key < p.N;
+  float sum = 0.f, peak = 0.f;   // S == 1: of the ranges so far, added up in the order of merge_columns_kernel
+  auto end_range = [&](int range) __attribute__((always_inline)) {
+    f32x4 c4[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) c4[g] = g < NG ? csum[g % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
+    const float s = MODE != kModeMax ? lanes16_scatter<false>(c4, lane) : 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) c4[g] = g < NG ? cmax[g % NG] : (f32x4){0.f, 0.f, 0.f, 0.f};
+    const float m = MODE != kModeSum ? fast_exp2(lanes16_scatter<true>(c4, lane)) : 0.f;
+    if (S == 1) {
+      sum += s;
+      peak = fmaxf(peak, m);
+    } else if (col_mine) {
+      const int64_t at = ((int64_t)range * p.bh_count + bh) * p.N + col_key;
+      if (MODE != kModeMax) static_cast<float*>(p.out)[at] = s;
+      if (MODE != kModeSum) static_cast<float*>(MODE == kModeBoth ? p.out2 : p.out)[at] = m;
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      csum[g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      cmax[g] = (f32x4){kNegInf, kNegInf, kNegInf, kNegInf};
+    }
+  };
+  auto finish_chunk = [&](int i) __attribute__((always_inline)) {
+    read_partials(i);
+    if (some_hidden) columns(std::true_type());
+    else columns(std::false_type());
+  };
+  // Chunk i: the columns of the chunk before, its own products, their exponents.
+  int range = split, in_range = 0, q0 = split * L * CR;
+#pragma unroll 1
+  for (int i = 0; i < chunks; ++i) {
+    if (i > 0) ring_sync<63>();
+    const bool exact = res_bad || (i == 0 ? first_bad : rg.is_bad(i));
+    const char* stage = rg.stage_of(i);
+    f32x4 acc[NG][SQ];
+    largest = 0;
+    if (i > 0) {
+      finish_chunk(i - 1);
+      if (in_range == 0) end_range(range - S);
+    }
+    if (exact || q0 < full_row || q0 + CR > p.M) {
+      const int in_use = live_groups(q0);
+      put(i + 1);
+      fetch();
+      if (exact) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int sq = 0; sq < SQ; ++sq) acc[g][sq] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        exact_scores<true>(acc, kb, p.k_sr, k0, p.N, qb, p.q_sr, q0, p.M, p.dgran, lane);
+      } else if (in_use > NG / 2) {
+        products(acc, stage, std::integral_constant<int, NG>(), [](int) {});
+      } else if (in_use > 0) {
+        products(acc, stage, std::integral_constant<int, NG / 2>(), [](int) {});
+      }
+      live = in_use;
+      kept_row = q0;
+      some_hidden = true;
+      exponents(i, acc, exact, std::true_type());
+    } else {
+      products(acc, stage, std::integral_constant<int, NG>(), [&](int ks) {
+        if (ks == 0) {
+          put(i + 1);
+          fetch();
+        }
+      });
+      live = NG;
+      kept_row = q0;
+      some_hidden = false;
+      exponents(i, acc, false, std::false_type());
+    }
+    rg.note(i + 1, largest);
+    q0 += CR;
+    if (++in_range == L) {
+      in_range = 0;
+      range += S;
+      q0 += (S - 1) * L * CR;
+    }
+  }
+  ring_sync<63>();
+  finish_chunk(chunks - 1);
+  end_range(in_range == 0 ? range - S : range);
+  if (S == 1 && col_mine) {
+    if (MODE != kModeMax) store_column(p, p.out, true, bh, col_key, sum);
+    if (MODE != kModeSum) store_column(p, MODE == kModeBoth ? p.out2 : p.out, false, bh, col_key, peak);
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -4537,7 +4871,7 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   p.teams = 0;
   p.sync = nullptr;
   p.spin_limit = 0;
-  p.col_tiles = p.col_group = p.row_blocks = p.col_blocks = 0;
+  p.col_tiles = p.col_group = p.row_blocks = p.col_blocks = p.parts = 0;
   return 0;
 }
 
@@ -4669,16 +5003,69 @@ OneQueryPlan one_query_plan(int dtype, int64_t bh, int N, int D, int64_t base_fl
 struct FewKeysPlan {
   int form;          // keys of a workgroup: 128 << form
   int splits;        // workgroups per pair
-  int64_t part_at, floats;   // where the columns of the splits start and the workspace ends, in floats
+  int parts;         // sets of columns that they leave (16-bit operands: one each)
+  int64_t part_at, floats;   // where the columns of the parts start and the workspace ends, in floats
 };
+// The same for fp32 operands in parts (few_keys_f32_kernel): up to 256 keys, in four waves up to 128 and in eight beyond; ks: k-steps of
+// 32 d.  Against the two kernels, 11600 shapes of 1 to 1500 pairs, 40 to 8192 queries, all reductions, with and without the mask: 0.66 of
+// their time where it is taken, 0.47 where several workgroups share a pair (2 pairs of 256 x 256 x 64 13.7 -> 8.9 us, 32 of 256 x 256 x 128 20.8 -> 11.9,
+// 512 of them 77 -> 52, 4 of 4096 x 256 x 128 117 -> 17, 256 of them 480 -> 294).
+// Below 1024 queries the path and the ranges of queries whose columns are added up apart (at most eight) follow from M, N and D alone, so that
+// the bits of a result do not depend on the number of pairs; left out are rows of up to 128 bytes against so many queries that the sweeps, which stage
+// four times the rows between two barriers, win for most numbers of pairs (206 of 900 x 172 x 48 1.15 times their time, 166 of 497 x 164 x 32 1.28).
+// From 1024 on ranges are one to a workgroup, and long calls of short rows that fill neither the chip nor the registers are left out, as few_keys_plan
+// does (`least`: 280 pairs of 5698 x 39 x 32, both, 199 -> 344; 137 of 7618 x 226 x 48 368 -> 479; 316 of 2605 x 14 x 32 93 -> 143).
+// Of what is taken 2 % lose 3 % or more, nearly all rows of D <= 64.  Two chunks (three of at most 128 keys) go to one workgroup, whose launch is
+// the only one (2 pairs of 64 x 64 x 64 7.3 -> 6.5, but of 128 x 64 x 64 9.1 and 10.6).
+FewKeysPlan few_keys_f32_plan(FewKeysPlan o, int64_t bh, int M, int N, int ks, bool both, int64_t base_floats) {
+  if (N > 256) return o;
+  const int form = N > 128 ? 1 : 0, rows = 16 * f32_groups(ks);
+  const int64_t chunks = ((int64_t)M + rows - 1) / rows, places = (form == 1 ? 1 : 2) * (int64_t)chip_cus();
+  const bool short_call = M < 1024;
+  int64_t s = places / bh;
+  if (s > chunks) s = chunks;
+  if (s < 1 || chunks <= (form == 1 ? 2 : 3)) s = 1;
+  const int64_t len = short_call ? (chunks + 7) / 8 : (chunks + s - 1) / s, parts = (chunks + len - 1) / len;   // (no part is empty)
+  if (s > parts) s = parts;
+  if (short_call) {
+    if (ks == 1 ? chunks >= (form == 1 ? 8 : 16) : ks == 2 && form == 1 && chunks >= 16) return o;
+  } else if (s <= 3) {
+    // chunks one behind the other, and the share of the chip's workgroups and of their keys that is there
+    const int64_t rounds = (bh * s + places - 1) / places, steps = rounds * ((chunks + s - 1) / s);
+    const double filled = (double)(bh * s) / (double)(rounds * places) * N / (128 << form);
+    double least = 0.0;
+    if (form == 1) {
+      if (ks == 1) least = 2.0;
+      else if (ks == 2) least = steps >= 64 ? 0.85 : steps >= 32 ? 0.6 : 0.4;
+      else if (steps >= 64) least = ks == 8 ? 0.3 : ks == 4 ? 0.4 : 0.5;
+      else if (ks == 3) least = 0.4;
+    } else if (ks == 1) {
+      least = steps >= 64 ? 0.6 : steps >= 32 ? 0.4 : 0.3;
+    } else if (ks == 2) {
+      least = steps >= 64 ? 0.3 : steps >= 32 ? 0.2 : 0.1;
+    } else if (ks > 4 && s == 1 && steps >= 64) {
+      least = 0.1;
+    }
+    if (filled < least) return o;
+  }
+  o.form = form;
+  o.splits = (int)s;
+  o.parts = (int)parts;
+  if (s > 1) {
+    o.part_at = (base_floats + 63) / 64 * 64;
+    o.floats = o.part_at + (both ? 2 : 1) * parts * bh * N;
+  }
+  return o;
+}
 FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool both, int64_t base_floats) {
   FewKeysPlan o;
   o.form = -1;
-  o.splits = 1;
+  o.splits = o.parts = 1;
   o.part_at = o.floats = base_floats;
   const int ks = ksteps_of(dtype, D);
   const int64_t bh = (int64_t)B * H;
-  if (dtype == FCR_DTYPE_F32 || ks > kMaxKSteps || M < 2 || B > 65535 || bh >= kMaxWorkgroups / 2) return o;   // (the grid's limits)
+  if ((dtype == FCR_DTYPE_F32 ? !in_parts(dtype, D) : ks > kMaxKSteps) || M < 2 || B > 65535 || bh >= kMaxWorkgroups / 2) return o;   // (the grid's limits)
+  if (dtype == FCR_DTYPE_F32) return few_keys_f32_plan(o, bh, M, N, f32_ksteps(ks), both, base_floats);
   const int groups = few_keys_groups(ks), most = groups == 4 ? 2 : 1;
   int form = 0;
   while (form <= most && N > (128 << form)) ++form;
@@ -4709,7 +5096,7 @@ FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool bot
       return o;
     }
   }
-  o.splits = (int)s;
+  o.splits = o.parts = (int)s;
   if (s > 1) {
     o.part_at = (base_floats + 63) / 64 * 64;
     o.floats = o.part_at + (both ? 2 : 1) * s * bh * N;
@@ -4975,6 +5362,24 @@ void launch_few_keys(const Params& p, bool causal, int mode, int form, hipStream
   else launch_few_keys_mode<DT, KS, kModeBoth>(p, causal, form, s);
 }
 
+template <int KS, int MODE, int NG, int NW>
+void launch_few_keys_f32_form(const Params& p, bool causal, hipStream_t s) {
+  const dim3 grid((unsigned)p.H, (unsigned)(p.bh_count / p.H), (unsigned)p.splits), block(64 * NW);
+  if (causal) hipLaunchKernelGGL((few_keys_f32_kernel<KS, true, MODE, NG, NW>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((few_keys_f32_kernel<KS, false, MODE, NG, NW>), grid, block, 0, s, p);
+}
+template <int KS, int MODE>
+void launch_few_keys_f32_mode(const Params& p, bool causal, int form, hipStream_t s) {
+  if (form == 0) return launch_few_keys_f32_form<KS, MODE, 2, 4>(p, causal, s);
+  launch_few_keys_f32_form<KS, MODE, 2, 8>(p, causal, s);
+}
+template <int KS>
+void launch_few_keys_f32(const Params& p, bool causal, int mode, int form, hipStream_t s) {
+  if (mode == kModeSum) launch_few_keys_f32_mode<KS, kModeSum>(p, causal, form, s);
+  else if (mode == kModeMax) launch_few_keys_f32_mode<KS, kModeMax>(p, causal, form, s);
+  else launch_few_keys_f32_mode<KS, kModeBoth>(p, causal, form, s);
+}
+
 template <int DT, int KS, int MODE, int NBR, int NBC>
 void launch_both_tiles(const Params& p, bool causal, hipStream_t s) {
   const dim3 grid((unsigned)(((p.total + 7) & ~7) + p.bh_count * p.col_tiles)), block(kThreads);
@@ -5078,6 +5483,20 @@ void fcr_detail::sweeps_f16_both(const Params& p, int ksteps, bool causal, int m
 #if FCR_HAS(12)
 void fcr_detail::sweeps_bf16_both(const Params& p, int ksteps, bool causal, int mode, hipStream_t s) {
   FCR_DISPATCH_KS(FCR_DTYPE_BF16, ksteps, FCR_CALL_BOTH)
+}
+#endif
+#if FCR_HAS(13)
+void fcr_detail::sweeps_f32_few_keys(const Params& p, int ksteps, bool causal, int mode, int form, hipStream_t s) {
+  switch (f32_ksteps(ksteps)) {
+    case 1: launch_few_keys_f32<1>(p, causal, mode, form, s); break;
+    case 2: launch_few_keys_f32<2>(p, causal, mode, form, s); break;
+    case 3: launch_few_keys_f32<3>(p, causal, mode, form, s); break;
+    case 4: launch_few_keys_f32<4>(p, causal, mode, form, s); break;
+    case 5: launch_few_keys_f32<5>(p, causal, mode, form, s); break;
+    case 6: launch_few_keys_f32<6>(p, causal, mode, form, s); break;
+    case 7: launch_few_keys_f32<7>(p, causal, mode, form, s); break;
+    default: launch_few_keys_f32<8>(p, causal, mode, form, s); break;
+  }
 }
 #endif
 #if FCR_HAS(3)
@@ -5253,17 +5672,18 @@ int launch_few_keys(Params& p, int dtype, int ksteps, const FewKeysPlan& o, floa
   p.lse = ws;
   Params sweep = p;
   sweep.splits = o.splits;
+  sweep.parts = o.parts;
   if (o.splits > 1) {
     sweep.out = ws + o.part_at;
-    sweep.out2 = ws + o.part_at + (mode == kModeBoth ? (int64_t)o.splits * p.bh_count * p.N : 0);
+    sweep.out2 = ws + o.part_at + (mode == kModeBoth ? (int64_t)o.parts * p.bh_count * p.N : 0);
     sweep.out_fmt = FCR_DTYPE_F32;
     sweep.mean_from = -1;
   }
-  (dtype == FCR_DTYPE_F16 ? fcr_detail::sweeps_f16_few_keys : fcr_detail::sweeps_bf16_few_keys)(sweep, ksteps, causal, mode, o.form, s);
+  (dtype == FCR_DTYPE_F32 ? fcr_detail::sweeps_f32_few_keys : dtype == FCR_DTYPE_F16 ? fcr_detail::sweeps_f16_few_keys : fcr_detail::sweeps_bf16_few_keys)(sweep, ksteps, causal, mode, o.form, s);
   const int rc = launched("few_keys_kernel");
   if (rc || o.splits == 1) return rc;
   p.part = ws + o.part_at;
-  p.splits = o.splits;
+  p.splits = o.parts;
   const dim3 grid((unsigned)((p.bh_count * (int64_t)p.N + 255) / 256)), block(256);
   if (mode == kModeSum) hipLaunchKernelGGL(merge_columns_kernel<kModeSum>, grid, block, 0, s, p);
   else if (mode == kModeMax) hipLaunchKernelGGL(merge_columns_kernel<kModeMax>, grid, block, 0, s, p);

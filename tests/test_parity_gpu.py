@@ -1874,9 +1874,94 @@ def test_few_keys_small_probabilities_of_small_sums(m, n, d, causal):
     assert ((low.double() - want).abs() <= 2.0 ** -8 * want).all()
 
 
-def test_few_keys_under_graph_capture():
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [
+    (1, 2, 1, 32), (3, 31, 15, 64), (2, 33, 129, 128), (300, 65, 128, 72), (5, 300, 256, 128), (2, 257, 255, 60), (20, 200, 200, 40),
+    (2, 1000, 17, 96), (9, 1056, 33, 128), (3, 5000, 250, 64), (3, 100, 256, 256), (4, 16, 130, 192), (150, 49, 250, 160), (260, 15, 127, 224), (2, 256, 256, 64),
+    # on both sides of the lines that leave long calls, and more keys, to the two kernels
+    (128, 257, 256, 32), (2, 224, 200, 32), (130, 520, 40, 64), (130, 512, 200, 64), (260, 1100, 30, 64), (260, 1500, 20, 36), (4, 90, 257, 64)])
+def test_few_keys_f32(h, m, n, d, causal):
+    """fp32 pairs whose keys fit a workgroup's registers: sums, maxima, both and the row statistics against 64 bits, to the 1e-5 that fp32
+    operands are held to everywhere, and no further off than 1.15 times the two kernels (their own spread between shapes) in any of them."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(h + m + n)
+    q, k = (torch.randn(2, h, r, d, device="cuda", generator=g) for r in (m, n))
+    sums, most = _columns_f64(q, k, causal)
+    err = {}
+    for option in (1, 0):
+        lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+        try:
+            one = [fca.flash_colreduce(q, k, red, causal) for red in ("sum", "max")]
+            two = fca.flash_colreduce_multi(q, k, ["sum", "max"], causal)
+            ws = torch.empty(lib.fcr_workspace_bytes(_lib.DTYPE_F32, 2, h, m, n, d) // 4, device="cuda")
+            out = torch.empty(2 * h, n, device="cuda")
+            _lib.check(lib.fcr_colreduce_ws(
+                q.data_ptr(), k.data_ptr(), out.data_ptr(), None, _lib.DTYPE_F32, ws.data_ptr(), 4 * ws.numel(), _lib.DTYPE_F32, 2, h, m, n, d,
+                _lib.strides4(q.stride()), _lib.strides4(k.stride()), d ** -0.5, _lib.REDUCE_SUM, int(causal), torch.cuda.current_stream().cuda_stream))
+        finally:
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+        torch.testing.assert_close(ws[: 2 * h * m].view(2, h, m), fca.row_lse2(q, k, causal), rtol=1e-5, atol=1e-5)
+        assert torch.equal(out.view(2, h, n), one[0])
+        err[option] = [_rel(x, want) for x, want in ((one[0], sums), (one[1], most), (two[0], sums), (two[1], most))]
+    for now, before in zip(err[1], err[0]):
+        assert now <= 1e-5 and now <= max(1.15 * before, 1.2e-7), err
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(2, 70, 70, 64), (3, 100, 250, 128), (300, 40, 100, 32), (2, 65, 250, 256)])
+def test_few_keys_f32_special_rows(h, m, n, d, causal):
+    """fp32 rows that the parts do not take (not finite, from 2^104 on, elements of 600 on both sides), scores far from zero, scales of any
+    sign, token-major and padded layouts: NaN in the columns of the two kernels, the others the same to what scores of magnitude 2^9 leave."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g) for r in (m, n))
+    cases = [(q, k, None), (q, k, 0.0), (q, k, -0.2), (q * 30, k, 1.0 / d ** 0.5), (q + 5, k - 5, None), (torch.zeros_like(q), k, None)]
+    for value in (float("nan"), float("inf"), float("-inf")):
+        bad_q, bad_k = q.clone(), k.clone()
+        bad_q[:, 0, m // 3, 1] = value
+        bad_k[:, -1, n // 2, 0] = value
+        cases += [(bad_q, k, None), (q, bad_k, None), (bad_q, bad_k, -0.1)]
+    big_q, big_k = q.clone(), k.clone()
+    big_q[:, :, m - 1] *= 2.0 ** 110
+    big_k[:, 0, n - 1] *= 2.0 ** 105
+    cases += [(big_q, k, 2.0 ** -110), (q, big_k, 2.0 ** -106)]
+    one_q, one_k = q.clone(), k.clone()
+    one_q[:, :, 5:7, 0] = 600.0   # (past 300 on both sides, with scores below 2^9)
+    one_k[:, :, :3, 1] = 600.0
+    cases += [(one_q, one_k, None)]
+    wide = torch.randn(1, n, h, d + 4, device="cuda", generator=g)[..., :d].transpose(1, 2)
+    cases += [(q.transpose(1, 2).contiguous().transpose(1, 2), wide, None)]
+    for at, (x, y, scale) in enumerate(cases):
+        for red in ("sum", "max", "pair"):
+            got = {}
+            for option in (1, 0):
+                lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+                try:
+                    got[option] = (torch.stack(list(fca.flash_colreduce_multi(x, y, ["sum", "max"], causal, scale))) if red == "pair"
+                                   else fca.flash_colreduce(x, y, red, causal, scale))
+                finally:
+                    lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+            assert torch.equal(got[1].isnan(), got[0].isnan()), (at, red)
+            torch.testing.assert_close(got[1], got[0], rtol=2e-4, atol=1e-6, equal_nan=True, msg=lambda t: f"case {at} {red}: {t}")
+
+
+@pytest.mark.parametrize("h,m,n,d", [(1, 500, 250, 64), (3, 130, 70, 64), (1, 1023, 200, 128), (2, 700, 100, 256), (5, 97, 129, 40), (1, 66, 256, 192)])
+def test_few_keys_f32_bits_do_not_depend_on_the_number_of_pairs(h, m, n, d):
+    """Shared pairs, whose columns a second launch adds up, pairs of one workgroup each and pairs in several rounds, in the ranges of
+    queries that sizes alone set."""
+    q, k = (x.cuda() for x in _inputs.randn_pair(1, h, m, n, d, seed=m + n, dtype=torch.float32))
+    for copies in (60 // h, 600 // h):
+        qs, ks = q.repeat(copies, 1, 1, 1), k.repeat(copies, 1, 1, 1)
+        for red in REDUCTIONS:
+            assert torch.equal(fca.flash_colreduce(q, k, red, True)[0], fca.flash_colreduce(qs, ks, red, True)[-1]), (red, copies)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_few_keys_under_graph_capture(dtype):
     """Shared pairs (two launches) in a captured graph, replayed with other contents and eager calls between."""
-    q, k = (torch.randn(1, 4, r, 64, device="cuda").half() for r in (300, 200))
+    q, k = (torch.randn(1, 4, r, 64, device="cuda").to(dtype) for r in (300, 200))
     fca.flash_colreduce(q, k, "mean", True)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
