@@ -1028,7 +1028,7 @@ __device__ __forceinline__ void col_sweep(const Params& p, char* smem, int v) {
       }
       __builtin_amdgcn_s_sleep(8);
     }
-    reinterpret_cast<uint32_t*>(lse_slot(t))[lane] = x;
+    if (x != kNotYet) reinterpret_cast<uint32_t*>(lse_slot(t))[lane] = x;   // (a wave that gave up leaves what another has got)
   };
   auto advance = [&](int t) {
     ring_sync<(Rg::kN - 2) * (Rg::kPer + 1)>();
