@@ -3252,11 +3252,15 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
       for (int w = 0; w < kRowWaves; ++w) l += red_row[64 * w];
       // 2^-60 <= l < 2^100: terms flushed to zero are far below the sum's last bit, and 2^score times 2^-lse
       // (the lse of all keys is at least this one) neither overflows nor loses anything above 2^-26
-      const bool good = (l >= 8.6736174e-19f) && (l < 1.2676506e30f);
+      // A row that the mask lets see none of this workgroup's keys adds nothing, and that is its sum: no reason to sweep them again.  The last
+      // workgroup of a team, with fewer keys than there are queries, made all of it wait for that: 7400 shapes of 33 to 128 queries 0.93 of the
+      // time in the geometric mean, one in ten below 0.68, 0.48 at best (maxima and both, reduced again from registers: 0.97, 0.74).
+      const bool none = CAUSAL && tid + p.c < key0;
+      const bool good = none || ((l >= 8.6736174e-19f) && (l < 1.2676506e30f));
       if (!good && tid < p.M) flag[0] = 1;   // (written by whoever finds a bad row; thread 0 resets it below)
       if (!KEEP && tid >= p.M && !(l < kPosInf)) flag[0] = 1;   // a row of zeros met a non-finite key
       if (tid == 0) flag[1] = 1;
-      if (good || tid >= p.M) publish(tid, 0u, good ? l : 1.f);   // (rows that do not exist: anything finite)
+      if (good || tid >= p.M) publish(tid, 0u, none ? 0.f : good ? l : 1.f);   // (rows that do not exist: anything finite)
     }
     lds_barrier();
     return flag[0] != 0;   // uniform over the workgroup

@@ -1736,6 +1736,33 @@ def test_few_keys(h, m, n, d, dtype, causal):
     assert torch.equal(out.view(2, h, n), got)
 
 
+@pytest.mark.parametrize("h,m,n,d", [(2, 100, 1025, 128), (3, 128, 1600, 64), (70, 65, 2048 + 64, 128), (2, 64, 2049, 64), (3, 33, 2100, 128),
+                                     (80, 40, 4096 + 39, 96), (300, 30, 1024 + 3, 128), (9, 32, 3072 + 31, 64)])
+def test_single_sweep_rows_that_see_none_of_the_last_keys(h, m, n, d):
+    """Causal, and the last workgroup of a team has fewer keys than there are queries: the first rows see none of them, which is a sum of 0 and
+    no reason to sweep again.  Every form of the sweep (65 to 128, 33 to 64, up to 32 queries with eight and four waves), against 64 bits (see
+    test_few_keys for the bound); a NaN query in such a row against the two kernels."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g).bfloat16() for r in (m, n))
+    sums, most = _columns_f64(q, k, True)
+    got = [fca.flash_colreduce(q, k, red, True, out_dtype=torch.float32) for red in ("sum", "max")]
+    got += fca.flash_colreduce_multi(q, k, ["sum", "max"], True, out_dtype=torch.float32)
+    for x, want in zip(got, (sums, most, sums, most)):
+        assert torch.isfinite(x).all() and _rel(x, want) <= 1e-5
+    q[:, 0, 0, 0] = float("nan")
+    for red in ("sum", "max"):
+        both = []
+        for option in (1, 0):
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+            try:
+                both.append(fca.flash_colreduce(q, k, red, True, out_dtype=torch.float32))
+            finally:
+                lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+        torch.testing.assert_close(both[0], both[1], rtol=1e-4, atol=1e-6, equal_nan=True)
+
+
 def _lib_workspace(q, k):
     from flash_colreduce_amd import _lib
     b, h, m, d = q.shape
