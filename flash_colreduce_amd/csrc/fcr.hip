@@ -2817,7 +2817,8 @@ __global__ __launch_bounds__(kThreads, (NG <= 4 ? 3 : 2)) void col_small_kernel(
 #pragma unroll
         for (int r2 = 0; r2 < 4; ++r2) {
           float x = fmaf(acc[g][r2], p.scale2, nlse[gb + g][r2]);
-          if (need_mask) x = (16 * (gb + g) + r2 >= first) ? x : kNegInf;
+          // (rows past M are copies of others, which an infinite key that only later rows see makes a NaN)
+          if (need_mask) x = (16 * (gb + g) + r2 >= first && 16 * (gb + g) + r2 < p.M - qrow) ? x : kNegInf;
           if (MODE != kModeSum) vmax = fmaxf(vmax, x);
           if (MODE != kModeMax) vsum += fast_exp2(x);
         }

@@ -1763,6 +1763,43 @@ def test_single_sweep_rows_that_see_none_of_the_last_keys(h, m, n, d):
         torch.testing.assert_close(both[0], both[1], rtol=1e-4, atol=1e-6, equal_nan=True)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(3, 33, 1500, 64), (2, 63, 2111, 128), (70, 65, 1111, 128), (3, 127, 1024, 96), (3, 128, 1100, 64),
+                                     (80, 17, 4100, 128), (300, 31, 1030, 128)])
+def test_single_sweep_hidden_scores_beside_odd_rows(h, m, n, d, causal):
+    """What the mask hides and rows of padding (query counts that fill no tile) are told apart by their values unless some row's are not finite: keys of
+    both signs of infinity and NaN, which rows of padding meet as NaN, and NaN queries, in sums, maxima and both, in every form of the sweep, against the
+    two kernels: NaN in the same columns, the others the same to rounding."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g).half() for r in (m, n))
+    cases = []
+    for value in (float("inf"), float("-inf"), float("nan")):
+        bad = k.clone()
+        bad[:, 0, n // 2, 1] = value
+        bad[:, -1, n - 1, 0] = value
+        cases += [(q, bad)]
+    same_sign = q.clone()
+    same_sign[..., 1] = -same_sign[..., 1].abs() - 0.1   # (every score of the infinite key is -inf)
+    dead = k.clone()
+    dead[:, :, n // 2, 1] = float("inf")
+    bad_q = q.clone()
+    bad_q[:, 0, m // 2, 0] = float("nan")
+    cases += [(same_sign, dead), (bad_q, k), (bad_q, dead)]
+    for at, (x, y) in enumerate(cases):
+        got = {}
+        for option in (1, 0):
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+            try:
+                got[option] = [fca.flash_colreduce(x, y, red, causal, out_dtype=torch.float32) for red in ("sum", "max")]
+                got[option] += fca.flash_colreduce_multi(x, y, ["sum", "max"], causal, out_dtype=torch.float32)
+            finally:
+                lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+        for a, b in zip(got[1], got[0]):
+            torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-6, equal_nan=True, msg=lambda t: f"case {at}: {t}")
+
+
 def _lib_workspace(q, k):
     from flash_colreduce_amd import _lib
     b, h, m, d = q.shape
