@@ -3120,6 +3120,7 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
     // the scores are gone by the time it shows, and the keys of the pair are streamed once more.
     f32x4 sc[KG][NQ];
     f32x4 rs[NQ];   // per row (register) and key (lane): sum of 2^score over the steps
+    bool odd_padding = false;   // row tid does not exist and has met a non-finite key
     float my_lse = kNegInf;   // of row tid over this workgroup's keys, for tid < kRowsWg (where the plain sums are not usable)
     // A partial value and the number of its round travel as ONE 64-bit word, so a word that carries this round's number carries this
     // round's value: nobody waits for a store to complete and there is no counter.  The slots start at zero (round
@@ -3183,10 +3184,9 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
       const int kbase = (c0a + j * KH + kh) * kChunk;
       const int key = kbase + 16 * wq + (lane & 15);
       // Rows past M are rows of zeros: their scores are 0 and their 2^score is 1, which nothing downstream uses
-      // (their factor in step 4 is 0), so the fast form of the sweep does not hide them.  Only a key with a
-      // non-finite element makes them NaN; the row threads below look for that and ask for the second sweep,
-      // which hides them as every sweep that keeps scores does.
-      const bool need_mask = (KEEP && ragged_rows) || kbase + kChunk > p.N || (CAUSAL && kbase + kChunk - 1 > p.c + 64 * qh);
+      // (step 4 multiplies by 0 or adds -inf), so they are not hidden.  Only a key with a non-finite element makes them
+      // NaN; the row threads below look for that, and step 4 then hides them (of plain sums after a second sweep).
+      const bool need_mask = kbase + kChunk > p.N || (CAUSAL && kbase + kChunk - 1 > p.c + 64 * qh);
       if (need_mask) {
         int first = CAUSAL ? key - p.c - 64 * qh - qrow : -(1 << 30);
         if (key >= p.N) first = 1 << 30;
@@ -3259,7 +3259,8 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
       const bool none = CAUSAL && tid + p.c < key0;
       const bool good = none || ((l >= 8.6736174e-19f) && (l < 1.2676506e30f));
       if (!good && tid < p.M) flag[0] = 1;   // (written by whoever finds a bad row; thread 0 resets it below)
-      if (!KEEP && tid >= p.M && !(l < kPosInf)) flag[0] = 1;   // a row of zeros met a non-finite key
+      odd_padding = tid >= p.M && !(l < kPosInf);   // a row of zeros met a non-finite key
+      if (!KEEP && odd_padding) flag[0] = 1;
       if (tid == 0) flag[1] = 1;
       if (good || tid >= p.M) publish(tid, 0u, none ? 0.f : good ? l : 1.f);   // (rows that do not exist: anything finite)
     }
@@ -3440,7 +3441,8 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
       }
       // what step 4 adds to a score, or multiplies 2^score by (nothing for rows that do not exist)
       // (a NaN lse stays a NaN factor: the row's visible columns become NaN, as in the other kernels)
-      rowv[tid] = keep_scores ? -lse : (tid < p.M ? factor : 0.f);
+      if (keep_scores) rowv[tid] = tid < p.M ? -lse : odd_padding ? __builtin_nanf("") : kNegInf;
+      else rowv[tid] = tid < p.M ? factor : 0.f;
       if (split == 0 && tid < p.M) p.lse[(int64_t)bh * p.M + tid] = lse;   // (not meaningful if the team was not met)
     }
     lds_barrier();
@@ -3451,6 +3453,13 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
     f32x4 nl[NQ];
 #pragma unroll
     for (int g = 0; g < NQ; ++g) nl[g] = *reinterpret_cast<const f32x4*>(rowv + 64 * qh + 16 * g + qrow);
+    // What is hidden is 0 (sums) or -inf in the registers and stays so beside rows whose value is below infinity: no masks, then.
+    bool odd = false;
+#pragma unroll
+    for (int g = 0; g < NQ; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) odd = odd || !(nl[g][r] < kPosInf);
+    const bool plain_rows = __builtin_amdgcn_ballot_w64(odd) == 0;
     float* const osum = obuf + qh * (kRes * kBatchKeys);
     float* const omax = osum + (MODE == kModeBoth ? kBatchKeys : 0);
     int c0b = c0;
@@ -3458,9 +3467,28 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
     auto columns = [&](auto batch_tag) __attribute__((always_inline)) {   // eight steps at a time through the column buffer
     constexpr int bt = decltype(batch_tag)::value;
     float vs[kFusedSteps], vm[kFusedSteps];   // per step: the lane's key, reduced over the lane's queries
-    const int kend = (c0b + (bt + 1) * kFusedSteps * KH) * kChunk;   // of the batch's keys
-    if (MODE == kModeSum && !keep_scores && kend <= p.N && (!CAUSAL || kend - 1 <= p.c + 64 * qh)) {
-      // the usual case, without a question per step: 3000 -> 1100 cycles on 1024 keys and 64 queries
+    // The usual cases, without a question per step.  (Per call, step by step and so, in the geometric mean of 13500 shapes: maxima of up to 64 queries 0.76, of
+    // up to 128 0.81, both 0.82 and 0.86, sums, which asked wherever the mask cut a workgroup's keys, 0.93 and 0.95: 512 pairs of 64 x 16384 x 128
+    // fp16 399 -> 384 us, 32 of 128 x 4096 17.7 -> 16.9.  Part of it is that sweeps that keep scores hide no rows of padding any more.)
+    if (MODE != kModeSum && plain_rows) {
+#pragma unroll
+      for (int jj = 0; jj < kFusedSteps; ++jj) {
+        f32x4 part = {0.f, 0.f, 0.f, 0.f};
+        float vmax = kNegInf;
+#pragma unroll
+        for (int g = 0; g < NQ; ++g) {
+          const f32x4 x = sc[bt * kFusedSteps + jj][g] + nl[g];
+          vmax = fmaxf(fmaxf(vmax, x[0]), x[1]);
+          vmax = fmaxf(fmaxf(vmax, x[2]), x[3]);
+          if (MODE == kModeBoth) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[r] += fast_exp2(x[r]);
+          }
+        }
+        vs[jj] = (part[0] + part[1]) + (part[2] + part[3]);
+        vm[jj] = vmax;
+      }
+    } else if (MODE == kModeSum && !keep_scores && plain_rows) {   // 3000 -> 1100 cycles on 1024 keys and 64 queries
 #pragma unroll
       for (int jj = 0; jj < kFusedSteps; ++jj) {
         f32x4 part = sc[bt * kFusedSteps + jj][0] * nl[0];
