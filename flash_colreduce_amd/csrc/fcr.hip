@@ -90,6 +90,7 @@ struct Params {
   // both_sweeps_kernel: `tiles`, `group`, `fill` and `total` are of the row sweeps
   int col_tiles, col_group;
   int row_blocks, col_blocks;
+  int run_chunks;    // col_fused_kernel: chunks of keys a workgroup takes of a pair
   int parts;         // few_keys_f32_kernel: ranges of a pair's queries whose columns are added up apart
 };
 // which: 0 = row statistics, 1 = column sweep, 2 = column sweep for few queries, 3 = both sweeps in one for few
@@ -2917,8 +2918,8 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ 
 // NQ: groups of sixteen queries a wave holds (4; 2 for at most 32 queries: the registers then hold the scores of
 // twice as many keys per pair, and the time between two sweeps is spread over that many.  One group and four
 // times the keys was built as well and was slower than two: 1568 against 1499 us on 64 x 32 pairs of 16384 keys).
-// SKIP: chunks past the last key are left out instead of being computed and hidden score by score.  The team waits for its last
-// workgroup, which holds them: 6 x 40 pairs of 111 x 7284 x 128 206 -> 165 us per call, 5 x 24 of 89 x 3776 x 64 51 -> 43,
+// SKIP: chunks past a workgroup's last key (spread_keys deals them evenly, so these are its last ones) are left out instead of being computed
+// and hidden score by score.  When the team's last workgroup held all of them, it waited for that one: 6 x 40 pairs of 111 x 7284 x 128 206 -> 165 us per call, 5 x 24 of 89 x 3776 x 64 51 -> 43,
 // 7 x 24 of 100 x 15756 x 128 249 -> 237 (bf16, sums).
 // NW: waves.  Four (a step is one chunk, and a pair's keys are shared by twice the workgroups) leave room for two
 // workgroups on a CU, of different teams or key ranges: one streams while the other exchanges its row sums.  For at most 32 queries
@@ -2938,7 +2939,6 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
   constexpr int kQBytes = QH * Rg::kRows;        // the queries of a pair, staged like a chunk of keys per 64 rows
   constexpr int kNumThreads = 64 * NW;
   constexpr int kRowsWg = 16 * NQ * QH;          // query rows a workgroup holds
-  constexpr int kItemKeys = KG * KH * kChunk;    // keys of a workgroup per pair
   constexpr int kBatchKeys = kFusedSteps * KH * kChunk;   // finished columns leave eight steps at a time
   constexpr int kBatches = KG / kFusedSteps;
   constexpr int kRes = (MODE == kModeBoth) ? 2 : 1;
@@ -2949,9 +2949,9 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
   constexpr int kMergeWaves = (NW / QH) / ((kRes == 2 && QH == 1 && NW == 8) ? 2 : 1);
   constexpr int kBatch = 4 * QH * (8 / NW);                 // slots a lane fetches together: one round trip for teams of up to 32
   constexpr int kMrgFloats = kMergeWaves * kRowsWg * 2;
-  // Column sums: the row sums are taken as the scores come, while the sweep waits for memory, or, where that costs sixteen registers
-  // too many, after it.
-  constexpr bool kSumsInSweep = QH == 1 && NQ == 4;
+  // Column sums: the row sums are taken as the scores come, while the sweep waits for memory, or, where the registers do not reach for that (five in
+  // memory for 65 to 128 queries that skip nothing, many more for two query groups), after it.  65 to 128 queries that skip: 0.97 of the time.
+  constexpr bool kSumsInSweep = NQ == 4 && (QH == 1 || SKIP);
   constexpr int kAhead = NS / KH - 1;            // steps in flight in front of the one being computed
   constexpr int kInFlight = (NS / KH - 2) * Rg::kPer;   // loads a loading wave may have outstanding when a step starts
   // (one LDS object: see col_small_kernel)
@@ -2972,9 +2972,9 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
   const bool loader = (KH == 2) || (wave < 4);   // (four waves: all)
   const int S = p.splits, T = p.teams;
   const int team = (int)blockIdx.x / S, split = (int)blockIdx.x - team * S;
-  const int c0 = split * (KG * KH);              // first chunk of this workgroup's keys
+  const int c0 = split * p.run_chunks;           // first chunk of this workgroup's keys
   const int key0 = c0 * kChunk;
-  const int keys_end = min(p.N, key0 + kItemKeys);
+  const int keys_end = min(p.N, key0 + p.run_chunks * kChunk);
   const int rounds = (p.bh_count - team + T - 1) / T;
   const int qrow0 = 4 * (lane0 >> 4);
   int spin_limit = p.spin_limit;
@@ -3164,7 +3164,7 @@ __global__ __launch_bounds__(64 * NW, 2) void col_fused_kernel(const Params p) {
         waiting = false;
       }
       const char* lds = stage_of(cons_chunk + j * KH + kh);
-      if (SKIP && (c0a + j * KH + kh) * kChunk >= p.N) {
+      if (SKIP && (c0a + j * KH + kh) * kChunk >= keys_end) {
         const float none = KEEP ? kNegInf : 0.f;
 #pragma unroll
         for (int g = 0; g < NQ; ++g) {
@@ -4904,7 +4904,7 @@ int make_params(Params& p, const void* q, const void* k, int dtype, int B, int H
   p.teams = 0;
   p.sync = nullptr;
   p.spin_limit = 0;
-  p.col_tiles = p.col_group = p.row_blocks = p.col_blocks = p.parts = 0;
+  p.col_tiles = p.col_group = p.row_blocks = p.col_blocks = p.parts = p.run_chunks = 0;
   return 0;
 }
 
@@ -4992,6 +4992,24 @@ FusedPairPlan fused_pair_plan(int64_t bh, int M, int N, int ksteps, const FusedP
   o.teams = (int)((cap / splits) < bh ? cap / splits : bh);
   o.floats = o.part_at + 2 * (2ll * o.teams * o.splits * 32);
   return o;
+}
+
+// The single sweep's keys of a pair, dealt evenly to the workgroups of its team (p.splits: as few as can hold them), in steps of
+// `chunks_per_step`; and to as many workgroups as there are CUs for where one round is all there is and that leaves a workgroup at most
+// five eighths of its steps, two or more (a smaller part does not pay for the exchange, and in several rounds the next pair's loads run under it): 0.91
+// to 0.94 of the time for 2850 such shapes.  Not where two query groups per wave hold twice the keys (1.05 for 85 shapes; the estimate that
+// chose them counts on those).
+void spread_keys(Params& p, int N, int chunks_per_step, int cap, bool may_widen) {
+  const int steps = (N + chunks_per_step * kChunk - 1) / (chunks_per_step * kChunk);
+  int per = (steps + p.splits - 1) / p.splits;
+  if (may_widen && p.teams == p.bh_count) {
+    const int places = cap / p.teams;
+    int wide = (steps + places - 1) / places;
+    if (wide < 2) wide = 2;
+    if (8 * wide <= 5 * per) per = wide;
+  }
+  p.splits = (steps + per - 1) / per;
+  p.run_chunks = per * chunks_per_step;
 }
 
 // The path for one query (one_query_*_kernel): sizes of its launches and its scratch, which lies behind everything
@@ -5330,15 +5348,13 @@ void launch_col_fused_form(const Params& p, bool causal, hipStream_t s) {
   else hipLaunchKernelGGL((col_fused_kernel<DT, KS, false, MODE, QH, NQ, SKIP, NW>), grid, block, 0, s, p);
 }
 
-// More than 64 queries: maxima gain nothing by leaving chunks out (ragged rows are hidden one by one in any case; sums and
-// maxima 323 -> 325 us), and where there is nothing to leave out the question alone costs (4 x 32 pairs of 89 x 4096 x 64
-// 40.7 -> 42.6 us, 32 of 128 x 4096 x 128 17.6 -> 17.8), so the host asks it.
+// More than 64 queries: where there is nothing to leave out the question alone costs (4 x 32 pairs of 89 x 4096 x 64
+// 40.7 -> 42.6 us, 32 of 128 x 4096 x 128 17.6 -> 17.8), so the host asks it; elsewhere leaving chunks out takes 0.94 (maxima, both) of the time.
 template <int DT, int KS, int MODE, int QH, int NQ, int NW>
 void launch_col_fused_mode(const Params& p, bool causal, hipStream_t s) {
-  if constexpr (QH == 2 && MODE != kModeSum) return launch_col_fused_form<DT, KS, MODE, QH, NQ, false, NW>(p, causal, s);
-  else if constexpr (QH == 2) {
+  if constexpr (QH == 2) {
     const int chunks = (p.N + kChunk - 1) / kChunk;
-    if (chunks % fused_chunks(QH, NQ) != 0) return launch_col_fused_form<DT, KS, MODE, QH, NQ, true, NW>(p, causal, s);
+    if (p.run_chunks != fused_chunks(QH, NQ) || chunks % p.run_chunks != 0) return launch_col_fused_form<DT, KS, MODE, QH, NQ, true, NW>(p, causal, s);
     launch_col_fused_form<DT, KS, MODE, QH, NQ, false, NW>(p, causal, s);
   } else {
     launch_col_fused_form<DT, KS, MODE, QH, NQ, true, NW>(p, causal, s);
@@ -6064,6 +6080,7 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
       form = 16;
       rows = 32;
     }
+    spread_keys(p, N, form == 16 || f.qh == 2 ? 1 : 2, chip_cus(), f.nq == 4 && form != 16);
     // the slots that the launch polls (one set of them for one round) and the status word start at zero
     const int words = (p.bh_count > p.teams ? 2 : 1) * p.teams * p.splits * rows * 2;
     p.total = p.teams * p.splits;

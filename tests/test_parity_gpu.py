@@ -1800,6 +1800,21 @@ def test_single_sweep_hidden_scores_beside_odd_rows(h, m, n, d, causal):
             torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-6, equal_nan=True, msg=lambda t: f"case {at}: {t}")
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(2, 100, 1024, 128), (3, 128, 1100, 64), (30, 65, 2049, 128), (100, 70, 1600, 64), (129, 128, 1025, 96), (2, 64, 2100, 128),
+                                     (1, 33, 65536, 64), (40, 40, 3000, 96), (100, 48, 1025, 128), (300, 60, 1200, 128), (300, 20, 2900, 128), (7, 32, 5000, 64)])
+def test_single_sweep_keys_dealt_evenly(h, m, n, d, causal):
+    """Keys dealt to as few workgroups as can hold them and, in one round, to as many as there are CUs for: two steps each, one more or
+    less in the last, ragged chunks, in every form of the sweep; against 64 bits (see test_few_keys for the bound)."""
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g).half() for r in (m, n))
+    sums, most = _columns_f64(q, k, causal)
+    got = [fca.flash_colreduce(q, k, red, causal, out_dtype=torch.float32) for red in ("sum", "max")]
+    got += fca.flash_colreduce_multi(q, k, ["sum", "max"], causal, out_dtype=torch.float32)
+    for x, want in zip(got, (sums, most, sums, most)):
+        assert torch.isfinite(x).all() and _rel(x, want) <= 1e-5
+
+
 def _lib_workspace(q, k):
     from flash_colreduce_amd import _lib
     b, h, m, d = q.shape
