@@ -1119,8 +1119,8 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 // (which keeps the XCDs) column tiles as col_reduce_kernel.  The row statistics start as kNotYet (fill_words_kernel), a row sweep stores its rows' values with
 // device scope, and a column sweep takes a chunk of queries once their values are there: every word says so by itself, so there are
 // no flags, no order between words and no fences.  Workgroups are dispatched in order, on every XCD the row tiles first, and a row tile
-// waits for nobody: whatever a column sweep waits for is running or done.  Should that not hold the wait ends after p.spin_limit polls and
-// the columns become NaN.
+// waits for nobody, so every wait ends, beside kernels that wait for nobody too.  Launches that wait (these and single sweeps) are kept apart by the
+// host (SweepOrder), and a captured graph gets the two launches.  Should a wait not end, it does after p.spin_limit polls and the columns become NaN.
 // What it is for: a launch that waits for its longest or last sweeps keeps CUs idle at its end, and here only the second one does.  With
 // the mask, the first column tile needs only the rows of the first row tile at first, which end early, and follows the row sweeps chunk
 // by chunk.  A column sweep looks at a chunk's values a chunk ahead, one LDS read and one branch per chunk, within 1 % of a sweep of its
@@ -5980,7 +5980,8 @@ namespace {
 // different streams could be dispatched side by side, each holding CUs the other needs, until their bounded
 // waits run out.  So inside a process they are chained: a single sweep on another stream than the one before
 // first waits (on the GPU; the host never blocks) for an event recorded at the end of that stream.  Calls that
-// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call).  Not under stream
+// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call).  So is both_sweeps_kernel: beside another waiting launch its
+// column tiles on one die could hold the CUs that the other needs while its last row tiles on another die wait for theirs.  Not under stream
 // capture (a graph carries no such edge; graphs holding single sweeps must not replay side by side on one GPU),
 // not for other processes on the same GPU, and not for fcr_colreduce_static, whose calls must not overlap anyway.
 struct SweepOrder {
@@ -6095,7 +6096,15 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
   }
   if (single) {
     const BothPlan o = both_plan(dtype, ksteps, p.bh_count, M, N, causal != 0);
-    if (o.row_blocks > 0) return launch_both(p, dtype, ksteps, o, ws, mode, causal != 0, static_cast<hipStream_t>(stream));
+    if (o.row_blocks > 0) {
+      hipStream_t s = static_cast<hipStream_t>(stream);
+      SweepOrder* const order = order_begin(s);
+      if (order) {   // (a graph that is being captured takes the two launches below: nothing orders its replays)
+        const int brc = launch_both(p, dtype, ksteps, o, ws, mode, causal != 0, s);
+        order_end(order, s, true);
+        return brc;
+      }
+    }
   }
   rc = fcr_row_lse(q, k, ws, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream);
   if (rc) return rc;

@@ -257,11 +257,12 @@ int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, in
  * fcr_colreduce_status waits for the stream and returns FCR_E_WAIT if that happened in the last call that
  * used lse_ws with these sizes, 0 otherwise (also for problems that do not take the single sweep).
  * A single sweep fills the chip, one or two workgroups per CU, and two of them dispatched side by side would
- * starve each other until their waits run out.  Inside a process the library prevents that: a single
- * sweep issued on another stream than the previous one is made to wait on the GPU (an event recorded on
+ * starve each other until their waits run out, and so could one and a call whose column sweeps wait in
+ * one launch with its row sweeps.  Inside a process the library prevents that: such a call
+ * issued on another stream than the previous one is made to wait on the GPU (an event recorded on
  * that stream, hipStreamWaitEvent on the new one; the host does not block, calls that stay on one stream
  * pay nothing).  Outside its reach: launches recorded under stream capture (graphs that hold single
- * sweeps must not replay side by side on one GPU), other processes on the same GPU, and
+ * sweeps must not replay side by side on one GPU; the other kind takes two launches there), other processes on the same GPU, and
  * fcr_colreduce_static, whose calls must not overlap anyway.  There, switch the single sweep off or
  * keep such calls apart.
  * No counterpart in the reference, whose kernel has no cross-program dependencies.

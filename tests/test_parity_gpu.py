@@ -2359,15 +2359,39 @@ def test_both_sweeps_wait_is_bounded(reduction):
 
 
 def test_both_sweeps_under_graph_capture():
-    """The fill, the row sweeps and the column sweeps are kernels of one graph: replays on new operands, with eager calls and
-    synchronizations between them, give the eager result."""
+    """A captured call takes the two launches, whose replays wait for nothing beside them: replays on new operands, with eager calls and
+    synchronizations between them, give the bits of two launches and the eager result to rounding."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
     q, k = (x.cuda() for x in _inputs.randn_pair(2, 6, 900, 900, 128, seed=3, dtype=torch.bfloat16))
     fca.flash_colreduce(q, k, "sum", True)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        out = fca.flash_colreduce(q, k, "sum", True)
+        out = fca.flash_colreduce(q, k, "sum", True, out_dtype=torch.float32)
     for step in range(4):
         q.copy_(torch.randn_like(q))
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out, fca.flash_colreduce(q, k, "sum", True)), step
+        torch.testing.assert_close(out, fca.flash_colreduce(q, k, "sum", True, out_dtype=torch.float32), rtol=1e-5, atol=1e-6)
+        lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 0)
+        try:
+            assert torch.equal(out, fca.flash_colreduce(q, k, "sum", True, out_dtype=torch.float32)), step
+        finally:
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+
+
+def test_launches_that_wait_on_two_streams():
+    """Both sweeps in one launch and single sweeps, issued in turn on two streams without a wait between them: the host chains them, and every
+    result is the one of a call by itself."""
+    shapes = [(6, 900, 900, 128), (32, 100, 4096, 128), (3, 1100, 1100, 64), (64, 64, 8192, 128)]
+    ops = [tuple(torch.randn(1, h, r, d, device="cuda").half() for r in (m, n)) for h, m, n, d in shapes]
+    want = [fca.flash_colreduce(q, k, "sum", True) for q, k in ops]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got = []
+    for step in range(12):
+        for i, (q, k) in enumerate(ops):
+            with torch.cuda.stream(streams[(step + i) % 2]):
+                got.append((i, fca.flash_colreduce(q, k, "sum", True)))
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, want[i]) for i, x in got)
