@@ -5169,6 +5169,9 @@ FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool bot
 //   Without the mask, or with many more keys than queries, no column can start before the rows of its pair end: there have to be row
 //   tiles for every CU (24 of 2893 x 128 144 -> 121, 48 of 2929 244 -> 207, 61 of 2223 174 -> 143, 18 of 7902 x 64 449 -> 355; but 17 of 2873 x 128 88 -> 89, 5 of 3039 50 -> 64;
 //   with 128 queries per 1000 keys 68 of 1090 x 8104 318 -> 334).
+//   Many rounds: the last one is a small part of them, and one launch is as fast in the mean and up to 1.07 of the time (640 of 1479 x 96 391 -> 424).
+//   Geometric means over 2600 squares of 1030 to 6000, `rows` of 4 to 6, 6 to 10, 10 to 16 and beyond: with the mask D = 64 0.80, 0.88, 0.92, 0.98, 128 0.90, 0.95,
+//   0.99, 1.00, 256 0.97, 1.00, 1.00, 1.00; without it 64 0.92, 0.95, 0.99, 1.02, 128 0.95, 0.98, 1.00, 1.01, 256 0.99, 1.00, 1.00, 1.00.
 struct BothPlan {
   int row_blocks = 0, col_blocks = 0;
 };
@@ -5182,6 +5185,7 @@ BothPlan both_plan(int dtype, int ksteps, int64_t bh, int M, int N, bool causal)
   const double small = (double)tiles / cus, rows = (double)(bh * ((M + 255) / 256)) / cus;
   const bool longer = 2 * (int64_t)N > 3 * (int64_t)M, level = causal && !longer;   // level: the column sweeps can follow the row sweeps
   int nr = 1, nc = 1;
+  if (rows >= (ksteps > 4 ? 6.0 : ksteps <= 2 && level ? 16.0 : 10.0)) return o;
   if (ksteps > 4) {
     if (!level && small < 1.05) return o;
   } else if (ksteps <= 2) {
