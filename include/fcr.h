@@ -207,8 +207,8 @@ int fcr_colreduce_to(const void* q, const void* k, void* out, int out_dtype, flo
  * fcr_colreduce_sum_max_to (out_max given; reduction then names what `out` holds, sum or mean) compute, and with
  * fcr_workspace_bytes(dtype, B, H, M, N, D) bytes by the fastest path for the problem: one query is read
  * once, without the matrix instructions, and its scores wait in the workspace (4 bytes per key) for their row's
- * sum (64 sequences of 32 heads and 65536 keys: 0.5 GB); 16-bit keys that fit the registers of a workgroup (at most
- * 512, or 256 in rows of more than 256 bytes) form each score once, and where several workgroups share a pair their columns
+ * sum (64 sequences of 32 heads and 65536 keys: 0.5 GB); keys that fit the registers of a workgroup (16-bit ones at most
+ * 512, or 256 in rows of more than 256 bytes, fp32 ones of D >= 32 at most 256) form each score once, and where several workgroups share a pair their columns
  * wait in the workspace for a second launch.  With less, but at least fcr_lse_bytes, the call takes the
  * path of the entry points above, as it does for long calls of few keys that would fill neither the chip nor a workgroup's
  * registers (FCR_E_SCRATCH below that); results agree to rounding either way.  ws must be 16-byte aligned, its first
