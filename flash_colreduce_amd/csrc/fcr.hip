@@ -695,13 +695,11 @@ struct NoAux {};
 // default policy is the faster one.
 // TELL: column sweeps of the same launch wait for the values (both_sweeps_kernel).
 template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE, bool TELL>
-__device__ __forceinline__ void row_sweep(const Params& p, char* smem, int v) {
+__device__ __forceinline__ void row_sweep(const Params& p, char* smem, int tid, int bh, int tile, int split) {
   using Rg = Ring<KS>;
   constexpr int NG = wave_group_count(NB);
   constexpr int kTileRows = kWaves * 16 * NG;
-  int bh, tile, split;
-  map_block_split(p, v, CAUSAL, bh, tile, split);
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, keeps the row views scalar
   const int b = bh / p.H, h = bh - b * p.H;
   const char* qb = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
@@ -810,7 +808,9 @@ __device__ __forceinline__ void row_sweep(const Params& p, char* smem, int v) {
 template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE>
 __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(const Params p) {
   __shared__ __attribute__((aligned(1024))) char smem[Ring<KS>::kBytes];
-  row_sweep<DT, KS, CAUSAL, NB, STREAM_ONCE, false>(p, smem, (int)blockIdx.x);
+  int bh, tile, split;
+  map_block_split(p, (int)blockIdx.x, CAUSAL, bh, tile, split);
+  row_sweep<DT, KS, CAUSAL, NB, STREAM_ONCE, false>(p, smem, (int)threadIdx.x, bh, tile, split);
 }
 
 // lse[r] = log2 sum_s 2^part[s][r] over the key ranges of a split row sweep.  One thread per row; the
@@ -946,7 +946,9 @@ inline int col_tile_blocks(int ksteps, int mode, int N, int64_t bh, bool causal)
 }
 
 // FOLLOW: row sweeps of the same launch may not have stored the lse of the streamed rows yet (both_sweeps_kernel).
-constexpr uint32_t kNotYet = 0xffffffffu;   // an lse that is still to come: no row sweep stores this NaN
+constexpr uint32_t kNotYet = 0xffffffffu;   // an lse that is still to come: no row sweep stores this NaN,
+constexpr uint32_t kBegun = 0xfffffffeu;    // nor this one, which stands at the first row of a tile that a running workgroup has in hand
+__device__ __forceinline__ bool still_to_come(uint32_t lse) { return lse >= kBegun; }
 constexpr int kLseSlots = 8;                // of 64 rows each
 template <int KS, int NB, bool FOLLOW>
 __host__ __device__ constexpr int col_sweep_bytes() {
@@ -955,13 +957,11 @@ __host__ __device__ constexpr int col_sweep_bytes() {
   return ring > red ? ring : red;
 }
 template <int DT, int KS, bool CAUSAL, int MODE, int NB, bool FOLLOW>
-__device__ __forceinline__ void col_sweep(const Params& p, char* smem, int v) {
+__device__ __forceinline__ void col_sweep(const Params& p, char* smem, int bh, int tile) {
   using Rg = Ring<KS>;
   static_assert(!FOLLOW || Rg::kN + 1 <= kLseSlots, "a slot for every chunk whose lse is read or on its way");
   constexpr int NG = wave_group_count(NB);
   constexpr int kTileRows = kWaves * 16 * NG;
-  int bh, tile;
-  map_block(p, v, false, bh, tile);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, keeps the row views scalar
   const int b = bh / p.H, h = bh - b * p.H;
@@ -1022,20 +1022,20 @@ __device__ __forceinline__ void col_sweep(const Params& p, char* smem, int v) {
     uint32_t x = kNotYet;
     for (;;) {
       x = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (__builtin_amdgcn_ballot_w64(x == kNotYet) == 0) break;
+      if (__builtin_amdgcn_ballot_w64(still_to_come(x)) == 0) break;
       if (given_up || ++polls > p.spin_limit) {
         given_up = true;
         break;
       }
       __builtin_amdgcn_s_sleep(8);
     }
-    if (x != kNotYet) reinterpret_cast<uint32_t*>(lse_slot(t))[lane] = x;   // (a wave that gave up leaves what another has got)
+    if (!still_to_come(x)) reinterpret_cast<uint32_t*>(lse_slot(t))[lane] = x;   // (a wave that gave up leaves what another has got)
   };
   auto advance = [&](int t) {
     ring_sync<(Rg::kN - 2) * (Rg::kPer + 1)>();
     if constexpr (FOLLOW) {
       if (t == t0) word = reinterpret_cast<const uint32_t*>(lse_slot(t))[lane];
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(word == kNotYet) != 0, 0)) wait_for(t);
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(still_to_come(word)) != 0, 0)) wait_for(t);
       word = reinterpret_cast<const uint32_t*>(lse_slot(t + 1))[lane];
     }
     issue(t + Rg::kN - 1);
@@ -1112,37 +1112,93 @@ __device__ __forceinline__ void col_sweep(const Params& p, char* smem, int v) {
 template <int DT, int KS, bool CAUSAL, int MODE, int NB>
 __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_reduce_kernel(const Params p) {
   __shared__ __attribute__((aligned(1024))) char smem[col_sweep_bytes<KS, NB, false>()];
-  col_sweep<DT, KS, CAUSAL, MODE, NB, false>(p, smem, (int)blockIdx.x);
+  int bh, tile;
+  map_block(p, (int)blockIdx.x, false, bh, tile);
+  col_sweep<DT, KS, CAUSAL, MODE, NB, false>(p, smem, bh, tile);
 }
 
 // Both sweeps in one launch: workgroups [0, p.total) take row tiles as row_lse_kernel does, those from the next multiple of eight on
 // (which keeps the XCDs) column tiles as col_reduce_kernel.  The row statistics start as kNotYet (fill_words_kernel), a row sweep stores its rows' values with
-// device scope, and a column sweep takes a chunk of queries once their values are there: every word says so by itself, so there are
-// no flags, no order between words and no fences.  Workgroups are dispatched in order, on every XCD the row tiles first, and a row tile
-// waits for nobody, so every wait ends, beside kernels that wait for nobody too.  Launches that wait (these and single sweeps) are kept apart by the
-// host (SweepOrder), and a captured graph gets the two launches.  Should a wait not end, it does after p.spin_limit polls and the columns become NaN.
+// device scope, and a column sweep takes a chunk of queries once their values are there: every word says so by itself, so there is
+// no order between words and there are no fences.  A column sweep first looks whether every row tile that it needs has begun: the workgroup whose place
+// it is marks the tile's first row with kBegun when it starts.  If one has not (another die is behind, other kernels hold its CUs), the workgroup gives it
+// kPatience polls, then takes the tile in hand itself, marks it and sweeps it (the place's own workgroup will store the same bits once more).  So a
+// column sweep waits only for row tiles that a running workgroup has in hand, and those wait for nobody: every wait ends, whatever the order in which
+// workgroups start and whatever else holds CUs meanwhile, be it kernels that wait for each other, and no launch has to be kept apart from another.
+// The bound on a wait (p.spin_limit polls, then the columns become NaN) is for a host that lowers it.
+// The look costs 0.25 % in the geometric mean of 1600 shapes (a round trip to memory per column tile, beside another workgroup's sweep), all of it,
+// the mark and the loop 1.0 %.  Started in the reverse order, columns first, the launch gives the same bits in 1.2 to 2.3 times the time.  (Tickets
+// for all tiles instead, rows first, cost 4.9 %, up to half of a short call: 64 to 128 atomics on a line before the first load of a
+// workgroup, and workgroups that share a CU no longer get a long tile and a short one.)
+// A captured graph gets the two launches, whose bits it has always had.
 // What it is for: a launch that waits for its longest or last sweeps keeps CUs idle at its end, and here only the second one does.  With
 // the mask, the first column tile needs only the rows of the first row tile at first, which end early, and follows the row sweeps chunk
 // by chunk.  A column sweep looks at a chunk's values a chunk ahead, one LDS read and one branch per chunk, within 1 % of a sweep of its
 // own (32 heads of 8192 x 8192 x 128 467 -> 472 us, where nothing is gained).  When a CU holds two workgroups the older one runs at nearly its
 // full speed and the younger one on what is left (1.15 us and 3.3 per chunk of 64 rows against 1.05 alone), so the order of
 // dispatch decides what ends together: see map_group, and both_plan for what was measured.
+constexpr int kPatience = 32;   // polls, a microsecond or so each
 template <int DT, int KS, bool CAUSAL, int MODE, int NBR, int NBC>
 __global__ __launch_bounds__(kThreads, 2) void both_sweeps_kernel(const Params p) {
   constexpr int kCols = col_sweep_bytes<KS, NBC, true>();
   __shared__ __attribute__((aligned(1024))) char smem[kCols > Ring<KS>::kBytes ? kCols : Ring<KS>::kBytes];
-  const int v = (int)blockIdx.x, rows = (p.total + 7) & ~7;
-  if (v < rows) {
-    if (v < p.total) row_sweep<DT, KS, CAUSAL, NBR, false, true>(p, smem, v);
-    return;
+  constexpr int kRowTile = kWaves * 16 * wave_group_count(NBR), kColTile = kWaves * 16 * wave_group_count(NBC);
+  const int v = (int)blockIdx.x, rows = (p.total + 7) & ~7, tid = (int)threadIdx.x, lane = tid & 63;
+  const bool own = v < rows;   // a row tile's place
+  int bh, tile, split = 0, row = -1, next = 0, patience = min(p.spin_limit, kPatience);
+  if (own) {
+    if (v >= p.total) return;
+    map_block_split(p, v, CAUSAL, bh, row, split);
+  } else {
+    Params c = p;
+    c.tiles = p.col_tiles;
+    c.group = p.col_group;
+    c.fill = 0;
+    map_block(c, v - rows, false, bh, tile);
+    if (CAUSAL) next = max(0, tile * kColTile - p.c) / kChunk * kChunk / kRowTile;   // the first row tile that it needs
   }
-  Params c = p;
-  c.tiles = p.col_tiles;
-  c.group = p.col_group;
-  c.fill = 0;
-  col_sweep<DT, KS, CAUSAL, MODE, NBC, true>(c, smem, v - rows);
+  uint32_t* const words = reinterpret_cast<uint32_t*>(p.lse) + (int64_t)bh * p.M;
+  auto mark = [&](int r) {   // whether the tile was not marked before
+    uint32_t none = kNotYet;
+    return __hip_atomic_compare_exchange_strong(words + r * kRowTile, &none, kBegun, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (own && tid == 0) mark(row);   // (the answer is not waited for)
+  for (;;) {
+    if (row < 0) {   // a row tile of the pair that nobody has begun
+      if (tid < 64) {
+        const int last = (p.M - 1) / kRowTile;
+        while (next <= last) {
+          const uint32_t x = __hip_atomic_load(words + min(next + lane, last) * kRowTile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          const uint64_t missing = __builtin_amdgcn_ballot_w64(x == kNotYet);
+          if (missing == 0) {
+            next += 64;
+            continue;
+          }
+          next += __builtin_ctzll(missing);
+          if (patience > 0) {
+            --patience;
+            __builtin_amdgcn_s_sleep(8);
+          } else if (__builtin_amdgcn_ballot_w64(lane == 0 && mark(next)) != 0) {
+            break;
+          }
+        }
+        if (lane == 0) *reinterpret_cast<int*>(smem) = next <= last ? next : -1;
+      }
+      lds_barrier();
+      row = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(smem));
+      lds_barrier();
+      if (row < 0) break;
+    }
+    // (opaque: what the sweep derives from these is not to be kept in registers around the loop)
+    const __attribute__((address_space(4))) Params* at = (const __attribute__((address_space(4))) Params*)__builtin_amdgcn_kernarg_segment_ptr();
+    int thread = tid;
+    asm volatile("" : "+s"(at), "+v"(thread));
+    row_sweep<DT, KS, CAUSAL, NBR, false, true>(*(const Params*)at, smem, thread, bh, row, split);
+    if (own) return;
+    row = -1;
+  }
+  col_sweep<DT, KS, CAUSAL, MODE, NBC, true>(p, smem, bh, tile);
 }
-
 
 // ---------------------------------------------------------------------------------------------
 // Both sweeps in one for a pair whose keys all fit the registers of one workgroup: every wave keeps 16 * NG keys (groups w, w + NW,
@@ -5980,12 +6036,19 @@ int fcr_pack_f32(const float* src, void* dst, int64_t rows, int D, int terms, in
 }
 
 namespace {
+// Whether a stream is being captured, or that cannot be told.
+bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone) return false;
+  (void)hipGetLastError();
+  return true;
+}
+
 // A single sweep expects the whole chip: its workgroups wait for each other, one of eight waves or two of four per CU.  Two of them issued on
 // different streams could be dispatched side by side, each holding CUs the other needs, until their bounded
 // waits run out.  So inside a process they are chained: a single sweep on another stream than the one before
 // first waits (on the GPU; the host never blocks) for an event recorded at the end of that stream.  Calls that
-// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call).  So is both_sweeps_kernel: beside another waiting launch its
-// column tiles on one die could hold the CUs that the other needs while its last row tiles on another die wait for theirs.  Not under stream
+// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call).  Not under stream
 // capture (a graph carries no such edge; graphs holding single sweeps must not replay side by side on one GPU),
 // not for other processes on the same GPU, and not for fcr_colreduce_static, whose calls must not overlap anyway.
 struct SweepOrder {
@@ -5998,11 +6061,7 @@ std::mutex g_order_mu;
 
 // Takes the lock and returns the device's entry when the launch on stream s is to be chained, else nullptr.
 SweepOrder* order_begin(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
+  if (is_capturing(s)) return nullptr;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
     (void)hipGetLastError();
@@ -6098,17 +6157,9 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
     order_end(order, s, !fcr_detail::fused_refused && lrc == 0);
     if (!fcr_detail::fused_refused) return lrc;
   }
-  if (single) {
+  if (single && !is_capturing(static_cast<hipStream_t>(stream))) {   // (a captured call keeps the bits of the two launches)
     const BothPlan o = both_plan(dtype, ksteps, p.bh_count, M, N, causal != 0);
-    if (o.row_blocks > 0) {
-      hipStream_t s = static_cast<hipStream_t>(stream);
-      SweepOrder* const order = order_begin(s);
-      if (order) {   // (a graph that is being captured takes the two launches below: nothing orders its replays)
-        const int brc = launch_both(p, dtype, ksteps, o, ws, mode, causal != 0, s);
-        order_end(order, s, true);
-        return brc;
-      }
-    }
+    if (o.row_blocks > 0) return launch_both(p, dtype, ksteps, o, ws, mode, causal != 0, static_cast<hipStream_t>(stream));
   }
   rc = fcr_row_lse(q, k, ws, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream);
   if (rc) return rc;

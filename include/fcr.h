@@ -170,8 +170,8 @@ int fcr_pack_f32(const float* src, void* dst, int64_t rows, int D, int terms, in
 
 /*
  * Both kernels on one stream, back to back or, where that is the faster way, in one launch whose column sweeps wait for the
- * row statistics they need (16-bit operands; a wait ends after FCR_OPT_WAIT_POLLS polls, with NaN columns, which takes a GPU
- * that does not dispatch the workgroups of a launch in order): the whole of _flash_colreduce (flash.py:277-308)
+ * row statistics they need (16-bit operands, not under stream capture; they wait only for what a running workgroup has in
+ * hand, so every wait ends whatever else the GPU runs, and after FCR_OPT_WAIT_POLLS polls at the latest, with NaN columns): the whole of _flash_colreduce (flash.py:277-308)
  * except the final cast to the input dtype, which stays with the host.  lse_ws is scratch of
  * fcr_lse_bytes(B,H,M,N,D) bytes whose first B*H*M floats hold the row statistics on return.
  */
@@ -257,12 +257,11 @@ int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, in
  * fcr_colreduce_status waits for the stream and returns FCR_E_WAIT if that happened in the last call that
  * used lse_ws with these sizes, 0 otherwise (also for problems that do not take the single sweep).
  * A single sweep fills the chip, one or two workgroups per CU, and two of them dispatched side by side would
- * starve each other until their waits run out, and so could one and a call whose column sweeps wait in
- * one launch with its row sweeps.  Inside a process the library prevents that: such a call
- * issued on another stream than the previous one is made to wait on the GPU (an event recorded on
+ * starve each other until their waits run out.  Inside a process the library prevents that: a single
+ * sweep issued on another stream than the previous one is made to wait on the GPU (an event recorded on
  * that stream, hipStreamWaitEvent on the new one; the host does not block, calls that stay on one stream
  * pay nothing).  Outside its reach: launches recorded under stream capture (graphs that hold single
- * sweeps must not replay side by side on one GPU; the other kind takes two launches there), other processes on the same GPU, and
+ * sweeps must not replay side by side on one GPU, nor beside single sweeps issued otherwise), other processes on the same GPU, and
  * fcr_colreduce_static, whose calls must not overlap anyway.  There, switch the single sweep off or
  * keep such calls apart.
  * No counterpart in the reference, whose kernel has no cross-program dependencies.

@@ -2395,3 +2395,66 @@ def test_launches_that_wait_on_two_streams():
                 got.append((i, fca.flash_colreduce(q, k, "sum", True)))
     torch.cuda.synchronize()
     assert all(torch.equal(x, want[i]) for i, x in got)
+
+
+def test_both_sweeps_wait_for_no_other_stream():
+    """A call that holds both sweeps in one launch runs while a stream on which the one before it was issued is busy with
+    something else: nothing of that stream is waited for."""
+    q, k = (x.cuda() for x in _inputs.randn_pair(1, 3, 700, 700, 128, seed=4, dtype=torch.float16))
+    want = fca.flash_colreduce(q, k, "sum", True)
+    first = torch.cuda.Stream()
+    one = torch.ones(1, device="cuda")
+    beside = None
+    for _ in range(8):   # a stream that runs beside the first one (they share hardware queues)
+        other = torch.cuda.Stream()
+        with torch.cuda.stream(other):
+            fca.flash_colreduce(q, k, "sum", True), one + one
+        torch.cuda.synchronize()
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(50_000_000)
+            busy = torch.cuda.Event()
+            busy.record()
+        with torch.cuda.stream(other):
+            one + one
+        other.synchronize()
+        if not busy.query():
+            beside = other
+            break
+    torch.cuda.synchronize()
+    assert beside is not None
+    with torch.cuda.stream(first):
+        fca.flash_colreduce(q, k, "sum", True)
+        torch.cuda._sleep(50_000_000)
+        busy = torch.cuda.Event()
+        busy.record()
+    with torch.cuda.stream(beside):
+        got = fca.flash_colreduce(q, k, "sum", True)
+    beside.synchronize()
+    assert not busy.query()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
+def test_prefill_beside_a_captured_decode():
+    """Eager calls that hold both sweeps in one launch on one stream, replays of a graph that holds a single sweep on another, with no
+    wait between the two streams: every result is that of a call by itself, again after synchronizations and with calls in between."""
+    g = torch.Generator(device="cuda").manual_seed(11)
+    make = lambda h, m, n, d: tuple(torch.randn(1, h, r, d, device="cuda", generator=g).half() for r in (m, n))
+    decode = make(64, 64, 8192, 128)
+    prefills = [make(12, 1100, 1100, 128), make(60, 1000, 1000, 128), make(3, 700, 700, 256), make(40, 1500, 1500, 64)]
+    want = [fca.flash_colreduce(q, k, "sum", True) for q, k in (decode, *prefills)]
+    graph, left, right = torch.cuda.CUDAGraph(), torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.graph(graph):
+        out = fca.flash_colreduce(*decode, "sum", True)
+    torch.cuda.synchronize()
+    for rounds in (1, 4, 8):
+        got = []
+        for step in range(rounds):
+            with torch.cuda.stream(left):
+                graph.replay()
+                got.append((0, out.clone()))
+            with torch.cuda.stream(right):
+                got += [(1 + i, fca.flash_colreduce(q, k, "sum", True)) for i, (q, k) in enumerate(prefills)]
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, want[i]) for i, x in got)
+        assert torch.equal(fca.flash_colreduce(*prefills[0], "sum", True), want[1])
