@@ -41,6 +41,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -6047,48 +6048,76 @@ bool is_capturing(hipStream_t s) {
 // A single sweep expects the whole chip: its workgroups wait for each other, one of eight waves or two of four per CU.  Two of them issued on
 // different streams could be dispatched side by side, each holding CUs the other needs, until their bounded
 // waits run out.  So inside a process they are chained: a single sweep on another stream than the one before
-// first waits (on the GPU; the host never blocks) for an event recorded at the end of that stream.  Calls that
-// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call).  Not under stream
+// first waits (on the GPU; the host blocks only if that stream was destroyed) for an event recorded at the end of that stream.  Calls that
+// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call; on hipStreamPerThread there is one).  Not under stream
 // capture (a graph carries no such edge; graphs holding single sweeps must not replay side by side on one GPU),
 // not for other processes on the same GPU, and not for fcr_colreduce_static, whose calls must not overlap anyway.
+// Where the order cannot be had the call takes the two kernels.
 struct SweepOrder {
   hipEvent_t done = nullptr;
   hipStream_t last = nullptr;
+  uint64_t thread = 0;      // of hipStreamPerThread, one handle for a stream of every thread: whose
   bool any = false;
+  bool recorded = false;    // `done` stands behind the last launch: always so on hipStreamPerThread, where no other thread can record it
 };
 SweepOrder g_order[64];
 std::mutex g_order_mu;
 
-// Takes the lock and returns the device's entry when the launch on stream s is to be chained, else nullptr.
-SweepOrder* order_begin(hipStream_t s) {
-  if (is_capturing(s)) return nullptr;
+uint64_t thread_number() {   // (the address of a thread's own variable may come back with another thread)
+  static std::atomic<uint64_t> count{0};
+  static thread_local const uint64_t mine = ++count;
+  return mine;
+}
+
+// Stream s waits for what is on the stream of the last single sweep.
+bool wait_for_last(SweepOrder* o, hipStream_t s) {
+  if (!o->recorded) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    hipError_t e = o->thread != 0 ? hipErrorInvalidHandle : hipStreamIsCapturing(o->last, &st);
+    if (e == hipSuccess && st != hipStreamCaptureStatusNone) return false;   // (what it was given before the capture may still run)
+    if (e == hipSuccess) e = hipEventRecord(o->done, o->last);
+    if (e != hipSuccess) {   // the stream is gone, its work perhaps not: the host waits for the device, whoever captures meanwhile
+      (void)hipGetLastError();
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
+      e = hipDeviceSynchronize();
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      return e == hipSuccess;
+    }
+  }
+  return hipStreamWaitEvent(s, o->done, 0) == hipSuccess;
+}
+
+// Whether a single sweep may be launched on stream s; then `o` is the device's entry, locked until order_end, or null for a captured launch,
+// which nothing orders.
+bool order_begin(hipStream_t s, SweepOrder*& o) {
+  o = nullptr;
+  if (is_capturing(s)) return true;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
     (void)hipGetLastError();
-    return nullptr;
+    return false;
   }
   g_order_mu.lock();
-  SweepOrder* o = &g_order[dev];
-  if (!o->done && hipEventCreateWithFlags(&o->done, hipEventDisableTiming) != hipSuccess) {
+  SweepOrder* const e = &g_order[dev];
+  if (!e->done && hipEventCreateWithFlags(&e->done, hipEventDisableTiming) != hipSuccess) e->done = nullptr;
+  const bool same = e->last == s && e->thread == (s == hipStreamPerThread ? thread_number() : 0);
+  if (!e->done || (e->any && !same && !wait_for_last(e, s))) {
     (void)hipGetLastError();
-    o->done = nullptr;
     g_order_mu.unlock();
-    return nullptr;
+    return false;
   }
-  if (o->any && o->last != s) {
-    // (a stream that is being captured now, or was destroyed, is left alone: nothing of it can still run)
-    hipStreamCaptureStatus lst = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(o->last, &lst) != hipSuccess || lst != hipStreamCaptureStatusNone ||
-        hipEventRecord(o->done, o->last) != hipSuccess || hipStreamWaitEvent(s, o->done, 0) != hipSuccess)
-      (void)hipGetLastError();
-  }
-  return o;
+  o = e;
+  return true;
 }
 void order_end(SweepOrder* o, hipStream_t s, bool launched_it) {
   if (!o) return;
   if (launched_it) {
     o->last = s;
+    o->thread = s == hipStreamPerThread ? thread_number() : 0;
     o->any = true;
+    o->recorded = o->thread != 0 && hipEventRecord(o->done, s) == hipSuccess;
+    if (o->thread != 0 && !o->recorded) (void)hipGetLastError();
   }
   g_order_mu.unlock();
 }
@@ -6150,12 +6179,14 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
     p.total = p.teams * p.splits;
     const long long polls = __atomic_load_n(&g_wait_polls, __ATOMIC_RELAXED);
     p.spin_limit = polls > 0x7fffffffll ? 0x7fffffff : (int)polls;
-    fcr_detail::fused_refused = false;
-    SweepOrder* const order = order_begin(s);
-    launch_sweeps(dtype, 3, p, ksteps, causal != 0, mode | form, s, reinterpret_cast<unsigned*>(p.part), words);
-    const int lrc = fcr_detail::fused_refused ? 0 : launched("col_fused_kernel");
-    order_end(order, s, !fcr_detail::fused_refused && lrc == 0);
-    if (!fcr_detail::fused_refused) return lrc;
+    SweepOrder* order;
+    if (order_begin(s, order)) {
+      fcr_detail::fused_refused = false;
+      launch_sweeps(dtype, 3, p, ksteps, causal != 0, mode | form, s, reinterpret_cast<unsigned*>(p.part), words);
+      const int lrc = fcr_detail::fused_refused ? 0 : launched("col_fused_kernel");
+      order_end(order, s, !fcr_detail::fused_refused && lrc == 0);
+      if (!fcr_detail::fused_refused) return lrc;
+    }
   }
   if (single && !is_capturing(static_cast<hipStream_t>(stream))) {   // (a captured call keeps the bits of the two launches)
     const BothPlan o = both_plan(dtype, ksteps, p.bh_count, M, N, causal != 0);
@@ -6163,8 +6194,12 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
   }
   rc = fcr_row_lse(q, k, ws, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream);
   if (rc) return rc;
-  return col_reduce_any(q, k, ws, out, out2, mode, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream,
-                        res);
+  rc = col_reduce_any(q, k, ws, out, out2, mode, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream,
+                      res);
+  if (rc || !single || !fused) return rc;
+  // a single sweep that was not launched, so nobody waited: fcr_colreduce_status looks there (behind the kernels, whose partial results may lie there)
+  hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), nullptr, 0, reinterpret_cast<unsigned*>(ws + f.sync_at));
+  return launched("zero_words_kernel");
 }
 }  // namespace
 

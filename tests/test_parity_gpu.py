@@ -2458,3 +2458,86 @@ def test_prefill_beside_a_captured_decode():
         torch.cuda.synchronize()
         assert all(torch.equal(x, want[i]) for i, x in got)
         assert torch.equal(fca.flash_colreduce(*prefills[0], "sum", True), want[1])
+
+
+def _decode_call(q, k, out, ws, stream):
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    _, h, m, d = q.shape
+    _lib.check(lib.fcr_colreduce(q.data_ptr(), k.data_ptr(), out.data_ptr(), ws.data_ptr(), _lib.DTYPE_F16, 1, h, m, k.shape[2], d,
+                                 _lib.strides4(q.stride()), _lib.strides4(k.stride()), d ** -0.5, 0, 1, stream))
+
+
+def test_single_sweeps_take_the_two_kernels_where_nothing_orders_them():
+    """While the stream of the last single sweep is being captured, nothing can be recorded behind what it was given before: a call on another
+    stream then takes the two kernels (their bits, and a status of 0 whatever the scratch held), and the single sweep again afterwards."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    h, m, n, d = 64, 64, 8192, 128
+    g = torch.Generator(device="cuda").manual_seed(9)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g).half() for r in (m, n))
+    floats = lib.fcr_lse_bytes(1, h, m, n, d) // 4
+    ws, side_ws = (torch.empty(floats, device="cuda") for _ in range(2))
+    out, side_out = (torch.empty(h, n, device="cuda") for _ in range(2))
+    main, side = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    want = {}
+    for option in (0, 1):
+        lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, option)
+        try:
+            _decode_call(q, k, out, ws, main.cuda_stream)
+            main.synchronize()
+            want[option] = out.clone()
+        finally:
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+    assert not torch.equal(want[0], want[1])
+    _decode_call(q, k, out, ws, main.cuda_stream)
+    graph = torch.cuda.CUDAGraph()
+    side_ws.fill_(-1.0)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=main, capture_error_mode="relaxed"):
+        _decode_call(q, k, out, ws, main.cuda_stream)
+        _decode_call(q, k, side_out, side_ws, side.cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(side_out, want[0])
+    assert lib.fcr_colreduce_status(side_ws.data_ptr(), _lib.DTYPE_F16, 1, h, m, n, d, side.cuda_stream) == 0
+    _decode_call(q, k, side_out, side_ws, side.cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(side_out, want[1])
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want[1])
+
+
+def test_single_sweeps_on_the_streams_of_several_threads():
+    """hipStreamPerThread is one handle for a stream of every thread: single sweeps that threads issue on theirs are kept apart, among
+    themselves and from those on an ordinary stream, and every result is right."""
+    import threading
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    per_thread = 2   # hipStreamPerThread
+    h, m, n, d = 64, 64, 8192, 128
+    g = torch.Generator(device="cuda").manual_seed(10)
+    q, k = (torch.randn(1, h, r, d, device="cuda", generator=g).half() for r in (m, n))
+    floats = lib.fcr_lse_bytes(1, h, m, n, d) // 4
+    streams = [per_thread, per_thread, torch.cuda.Stream().cuda_stream]
+    ws = [torch.empty(floats, device="cuda") for _ in range(4)]
+    out = [torch.zeros(h, n, device="cuda") for _ in range(4)]
+    _decode_call(q, k, out[3], ws[3], torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    errors = []
+
+    def run(i):
+        try:
+            for _ in range(6):
+                _decode_call(q, k, out[i], ws[i], streams[i])
+        except Exception as e:
+            errors.append(e)
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    assert all(torch.equal(x, out[3]) for x in out[:3])
