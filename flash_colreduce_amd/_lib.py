@@ -85,6 +85,8 @@ def _declare(lib):
     lib.fcr_set_option.argtypes = [c.c_int, c.c_longlong]
     lib.fcr_colreduce_status.restype = c.c_int
     lib.fcr_colreduce_status.argtypes = [c.c_void_p] + [c.c_int] * 6 + [c.c_void_p]
+    lib.fcr_colreduce_ws_status.restype = c.c_int
+    lib.fcr_colreduce_ws_status.argtypes = [c.c_void_p, c.c_size_t] + [c.c_int] * 6 + [c.c_void_p]
     return lib
 
 

@@ -86,7 +86,8 @@ struct Params {
   float inv_m;       //   multiplied by inv_m = 1/M, column j from there on is divided by N - j
   // col_fused_kernel: teams of `splits` workgroups, team t takes (b,h) = t, t + teams, ..
   int teams;
-  unsigned* sync;    // error word; zero at launch, like the slots at `part`
+  unsigned* sync;    // error word; zero at launch, like the slots at `part`.  both_sweeps_kernel: null if the workspace has no room for it;
+                     // row_lse_kernel clears it for the calls that take two launches instead
   int spin_limit;    // polls of the counter after which a wait gives up
   // both_sweeps_kernel: `tiles`, `group`, `fill` and `total` are of the row sweeps
   int col_tiles, col_group;
@@ -809,6 +810,7 @@ __device__ __forceinline__ void row_sweep(const Params& p, char* smem, int tid, 
 template <int DT, int KS, bool CAUSAL, int NB, bool STREAM_ONCE>
 __global__ __launch_bounds__(kThreads, (KS > 8 ? 1 : 2)) void row_lse_kernel(const Params p) {
   __shared__ __attribute__((aligned(1024))) char smem[Ring<KS>::kBytes];
+  if (p.sync != nullptr && blockIdx.x == 0 && threadIdx.x == 0) p.sync[0] = 0u;
   int bh, tile, split;
   map_block_split(p, (int)blockIdx.x, CAUSAL, bh, tile, split);
   row_sweep<DT, KS, CAUSAL, NB, STREAM_ONCE, false>(p, smem, (int)threadIdx.x, bh, tile, split);
@@ -1107,6 +1109,7 @@ __device__ __forceinline__ void col_sweep(const Params& p, char* smem, int bh, i
   for (int t = nfull; t < nchunks; ++t) general_chunk(t, std::true_type());
 
   ring_sync<0>();   // every load has landed (those past the last chunk write zeros): the LDS can be reused
+  if (FOLLOW && given_up && p.sync != nullptr) p.sync[0] = 1u;
   col_store<MODE, NG>(p, smem, bh, k0, csum, cmax, lane, wave, given_up);
 }
 
@@ -1126,7 +1129,7 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 // kPatience polls, then takes the tile in hand itself, marks it and sweeps it (the place's own workgroup will store the same bits once more).  So a
 // column sweep waits only for row tiles that a running workgroup has in hand, and those wait for nobody: every wait ends, whatever the order in which
 // workgroups start and whatever else holds CUs meanwhile, be it kernels that wait for each other, and no launch has to be kept apart from another.
-// The bound on a wait (p.spin_limit polls, then the columns become NaN) is for a host that lowers it.
+// The bound on a wait (p.spin_limit polls, then the columns become NaN and p.sync[0] is set) is for a host that lowers it.
 // The look costs 0.25 % in the geometric mean of 1600 shapes (a round trip to memory per column tile, beside another workgroup's sweep), all of it,
 // the mark and the loop 1.0 %.  Started in the reverse order, columns first, the launch gives the same bits in 1.2 to 2.3 times the time.  (Tickets
 // for all tiles instead, rows first, cost 4.9 %, up to half of a short call: 64 to 128 atomics on a line before the first load of a
@@ -2949,16 +2952,19 @@ __device__ __forceinline__ float row16_reduce(float v) {
   return v;
 }
 
-// n words from w on, and the word at `one`.  (A workspace of one of the calls without a size may start at any multiple of 8 bytes.)  A launch of its own in front of every single sweep: 16 bytes per
-// thread, and of a launch of one round one of the two sets of slots (32 pairs of 128 x 4096 x 128 17.8 -> 17.4 us per call).
-__global__ __launch_bounds__(256) void fill_words_kernel(unsigned* __restrict__ w, int64_t n, unsigned value) {
+// n words from w on get `value`, and the word at `zero`, if there is one, 0: in front of both_sweeps_kernel.
+__global__ __launch_bounds__(256) void fill_words_kernel(unsigned* __restrict__ w, int64_t n, unsigned value, unsigned* __restrict__ zero) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + (int)threadIdx.x) * 4;
   if ((reinterpret_cast<uintptr_t>(w) & 15) == 0 && i + 4 <= n) {
     *reinterpret_cast<u32x4*>(w + i) = (u32x4){value, value, value, value};
   } else {
     for (int64_t j = i; j < n && j < i + 4; ++j) w[j] = value;
   }
+  if (i == 0 && zero != nullptr) *zero = 0u;
 }
+
+// n words from w on, and the word at `one`.  (A workspace of one of the calls without a size may start at any multiple of 8 bytes.)  A launch of its own in front of every single sweep: 16 bytes per
+// thread, and of a launch of one round one of the two sets of slots (32 pairs of 128 x 4096 x 128 17.8 -> 17.4 us per call).
 __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ w, int n, unsigned* __restrict__ one) {
   const int i = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4;
   if ((reinterpret_cast<uintptr_t>(w) & 15) == 0 && i + 4 <= n) {
@@ -5262,6 +5268,17 @@ BothPlan both_plan(int dtype, int ksteps, int64_t bh, int M, int N, bool causal)
   return o;
 }
 
+// Where the status word of both_sweeps_kernel stands in a workspace of fcr_workspace_bytes, in floats, for problems that take it with the mask or
+// without (the size does not know which); -1 where there is none, as where few_keys_kernel is meant, whose columns may lie there.
+// base_floats: what fcr_lse_bytes asks for.
+constexpr int kStatusFloats = 32;
+int64_t both_status_at(int dtype, int B, int H, int M, int N, int D, int64_t base_floats) {
+  const int ksteps = ksteps_of(dtype, D);
+  const int64_t bh = (int64_t)B * H;
+  if (both_plan(dtype, ksteps, bh, M, N, true).row_blocks == 0 && both_plan(dtype, ksteps, bh, M, N, false).row_blocks == 0) return -1;
+  return few_keys_plan(dtype, B, H, M, N, D, false, base_floats).form >= 0 ? -1 : (base_floats + 63) / 64 * 64;
+}
+
 int launched(const char* what) {
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) return 0;
@@ -5771,7 +5788,7 @@ int launch_both(Params& p, int dtype, int ksteps, const BothPlan& o, float* ws, 
   const long long polls = __atomic_load_n(&g_wait_polls, __ATOMIC_RELAXED);
   p.spin_limit = polls > 0x7fffffffll ? 0x7fffffff : (int)polls;
   const int64_t words = (int64_t)p.bh_count * p.M;
-  hipLaunchKernelGGL(fill_words_kernel, dim3((unsigned)((words + 1023) / 1024)), dim3(256), 0, s, reinterpret_cast<unsigned*>(ws), words, kNotYet);
+  hipLaunchKernelGGL(fill_words_kernel, dim3((unsigned)((words + 1023) / 1024)), dim3(256), 0, s, reinterpret_cast<unsigned*>(ws), words, kNotYet, p.sync);
   const int rc = launched("fill_words_kernel");
   if (rc) return rc;
   (dtype == FCR_DTYPE_F16 ? fcr_detail::sweeps_f16_both : fcr_detail::sweeps_bf16_both)(p, ksteps, causal, mode, s);
@@ -5891,14 +5908,16 @@ size_t fcr_lse_bytes(int B, int H, int M, int N, int D) {
   return fcr_lse_bytes_two_kernels(B, H, M, N);
 }
 
-int fcr_row_lse(const void* q, const void* k, float* lse, int dtype, int B, int H, int M, int N, int D,
-                const int64_t q_strides[4], const int64_t k_strides[4], float scale, int causal,
-                void* stream) {
+namespace {
+// status: a word to clear, or null
+int row_lse_any(const void* q, const void* k, float* lse, unsigned* status, int dtype, int B, int H, int M, int N, int D,
+                const int64_t q_strides[4], const int64_t k_strides[4], float scale, int causal, void* stream) {
   Params p;
   if (!lse) return fail(FCR_E_NULL, "null pointer argument");
   int rc = make_params(p, q, k, dtype, B, H, M, N, D, q_strides, k_strides, scale, false, causal != 0);
   if (rc) return rc;
   p.lse = lse;
+  p.sync = status;
   p.splits = row_splits(dtype, B, H, M, N, D);
   p.part = lse + (int64_t)B * H * M;  // only touched when splits > 1 (see fcr_lse_bytes)
   p.total *= p.splits;
@@ -5913,6 +5932,13 @@ int fcr_row_lse(const void* q, const void* k, float* lse, int dtype, int B, int 
   hipLaunchKernelGGL(lse_combine_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, p.part, lse, rows,
                      p.splits);
   return launched("lse_combine_kernel");
+}
+}  // namespace
+
+int fcr_row_lse(const void* q, const void* k, float* lse, int dtype, int B, int H, int M, int N, int D,
+                const int64_t q_strides[4], const int64_t k_strides[4], float scale, int causal,
+                void* stream) {
+  return row_lse_any(q, k, lse, nullptr, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream);
 }
 
 namespace {
@@ -6188,11 +6214,17 @@ int whole_call(const void* q, const void* k, void* out, const ResultSpec& res, f
       if (!fcr_detail::fused_refused) return lrc;
     }
   }
+  unsigned* status = nullptr;
+  if (ws_bytes != 0) {
+    const int64_t at = both_status_at(dtype, B, H, M, N, D, (int64_t)(lse_bytes / sizeof(float)));
+    if (at >= 0 && (size_t)(at + kStatusFloats) * sizeof(float) <= ws_bytes) status = reinterpret_cast<unsigned*>(ws + at);
+  }
   if (single && !is_capturing(static_cast<hipStream_t>(stream))) {   // (a captured call keeps the bits of the two launches)
     const BothPlan o = both_plan(dtype, ksteps, p.bh_count, M, N, causal != 0);
+    p.sync = status;
     if (o.row_blocks > 0) return launch_both(p, dtype, ksteps, o, ws, mode, causal != 0, static_cast<hipStream_t>(stream));
   }
-  rc = fcr_row_lse(q, k, ws, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream);
+  rc = row_lse_any(q, k, ws, status, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream);
   if (rc) return rc;
   rc = col_reduce_any(q, k, ws, out, out2, mode, dtype, B, H, M, N, D, q_strides, k_strides, scale, causal, stream,
                       res);
@@ -6289,6 +6321,8 @@ size_t fcr_workspace_bytes(int dtype, int B, int H, int M, int N, int D) {
   if (row_width_ok(dtype, D)) {
     const int64_t floats = (int64_t)(base / sizeof(float));
     int64_t most = few_keys_plan(dtype, B, H, M, N, D, true, floats).floats;   // (one result takes half of it)
+    const int64_t status_at = both_status_at(dtype, B, H, M, N, D, floats);
+    if (status_at >= 0 && status_at + kStatusFloats > most) most = status_at + kStatusFloats;
     FusedPlan f;
     if (dtype != FCR_DTYPE_F32 && ksteps_of(dtype, D) <= 4 && fused_shape((int64_t)B * H, M, N, f)) {
       const FusedPairPlan two = fused_pair_plan((int64_t)B * H, M, N, ksteps_of(dtype, D), f);
@@ -6366,22 +6400,35 @@ int fcr_set_option(int option, long long value) {
   return fail(FCR_E_SHAPE, "unknown option");
 }
 
-int fcr_colreduce_status(const float* lse_ws, int dtype, int B, int H, int M, int N, int D, void* stream) {
-  if (!lse_ws) return fail(FCR_E_NULL, "null pointer argument");
-  if (B < 1 || H < 1 || M < 1 || N < 1 || D < 1) return fail(FCR_E_SHAPE, "B, H, M, N, D must be >= 1");
-  FusedPlan f;
-  if (dtype == FCR_DTYPE_F32 || ksteps_of(dtype, D) > 4 || !fused_shape((int64_t)B * H, M, N, f)) return 0;
+namespace {
+// FCR_E_WAIT if the word on the device is set, once the stream's work is done.
+int read_status(const unsigned* at, const char* text, hipStream_t s) {
   unsigned word = 0;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  hipError_t e = hipMemcpyAsync(&word, reinterpret_cast<const unsigned*>(lse_ws + f.sync_at), sizeof(word),
-                                hipMemcpyDeviceToHost, s);
+  hipError_t e = hipMemcpyAsync(&word, at, sizeof(word), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     snprintf(g_err, sizeof(g_err), "reading the status word failed: %s", hipGetErrorString(e));
     return (int)e;
   }
-  if (word != 0) return fail(FCR_E_WAIT, "a workgroup of the single sweep gave up waiting for its team; the columns of that (b,h) pair are NaN");
-  return 0;
+  return word != 0 ? fail(FCR_E_WAIT, text) : 0;
+}
+}  // namespace
+
+int fcr_colreduce_status(const float* lse_ws, int dtype, int B, int H, int M, int N, int D, void* stream) {
+  if (!lse_ws) return fail(FCR_E_NULL, "null pointer argument");
+  if (B < 1 || H < 1 || M < 1 || N < 1 || D < 1) return fail(FCR_E_SHAPE, "B, H, M, N, D must be >= 1");
+  FusedPlan f;
+  if (dtype == FCR_DTYPE_F32 || ksteps_of(dtype, D) > 4 || !fused_shape((int64_t)B * H, M, N, f)) return 0;
+  return read_status(reinterpret_cast<const unsigned*>(lse_ws + f.sync_at),
+                     "a workgroup of the single sweep gave up waiting for its team; the columns of that (b,h) pair are NaN", static_cast<hipStream_t>(stream));
+}
+
+int fcr_colreduce_ws_status(const void* ws, size_t ws_bytes, int dtype, int B, int H, int M, int N, int D, void* stream) {
+  const int rc = fcr_colreduce_status(static_cast<const float*>(ws), dtype, B, H, M, N, D, stream);
+  if (rc || (dtype != FCR_DTYPE_F16 && dtype != FCR_DTYPE_BF16) || !row_width_ok(dtype, D)) return rc;
+  const int64_t at = both_status_at(dtype, B, H, M, N, D, (int64_t)(fcr_lse_bytes(B, H, M, N, D) / sizeof(float)));
+  if (at < 0 || (size_t)(at + kStatusFloats) * sizeof(float) > ws_bytes) return 0;
+  return read_status(static_cast<const unsigned*>(ws) + at, "a column sweep gave up waiting for row statistics; its columns are NaN", static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -72,7 +72,7 @@ extern "C" {
 #define FCR_E_REDUCTION -5 /* reduction is not FCR_REDUCE_* */
 #define FCR_E_SCALE -6     /* scale is not finite */
 #define FCR_E_SCRATCH -7   /* fcr_colreduce_static: the problem needs more than FCR_STATIC_SCRATCH_BYTES */
-#define FCR_E_WAIT -8      /* fcr_colreduce_status: a workgroup of the single sweep gave up waiting for its team */
+#define FCR_E_WAIT -8      /* fcr_colreduce_status, _ws_status: a workgroup gave up waiting (see FCR_OPT_WAIT_POLLS), columns are NaN */
 
 /* fcr_set_option */
 #define FCR_OPT_SINGLE_SWEEP 0 /* 0: every call takes the two kernels, in two launches (default 1) */
@@ -268,6 +268,12 @@ int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, in
  * No counterpart in the reference, whose kernel has no cross-program dependencies.
  */
 int fcr_colreduce_status(const float* lse_ws, int dtype, int B, int H, int M, int N, int D, void* stream);
+
+/*
+ * The same for the last fcr_colreduce_ws on a workspace of fcr_workspace_bytes bytes or more, ws_bytes as that call got it: it also tells
+ * whether a column sweep in one launch with the row sweeps gave up waiting.  (The calls without ws_bytes have no word for that.)
+ */
+int fcr_colreduce_ws_status(const void* ws, size_t ws_bytes, int dtype, int B, int H, int M, int N, int D, void* stream);
 
 /*
  * Process-wide switches (FCR_OPT_*), read by every later call: every path but the two launches on or off (results agree

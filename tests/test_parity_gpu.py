@@ -2541,3 +2541,33 @@ def test_single_sweeps_on_the_streams_of_several_threads():
     torch.cuda.synchronize()
     assert not errors
     assert all(torch.equal(x, out[3]) for x in out[:3])
+
+
+def test_both_sweeps_report_a_wait_that_gave_up():
+    """fcr_colreduce_ws_status says so after the call whose columns are NaN, and 0 after any other call on that workspace: the next one, one in two
+    launches, one on a workspace whose word was never written, one without room for the word."""
+    from flash_colreduce_amd import _lib
+    lib = _lib.load()
+    h, m, d = 4, 1200, 128
+    q, k = (x.cuda() for x in _inputs.randn_pair(1, h, m, m, d, seed=5, dtype=torch.float16))
+    ws, out = torch.full((_lib_workspace(q, k),), -1.0, device="cuda"), torch.empty(h, m, device="cuda")
+    least = lib.fcr_lse_bytes(1, h, m, m, d) // 4
+    assert ws.numel() > least
+    state = lambda w: lib.fcr_colreduce_ws_status(w.data_ptr(), 4 * w.numel(), _lib.DTYPE_F16, 1, h, m, m, d, torch.cuda.current_stream().cuda_stream)
+
+    def call(w, causal, options=()):
+        for option, value in options:
+            lib.fcr_set_option(option, value)
+        try:
+            _ws_call(q, k, out, w, causal)
+        finally:
+            lib.fcr_set_option(_lib.OPT_WAIT_POLLS, 1 << 20)
+            lib.fcr_set_option(_lib.OPT_SINGLE_SWEEP, 1)
+        return state(w)
+    no_polls, two_launches = [(_lib.OPT_WAIT_POLLS, 0)], [(_lib.OPT_SINGLE_SWEEP, 0)]
+    assert call(ws, True, two_launches) == 0     # first of all: nothing else has cleared the word
+    for after in ((True, ()), (True, two_launches), (False, ())):
+        assert call(ws, True, no_polls) == -8 and out.isnan().any()
+        assert call(ws, *after) == 0 and out.isfinite().all()
+    assert call(ws[:least], True, no_polls) == 0 and out.isnan().any()
+    assert lib.fcr_colreduce_ws_status(None, 1 << 20, 0, 1, 1, 8, 8, 64, None) == -1
