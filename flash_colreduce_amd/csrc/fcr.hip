@@ -5220,21 +5220,16 @@ FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool bot
 
 // Both sweeps in one launch (both_sweeps_kernel): 32-row blocks per wave of its row and its column tiles; row_blocks 0: two launches.
 // The column sweeps start where row sweeps leave a CU, so a launch that does not fill its last round no longer costs a round twice, and
-// where the mask gives row tiles that end early the column sweeps follow them.  us per call, two launches -> one, against 256-row tiles per CU (`rows`), of
-// 480 shapes of 4 to 512 pairs, 530 to 9000 queries, fp16 and bf16, all reductions:
-//   With the mask and as many keys as queries, rows of more than 128 bytes: up to 0.9 both tiles have 128 rows (18 pairs of 2240 x 128 55.5 -> 41,
-//   11 of 4078 x 128 103 -> 67, 4 of 570 x 128 18.9 -> 16.6), up to 1.9 the column tiles (27 of 2240 65 -> 54, 37 of 2810 106 -> 92), and from 2.65 on
-//   neither (155 of 1538 151 -> 133, 43 of 6338 514 -> 447).  In between two launches, each with its second helping dealt
-//   backwards (map_group), are as fast (48 of 2929 118 -> 120, 25 of 5834 212 -> 220, 32 of 4954 199 -> 197), and so are they for a few rounds of long sweeps, whose
-//   last round is a small part (32 of 8192 468 -> 472, of 16384 1798 -> 1810).  Rows of 129 to 192 bytes lose between 1.0 and 1.3 as well (60 of 1045 x 80 27.3 -> 29.5).
-//   Rows of up to 128 bytes: 128-row tiles, four workgroups to a CU; two launches between 1.1 and 2.6 (10 of 8777 x 64 138 -> 148, 61 of 2304 68 -> 75; but 259 of
-//   626 41 -> 34, 206 of 1100 77 -> 60).  Rows of more than 256 bytes: 128-row tiles, always (10 of 1895 x 256 54 -> 41, 32 of 2048 79 -> 68, 77 of 4305 692 -> 675).
-//   Without the mask, or with many more keys than queries, no column can start before the rows of its pair end: there have to be row
-//   tiles for every CU (24 of 2893 x 128 144 -> 121, 48 of 2929 244 -> 207, 61 of 2223 174 -> 143, 18 of 7902 x 64 449 -> 355; but 17 of 2873 x 128 88 -> 89, 5 of 3039 50 -> 64;
-//   with 128 queries per 1000 keys 68 of 1090 x 8104 318 -> 334).
-//   Many rounds: the last one is a small part of them, and one launch is as fast in the mean and up to 1.07 of the time (640 of 1479 x 96 391 -> 424).
-//   Geometric means over 2600 squares of 1030 to 6000, `rows` of 4 to 6, 6 to 10, 10 to 16 and beyond: with the mask D = 64 0.80, 0.88, 0.92, 0.98, 128 0.90, 0.95,
-//   0.99, 1.00, 256 0.97, 1.00, 1.00, 1.00; without it 64 0.92, 0.95, 0.99, 1.02, 128 0.95, 0.98, 1.00, 1.01, 256 0.99, 1.00, 1.00, 1.00.
+// where the mask gives row tiles that end early the column sweeps follow them.  What two launches have and one has not: keys split over workgroups where there are few
+// row tiles, rounds that tiles fill exactly, both second helpings dealt backwards (map_group), and no words to fill, which counts in calls of 20 us.
+// `rows` and `small`: tiles of 256 and of 128 rows per CU.  Figures: one launch's time against two's, of 29000 shapes of 1 to 1200 pairs, 400 to 9000 queries, 370 to 35000
+// keys, fp16 and bf16, all reductions, as a geometric mean and the share that loses 3 % or more.  What is taken: 0.922, 2 % (0.843 below one round); what the cuts beside each
+// `if` leave to two launches: 0.992, 20 %.  us, two launches -> one:
+//   With the mask and at most 1.5 keys per query (`level`) the column sweeps can follow the row sweeps from the start: 0.911.  Rows of 129 to 256 bytes have 128-row tiles up
+//   to 0.9 (11 of 4078 x 128 103 -> 68), 256-row ones for rows up to 1.9 (27 of 2240 65 -> 55), for both beyond (155 of 1538 151 -> 134); others 128-row tiles (10 of
+//   1895 x 256 54 -> 41, 32 of 2048 79 -> 69, 259 of 626 x 64 41 -> 35).
+//   With the mask and more keys than that 0.961, without it 0.929: no column can start before the rows of its pair end, so there has to be a row tile for every
+//   CU (24 of 2893 x 128 144 -> 122, 18 of 7902 x 64 449 -> 359).
 struct BothPlan {
   int row_blocks = 0, col_blocks = 0;
 };
@@ -5246,22 +5241,34 @@ BothPlan both_plan(int dtype, int ksteps, int64_t bh, int M, int N, bool causal)
   const int64_t tiles = bh * ((M + 127) / 128), cols = bh * ((N + 127) / 128);   // of 128 rows
   if (tiles + cols >= kMaxWorkgroups / 2) return o;
   const double small = (double)tiles / cus, rows = (double)(bh * ((M + 255) / 256)) / cus;
-  const bool longer = 2 * (int64_t)N > 3 * (int64_t)M, level = causal && !longer;   // level: the column sweeps can follow the row sweeps
+  const bool longer = 2 * (int64_t)N > 3 * (int64_t)M, level = causal && !longer;
+  auto within = [&](double from, double to) { return rows >= from && rows < to; };
+  // few tiles, whose keys two launches split: 1.05, 57 % (1 pair of 6891 x 8176 x 32 46 -> 64), and 1.02, 35 %; the rest below 0.4 0.876
+  if (level && ((small < 0.26 && 20 * (int64_t)N > 23 * (int64_t)M) || (small < 0.4 && bh == 1 && ksteps <= 2))) return o;
   int nr = 1, nc = 1;
-  if (rows >= (ksteps > 4 ? 6.0 : ksteps <= 2 && level ? 16.0 : 10.0)) return o;
   if (ksteps > 4) {
+    if (rows >= 5.0) return o;                                                   // 0.99 (216 pairs of 1562 x 256 290 -> 309)
     if (!level && small < 1.05) return o;
-  } else if (ksteps <= 2) {
-    if (level ? rows >= 1.1 && (rows < 2.7 || N >= 10000) : longer ? rows < 1.1 : small < 1.02 || (small >= 1.5 && rows < 1.1)) return o;
+    if (longer && causal && N >= 11000 && rows < 2.0) return o;                  // 1.004, 10 % (17 of 6554 x 20777 x 256 1771 -> 1987); the rest 0.975
+    if (!causal && rows < 1.0 && (small >= 1.5 || 10 * (int64_t)N < 9 * (int64_t)M)) return o;   // 0.994, 12 %; the rest below one round 0.895
+  } else if (level && ksteps <= 2) {
+    if (rows >= 16.0 || within(1.1, 2.7) || (rows >= 2.7 && N >= 10000)) return o;   // (61 of 2304 x 64 68 -> 75, 10 of 8777 138 -> 148)
+    if (N < 700 && within(0.6, 1.1)) return o;                                   // 1.03, 56 % (58 of 671 x 562 x 32 14.1 -> 15.5); with more keys 0.814
   } else if (level) {
-    if (rows >= 1.85 && (rows < 2.1 ? N > 8500 : rows < 2.65 || N >= 8000)) return o;
-    if (ksteps == 3 && rows >= 1.0 && rows < 1.3) return o;
+    if (rows >= 10.0 || within(2.1, 2.65) || (rows >= 2.65 && N >= 8000)) return o;  // as fast (48 of 2929 x 128 118 -> 120, 32 of 8192 468 -> 472)
+    if (N >= 3400 && within(1.85, 2.1)) return o;                                // 0.97, 18 %; with fewer keys 0.936
+    if (ksteps == 3 && within(1.0, 2.65)) return o;                              // 0.99, 21 % (25 of 4880 x 80 145 -> 168)
+    if (N < 1000 && (ksteps == 3 ? within(0.6, 1.0) : within(0.9, 1.1))) return o;   // 0.99, 33 %, and 0.985, 39 %; with more keys 0.786 and 0.912
     nr = rows >= 0.9 ? 2 : 1;
     nc = rows >= 1.9 ? 2 : 1;
   } else {
-    if (longer ? rows < 1.85 : small < 1.02 || (small >= 1.5 && rows < 1.0)) return o;
-    nr = rows >= 1.5 ? 2 : 1;
-    nc = rows >= 1.85 ? 2 : 1;
+    if (rows >= 10.0 || (longer && rows < (ksteps <= 2 ? 1.1 : 1.85))) return o; // (68 of 1090 x 8104 x 128 318 -> 334)
+    if (!longer && (small < 1.02 || rows < (ksteps <= 2 ? 0.67 : 1.0))) return o;   // 0.997, 23 %, and 0.98, 26 % (5 of 7839 x 6211 x 128 148 -> 198); beyond 0.92
+    if (!longer && ksteps <= 2 && small >= 1.5 && rows < 1.1) return o;
+    if (ksteps > 2) {
+      nr = rows >= 1.5 ? 2 : 1;
+      nc = rows >= 1.85 ? 2 : 1;
+    }
   }
   o.row_blocks = nr;
   o.col_blocks = nc;

@@ -284,3 +284,18 @@ def test_fp32_tiles_with_the_mask(f32_tiles):
         assert row(m, n, bh, 1, 256)[0] == waves, (m, n)
     assert col(4, 0, 2000, 2000, 20, 0, 256) == (8, 2) and col(4, 0, 2000, 2000, 48, 1, 256) == (8, 2)   # no mask; three per CU
     assert col(2, 1, 12, 15478, 2, 0, 256) == (4, 2) and col(8, 1, 128, 1024, 32, 1, 256) == (8, 1)
+
+
+def test_which_calls_have_room_for_the_word_of_both_sweeps():
+    """fcr_workspace_bytes holds a status word for 16-bit problems whose sweeps share a launch (with the mask or without), restated for 256 CUs
+    at shapes on both sides of the rule's cuts: those on the second side lose by it, or gain nothing."""
+    lib = _lib.load()
+    if torch.cuda.is_available():
+        pytest.skip("the rule is restated for the 256 CUs that the library assumes without a device")
+    more = lambda h, m, n, d, dtype=0: lib.fcr_workspace_bytes(dtype, 1, h, m, n, d) - lib.fcr_lse_bytes(1, h, m, n, d)
+    for shape in ((32, 2048, 2048, 256), (11, 4078, 4078, 128), (27, 2240, 2240, 128), (155, 1538, 1538, 128), (3, 700, 700, 128), (24, 2893, 2893, 128),
+                  (10, 1895, 1895, 256), (18, 7902, 7902, 64), (60, 1000, 1000, 128), (2, 1000, 1100, 128), (250, 520, 1500, 128)):
+        assert 0 < more(*shape) <= 512 and 0 < more(*shape, 1) <= 512 and more(*shape, 2) == 0, shape
+    for shape in ((4, 128, 700, 128), (32, 512, 32768, 128), (68, 1090, 8104, 128), (300, 2000, 2000, 256), (216, 1562, 1562, 256), (1, 6891, 8176, 32),
+                  (1, 7061, 7061, 32), (80, 570, 570, 48), (85, 601, 601, 32), (60, 800, 800, 96), (72, 670, 670, 80)):
+        assert more(*shape) == 0, shape
