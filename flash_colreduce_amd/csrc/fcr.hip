@@ -5222,9 +5222,9 @@ FewKeysPlan few_keys_plan(int dtype, int B, int H, int M, int N, int D, bool bot
 // The column sweeps start where row sweeps leave a CU, so a launch that does not fill its last round no longer costs a round twice, and
 // where the mask gives row tiles that end early the column sweeps follow them.  What two launches have and one has not: keys split over workgroups where there are few
 // row tiles, rounds that tiles fill exactly, both second helpings dealt backwards (map_group), and no words to fill, which counts in calls of 20 us.
-// `rows` and `small`: tiles of 256 and of 128 rows per CU.  Figures: one launch's time against two's, of 29000 shapes of 1 to 1200 pairs, 400 to 9000 queries, 370 to 35000
-// keys, fp16 and bf16, all reductions, as a geometric mean and the share that loses 3 % or more.  What is taken: 0.922, 2 % (0.843 below one round); what the cuts beside each
-// `if` leave to two launches: 0.992, 20 %.  us, two launches -> one:
+// `rows` and `small`: tiles of 256 and of 128 rows per CU.  Figures: one launch's time against two's, of 30700 shapes of 1 to 2500 pairs, 130 to 9000 queries, 513 to 50000
+// keys, fp16 and bf16, all reductions, as a geometric mean and the share that loses 3 % or more.  What is taken: 0.922, 1.7 % (0.845 below one round; 1.15 at worst); what the
+// cuts below leave to two launches: 0.994, 21 % (1.39).  us, two launches -> one:
 //   With the mask and at most 1.5 keys per query (`level`) the column sweeps can follow the row sweeps from the start: 0.911.  Rows of 129 to 256 bytes have 128-row tiles up
 //   to 0.9 (11 of 4078 x 128 103 -> 68), 256-row ones for rows up to 1.9 (27 of 2240 65 -> 55), for both beyond (155 of 1538 151 -> 134); others 128-row tiles (10 of
 //   1895 x 256 54 -> 41, 32 of 2048 79 -> 69, 259 of 626 x 64 41 -> 35).
@@ -5243,8 +5243,14 @@ BothPlan both_plan(int dtype, int ksteps, int64_t bh, int M, int N, bool causal)
   const double small = (double)tiles / cus, rows = (double)(bh * ((M + 255) / 256)) / cus;
   const bool longer = 2 * (int64_t)N > 3 * (int64_t)M, level = causal && !longer;
   auto within = [&](double from, double to) { return rows >= from && rows < to; };
-  // few tiles, whose keys two launches split: 1.05, 57 % (1 pair of 6891 x 8176 x 32 46 -> 64), and 1.02, 35 %; the rest below 0.4 0.876
-  if (level && ((small < 0.26 && 20 * (int64_t)N > 23 * (int64_t)M) || (small < 0.4 && bh == 1 && ksteps <= 2))) return o;
+  // few tiles, whose keys two launches split: 0.99, 28 %, and 1.006, 33 % (1 pair of 6891 x 8176 x 32 46 -> 64); the rest below 0.4 0.875
+  if (level && ((small < 0.26 && 20 * (int64_t)N > 23 * (int64_t)M) || (small < 0.4 && bh == 1 && ksteps <= 3))) return o;
+  // Multiples of eight pairs, which deal every die whole pairs, leave two launches less to gain: 0.999, 28 % between 0.9 and 2.7 rounds of 193 to 256 bytes (72 of
+  // 840 x 128 26 -> 32; other numbers of pairs 0.947, 6 %), 0.985, 12 % of 129 to 192 (0.966, 5 %), 0.983, 8 % of more than 256 (0.969, 1 %).
+  const bool whole = bh % 8 == 0 && level;
+  if (whole && (ksteps > 4 ? within(1.3, 1.9) : ksteps == 4 ? within(0.9, 2.7) : ksteps == 3 && within(0.9, 4.0))) return o;
+  // A few hundred queries against many keys: 0.997, 30 % (246 of 314 x 8281 x 96 387 -> 440: 256-row tiles, where two launches have three of 128); the rest of up to 384 queries 0.945.
+  if (longer && M <= 384 && (ksteps <= 2 ? M <= 256 || rows >= 4.0 : ksteps <= 4 ? M > 256 : M <= 256 && rows >= 2.0)) return o;
   int nr = 1, nc = 1;
   if (ksteps > 4) {
     if (rows >= 5.0) return o;                                                   // 0.99 (216 pairs of 1562 x 256 290 -> 309)

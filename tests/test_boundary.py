@@ -297,5 +297,5 @@ def test_which_calls_have_room_for_the_word_of_both_sweeps():
                   (10, 1895, 1895, 256), (18, 7902, 7902, 64), (60, 1000, 1000, 128), (2, 1000, 1100, 128), (250, 520, 1500, 128)):
         assert 0 < more(*shape) <= 512 and 0 < more(*shape, 1) <= 512 and more(*shape, 2) == 0, shape
     for shape in ((4, 128, 700, 128), (32, 512, 32768, 128), (68, 1090, 8104, 128), (300, 2000, 2000, 256), (216, 1562, 1562, 256), (1, 6891, 8176, 32),
-                  (1, 7061, 7061, 32), (80, 570, 570, 48), (85, 601, 601, 32), (60, 800, 800, 96), (72, 670, 670, 80)):
+                  (1, 7061, 7061, 32), (246, 314, 8281, 96), (80, 570, 570, 48), (85, 601, 601, 32), (60, 800, 800, 96), (72, 670, 670, 80)):
         assert more(*shape) == 0, shape
