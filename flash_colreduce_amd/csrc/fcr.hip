@@ -5060,13 +5060,14 @@ FusedPairPlan fused_pair_plan(int64_t bh, int M, int N, int ksteps, const FusedP
 // The single sweep's keys of a pair, dealt evenly to the workgroups of its team (p.splits: as few as can hold them), in steps of
 // `chunks_per_step`; and to as many workgroups as there are CUs for where one round is all there is and that leaves a workgroup at most
 // five eighths of its steps, two or more (a smaller part does not pay for the exchange, and in several rounds the next pair's loads run under it): 0.91
-// to 0.94 of the time for 2850 such shapes.  Not where two query groups per wave hold twice the keys (1.05 for 85 shapes; the estimate that
-// chose them counts on those).
+// to 0.94 of the time for 2850 such shapes.  To 64 at most, as every member reads every other's sums: one pair of 65 to 128 queries and 24576 to 32768 keys
+// 18.0 us with as few as can hold them, 18.1 with a member per CU, 14.7 with 64, 14.6 with 96, 15.2 with 128; of 2 to 32 and 49152 to 65536 keys 17.2, 17.2, 14.8, 14.7 and
+// 14.8.  Not where two query groups per wave hold twice the keys (1.05 for 85 shapes; the estimate that chose them counts on those).
 void spread_keys(Params& p, int N, int chunks_per_step, int cap, bool may_widen) {
   const int steps = (N + chunks_per_step * kChunk - 1) / (chunks_per_step * kChunk);
   int per = (steps + p.splits - 1) / p.splits;
   if (may_widen && p.teams == p.bh_count) {
-    const int places = cap / p.teams;
+    const int places = cap / p.teams < 64 ? cap / p.teams : 64;
     int wide = (steps + places - 1) / places;
     if (wide < 2) wide = 2;
     if (8 * wide <= 5 * per) per = wide;

@@ -2588,3 +2588,10 @@ def test_both_sweeps_share_a_launch(h, m, n, d, dtype, causal):
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:   # (the shapes are chosen for that)
         assert lib.fcr_workspace_bytes(dt, 1, h, m, n, d) > lib.fcr_lse_bytes(1, h, m, n, d)
     test_both_sweeps_in_one_launch(h, m, n, d, dtype, causal)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,m,n,d", [(1, 100, 29647, 64), (1, 2, 63379, 96), (2, 128, 20001, 128), (3, 33, 33000, 64), (1, 64, 40000, 128)])
+def test_single_sweep_teams_of_one_to_three_pairs(h, m, n, d, causal):
+    """Long caches of few pairs, whose teams stop growing at 64 members: the last of them with few keys, ragged chunks."""
+    test_single_sweep_keys_dealt_evenly(h, m, n, d, causal)
