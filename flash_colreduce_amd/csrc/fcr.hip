@@ -2426,7 +2426,8 @@ __global__ __launch_bounds__(64 * NW, 2) void col_reduce_f32_kernel(const Params
 // behind the barrier of the next chunk the waves' (maximum, sum) are merged, so no scores need another form.  Forming a score
 // is three matrix instructions per k-step and the split of its row, which the maximum adds little to.  At most 256 keys: two groups per
 // wave are what the registers hold in parts beside a chunk's scores (four groups of D <= 64 and 16 queries per chunk were built: 256 pairs of 512 x
-// 512 x 64 77 -> 63 us, with the mask 60 -> 67, and some forms kept registers in memory).  Bound by the chain of a chunk, barrier, merge,
+// 512 x 64 77 -> 63 us, with the mask 60 -> 67, and some forms kept registers in memory; of what is kept the forms for D > 224, at most 128 keys, maxima
+// and both keep 2 to 7, 12 to 20 bytes per lane, at 0.61 of the two kernels' time all the same).  Bound by the chain of a chunk, barrier, merge,
 // products, maximum, exponents, sum, on two waves per SIMD: 4700 cycles per chunk of 32 queries against 256 keys of 128, of which 1540 are
 // matrix and 3000 port cycles.  Per call, two kernels -> this one: see few_keys_f32_plan.
 
@@ -5130,7 +5131,8 @@ struct FewKeysPlan {
 // four times the rows between two barriers, win for most numbers of pairs (206 of 900 x 172 x 48 1.15 times their time, 166 of 497 x 164 x 32 1.28).
 // From 1024 on ranges are one to a workgroup, and long calls of short rows that fill neither the chip nor the registers are left out, as few_keys_plan
 // does (`least`: 280 pairs of 5698 x 39 x 32, both, 199 -> 344; 137 of 7618 x 226 x 48 368 -> 479; 316 of 2605 x 14 x 32 93 -> 143).
-// Of what is taken 2 % lose 3 % or more, nearly all rows of D <= 64.  Two chunks (three of at most 128 keys) go to one workgroup, whose launch is
+// Of 30000 shapes that are taken (8 to 256 keys, D of 32 to 256; 0.579 of the time) 1.8 % lose 3 % or more, nearly all of them rows of D < 64 with 100 pairs or more (353 of 462 x 24 x 32, both,
+// 24.3 -> 36.6; D = 64: 527 of 484 x 20 47 -> 59), where fewer pairs gain 10 to 25 %: the path must not follow from the number of pairs.  Two chunks (three of at most 128 keys) go to one workgroup, whose launch is
 // the only one (2 pairs of 64 x 64 x 64 7.3 -> 6.5, but of 128 x 64 x 64 9.1 and 10.6).
 FewKeysPlan few_keys_f32_plan(FewKeysPlan o, int64_t bh, int M, int N, int ks, bool both, int64_t base_floats) {
   if (N > 256) return o;
@@ -5686,6 +5688,7 @@ void fcr_detail::sweeps_bf16_long_rows(int which, const Params& p, int ksteps, b
 
 #if FCR_HAS(0)
 namespace {
+// process-wide switches (fcr_set_option)
 int g_single_sweep = 1;
 long long g_wait_polls = 1ll << 20;
 
@@ -5898,7 +5901,6 @@ size_t fcr_lse_bytes_two_kernels(int B, int H, int M, int N) {
   return rows * sizeof(float) * (splits > 1 ? 1 + (size_t)splits : 1);
 }
 
-// process-wide switches (fcr_set_option)
 }  // namespace
 thread_local bool fcr_detail::fused_refused = false;
 
@@ -6088,8 +6090,8 @@ bool is_capturing(hipStream_t s) {
 // A single sweep expects the whole chip: its workgroups wait for each other, one of eight waves or two of four per CU.  Two of them issued on
 // different streams could be dispatched side by side, each holding CUs the other needs, until their bounded
 // waits run out.  So inside a process they are chained: a single sweep on another stream than the one before
-// first waits (on the GPU; the host blocks only if that stream was destroyed) for an event recorded at the end of that stream.  Calls that
-// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call; on hipStreamPerThread there is one).  Not under stream
+// first waits (on the GPU; the host blocks only if that stream was destroyed or, once, was another thread's hipStreamPerThread) for an event recorded at the end of that stream.  Calls that
+// stay on one stream pay nothing (an event behind every call costs 5 us of a 18 us call; on hipStreamPerThread there is one as soon as others follow there).  Not under stream
 // capture (a graph carries no such edge; graphs holding single sweeps must not replay side by side on one GPU),
 // not for other processes on the same GPU, and not for fcr_colreduce_static, whose calls must not overlap anyway.
 // Where the order cannot be had the call takes the two kernels.
@@ -6098,7 +6100,8 @@ struct SweepOrder {
   hipStream_t last = nullptr;
   uint64_t thread = 0;      // of hipStreamPerThread, one handle for a stream of every thread: whose
   bool any = false;
-  bool recorded = false;    // `done` stands behind the last launch: always so on hipStreamPerThread, where no other thread can record it
+  bool recorded = false;    // `done` stands behind the last launch
+  bool mixed = false;       // other streams follow on hipStreamPerThread, where no other thread can record `done`: each launch there does
 };
 SweepOrder g_order[64];
 std::mutex g_order_mu;
@@ -6116,8 +6119,9 @@ bool wait_for_last(SweepOrder* o, hipStream_t s) {
     hipError_t e = o->thread != 0 ? hipErrorInvalidHandle : hipStreamIsCapturing(o->last, &st);
     if (e == hipSuccess && st != hipStreamCaptureStatusNone) return false;   // (what it was given before the capture may still run)
     if (e == hipSuccess) e = hipEventRecord(o->done, o->last);
-    if (e != hipSuccess) {   // the stream is gone, its work perhaps not: the host waits for the device, whoever captures meanwhile
+    if (e != hipSuccess) {   // the stream is gone or another thread's, its work perhaps still there: the host waits for the device, whoever captures meanwhile
       (void)hipGetLastError();
+      o->mixed = o->mixed || o->thread != 0;
       hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
       if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
       e = hipDeviceSynchronize();
@@ -6132,7 +6136,12 @@ bool wait_for_last(SweepOrder* o, hipStream_t s) {
 // which nothing orders.
 bool order_begin(hipStream_t s, SweepOrder*& o) {
   o = nullptr;
-  if (is_capturing(s)) return true;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (st != hipStreamCaptureStatusNone) return true;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
     (void)hipGetLastError();
@@ -6156,8 +6165,8 @@ void order_end(SweepOrder* o, hipStream_t s, bool launched_it) {
     o->last = s;
     o->thread = s == hipStreamPerThread ? thread_number() : 0;
     o->any = true;
-    o->recorded = o->thread != 0 && hipEventRecord(o->done, s) == hipSuccess;
-    if (o->thread != 0 && !o->recorded) (void)hipGetLastError();
+    o->recorded = o->mixed && o->thread != 0 && hipEventRecord(o->done, s) == hipSuccess;
+    if (!o->recorded) (void)hipGetLastError();
   }
   g_order_mu.unlock();
 }

@@ -259,8 +259,8 @@ int fcr_colreduce_static(const void* q, const void* k, float* out, int dtype, in
  * A single sweep fills the chip, one or two workgroups per CU, and two of them dispatched side by side would
  * starve each other until their waits run out.  Inside a process the library prevents that: a single
  * sweep issued on another stream than the previous one is made to wait on the GPU (an event recorded on
- * that stream, hipStreamWaitEvent on the new one; the host does not block unless that stream was destroyed, calls that stay on one stream
- * pay nothing; on hipStreamPerThread, a stream of every thread, an event is recorded behind each).  Where that cannot be had, for instance
+ * that stream, hipStreamWaitEvent on the new one; calls that stay on one stream pay nothing).  The host waits if that stream was destroyed,
+ * and once if it was another thread's hipStreamPerThread; from then on an event is recorded behind each call there.  Where that cannot be had, for instance
  * while the other stream is being captured, the call takes the two kernels.  Outside its reach: launches recorded under stream capture (graphs that hold single
  * sweeps must not replay side by side on one GPU, nor beside single sweeps issued otherwise), other processes on the same GPU, and
  * fcr_colreduce_static, whose calls must not overlap anyway.  There, switch the single sweep off or
