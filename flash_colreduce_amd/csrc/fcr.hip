@@ -1130,8 +1130,8 @@ __global__ __launch_bounds__(kThreads, ((NB > 2 || KS > 8) ? 1 : 2)) void col_re
 // column sweep waits only for row tiles that a running workgroup has in hand, and those wait for nobody: every wait ends, whatever the order in which
 // workgroups start and whatever else holds CUs meanwhile, be it kernels that wait for each other, and no launch has to be kept apart from another.
 // The bound on a wait (p.spin_limit polls, then the columns become NaN and p.sync[0] is set) is for a host that lowers it.
-// The look costs 0.25 % in the geometric mean of 1600 shapes (a round trip to memory per column tile, beside another workgroup's sweep), all of it,
-// the mark and the loop 1.0 %.  Started in the reverse order, columns first, the launch gives the same bits in 1.2 to 2.3 times the time.  (Tickets
+// Mark and look (a round trip to memory per column tile, beside another workgroup's sweep) cost 0.8 % in the geometric mean of 2900 shapes, up to 1.3 % of calls of
+// several rounds.  The row sweep stands here twice: in one loop for both kinds of places it cost another 0.4 %.  Started in the reverse order, columns first, the launch gives the same bits in 1.2 to 2.3 times the time.  (Tickets
 // for all tiles instead, rows first, cost 4.9 %, up to half of a short call: 64 to 128 atomics on a line before the first load of a
 // workgroup, and workgroups that share a CU no longer get a long tile and a short one.)
 // A captured graph gets the two launches, whose bits it has always had.
@@ -1147,32 +1147,43 @@ __global__ __launch_bounds__(kThreads, 2) void both_sweeps_kernel(const Params p
   constexpr int kCols = col_sweep_bytes<KS, NBC, true>();
   __shared__ __attribute__((aligned(1024))) char smem[kCols > Ring<KS>::kBytes ? kCols : Ring<KS>::kBytes];
   constexpr int kRowTile = kWaves * 16 * wave_group_count(NBR), kColTile = kWaves * 16 * wave_group_count(NBC);
-  const int v = (int)blockIdx.x, rows = (p.total + 7) & ~7, tid = (int)threadIdx.x, lane = tid & 63;
-  const bool own = v < rows;   // a row tile's place
-  int bh, tile, split = 0, row = -1, next = 0, patience = min(p.spin_limit, kPatience);
-  if (own) {
-    if (v >= p.total) return;
-    map_block_split(p, v, CAUSAL, bh, row, split);
-  } else {
-    Params c = p;
-    c.tiles = p.col_tiles;
-    c.group = p.col_group;
-    c.fill = 0;
-    map_block(c, v - rows, false, bh, tile);
-    if (CAUSAL) next = max(0, tile * kColTile - p.c) / kChunk * kChunk / kRowTile;   // the first row tile that it needs
-  }
-  uint32_t* const words = reinterpret_cast<uint32_t*>(p.lse) + (int64_t)bh * p.M;
-  auto mark = [&](int r) {   // whether the tile was not marked before
-    uint32_t none = kNotYet;
-    return __hip_atomic_compare_exchange_strong(words + r * kRowTile, &none, kBegun, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int v = (int)blockIdx.x, rows = (p.total + 7) & ~7, tid = (int)threadIdx.x;
+  auto words_of = [&](int bh) {
+    uint32_t* words = reinterpret_cast<uint32_t*>(p.lse) + (int64_t)bh * p.M;
+    asm volatile("" : "+v"(words));   // (opaque: per-lane arithmetic on it is not to draw that of the sweeps into vector registers)
+    return words;
   };
-  if (own && tid == 0) mark(row);   // (the answer is not waited for)
-  for (;;) {
-    if (row < 0) {   // a row tile of the pair that nobody has begun
-      if (tid < 64) {
-        const int last = (p.M - 1) / kRowTile;
+  auto mark = [&](uint32_t* word) {   // whether the tile was not marked before
+    uint32_t none = kNotYet;
+    return __hip_atomic_compare_exchange_strong(word, &none, kBegun, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (v < rows) {   // a row tile's place
+    if (v >= p.total) return;
+    int bh, tile, split;
+    map_block_split(p, v, CAUSAL, bh, tile, split);
+    int place = tile;
+    asm volatile("" : "+v"(place));   // (as words_of)
+    uint32_t* const words = words_of(bh);
+    if (tid == 0) mark(words + place * kRowTile);   // (the answer is not waited for)
+    row_sweep<DT, KS, CAUSAL, NBR, false, true>(p, smem, tid, bh, tile, split);
+    return;
+  }
+  Params c = p;
+  c.tiles = p.col_tiles;
+  c.group = p.col_group;
+  c.fill = 0;
+  int bh, tile;
+  map_block(c, v - rows, false, bh, tile);
+  {
+    const int last = (p.M - 1) / kRowTile;
+    int next = CAUSAL ? max(0, tile * kColTile - p.c) / kChunk * kChunk / kRowTile : 0;   // the first row tile that it needs
+    asm volatile("" : "+v"(next));
+    int patience = min(p.spin_limit, kPatience);
+    uint32_t* const words = words_of(bh);
+    for (;;) {
+      if (tid < 64) {   // a row tile of the pair that nobody has begun
         while (next <= last) {
-          const uint32_t x = __hip_atomic_load(words + min(next + lane, last) * kRowTile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          const uint32_t x = __hip_atomic_load(words + min(next + tid, last) * kRowTile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           const uint64_t missing = __builtin_amdgcn_ballot_w64(x == kNotYet);
           if (missing == 0) {
             next += 64;
@@ -1182,26 +1193,25 @@ __global__ __launch_bounds__(kThreads, 2) void both_sweeps_kernel(const Params p
           if (patience > 0) {
             --patience;
             __builtin_amdgcn_s_sleep(8);
-          } else if (__builtin_amdgcn_ballot_w64(lane == 0 && mark(next)) != 0) {
+          } else if (__builtin_amdgcn_ballot_w64(tid == 0 && mark(words + next * kRowTile)) != 0) {
             break;
           }
         }
-        if (lane == 0) *reinterpret_cast<int*>(smem) = next <= last ? next : -1;
+        if (tid == 0) *reinterpret_cast<int*>(smem) = next <= last ? next : -1;
       }
       lds_barrier();
-      row = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(smem));
+      const int row = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(smem));
       lds_barrier();
       if (row < 0) break;
+      // (opaque: what the sweep derives from these is not to be kept in registers around the loop, and a split of 0 that the compiler knows
+      // would put its chunk numbers into vector registers)
+      const __attribute__((address_space(4))) Params* at = (const __attribute__((address_space(4))) Params*)__builtin_amdgcn_kernarg_segment_ptr();
+      int thread = tid, split = 0;
+      asm volatile("" : "+s"(at), "+v"(thread), "+s"(split));
+      row_sweep<DT, KS, CAUSAL, NBR, false, true>(*(const Params*)at, smem, thread, bh, row, split);
     }
-    // (opaque: what the sweep derives from these is not to be kept in registers around the loop)
-    const __attribute__((address_space(4))) Params* at = (const __attribute__((address_space(4))) Params*)__builtin_amdgcn_kernarg_segment_ptr();
-    int thread = tid;
-    asm volatile("" : "+s"(at), "+v"(thread));
-    row_sweep<DT, KS, CAUSAL, NBR, false, true>(*(const Params*)at, smem, thread, bh, row, split);
-    if (own) return;
-    row = -1;
   }
-  col_sweep<DT, KS, CAUSAL, MODE, NBC, true>(p, smem, bh, tile);
+  col_sweep<DT, KS, CAUSAL, MODE, NBC, true>(c, smem, bh, tile);
 }
 
 // ---------------------------------------------------------------------------------------------
